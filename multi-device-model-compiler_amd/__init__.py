@@ -7,6 +7,11 @@ GEMM epilogues and the transformer layers).  This module only loads them and
 marshals arguments: device memory and streams come from the caller (PyTorch
 tensors in the tests and the bench), every computation happens inside the HIP
 libraries.  There is no fallback: a missing library or a failing call raises.
+
+The tensor functions go through ``lib/mdmc_torch_calls.so`` (csrc/python/torch_calls.cpp)
+for the ordinary call - contiguous operands of the expected types on the current
+device and stream - and through ctypes, with the checks and messages below, for
+every other.
 """
 from __future__ import annotations
 
@@ -19,6 +24,7 @@ LIB_DIR = os.path.join(_HERE, "lib")
 BIN_DIR = os.path.join(_HERE, "bin")
 RUNTIME_LIB = os.path.join(LIB_DIR, "libmgpu_hip_runtime.so")
 OPS_LIB = os.path.join(LIB_DIR, "libmgpu_hip_ops.so")
+CALLS_LIB = os.path.join(LIB_DIR, "mdmc_torch_calls.so")
 OPS_MODULE = os.path.join(LIB_DIR, "ops.hsaco")
 INCLUDE_DIR = os.path.join(os.path.dirname(_HERE), "include")
 
@@ -36,7 +42,7 @@ def build(force: bool = True, jobs: int = 8) -> None:
 
 
 def is_built() -> bool:
-    return os.path.exists(RUNTIME_LIB) and os.path.exists(OPS_LIB)
+    return all(os.path.exists(p) for p in (RUNTIME_LIB, OPS_LIB, CALLS_LIB))
 
 
 _c_void_p, _c_int32, _c_int64, _c_float, _c_size_t = (
@@ -186,8 +192,30 @@ def _check(lib) -> None:
 
 # --------------------------------------------------------------------------
 # Tensor-level helpers (torch tensors on the GPU; torch only supplies memory
-# and the stream handle).
+# and the stream handle).  Each one asks the native call first; None from it
+# means that the call is not the ordinary one, and the Python code below does it.
 # --------------------------------------------------------------------------
+
+_calls = None
+
+
+def _load_calls():
+    """The native calls; the kernel library they sit on is initialised with them (needs a GPU)."""
+    global _calls
+    ops()
+    if _calls is None:
+        import importlib.machinery
+        import importlib.util
+        import torch  # noqa: F401  (the extension links against its libraries)
+        if not os.path.exists(CALLS_LIB):
+            raise MgpuError(f"{CALLS_LIB} is not built; run `make -C {_HERE}` (or __graft_entry__.build())")
+        loader = importlib.machinery.ExtensionFileLoader("mdmc_torch_calls", CALLS_LIB)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
+        loader.exec_module(module)
+        module.set_error(MgpuError)
+        _calls = module
+    return _calls
+
 
 def _stream_handle(stream=None) -> int:
     import torch
@@ -211,6 +239,10 @@ def _suffix(dtype) -> str:
 
 
 def add(a, b, out=None, stream=None):
+    if stream is None:
+        done = (_calls or _load_calls()).add(a, b, out)
+        if done is not None:
+            return done
     import torch
     assert a.dtype == torch.float32 and b.dtype == torch.float32 and a.shape == b.shape
     if out is None:
@@ -222,6 +254,10 @@ def add(a, b, out=None, stream=None):
 
 
 def layer_norm(x, gamma, beta, eps: float = 1e-5, out=None, stream=None):
+    if stream is None:
+        done = (_calls or _load_calls()).layer_norm(x, gamma, beta, eps, out)
+        if done is not None:
+            return done
     import torch
     n = x.shape[-1]
     m = x.numel() // n if n else 0
@@ -236,6 +272,10 @@ def layer_norm(x, gamma, beta, eps: float = 1e-5, out=None, stream=None):
 
 def cast_layer_norm(x, gamma, beta, eps: float = 1e-5, stream=None):
     """fp32 x -> (fp16 copy of x, LayerNorm of that copy in fp16), one pass."""
+    if stream is None:
+        done = (_calls or _load_calls()).cast_layer_norm(x, gamma, beta, eps)
+        if done is not None:
+            return done
     import torch
     assert x.dtype == torch.float32
     n = x.shape[-1]
@@ -250,6 +290,10 @@ def cast_layer_norm(x, gamma, beta, eps: float = 1e-5, stream=None):
 
 
 def add_residual_layer_norm(x, residual, gamma, beta, eps: float = 1e-5, stream=None):
+    if stream is None:
+        done = (_calls or _load_calls()).add_residual_layer_norm(x, residual, gamma, beta, eps)
+        if done is not None:
+            return done
     import torch
     n = x.shape[-1]
     m = x.numel() // n if n else 0
@@ -265,6 +309,10 @@ def add_residual_layer_norm(x, residual, gamma, beta, eps: float = 1e-5, stream=
 
 def fused_mha(qkv, seqlens=None, scale=None, causal: bool = False, out=None, stream=None):
     """qkv [B,S,3,H,D] fp16/bf16 -> [B,S,H*D]."""
+    if stream is None:
+        done = (_calls or _load_calls()).fused_mha(qkv, seqlens, scale, causal, out)
+        if done is not None:
+            return done
     import torch
     B, S, three, H, D = qkv.shape
     assert three == 3
@@ -284,6 +332,10 @@ def fused_mha(qkv, seqlens=None, scale=None, causal: bool = False, out=None, str
 
 def fused_mha_cu_seqlens(qkv, cu_seqlens, max_s: int, scale=None, causal: bool = False, out=None, stream=None):
     """qkv [total,3,H,D] fp16/bf16 packed back to back, cu_seqlens int32 [B+1] -> [total,H*D]."""
+    if stream is None:
+        done = (_calls or _load_calls()).fused_mha_cu_seqlens(qkv, cu_seqlens, max_s, scale, causal, out)
+        if done is not None:
+            return done
     import torch
     total, three, H, D = qkv.shape
     assert three == 3 and cu_seqlens.dtype == torch.int32
@@ -300,6 +352,10 @@ def fused_mha_cu_seqlens(qkv, cu_seqlens, max_s: int, scale=None, causal: bool =
 
 
 def cast_f32_to_f16(x, stream=None):
+    if stream is None:
+        done = (_calls or _load_calls()).cast_f32_to_f16(x)
+        if done is not None:
+            return done
     import torch
     out = torch.empty(x.shape, dtype=torch.float16, device=x.device)
     lib = ops()
@@ -309,6 +365,10 @@ def cast_f32_to_f16(x, stream=None):
 
 
 def cast_f16_to_f32(x, stream=None):
+    if stream is None:
+        done = (_calls or _load_calls()).cast_f16_to_f32(x)
+        if done is not None:
+            return done
     import torch
     out = torch.empty(x.shape, dtype=torch.float32, device=x.device)
     lib = ops()
@@ -318,6 +378,10 @@ def cast_f16_to_f32(x, stream=None):
 
 
 def cast_f32_to_bf16(x, stream=None):
+    if stream is None:
+        done = (_calls or _load_calls()).cast_f32_to_bf16(x)
+        if done is not None:
+            return done
     import torch
     out = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
     lib = ops()
@@ -327,6 +391,10 @@ def cast_f32_to_bf16(x, stream=None):
 
 
 def cast_bf16_to_f32(x, stream=None):
+    if stream is None:
+        done = (_calls or _load_calls()).cast_bf16_to_f32(x)
+        if done is not None:
+            return done
     import torch
     out = torch.empty(x.shape, dtype=torch.float32, device=x.device)
     lib = ops()
@@ -337,6 +405,10 @@ def cast_bf16_to_f32(x, stream=None):
 
 def qkv_bias_transpose(qkv, bias, stream=None):
     """qkv [B,S,3,H,D] fp16 or bf16 (updated in place with the bias) -> q, k, v [B,H,S,D]."""
+    if stream is None:
+        done = (_calls or _load_calls()).qkv_bias_transpose(qkv, bias)
+        if done is not None:
+            return done
     import torch
     B, S, _, H, D = qkv.shape
     q = torch.empty((B, H, S, D), dtype=qkv.dtype, device=qkv.device)
@@ -368,6 +440,10 @@ def matmul_ex(x, w, bias=None, residual=None, act: int = ACT_NONE, stream=None, 
     """kernel "auto": mgpuMatmulEx*, i.e. the library or the hand-written MFMA kernel as
     the committed table and the fixed rule of the library say; "mfma": the hand-written kernel itself (fp16 / bf16, M a multiple
     of 128, N of 128 or 96, K of 32); "packed": mgpuMatmulExPacked*, w being the [N, K] copy pack_weight made."""
+    if stream is None and kernel in ("auto", "packed"):
+        done = (_calls or _load_calls()).matmul_ex(x, w, bias, residual, act, kernel == "packed")
+        if done is not None:
+            return done
     import torch
     M, K = x.shape
     if kernel == "packed":
@@ -397,6 +473,10 @@ def _conv_out(size, k, pl, pr, s, d=1):
 
 def conv2d(x, w, bias, post_add=None, pad=(0, 0, 0, 0), stride=(1, 1), dilation=(1, 1), relu=False, stream=None):
     """NCHW fp32; pad = (top, left, bottom, right)."""
+    if stream is None:
+        done = (_calls or _load_calls()).conv2d(x, w, bias, post_add, pad, stride, dilation, relu)
+        if done is not None:
+            return done
     import torch
     N, IC, H, W = x.shape
     OC, IC2, KH, KW = w.shape
@@ -414,6 +494,10 @@ def conv2d(x, w, bias, post_add=None, pad=(0, 0, 0, 0), stride=(1, 1), dilation=
 
 def pool2d(x, kernel, pad=(0, 0, 0, 0), stride=(1, 1), method="max", stream=None):
     """NCHW fp32; method "max" or "avg" (average counts the padding)."""
+    if stream is None:
+        done = (_calls or _load_calls()).pool2d(x, kernel, pad, stride, method != "max")
+        if done is not None:
+            return done
     import torch
     N, C, H, W = x.shape
     OH = _conv_out(H, kernel[0], pad[0], pad[2], stride[0])
@@ -428,6 +512,11 @@ def pool2d(x, kernel, pad=(0, 0, 0, 0), stride=(1, 1), method="max", stream=None
 
 def decoding_context_layer(x, wqkv, wo, bo, w1, b1, w2, b2, heads: int, causal: bool = True,
                            relu: bool = True, norm_first: bool = True, stream=None):
+    if stream is None:
+        done = (_calls or _load_calls()).decoding_context_layer(
+            x, wqkv, wo, bo, w1, b1, w2, b2, heads, causal, relu, norm_first)
+        if done is not None:
+            return done
     import torch
     B, S, d = x.shape
     ffn = w1.shape[1]
@@ -444,6 +533,11 @@ def bert_encoder_layer(x, wqkv, bqkv, wo, bo, g1, be1, w1, b1, w2, b2, g2, be2, 
                        seqlens=None, eps: float = 1e-5, out=None, stream=None, no_alloc: bool = False):
     """no_alloc: the entry point whose temporaries live in the library's fixed
     device array (the caller supplies ``out``: nothing is allocated then)."""
+    if stream is None:
+        done = (_calls or _load_calls()).bert_encoder_layer(
+            x, wqkv, bqkv, wo, bo, g1, be1, w1, b1, w2, b2, g2, be2, heads, seqlens, eps, out, no_alloc)
+        if done is not None:
+            return done
     import torch
     B, S, d = x.shape
     ffn = w1.shape[1]
