@@ -9,22 +9,27 @@
 // The convolution is an implicit GEMM on the fp32 matrix cores
 // (v_mfma_f32_32x32x2_f32: true fp32 products, fp32 accumulation):
 //   y[n][oc, p] = sum_k w[oc, k] * taps[k, p],  k = (ic, kh, kw), p = (oh, ow)
-// A 256-thread block owns 64 output channels x 128 (or 64) output pixels of one
-// image; its 4 wavefronts sit 2 x 2 over that tile, 32 channels x 64 (32)
-// pixels each.  The tap matrix is never written to memory: per chunk of 32
-// taps the block gathers its [32, pixels] slice from the image into LDS (zero
-// for padding and for taps past the end; a thread keeps one pixel and walks
-// a run of consecutive taps, so global reads run along image rows and the
-// (ic, kh, kw) decomposition costs one division per chunk) next to the
-// [64, 32] filter slice - both through registers, fetched one chunk ahead of
-// the MFMAs that use them - and every lane feeds the MFMAs with one filter
-// value and one tap value per instruction.  The accumulator layout puts 32 consecutive pixels of
-// one channel in the 32 lanes of a register, so the epilogue (bias, postAdd,
-// ReLU) writes whole 128-byte runs of the NCHW output: one pass over the
-// output, none over an intermediate.  Unlike the reference, asymmetric padding
-// is honoured (it passes only PHL / PWL to cuDNN).
+// in 32 x 32 tiles, channels in the rows and pixels - counted over the whole batch - in the
+// columns, so that a register of an accumulator is 32 consecutive pixels of a channel: whole
+// 128-byte runs of the NCHW output.  The tap matrix is never written to memory.  Taps come
+// through buffer loads, whose bounds check answers 0 for an offset outside the image: padding costs
+// no branch and no second instruction.  Four kernels share the work (conv2d below has the rule and
+// the measurements behind it):
+//   few taps  (K <= 32, a network's stem)  filter in registers, wavefronts walk over pixel tiles
+//   window    (1, 3, 5 or 7 square, few tiles)  operands straight from L1 / L2 into registers,
+//             four wavefronts per tile
+//   tile      (the same windows, many tiles)    operands shared through LDS by 64 x 64 tiles
+//   table     (every other window, and images beyond 2 GiB)  tap offsets from a table in LDS
+// What bounds them: one 32x32x2 MFMA takes 64 cycles of a SIMD (157 TFLOP/s on the chip) and the
+// vector instructions of the same wavefront do not overlap with it, so the loops are built to have
+// none; the stem is bound by its output (268 MB at 16 x 3 x 256 x 256 -> 64: 116 -> 70 us, a plain fill
+// of as many bytes takes 39).  Unlike the reference, asymmetric padding is honoured (it passes only
+// PHL / PWL to cuDNN).
 #include "common.hpp"
 #include "mgpu_ops_internal.hpp"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace mgpu {
 
@@ -35,154 +40,736 @@ struct ConvGeo {
 };
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kConvOC = 64; // output channels per block
+constexpr int kChunk = 16;     // taps per step of the reduction: 8 a lane half
+constexpr int kSegment = 2048; // taps the tap table holds at a time
+constexpr int kOutside = (int)0x80000000; // a byte offset past every resource: the hardware's bounds check reads 0 there
+constexpr int kNever = 0x3fff0000; // added to a row index it puts the tap outside every image
 
-template <int TP, int KC> // output pixels per block (128 or 64), taps staged per step
-__global__ __launch_bounds__(256) void conv_mfma_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                                        const float *__restrict__ bias, const float *__restrict__ add,
-                                                        float *__restrict__ y, ConvGeo g, int OC, int K, int P,
-                                                        int pTiles, bool relu) {
-  constexpr int PJ = TP / 64; // 32-pixel accumulators per wavefront
-  // +1: the 32 lanes of a filter read sit 33 words apart, one bank each
-  __shared__ float filt[kConvOC][KC + 1];
-  __shared__ float taps[KC][TP];
+// Where tap k of a pixel sits: the offset from the pixel's first tap (bytes; elements when WIDE)
+// and the window position (kw | kh << 5) or, for WIDE (images beyond 2 GiB, windows beyond 31
+// positions), the row and column distances.
+struct TapNarrow {
+  int off, pos;
+};
+struct TapWide {
+  int off, dh, dw, pad;
+};
 
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const int l32 = lane % 32, hl = lane / 32;
-  const int wm = wave / 2, wp = wave % 2;
-  const int n = blockIdx.x / pTiles;
-  const int p0 = (blockIdx.x % pTiles) * TP;
-  const int oc0 = blockIdx.y * kConvOC;
-  // block-uniform bases; everything a lane adds to them fits 32 bits (checked by the caller)
-  const float *image = x + (int64_t)n * g.IC * g.H * g.W;
-  const float *wtile = w + (int64_t)oc0 * K;
+// Division by a number that the host knows, for dividends below 2^31: (mulhi(n, mul) + n) >> shift.
+struct FastDiv {
+  unsigned mul, shift;
+};
+__device__ __forceinline__ int divide(int n, FastDiv d) {
+  return (int)((__umulhi((unsigned)n, d.mul) + (unsigned)n) >> d.shift);
+}
 
-  // this thread's pixel for the gathers (fixed: 256 is a multiple of TP)
-  const int gp = p0 + tid % TP;
-  const bool gpValid = gp < P;
-  const int goh = gpValid ? gp / g.OW : 0, gow = gpValid ? gp % g.OW : 0;
-  // a pixel past the end gets a first row above the image for every tap: it gathers zeros
-  const int ih0 = gpValid ? goh * g.SH - g.PHL : -g.KH * g.DH - 1, iw0 = gow * g.SW - g.PWL;
+// Which of `count` window rows (columns), `dilation` apart from `first` on, lie outside 0 .. size - 1: bit i for the i-th.
+__device__ __forceinline__ unsigned outsideBits(int first, int size, int count, int dilation) {
+  if (dilation == 1) { // (uniform) the bits below -first and from size - first on
+    const int lo = first < 0 ? -first : 0, hi = size - first;
+    const unsigned below = lo > 31 ? ~0u : (1u << lo) - 1u, above = hi > 31 ? 0u : hi < 0 ? ~0u : ~0u << hi;
+    return below | above;
+  }
+  unsigned bits = 0;
+  for (int i = 0; i < count; i++) bits |= (unsigned)(first + i * dilation) < (unsigned)size ? 0u : 1u << i;
+  return bits;
+}
 
-  f32x16 acc[PJ];
+// A buffer resource over `elems` floats (2 GiB of them at most: no offset reaches further), for the
+// builtins and, as its four words, for inline assembly.
+constexpr int kRawBuffer = 0x00027000;
+__device__ __forceinline__ int resourceBytes(int64_t elems) { return (int)(elems * 4 < 0x7fffffff ? elems * 4 : 0x7fffffff); }
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t resource(const float *p, int64_t elems) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, resourceBytes(elems), kRawBuffer);
+}
+__device__ __forceinline__ i32x4 resourceWords(const float *p, int64_t elems) {
+  const uint64_t at = (uint64_t)(uintptr_t)p;
+  return i32x4{(int)(uint32_t)at, (int)(uint32_t)(at >> 32) & 0xffff, resourceBytes(elems), kRawBuffer};
+}
+
+// The end of a wavefront's 32 channels x PT x 32 pixels: the sum over the KS wavefronts of the tile
+// (wavefront ks of them has slot `slot0` + ks of `partial`), bias, postAdd, ReLU, store.  pix and img:
+// the lane's pixels (-1: past the end) and their images less nFirst.  Lane: the type of a lane's byte
+// offset from image nFirst.
+template <int PT, int KS, typename Lane, int SLOTS, int WORDS>
+__device__ __forceinline__ void finishTile(f32x16 (&acc)[PT], float (&partial)[SLOTS][WORDS], int slot0, int ks, const float *bias,
+                                           const float *add, float *y, int OC, int P, int oc0, int nFirst, const int (&img)[PT],
+                                           const int (&pix)[PT], int lane, int relu) {
+  const int hl = lane / 32;
+  // accumulator register r of lane l: channel 8*(r/4) + 4*(l/32) + r%4, pixel l%32.  (Offsets are
+  // bytes next to a uniform base: a store takes its address from a scalar pair and one vector register.)
+  const int64_t first = ((int64_t)nFirst * OC + oc0) * P;
+  Lane at[PT];
 #pragma unroll
-  for (int j = 0; j < PJ; j++)
+  for (int j = 0; j < PT; j++) at[j] = (((Lane)img[j] * OC + 4 * hl) * P + (Lane)pix[j]) * 4;
+  constexpr int SHARE = 16 / KS; // registers this wavefront finishes
+  if constexpr (KS > 1) {
+    static_assert(PT == 1, "one accumulator per wavefront where the taps are split");
 #pragma unroll
-    for (int i = 0; i < 16; i++) acc[j][i] = 0.0f;
-
-  // Each chunk is fetched into registers one step ahead of its use, so the
-  // global loads of chunk c+1 are in flight while the MFMAs of chunk c run.
-  constexpr int FR = kConvOC * KC / 256; // filter values per thread and chunk
-  constexpr int TR = KC * TP / 256;      // consecutive taps per thread and chunk
-  const int tk0 = (tid / TP) * TR;            // first tap of this thread inside a chunk
-  float fv[FR], tv[TR];
-  auto fetch = [&](int k0) {
+    for (int r = 0; r < 16; r++) partial[slot0 + ks][r * 64 + lane] = acc[0][r];
+    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < FR; i++) { // consecutive threads along k
-      const int e = tid + 256 * i;
-      const int ocl = e / KC, kl = e % KC;
-      // Unconditional loads from a clamped address, the value selected afterwards:
-      // a load under a branch would have to land before the next one is issued.
-      const bool live = oc0 + ocl < OC && k0 + kl < K;
-      const float val = wtile[live ? (uint32_t)(ocl * K + k0 + kl) : 0u];
-      fv[i] = live ? val : 0.0f;
+    for (int i = 0; i < SHARE; i++) {
+      float v = 0.0f;
+#pragma unroll
+      for (int s = 0; s < KS; s++) v += partial[slot0 + s][(ks * SHARE + i) * 64 + lane];
+      acc[0][i] = v;
     }
-    // One division per chunk; from there the tap index walks like an odometer
-    // and the image offset follows it with additions only.
-    int k = k0 + tk0;
-    int kw = k % g.KW, kh = (k / g.KW) % g.KH;
-    int ih = ih0 + kh * g.DH, iw = iw0 + kw * g.DW;
-    int off = ((k / (g.KW * g.KH)) * g.H + ih) * g.W + iw;
+  }
+  const bool fullOc = oc0 + 32 <= OC; // (uniform: no channel test inside a full tile)
+  auto channel = [&](int i) { // of register i of the wavefront's share, less the lane's 4 hl
+    const int r = ks * SHARE + i;
+    return 8 * (r / 4) + r % 4;
+  };
+  float bv[SHARE];
 #pragma unroll
-    for (int i = 0; i < TR; i++) {
-      const bool inside = (unsigned)ih < (unsigned)g.H && (unsigned)iw < (unsigned)g.W && k < K;
-      const float val = image[inside ? (uint32_t)off : 0u];
-      tv[i] = inside ? val : 0.0f;
-      k++;
-      iw += g.DW;
-      off += g.DW;
-      if (++kw == g.KW) {
-        kw = 0;
-        iw = iw0;
-        ih += g.DH;
-        off += g.DH * g.W - g.KW * g.DW;
-        if (++kh == g.KH) {
-          kh = 0;
-          ih = ih0;
-          off += (g.H - g.KH * g.DH) * g.W;
-        }
+  for (int i = 0; i < SHARE; i++) {
+    const int oc = oc0 + channel(i) + 4 * hl;
+    bv[i] = bias[fullOc || oc < OC ? oc : OC - 1];
+  }
+  auto epilogue = [&](auto everyChannel, auto plain) {
+#pragma unroll
+    for (int j = 0; j < PT; j++) {
+      if (pix[j] < 0) continue;
+#pragma unroll
+      for (int i = 0; i < SHARE; i++) {
+        const int ocl = channel(i);
+        if (!decltype(everyChannel)::value && oc0 + ocl + 4 * hl >= OC) continue;
+        const int64_t row = first + (int64_t)ocl * P;
+        float v = acc[j][i] + bv[i];
+        if (!decltype(plain)::value) v += *reinterpret_cast<const float *>(reinterpret_cast<const char *>(add + row) + at[j]);
+        // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
+        *reinterpret_cast<float *>(reinterpret_cast<char *>(y + row) + at[j]) = relu ? fmaxf(v, 0.0f) : v;
       }
     }
   };
+  if (!add && fullOc) epilogue(std::true_type(), std::true_type());
+  else if (!add) epilogue(std::false_type(), std::true_type());
+  else if (fullOc) epilogue(std::true_type(), std::false_type());
+  else epilogue(std::false_type(), std::false_type());
+}
 
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += KC) {
-    __syncthreads(); // everybody is done with the previous chunk
+// ---- any window -----------------------------------------------------------------------------
+// The four wavefronts of a block share one 32 x 32 tile and split the taps.
+template <bool WIDE>
+__global__ __launch_bounds__(256, 2) void conv_table_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                            const float *__restrict__ bias, const float *__restrict__ add,
+                                                            float *__restrict__ y, ConvGeo g, int OC, int K, int P, int64_t pixelsArg,
+                                                            int relu) {
+  using Tap = typename std::conditional<WIDE, TapWide, TapNarrow>::type;
+  using Index = typename std::conditional<WIDE, int64_t, int>::type; // (64-bit divisions are long sequences)
+  const Index pixels = (Index)pixelsArg;
+  constexpr int KS = 4;
+  __shared__ __attribute__((aligned(16))) Tap table[kSegment];
+  __shared__ float partial[KS][16 * 64];
+
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int ks = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int l32 = lane % 32, hl = lane / 32;
+  const int oc0 = blockIdx.y * 32;
+  const Index q0 = (Index)blockIdx.x * 32; // (the grid has no block past the last pixel)
+  const int64_t imageElems = (int64_t)g.IC * g.H * g.W;
+
+  // The lane's pixel.  Which window rows and columns fall outside the image is a bit mask (bit 31
+  // always set: the position of a tap past the end); a pixel past the end has every bit set.
+  const int nFirst = __builtin_amdgcn_readfirstlane((int)(q0 / P));
+  const Index q = q0 + l32;
+  const bool live = q < pixels;
+  const int n = live ? (int)(q / P) : nFirst;
+  const int p = live ? (int)(q - (Index)n * P) : 0;
+  const int oh = p / g.OW, ow = p - oh * g.OW;
+  const int img[1] = {n - nFirst}, pix[1] = {live ? p : -1};
+  const int ih0 = live ? oh * g.SH - g.PHL : -kNever, iw0 = ow * g.SW - g.PWL;
+  Index base = (Index)img[0] * (Index)imageElems + (Index)(oh * g.SH - g.PHL) * g.W + iw0;
+  const float *image = x + nFirst * imageElems;
+  unsigned rowOut = 0, colOut = 0;
+  if constexpr (!WIDE) {
+    rowOut = live ? outsideBits(ih0, g.H, g.KH, g.DH) : ~0u;
+    colOut = outsideBits(iw0, g.W, g.KW, g.DW) | 0x80000000u;
+    base *= 4; // bytes from `image`, in the 32 bits that the host has checked they fit
+  }
+  const auto rsrc = resource(image, ((pixels - 1) / P + 1 - nFirst) * imageElems);
+  const float *wrow = w + (int64_t)(oc0 + l32 < OC ? oc0 + l32 : OC - 1) * K; // (a channel past the end is not stored)
+
+  f32x16 acc[1];
 #pragma unroll
-    for (int i = 0; i < FR; i++) {
-      const int e = tid + 256 * i;
-      filt[e / KC][e % KC] = fv[i];
-    }
+  for (int i = 0; i < 16; i++) acc[0][i] = 0.0f;
+
+  // One step's operands: the contraction does not care in which slot a tap sits, so lane half hl
+  // takes taps 8 hl .. 8 hl + 7 of the chunk (two 16-byte filter loads) and MFMA i of the step
+  // multiplies tap i of either half.
+  struct Operands {
+    float a[8], b[8];
+  };
+  auto fetch = [&](Operands &o, int seg, int k) { // taps k .. k + 15, k relative to the segment
+    const int kl = k + 8 * hl;
+    if (seg + k + kChunk <= K) { // (uniform)
+      const f32x4 lo = *reinterpret_cast<const f32x4 __attribute__((aligned(4))) *>(wrow + seg + kl);
+      const f32x4 hi = *reinterpret_cast<const f32x4 __attribute__((aligned(4))) *>(wrow + seg + kl + 4);
 #pragma unroll
-    for (int i = 0; i < TR; i++) taps[tk0 + i][tid % TP] = tv[i];
-    __syncthreads();
-    if (k0 + KC < K) fetch(k0 + KC);
-#pragma unroll
-    for (int kk = 0; kk < KC; kk += 2) {
-      const float a = filt[32 * wm + l32][kk + hl];
-#pragma unroll
-      for (int j = 0; j < PJ; j++) {
-        const float b = taps[kk + hl][wp * (TP / 2) + 32 * j + l32];
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[j], 0, 0, 0);
+      for (int i = 0; i < 4; i++) {
+        o.a[i] = lo[i];
+        o.a[4 + i] = hi[i];
       }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const bool in = seg + kl + i < K;
+        const float v = wrow[in ? seg + kl + i : 0];
+        o.a[i] = in ? v : 0.0f;
+      }
+    }
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const Tap tap = table[kl + i];
+        const bool in = (unsigned)(ih0 + tap.dh) < (unsigned)g.H && (unsigned)(iw0 + tap.dw) < (unsigned)g.W;
+        const float v = image[in ? base + tap.off : 0];
+        o.b[i] = in ? v : 0.0f;
+      }
+    } else {
+      i32x4 e[4]; // two taps each
+#pragma unroll
+      for (int i = 0; i < 4; i++) e[i] = reinterpret_cast<const i32x4 *>(&table[kl])[i];
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int off = e[i / 2][2 * (i % 2)], pos = e[i / 2][2 * (i % 2) + 1];
+        // all ones where the row or the column is outside: two bit-field extracts, an add and an or
+        const int out = __builtin_amdgcn_sbfe(rowOut, pos >> 5, 1) | __builtin_amdgcn_sbfe(colOut, pos, 1);
+        o.b[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, ((int)base + off) | out, 0, 0));
+      }
+    }
+  };
+  auto multiply = [&](const Operands &o) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(o.a[i], o.b[i], acc[0], 0, 0, 0);
+  };
+
+  for (int seg = 0; seg < K; seg += kSegment) {
+    const int taps = K - seg < kSegment ? K - seg : kSegment;
+    const int padded = (taps + kChunk - 1) / kChunk * kChunk;
+    if (seg) __syncthreads(); // everybody is done with the previous segment's table
+    for (int e = tid; e < padded; e += 256) {
+      const int k = seg + e;
+      const int ic = k / (g.KW * g.KH), r = k - ic * (g.KW * g.KH);
+      const int kh = r / g.KW, kw = r - kh * g.KW;
+      Tap tap;
+      tap.off = (ic * g.H + kh * g.DH) * g.W + kw * g.DW;
+      if constexpr (WIDE) {
+        tap.dh = k < K ? kh * g.DH : kNever;
+        tap.dw = kw * g.DW;
+        tap.pad = 0;
+      } else {
+        tap.off = k < K ? tap.off * 4 : 0;
+        tap.pos = k < K ? kw | kh << 5 : 31;
+      }
+      table[e] = tap;
+    }
+    __syncthreads();
+
+    const int chunks = padded / kChunk;
+    const int c0 = chunks * ks / KS, c1 = chunks * (ks + 1) / KS; // this wavefront's share
+    // each chunk's loads fly under the MFMAs of the one before
+    Operands even, odd;
+    if (c0 < c1) fetch(even, seg, c0 * kChunk);
+    for (int c = c0; c < c1; c += 2) {
+      if (c + 1 < c1) fetch(odd, seg, (c + 1) * kChunk);
+      multiply(even);
+      if (c + 1 >= c1) break;
+      if (c + 2 < c1) fetch(even, seg, (c + 2) * kChunk);
+      multiply(odd);
     }
   }
 
-  // accumulator register r of lane l: channel 8*(r/4) + 4*(l/32) + r%4, pixel l%32
-  const int ocl0 = 32 * wm + 4 * hl;        // channel of register 0 inside the tile
-  const bool fullOc = oc0 + kConvOC <= OC; // uniform: no channel test inside a full tile
-  const int64_t tileBase = ((int64_t)n * OC + oc0) * P + p0;
-  float *ytile = y + tileBase;
-  const float *atile = add ? add + tileBase : nullptr;
-  const float *btile = bias + oc0;
+  using Lane = typename std::conditional<WIDE, int64_t, uint32_t>::type;
+  finishTile<1, KS, Lane>(acc, partial, 0, ks, bias, add, y, OC, P, oc0, nFirst, img, pix, lane, relu);
+}
+
+// ---- square windows of 1, 3, 5 or 7 --------------------------------------------------------
+// No tap table: the reduction walks input channels in groups - pairs, one channel per lane half;
+// 1 x 1: sixteen, eight per half - and inside a group the window positions, with a register each for
+// the position's byte offset.  The channel enters through the scalar offset of the load, so a tap
+// costs no vector instruction (the table's five a tap were 40 % of a 32 x 32 tile's loop).
+template <int WIN> struct Window {
+  static constexpr int KK = WIN * WIN;
+  static constexpr int UNITS = WIN <= 3 ? 1 : WIN;        // fetched at a time: the window, or one of its rows
+  static constexpr int STEPS = WIN == 1 ? 8 : KK / UNITS; // MFMA steps per unit
+  static constexpr int HALF = WIN == 1 ? 8 : 1;           // channels per lane half and group
+};
+
+// A wavefront's tile is 32 channels x PT x 32 pixels; KS of a block's four wavefronts share a tile
+// and split the channel groups.
+template <int WIN, int PT, int KS>
+__global__ __launch_bounds__(256, 2) void conv_window_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                             const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
+                                                             int P, int N, FastDiv byP, FastDiv byOW, const float *__restrict__ add,
+                                                             int relu) {
+  using Win = Window<WIN>;
+  constexpr int KK = Win::KK, UNITS = Win::UNITS, STEPS = Win::STEPS, HALF = Win::HALF;
+  constexpr int TILES = 4 / KS;
+  __shared__ float partial[KS > 1 ? 4 : 1][KS > 1 ? 16 * 64 : 1];
+
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int l32 = lane % 32, hl = lane / 32;
+  const int ks = wave % KS, tile = wave / KS;
+  const int oc0 = blockIdx.y * 32;
+  const int q0 = ((int)blockIdx.x * TILES + tile) * (32 * PT);
+  const int HW4 = g.H * g.W * 4, pixels = N * P;
+
+  const int nFirst = __builtin_amdgcn_readfirstlane(divide(q0 < pixels ? q0 : pixels - 1, byP));
+  int pix[PT], img[PT], voff[PT][KK];
 #pragma unroll
-  for (int j = 0; j < PJ; j++) {
-    const int pl = wp * (TP / 2) + 32 * j + l32;
-    if (p0 + pl >= P) continue;
+  for (int j = 0; j < PT; j++) {
+    const int q = q0 + 32 * j + l32;
+    const bool live = q < pixels;
+    const int n = live ? divide(q, byP) : nFirst;
+    const int p = live ? q - n * P : 0;
+    const int oh = divide(p, byOW), ow = p - oh * g.OW;
+    img[j] = n - nFirst;
+    pix[j] = live ? p : -1;
+    const int ih0 = live ? oh * g.SH - g.PHL : -kNever, iw0 = ow * g.SW - g.PWL;
+    const int base = (img[j] * g.IC + hl * HALF) * HW4 + ((oh * g.SH - g.PHL) * g.W + iw0) * 4;
+#pragma unroll
+    for (int kh = 0; kh < WIN; kh++)
+#pragma unroll
+      for (int kw = 0; kw < WIN; kw++) {
+        const bool in = (unsigned)(ih0 + kh * g.DH) < (unsigned)g.H && (unsigned)(iw0 + kw * g.DW) < (unsigned)g.W;
+        voff[j][kh * WIN + kw] = in ? base + (kh * g.DH * g.W + kw * g.DW) * 4 : kOutside;
+      }
+  }
+  const int64_t imageElems = (int64_t)g.IC * g.H * g.W;
+  const auto image = resource(x + nFirst * imageElems, (N - nFirst) * imageElems);
+  const auto filter = resource(w + (int64_t)oc0 * g.IC * KK, (int64_t)(OC - oc0) * g.IC * KK);
+  // (a channel past the end reads the last one's filter and is not stored)
+  const int woff = ((oc0 + l32 < OC ? l32 : OC - 1 - oc0) * g.IC + hl * HALF) * (KK * 4);
+
+  f32x16 acc[PT];
+#pragma unroll
+  for (int j = 0; j < PT; j++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[j][i] = 0.0f;
+
+  struct Operands {
+    float a[STEPS], b[PT][STEPS];
+  };
+  auto loadF = [](const __amdgpu_buffer_rsrc_t &r, int voffset, int soffset) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voffset, soffset, 0));
+  };
+  auto fetch = [&](Operands &o, int group, auto unitConst) { // a group all of whose channels exist
+    constexpr int unit = decltype(unitConst)::value;
+    constexpr int AT = unit * STEPS * 4;
+    const int wbase = group * (2 * HALF * KK * 4);
+#pragma unroll
+    for (int i = 0; i + 4 <= STEPS; i += 4) {
+      const auto v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(filter, woff + AT + i * 4, wbase, 0));
+#pragma unroll
+      for (int e = 0; e < 4; e++) o.a[i + e] = v[e];
+    }
+#pragma unroll
+    for (int i = STEPS / 4 * 4; i < STEPS; i++) o.a[i] = loadF(filter, woff + AT + i * 4, wbase);
+#pragma unroll
+    for (int i = 0; i < STEPS; i++)
+#pragma unroll
+      for (int j = 0; j < PT; j++)
+        o.b[j][i] = loadF(image, voff[j][WIN == 1 ? 0 : unit * STEPS + i], (group * (2 * HALF) + (WIN == 1 ? i : 0)) * HW4);
+  };
+  auto multiply = [&](const Operands &o) {
+#pragma unroll
+    for (int i = 0; i < STEPS; i++)
+#pragma unroll
+      for (int j = 0; j < PT; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(o.a[i], o.b[j][i], acc[j], 0, 0, 0);
+  };
+
+  const int groups = g.IC / (2 * HALF);
+  const int g0 = groups * ks / KS, g1 = groups * (ks + 1) / KS; // this wavefront's share
+  // Two buffers; a unit's loads fly under the MFMAs of the one before.  With an odd number of units
+  // a group ends on the other buffer than it began: the loop body is two groups.
+  Operands buf[2];
+  if (g0 < g1) fetch(buf[0], g0, std::integral_constant<int, 0>());
+  auto oneGroup = [&](int group, auto phaseConst) {
+    constexpr int phase = decltype(phaseConst)::value;
+    auto step = [&](auto self, auto unitConst) {
+      constexpr int unit = decltype(unitConst)::value;
+      if constexpr (unit < UNITS) {
+        if constexpr (unit + 1 < UNITS) fetch(buf[(phase + unit + 1) % 2], group, std::integral_constant<int, unit + 1>());
+        else if (group + 1 < g1) fetch(buf[(phase + unit + 1) % 2], group + 1, std::integral_constant<int, 0>());
+        multiply(buf[(phase + unit) % 2]);
+        self(self, std::integral_constant<int, unit + 1>());
+      }
+    };
+    step(step, std::integral_constant<int, 0>());
+  };
+  for (int group = g0; group < g1; group += 2) {
+    oneGroup(group, std::integral_constant<int, 0>());
+    if (group + 1 < g1) oneGroup(group + 1, std::integral_constant<int, UNITS % 2>());
+  }
+  // The channels beyond the last whole group: what lies past the last channel is asked for at an
+  // offset outside the resource (and reads as 0), operand by operand.
+  const int rest = g.IC - groups * (2 * HALF);
+  if (rest && ks == KS - 1) {
+    auto tail = [&](auto self, auto unitConst) {
+      constexpr int unit = decltype(unitConst)::value;
+      if constexpr (unit < UNITS) {
+        const int wbase = groups * (2 * HALF * KK * 4);
+#pragma unroll
+        for (int i = 0; i < STEPS; i++) {
+          const int c = WIN == 1 ? i : 0; // channel of the step inside the lane half's
+          const bool in = hl * HALF + c < rest;
+          buf[0].a[i] = loadF(filter, in ? woff + (unit * STEPS + i) * 4 + wbase : kOutside, 0);
+#pragma unroll
+          for (int j = 0; j < PT; j++) {
+            const int at = voff[j][WIN == 1 ? 0 : unit * STEPS + i];
+            buf[0].b[j][i] = loadF(image, in && at != kOutside ? at + (groups * (2 * HALF) + c) * HW4 : kOutside, 0);
+          }
+        }
+        multiply(buf[0]);
+        self(self, std::integral_constant<int, unit + 1>());
+      }
+    };
+    tail(tail, std::integral_constant<int, 0>());
+  }
+  finishTile<PT, KS, uint32_t>(acc, partial, tile * KS, ks, bias, add, y, OC, P, oc0, nFirst, img, pix, lane, relu);
+}
+
+// ---- few taps -----------------------------------------------------------------------------
+// A reduction of at most 2 NS taps (a network's stem: 3 channels, 3 x 3).  A wavefront keeps the
+// filter of its OCT x 32 channels in registers, lane half hl the taps 2 s + hl of step s, and walks
+// over tiles of 32 pixels; the taps of the next tile are in flight while this one's are multiplied
+// and stored.
+template <int OCT, int NS>
+__global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                               const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
+                                                               int P, int N, FastDiv byP, FastDiv byOW, const float *__restrict__ add,
+                                                               int relu, int K, int tiles, int tileStep) {
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int l32 = lane % 32, hl = lane / 32;
+  const int oc0 = blockIdx.y * (32 * OCT);
+  const int pixels = N * P;
+
+  // Filter values, and where the lane half's tap of each step sits: its byte offset from the pixel's
+  // first tap and its window position (kw | kh << 5; 31 past the end, a column that is always outside).
+  float a[OCT][NS];
+  int toff[NS], tpos[NS];
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    const int k = 2 * s + hl;
+    const int ic = k / (g.KW * g.KH), r = k - ic * (g.KW * g.KH);
+    const int kh = r / g.KW, kw = r - kh * g.KW;
+    const bool in = k < K;
+    toff[s] = in ? ((ic * g.H + kh * g.DH) * g.W + kw * g.DW) * 4 : 0;
+    tpos[s] = in ? kw | kh << 5 : 31;
+#pragma unroll
+    for (int t = 0; t < OCT; t++) {
+      const int oc = oc0 + 32 * t + l32 < OC ? oc0 + 32 * t + l32 : OC - 1;
+      const float v = w[(int64_t)oc * K + (in ? k : 0)];
+      a[t][s] = in ? v : 0.0f;
+    }
+  }
+
+  struct Tile {
+    int pix, img, nFirst; // the lane's pixel (-1: past the end), its image less the tile's first, that image
+    float b[NS];
+  };
+  const int64_t imageElems = (int64_t)g.IC * g.H * g.W;
+  auto fetch = [&](Tile &o, int tile) {
+    const int q0 = tile * 32, q = q0 + l32;
+    const bool live = q < pixels;
+    o.nFirst = __builtin_amdgcn_readfirstlane(divide(q0, byP));
+    const int n = live ? divide(q, byP) : o.nFirst;
+    const int p = live ? q - n * P : 0;
+    const int oh = divide(p, byOW), ow = p - oh * g.OW;
+    o.img = n - o.nFirst;
+    o.pix = live ? p : -1;
+    const int ih0 = oh * g.SH - g.PHL, iw0 = ow * g.SW - g.PWL;
+    const unsigned rowOut = live ? outsideBits(ih0, g.H, g.KH, g.DH) : ~0u;
+    const unsigned colOut = outsideBits(iw0, g.W, g.KW, g.DW) | 0x80000000u;
+    const int base = (o.img * (int)imageElems + ih0 * g.W + iw0) * 4;
+    const auto rsrc = resource(x + o.nFirst * imageElems, (N - o.nFirst) * imageElems);
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      const int out = __builtin_amdgcn_sbfe(rowOut, tpos[s] >> 5, 1) | __builtin_amdgcn_sbfe(colOut, tpos[s], 1);
+      o.b[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (base + toff[s]) | out, 0, 0));
+    }
+  };
+  float bv[OCT][16]; // the accumulators start from the bias
+#pragma unroll
+  for (int t = 0; t < OCT; t++)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-      constexpr int kRow[16] = {0, 1, 2, 3, 8, 9, 10, 11, 16, 17, 18, 19, 24, 25, 26, 27};
-      const int ocl = ocl0 + kRow[r];
-      if (!fullOc && oc0 + ocl >= OC) continue;
-      const uint32_t off = (uint32_t)ocl * (uint32_t)P + (uint32_t)pl;
-      float v = acc[j][r] + btile[ocl];
-      if (atile) v += atile[off];
-      // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
-      ytile[off] = relu ? fmaxf(v, 0.0f) : v;
+      const int oc = oc0 + 32 * t + 8 * (r / 4) + r % 4 + 4 * hl;
+      bv[t][r] = bias[oc < OC ? oc : OC - 1];
     }
+  const bool fullOc = oc0 + 32 * OCT <= OC;
+  const int64_t outElems = (int64_t)OC * P;
+  auto finish = [&](Tile &o) {
+    f32x16 acc[OCT];
+#pragma unroll
+    for (int t = 0; t < OCT; t++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[t][i] = bv[t][i];
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+#pragma unroll
+      for (int t = 0; t < OCT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t][s], o.b[s], acc[t], 0, 0, 0);
+    // (stores through the bounds check too: a pixel or a channel past the end is dropped by it)
+    const auto out = resource(y + o.nFirst * outElems, (N - o.nFirst) * outElems);
+    const auto post = resource(add + (add ? o.nFirst * outElems : 0), (N - o.nFirst) * outElems);
+    const int at = o.pix < 0 ? kOutside : ((o.img * OC + oc0 + 4 * hl) * P + o.pix) * 4;
+    // (opaque, or the compiler keeps their multiples and comparisons in scalar registers across the loop)
+    int row = P * 4, channels = OC;
+    asm volatile("" : "+s"(row), "+s"(channels));
+    auto store = [&](int ocl, float v, int voffset, int soffset) {
+      if (add) v += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(post, voffset, soffset, 0));
+      // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, relu ? fmaxf(v, 0.0f) : v), out, voffset, soffset, 0);
+    };
+    if (fullOc) {
+#pragma unroll
+      for (int t = 0; t < OCT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int ocl = 32 * t + 8 * (r / 4) + r % 4;
+          store(ocl, acc[t][r], at, ocl * row);
+        }
+    } else {
+#pragma unroll
+      for (int t = 0; t < OCT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int ocl = 32 * t + 8 * (r / 4) + r % 4;
+          if (oc0 + ocl < channels) // (a scalar offset past the resource would wrap the check)
+            store(ocl, acc[t][r], oc0 + ocl + 4 * hl < channels ? at : kOutside, ocl * row);
+        }
+    }
+  };
+  Tile even, odd;
+  int tile = (int)blockIdx.x * 4 + wave;
+  if (tile < tiles) fetch(even, tile);
+  for (; tile < tiles; tile += 2 * tileStep) {
+    if (tile + tileStep < tiles) fetch(odd, tile + tileStep);
+    finish(even);
+    if (tile + tileStep >= tiles) break;
+    if (tile + 2 * tileStep < tiles) fetch(even, tile + 2 * tileStep);
+    finish(odd);
   }
 }
 
-__global__ __launch_bounds__(256) void pool_kernel(const float *__restrict__ x, float *__restrict__ y, int64_t planes,
-                                                   int H, int W, int OH, int OW, int KH, int KW, int PHL, int PWL,
-                                                   int SH, int SW, bool average) {
-  const int64_t total = planes * OH * OW;
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += stride) {
-    const int ow = (int)(i % OW), oh = (int)((i / OW) % OH);
-    const float *plane = x + (i / ((int64_t)OW * OH)) * H * W;
+// ---- square windows, operands shared through LDS ---------------------------------------------
+// A block owns 64 output channels x 64 output pixels: 2 x 2 wavefronts of a 32 x 32 tile each, KS
+// times over when KS groups of four wavefronts split the channel groups.  Per unit of a channel group
+// its taps and filter values go from memory straight into LDS (dword loads; the bounds check writes
+// the zeros) into a ring of three stages, two units ahead of the one multiplied, the loads dealt out
+// between the MFMAs.  Every byte from L2 feeds 64 channels or pixels instead of the window kernel's
+// 32, whose L2 traffic is what bounds that one on large grids (8 x 256 x 14 x 14 -> 512, 3 x 3: 70 us
+// there, 45 here).
+template <int WIN, int KS>
+__global__ __launch_bounds__(256 * KS, 2) void conv_tile_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                                const float *__restrict__ bias, float *__restrict__ y, ConvGeo g,
+                                                                int OC, int P, int N, FastDiv byP, FastDiv byOW,
+                                                                const float *__restrict__ add, int relu) {
+  using Win = Window<WIN>;
+  constexpr int KK = Win::KK, UNITS = Win::UNITS, STEPS = Win::STEPS, HALF = Win::HALF;
+  constexpr int TL = (STEPS + 1) / 2;         // tap loads per wavefront and unit: every other step of one channel half
+  constexpr int PITCH = 18;                   // words per channel of the filter slice (2 * STEPS of them used; even, so that 32 channels fall on 32 banks)
+  constexpr int WL = 5;                       // filter loads per wavefront and unit: 4 x 5 x 64 >= 64 x PITCH
+  constexpr int ND = TL + WL;                 // loads per wavefront and unit
+  constexpr int kTapWords = 2 * TL * 2 * 64;  // [step][half][pixel]
+  constexpr int kStageWords = kTapWords + 4 * WL * 64;
+  constexpr int kRing = 3;
+  constexpr int kLds = KS * kRing * kStageWords * 4;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kLds];
+  static_assert(KS == 1 || KS * 4 * 4096 <= kLds, "the partial sums take the ring's place");
+
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int l32 = lane % 32, hl = lane / 32;
+  const int ks = wave / 4, wv = wave % 4;
+  const int wm = wv / 2, wp = wv % 2; // 32-channel and 32-pixel half of the block's tile
+  const int oc0 = blockIdx.y * 64, q0 = (int)blockIdx.x * 64;
+  const int HW4 = g.H * g.W * 4, pixels = N * P;
+  const int nFirst = __builtin_amdgcn_readfirstlane(divide(q0, byP)); // (the grid has no block past the last pixel)
+
+  // ---- movers.  Wavefront wv moves channel half wv / 2 of the taps, the steps of parity wv % 2.  The
+  // upper half's pixels are kept with bit 5 flipped, so that the two halves a wavefront reads at once lie
+  // on different banks.
+  const int mhalf = wv / 2, mstep = wv % 2;
+  int voff[UNITS * TL];
+  {
+    const int q = q0 + (lane ^ (32 * mhalf));
+    const bool live = q < pixels;
+    const int n = live ? divide(q, byP) : nFirst;
+    const int p = live ? q - n * P : 0;
+    const int oh = divide(p, byOW), ow = p - oh * g.OW;
+    const int ih0 = live ? oh * g.SH - g.PHL : -kNever, iw0 = ow * g.SW - g.PWL;
+    const int base = ((n - nFirst) * g.IC + mhalf * HALF) * HW4 + ((oh * g.SH - g.PHL) * g.W + iw0) * 4;
+#pragma unroll
+    for (int u = 0; u < UNITS; u++)
+#pragma unroll
+      for (int i = 0; i < TL; i++) {
+        // (1 x 1: every step reads the same position of another channel)
+        const int pos = WIN == 1 ? 0 : u * STEPS + 2 * i + mstep;
+        const int kh = pos / WIN, kw = pos - kh * WIN;
+        const bool in = (unsigned)(ih0 + kh * g.DH) < (unsigned)g.H && (unsigned)(iw0 + kw * g.DW) < (unsigned)g.W;
+        voff[u * TL + i] = in ? base + (kh * g.DH * g.W + kw * g.DW) * 4 : kOutside;
+      }
+  }
+  // The filter slice: word e = channel * PITCH + half * STEPS + step.
+  int woff[WL], wch[WL]; // byte offset at group 0, unit 0; channel inside the group (beyond every group: nothing to fetch)
+  {
+    const int row = g.IC * (KK * 4); // bytes per output channel
+    int oc = (WL * 64 * wv + lane) / PITCH, k = (WL * 64 * wv + lane) - oc * PITCH;
+    int at = oc * row;
+#pragma unroll
+    for (int i = 0; i < WL; i++) { // the next load's word is 64 = 3 * PITCH + 10 further
+      const bool upper = k >= STEPS;
+      const bool used = oc < 64 && oc0 + oc < OC && k < 2 * STEPS;
+      woff[i] = used ? at + k * 4 + (WIN > 1 && upper ? (KK - STEPS) * 4 : 0) : kOutside;
+      wch[i] = !used ? 0x3fffffff : WIN == 1 ? k : upper ? 1 : 0;
+      const bool wrap = k >= PITCH - 10;
+      k += wrap ? 10 - PITCH : 10;
+      oc += wrap ? 4 : 3;
+      at += wrap ? 4 * row : 3 * row;
+    }
+  }
+  const int64_t imageElems = (int64_t)g.IC * g.H * g.W;
+  const i32x4 image = resourceWords(x + nFirst * imageElems, (N - nFirst) * imageElems);
+  const i32x4 filter = resourceWords(w + (int64_t)oc0 * g.IC * KK, (int64_t)(OC - oc0) * g.IC * KK);
+  const uint32_t ldsBase = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) unsigned char *)smem) + ks * (kRing * kStageWords * 4);
+  // (inline assembly: completion is tracked by hand, see gemm_mfma.hip)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  auto dma4 = [&](int voffset, const i32x4 &rsrc, int soffset, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dword %0, %1, %2 offen lds"
+                 :
+                 : "v"(voffset), "s"(rsrc), "s"(soffset), "s"(lds)
+                 : "memory", "m0");
+  };
+#pragma clang diagnostic pop
+
+  const int groups = (g.IC + 2 * HALF - 1) / (2 * HALF);
+  const int perKs = (groups + KS - 1) / KS; // every wavefront group walks as many; those past the end fetch zeros
+  const int gBegin = ks * perKs;
+  // Load k of the wavefront's for a unit.  `whole`: every channel of the group exists (uniform).
+  auto load = [&](int k, int group, int unit, uint32_t at, auto whole) {
+    const int c0 = group * (2 * HALF);
+    if (k < TL) {
+      const int step = 2 * k + mstep;
+      const int c = c0 + (WIN == 1 ? step : 0); // the channel these 64 lanes read, less mhalf * HALF
+      const bool in = step < STEPS && (decltype(whole)::value || c + mhalf * HALF < g.IC);
+      dma4(in ? voff[unit * TL + k] : kOutside, image, in ? c * HW4 : 0, at + (uint32_t)((step * 2 + mhalf) * 64 * 4));
+    } else {
+      const int i = k - TL;
+      const bool in = decltype(whole)::value || c0 + wch[i] < g.IC;
+      // (a scalar offset beyond the resource would wrap the bounds check: 0 where nothing is in range)
+      const int wbase = decltype(whole)::value || c0 < g.IC ? (c0 * KK + unit * STEPS) * 4 : 0;
+      dma4(in ? woff[i] : kOutside, filter, wbase, at + (uint32_t)((kTapWords + (WL * wv + i) * 64) * 4));
+    }
+  };
+
+  f32x16 acc[1];
+#pragma unroll
+  for (int i = 0; i < 16; i++) acc[0][i] = 0.0f;
+
+  const int total = perKs * UNITS;
+  auto unitOf = [&](int t, auto &&f) { // f(group, unit as a constant) of the t-th unit
+    if constexpr (UNITS == 1) f(gBegin + t, std::integral_constant<int, 0>());
+    else {
+      const int grp = gBegin + t / UNITS, u = t % UNITS;
+      auto pick = [&](auto self, auto c) {
+        constexpr int k = decltype(c)::value;
+        if constexpr (k < UNITS) {
+          if (u == k) f(grp, c);
+          else self(self, std::integral_constant<int, k + 1>());
+        }
+      };
+      pick(pick, std::integral_constant<int, 0>());
+    }
+  };
+  auto loadUnit = [&](int t, int stage, auto &&take) { // take(load index -> void) issues the loads of unit t
+    unitOf(t, [&](int grp, auto u) {
+      const uint32_t into = ldsBase + (uint32_t)stage * (kStageWords * 4);
+      if ((grp + 1) * (2 * HALF) <= g.IC) take([&](int k) { load(k, grp, decltype(u)::value, into, std::true_type()); });
+      else take([&](int k) { load(k, grp, decltype(u)::value, into, std::false_type()); });
+    });
+  };
+  auto allAtOnce = [&](auto &&one) {
+#pragma unroll
+    for (int k = 0; k < ND; k++) one(k);
+  };
+  loadUnit(0, 0, allAtOnce);
+  if (total > 1) loadUnit(1, 1, allAtOnce);
+  // One unit: the MFMAs of its steps, each step's operands read from LDS one step ahead, and the
+  // loads of a later unit dealt out between the steps.
+  auto compute = [&](int stage, auto &&between) {
+    const auto *at = reinterpret_cast<const float __attribute__((address_space(3))) *>((uintptr_t)(ldsBase + (uint32_t)stage * (kStageWords * 4)));
+    const auto *ap = at + kTapWords + (32 * wm + l32) * PITCH + hl * STEPS;
+    const auto *bp = at + hl * 64 + ((wp * 32 + l32) ^ (32 * hl));
+    float a[2], b[2];
+    a[0] = ap[0];
+    b[0] = bp[0];
+#pragma unroll
+    for (int i = 0; i < STEPS; i++) {
+      if (i + 1 < STEPS) {
+        a[(i + 1) % 2] = ap[i + 1];
+        b[(i + 1) % 2] = bp[(i + 1) * 2 * 64];
+      }
+      acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i % 2], b[i % 2], acc[0], 0, 0, 0);
+      between(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int stage = 0;
+  for (int t = 0; t < total; t++) {
+    // unit t has landed (the one after may fly); everybody is done with unit t - 1, whose stage the
+    // loads of unit t + 2 overwrite
+    if (t + 1 < total) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ND) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (t + 2 < total)
+      loadUnit(t + 2, stage >= 1 ? stage - 1 : stage + 2, [&](auto &&one) {
+        compute(stage, [&](int i) {
+#pragma unroll
+          for (int k = i * ND / STEPS; k < (i + 1) * ND / STEPS; k++) one(k);
+        });
+      });
+    else compute(stage, [](int) {});
+    stage = stage == kRing - 1 ? 0 : stage + 1;
+  }
+
+  const int q = q0 + wp * 32 + l32;
+  const bool live = q < pixels;
+  const int n = live ? divide(q, byP) : nFirst;
+  const int img[1] = {n - nFirst}, pix[1] = {live ? q - n * P : -1};
+  if (KS > 1) __syncthreads(); // the partial sums take the ring's place
+  auto &partial = *reinterpret_cast<float(*)[KS > 1 ? 4 * KS : 1][KS > 1 ? 16 * 64 : 1]>(smem);
+  finishTile<1, KS, uint32_t>(acc, partial, wv * KS, ks, bias, add, y, OC, P, oc0 + 32 * wm, nFirst, img, pix, lane, relu);
+}
+
+// One output a thread.  Index: 32 bits where input and output allow (64-bit divisions are sequences of
+// a hundred instructions, longer than the window's loads; 4 x 64 x 28 x 28, 2 x 2: 2.5 -> 2.1 us).
+template <typename Index>
+__global__ __launch_bounds__(256) void pool_kernel(const float *__restrict__ x, float *__restrict__ y, Index total, Index stride,
+                                                   int H, int W, int OH, int OW, int KH, int KW, int PHL, int PWL, int SH,
+                                                   int SW, bool average) {
+  for (Index i = (Index)blockIdx.x * 256 + threadIdx.x; i < total; i += stride) {
+    const Index row = i / OW; // output row over all planes
+    const int ow = (int)(i - row * OW), oh = (int)(row % OH);
+    const float *plane = x + (row / OH) * (Index)H * W;
+    // the part of the window inside the image
+    const int h0 = oh * SH - PHL, w0 = ow * SW - PWL;
+    const int hFrom = h0 < 0 ? 0 : h0, hTo = h0 + KH < H ? h0 + KH : H;
+    const int wFrom = w0 < 0 ? 0 : w0, wTo = w0 + KW < W ? w0 + KW : W;
     float acc = average ? 0.0f : -INFINITY;
-    for (int kh = 0; kh < KH; kh++) {
-      const int ih = oh * SH - PHL + kh;
-      if (ih < 0 || ih >= H) continue;
-      for (int kw = 0; kw < KW; kw++) {
-        const int iw = ow * SW - PWL + kw;
-        if (iw < 0 || iw >= W) continue;
-        const float v = plane[(int64_t)ih * W + iw];
+    for (int ih = hFrom; ih < hTo; ih++)
+      for (int iw = wFrom; iw < wTo; iw++) {
+        const float v = plane[(Index)ih * W + iw];
         acc = average ? acc + v : fmaxf(acc, v);
       }
-    }
     y[i] = average ? acc / (float)(KH * KW) : acc;
   }
 }
@@ -194,6 +781,12 @@ unsigned blocksFor(int64_t items) {
 }
 
 bool fitsInt(int64_t v) { return v >= 0 && v <= 0x7fffffff; }
+
+FastDiv fastDiv(int d) {
+  unsigned shift = 0;
+  while ((1u << shift) < (unsigned)d) shift++;
+  return {(unsigned)((((uint64_t)1 << 32) * (((uint64_t)1 << shift) - d)) / d + 1), shift};
+}
 
 } // namespace
 
@@ -218,23 +811,91 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
   if (OH == 0 || OW == 0) return;
   const ConvGeo g{(int)IC, (int)H, (int)W, (int)KH, (int)KW, (int)OH, (int)OW, (int)PHL, (int)PWL,
                   (int)SH, (int)SW, (int)DH, (int)DW};
-  const int64_t ocTiles = (OC + kConvOC - 1) / kConvOC;
-  if (ocTiles > 65535) fail("mgpuConv2d: too many output channels for one launch");
-  // 128-pixel tiles unless that leaves fewer than two blocks per compute unit
-  const bool wide = N * ((P + 127) / 128) * ocTiles >= 512;
-  const int64_t pTiles = wide ? (P + 127) / 128 : (P + 63) / 64;
-  if (!fitsInt(N * pTiles)) fail("mgpuConv2d: too many output tiles for one launch");
-  // lane offsets inside a block's filter and output tiles are 32-bit
-  if (!fitsInt(kConvOC * K + K) || !fitsInt((kConvOC + 1) * P)) fail("mgpuConv2d: dimension too large");
-  const dim3 grid((unsigned)(N * pTiles), (unsigned)ocTiles);
   const float *add = hasPostAdd ? postAdd : nullptr;
-  if (wide)
-    conv_mfma_kernel<128, 32><<<grid, dim3(256), 0, stream>>>(input, weight, bias, add, output, g, (int)OC, (int)K,
-                                                              (int)P, (int)pTiles, relu);
-  else
-    conv_mfma_kernel<64, 32><<<grid, dim3(256), 0, stream>>>(input, weight, bias, add, output, g, (int)OC, (int)K,
-                                                             (int)P, (int)pTiles, relu);
-  MGPU_CHECK_LAUNCH("conv_mfma_kernel");
+  const int64_t pixels = N * P, pix32 = (pixels + 31) / 32;
+  const FastDiv byP = fastDiv((int)P), byOW = fastDiv((int)OW);
+  auto gridOf = [&](int64_t blocks, int64_t channels) {
+    const int64_t ocTiles = (OC + channels - 1) / channels;
+    if (ocTiles > 65535) fail("mgpuConv2d: too many output channels for one launch");
+    if (!fitsInt(blocks)) fail("mgpuConv2d: too many output tiles for one launch");
+    return dim3((unsigned)blocks, (unsigned)ocTiles);
+  };
+  // Everything but the table kernel's wide form keeps pixel indices and, from the first image a tile
+  // touches, byte offsets in 32 bits (a tile is at most 64 pixels), and window positions in 5.
+  const int64_t images = 63 / P + 2;
+  const bool narrow = fitsInt(pixels) && fitsInt(images * IC * H * W * 4) && fitsInt(images * OC * P * 4) &&
+                      fitsInt(65 * K * 4) && KH <= 31 && KW <= 31;
+  auto few = [&](auto octs, auto nss) {
+    constexpr int OCT = decltype(octs)::value, NS = decltype(nss)::value;
+    // two blocks per CU and channel tile at the registers of OCT = 2, four at those of OCT = 1
+    const int64_t most = std::max<int64_t>(1, (int64_t)numComputeUnits() * (4 / OCT) / ((OC + 32 * OCT - 1) / (32 * OCT)));
+    const int64_t blocks = std::min((pix32 + 3) / 4, most);
+    conv_few_taps_kernel<OCT, NS><<<gridOf(blocks, 32 * OCT), dim3(256), 0, stream>>>(
+        input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu, (int)K, (int)pix32, (int)(4 * blocks));
+  };
+  auto window = [&](auto win, auto pts, auto kss) {
+    constexpr int WIN = decltype(win)::value, PT = decltype(pts)::value, KS = decltype(kss)::value;
+    const int64_t perBlock = 4 / KS * 32 * PT;
+    conv_window_kernel<WIN, PT, KS><<<gridOf((pixels + perBlock - 1) / perBlock, 32), dim3(256), 0, stream>>>(
+        input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu);
+  };
+  auto tile = [&](auto win, auto kss) {
+    constexpr int WIN = decltype(win)::value, KS = decltype(kss)::value;
+    conv_tile_kernel<WIN, KS><<<gridOf((pixels + 63) / 64, 64), dim3(256 * KS), 0, stream>>>(
+        input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu);
+  };
+  auto table = [&](auto wide) {
+    conv_table_kernel<decltype(wide)::value><<<gridOf(pix32, 32), dim3(256), 0, stream>>>(
+        input, weight, bias, add, output, g, (int)OC, (int)K, (int)P, pixels, relu);
+  };
+  using std::integral_constant;
+  const integral_constant<int, 1> c1{};
+  const integral_constant<int, 2> c2{};
+  const integral_constant<int, 4> c4{};
+  // A 32 x 32 tile per wavefront group: `tiles` of them.  Measured where the lines lie (us, the
+  // kernels in turn, 3 x 3 unless said otherwise):
+  //  * 196 tiles (4 x 64 x 28 x 28 -> 64): window x 4 wavefronts 7.0, LDS tiles 14.7-18; 136 tiles
+  //    (256 x 13 x 41 -> 256): 18.0 against 45-62; 784 tiles (8 x 256 x 14 x 14 -> 512): 70 against 45;
+  //  * LDS tiles: 200 blocks of 128 units 45.5 with four groups, 49.3 with two, 62.8 with one; 392 blocks
+  //    of 32 units 29.9 / 25.9 / 27.9; 284 blocks of 16 units (1 x 1) 29.8 / 24.8 / 23.5;
+  //  * 96 channels are two 64-channel tiles with a quarter of nothing: 12 x 32 x 100 x 90 -> 96 takes 87 in LDS
+  //    tiles and 66-75 in window tiles of two accumulators.
+  const int64_t tiles = pix32 * ((OC + 31) / 32);
+  const bool squareWindow = KH == KW && (KH == 1 || KH == 3 || KH == 5 || KH == 7);
+  if (!narrow) {
+    table(std::true_type());
+  } else if (K <= 32) {
+    auto steps = [&](auto octs) {
+      if (K <= 10) few(octs, integral_constant<int, 5>());
+      else if (K <= 16) few(octs, integral_constant<int, 8>());
+      else if (K <= 28) few(octs, integral_constant<int, 14>());
+      else few(octs, integral_constant<int, 16>());
+    };
+    // (two accumulators share the gathered taps; few pixels are spread over more wavefronts instead)
+    if (OC > 32 && pix32 >= 4 * numComputeUnits()) steps(c2);
+    else steps(c1);
+  } else if (squareWindow) {
+    auto pick = [&](auto win) {
+      constexpr int WIN = decltype(win)::value;
+      const int64_t units = ((IC + 2 * Window<WIN>::HALF - 1) / (2 * Window<WIN>::HALF)) * Window<WIN>::UNITS;
+      const int64_t blocks = (pixels + 63) / 64 * ((OC + 63) / 64);
+      if (tiles <= 400) window(win, c1, c4);
+      else if ((OC - 1) % 64 >= 32) {
+        if (blocks <= numComputeUnits() && units >= 64) tile(win, c4);
+        else if (blocks <= 2 * numComputeUnits() && units >= 24) tile(win, c2);
+        else tile(win, c1);
+      } else if (tiles <= 2048) window(win, c1, c2);
+      else if constexpr (WIN <= 3) window(win, c2, c1);
+      else window(win, c1, c1);
+    };
+    if (KH == 1) pick(c1);
+    else if (KH == 3) pick(integral_constant<int, 3>());
+    else if (KH == 5) pick(integral_constant<int, 5>());
+    else pick(integral_constant<int, 7>());
+  } else {
+    table(std::false_type());
+  }
+  MGPU_CHECK_LAUNCH("mgpuConv2d");
 }
 
 void pool2d(const float *input, float *output, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OH, int64_t OW,
@@ -251,9 +912,16 @@ void pool2d(const float *input, float *output, int64_t N, int64_t C, int64_t H, 
   if (!input || !output) fail("mgpuPool2d: null pointer");
   for (int64_t v : {H, W, OH, OW, KH, KW, PHL, PWL, SH, SW})
     if (!fitsInt(v)) fail("mgpuPool2d: dimension too large");
-  pool_kernel<<<dim3(blocksFor(N * C * OH * OW)), dim3(256), 0, stream>>>(
-      input, output, N * C, (int)H, (int)W, (int)OH, (int)OW, (int)KH, (int)KW, (int)PHL, (int)PWL, (int)SH, (int)SW,
-      method == 1);
+  const int64_t total = N * C * OH * OW;
+  const unsigned blocks = blocksFor(total);
+  auto launch = [&](auto index) {
+    using Index = decltype(index);
+    pool_kernel<Index><<<dim3(blocks), dim3(256), 0, stream>>>(input, output, (Index)total, (Index)blocks * 256, (int)H, (int)W, (int)OH,
+                                                               (int)OW, (int)KH, (int)KW, (int)PHL, (int)PWL, (int)SH, (int)SW, method == 1);
+  };
+  // (the stride is added past the last index once)
+  if (N * C * H * W <= 0x7fffffff && total + (int64_t)blocks * 256 <= 0xffffffffll) launch(uint32_t());
+  else launch(int64_t());
   MGPU_CHECK_LAUNCH("pool_kernel");
 }
 

@@ -75,3 +75,40 @@ def test_conv_pool_reject_bad_arguments(pkg, gpu):
     lib.mgpuPool2d(x.data_ptr(), out.data_ptr(), 1, 2, 8, 8, 5, 5, 2, 2, 2, 2, 0, 0, 2, 2, 0, None)
     assert b"padding must be smaller" in lib.mgpuOpsTakeLastError()
     assert lib.mgpuOpsTakeLastError() is None
+
+
+@pytest.mark.parametrize("N,IC,H,W,OC,K,pad,stride,dilation,relu,add", [
+    # few taps (K <= 32): the step counts 5, 8, 14 and 16, one and two accumulators, a last channel tile of one, dilation
+    (3, 1, 9, 7, 33, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, True), (2, 16, 6, 5, 1, (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), False, False),
+    (40, 3, 33, 31, 65, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, True), (5, 2, 17, 19, 40, (4, 4), (2, 1, 1, 2), (2, 1), (1, 2), False, False),
+    # window kernel: odd channels, 5 x 5 and 7 x 7 rows, images smaller than a tile
+    (5, 5, 7, 7, 33, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False), (2, 3, 21, 18, 32, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), False, True),
+    (1, 4, 20, 23, 8, (7, 7), (3, 3, 3, 3), (2, 2), (1, 1), True, False), (9, 37, 3, 3, 64, (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), False, True),
+    (6, 8, 60, 61, 96, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False), (10, 36, 60, 61, 32, (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), False, False),
+    (8, 3, 90, 90, 24, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), False, False), (3, 8, 60, 61, 32, (3, 3), (1, 1, 1, 1), (1, 1), (2, 2), False, False),
+    # LDS tiles: one, two and four wavefront groups, channels that do not fill the last group
+    (8, 9, 50, 51, 64, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, True), (8, 50, 40, 40, 48, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, False),
+    (6, 131, 30, 31, 100, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False), (8, 72, 41, 40, 130, (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), False, True),
+    (5, 6, 64, 64, 64, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), False, False), (6, 4, 90, 90, 64, (7, 7), (3, 3, 3, 3), (1, 1), (1, 1), True, False),
+    # the table: windows that are no square of 1, 3, 5 or 7; more than one segment of it
+    (2, 12, 20, 22, 40, (1, 7), (0, 3, 0, 3), (1, 1), (1, 1), True, True), (2, 300, 9, 11, 33, (2, 4), (1, 1, 0, 2), (1, 1), (2, 1), False, False),
+    # windows and dilations beyond the table's narrow form
+    (1, 1, 70, 3, 2, (40, 1), (0, 0, 0, 0), (1, 1), (1, 1), False, False), (1, 2, 4000, 1, 3, (3, 1), (1, 0, 0, 0), (7, 1), (1500, 1), True, False)])
+def test_conv2d_every_kernel(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add):
+    conv_case(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add)
+
+
+def test_conv2d_padding_and_filler_do_not_multiply_garbage(pkg, gpu):
+    """Operands the kernels make up (taps outside the image, channels and taps past the end) are zeros on both sides:
+    an Inf or NaN in a neighbouring channel, filter row or image never reaches another output."""
+    import torch
+    for IC, OC, K, HW in ((3, 34, 3, 20), (5, 34, 3, 20), (5, 64, 3, 70), (33, 40, 1, 12), (7, 33, 2, 9)):
+        g = torch.Generator(device=gpu).manual_seed(IC)
+        x, w = torch.randn(2, IC, HW, HW, device=gpu, generator=g), torch.randn(OC, IC, K, K, device=gpu, generator=g)
+        b = torch.zeros(OC, device=gpu)
+        p = K // 2
+        clean = pkg.conv2d(x, w, b, pad=(p,) * 4)
+        x[1], w[1] = float("nan"), float("inf")
+        dirty = pkg.conv2d(x, w, b, pad=(p,) * 4)
+        keep = [o for o in range(OC) if o != 1]
+        assert torch.equal(clean[0, keep], dirty[0, keep]), (IC, OC, K)
