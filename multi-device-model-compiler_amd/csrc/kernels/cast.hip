@@ -248,10 +248,6 @@ namespace mgpu {
 
 namespace {
 
-__device__ __forceinline__ float gelu_erf(float x) {
-  return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void gelu_h_vec8_kernel(u32x4 *__restrict__ data, size_t n8) {
   const size_t stride = (size_t)gridDim.x * 256;

@@ -74,6 +74,11 @@ __device__ __forceinline__ float gelu_erfc(float x) {
   return x * (x > 0.0f ? 1.0f - halfErfc : halfErfc);
 }
 
+// ... and for fp32 results, by the library's erf.
+__device__ __forceinline__ float gelu_erf(float x) {
+  return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));
+}
+
 // ---- cross-lane sums on a 64-wide wavefront ------------------------------
 // DPP moves inside a row of 16 lanes (no LDS traffic), then lane exchanges
 // across rows.  After the call every participating lane holds the same sum.

@@ -10,9 +10,9 @@
 //    asks for fp16 accumulation (Ops.cu:164-167);
 //  * GELU is applied by an exact-erf kernel after a bias-only epilogue, because
 //    the library's fused GELU is the tanh approximation;
-//  * a call only enqueues: which of the two kernels serves a shape - the
-//    library or the hand-written MFMA kernel of gemm_mfma.hip - comes from a
-//    table decided offline (gemm_table.inc, written by `bench.py --tune-gemm`
+//  * a call only enqueues: which of the kernels serves a shape - the library or
+//    a hand-written one (gemm_mfma.hip, gemm_ksplit.hip, gemm_f32_small.hip) - comes
+//    from a table decided offline (gemm_table.inc, written by `bench.py --tune-gemm`
 //    from measurements on an MI355X) and, for shapes the table does not hold,
 //    from a fixed rule; the library runs the heuristic's first algorithm.
 //    MGPU_GEMM_KERNEL=library or =mfma in the environment overrides both.
@@ -79,7 +79,6 @@ struct Plan {
   size_t algoWorkspace = 0;
   hipblasLtMatmulAlgo_t algoNoWs;      // the first answer that needs no workspace
   bool hasNoWs = false;
-  bool handWritten = false; // serve the shape with gemm_mfma.hip when the operands allow it
 };
 
 // Shapes decided offline: {type (1 fp16, 2 bf16), M, N, K, hasBias, act, hasResidual, hand-written kernel
@@ -94,7 +93,7 @@ const TableEntry kTable[] = {
 #include "gemm_table.inc"
 };
 
-// Which kernel serves a shape nobody measured: the hand-written one where it can pay -
+// Which kernel serves an aligned shape nobody measured: the hand-written one where it can pay -
 // reductions up to 1024 deep, a GELU to fuse, or at most one 128-row tile per CU (its
 // eight-wavefront form).  On long reductions over many tiles the library's steady state
 // is ahead.
@@ -126,6 +125,49 @@ const TableEntry *tableRow(DType dt, int64_t M, int64_t N, int64_t K, bool hasBi
   return nullptr;
 }
 
+enum class Served { Library, Mfma, KSplit, F32Small };
+
+// The kernel for a call, decided without a lookup of the library's plans (a library call costs 6-7 us of
+// host time, a hand-written one a launch).
+//  * fp32: the small kernel up to 131072 tile-k (256 tiles of 32 x 32, 512 deep: 6.1 us against 6.7; 240 tiles
+//    768 deep 9.1 against 7.9; 1024 tiles 300 deep 17.9 against 14.9).
+//  * fp16 / bf16: the aligned shapes of the table as it says; otherwise the cheaper of gemm_mfma and
+//    gemm_ksplit by their estimates, as long as it is no large problem, where the library is ahead: more than
+//    400 tiles of 128 x 128 without a GELU to fuse (5000 x 2304 x 768 24.5 us against 27, 2000 x 6144 x 2048
+//    53.5 against 59; below, 2500 x 2304 x 768 16.9 against 16.7, 1200 x 1024 x 4096 36.6 against 31.7, 600 x 768 x
+//    768 7.5 against 5.4) - except for aligned shapes that the rule above gives to gemm_mfma.
+//  * K-major weights: gemm_ksplit while its tiles are at most one round of the CUs (beyond, the library, for
+//    which the layout was made).
+Served chooseKernel(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
+                    int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor) {
+  if (forcedKernel() == 1) return Served::Library;
+  if (dt == DType::F32) {
+    const int64_t tiles = (M + 31) / 32 * ((N + 31) / 32);
+    return !forcedKernel() && !weightKMajor && K <= 512 && tiles <= 131072 / K ? Served::F32Small : Served::Library;
+  }
+  const bool kSplitOk = gemmKSplitSupports(dt, in, weight, bias, residual, out, M, N, K);
+  double kSplitCost = 0.0;
+  const KSplitTile tile = gemmKSplitBest(M, N, K, act, &kSplitCost);
+  if (weightKMajor) {
+    const int64_t bm = tile == KSplitTile::T64x64 ? 64 : 32, bn = tile == KSplitTile::T32x32 ? 32 : 64;
+    return kSplitOk && !forcedKernel() && (M + bm - 1) / bm * ((N + bn - 1) / bn) <= numComputeUnits() ? Served::KSplit : Served::Library;
+  }
+  const bool mfmaOk = gemmMfmaSupportsRagged(dt, in, weight, bias, residual, out, M, N, K);
+  if (forcedKernel() == 2) return mfmaShape(dt, M, N, K) && mfmaOk ? Served::Mfma : Served::Library;
+  const bool aligned = mfmaOk && mfmaShape(dt, M, N, K);
+  if (aligned)
+    if (const TableEntry *e = tableRow(dt, M, N, K, hasBias, act, hasResidual)) return e->handWritten ? Served::Mfma : Served::Library;
+  const bool large = (M + 127) / 128 * ((N + 127) / 128) > 400;
+  if (large) {
+    if (mfmaOk && (act == ACT_GELU || (aligned && ruleSaysHandWritten(M, N, K, act)))) return Served::Mfma;
+    return Served::Library;
+  }
+  const double mfmaCost = gemmMfmaCost(M, N, K, act);
+  if (mfmaOk && mfmaCost < kSplitCost) return Served::Mfma;
+  // (where gemm_mfma cannot go - K no multiple of 32 - its estimate stands for the library's time)
+  return kSplitOk && kSplitCost < 1.2 * mfmaCost ? Served::KSplit : Served::Library;
+}
+
 using Key = std::tuple<int64_t, int64_t, int64_t, int, int, int, int, int>;
 std::map<Key, Plan> plans;
 
@@ -151,8 +193,7 @@ void destroyPlan(Plan &p) {
 constexpr int kCandidates = 16; // heuristic answers looked through for one that needs no workspace
 
 // Builds (once per shape, flags and type) the library's descriptors and picks its
-// algorithms; decides which kernel serves the shape.  No measurement, no allocation
-// beyond the library's host-side descriptors.
+// algorithms.  No measurement, no allocation beyond the library's host-side descriptors.
 Plan &getPlan(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor) {
   const bool relu = act == ACT_RELU;
   const Key key{M, N, K, (int)hasBias, act, (int)hasResidual, (int)dt, (int)weightKMajor};
@@ -211,11 +252,6 @@ Plan &getPlan(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, 
       p.hasNoWs = true;
     }
 
-  // The kernel: the table, else the rule.
-  p.handWritten = mfmaShape(dt, M, N, K) && ruleSaysHandWritten(M, N, K, act);
-  if (const TableEntry *e = tableRow(dt, M, N, K, hasBias, act, hasResidual)) p.handWritten = mfmaShape(dt, M, N, K) && e->handWritten != 0;
-  if (forcedKernel()) p.handWritten = forcedKernel() == 2;
-  if (weightKMajor) p.handWritten = false; // the hand-written kernel reads [K, N] weights only
   return plans.emplace(key, p).first->second;
 }
 
@@ -260,14 +296,26 @@ void matmulEx(DType dt, const void *input, const void *weight, const void *bias,
   if (act != ACT_NONE && hasResidual)
     fail("matmul: an activation cannot be combined with a residual");
 
-  std::lock_guard<std::mutex> lock(planMutex);
-  const Plan &p = getPlan(dt, M, N, K, hasBias, act, hasResidual, weightKMajor);
-  if (p.handWritten && gemmMfmaSupports(dt, input, weight, hasBias ? bias : nullptr,
-                                        hasResidual ? residual : nullptr, output, M, N, K)) {
-    gemmMfma(dt, input, weight, hasBias ? bias : nullptr, hasResidual ? residual : nullptr, output, M, N, K, act,
-             stream);
+  const void *b = hasBias ? bias : nullptr, *r = hasResidual ? residual : nullptr;
+  switch (chooseKernel(dt, input, weight, b, r, output, M, N, K, hasBias, act, hasResidual, weightKMajor)) {
+  case Served::Mfma:
+    gemmMfmaRagged(dt, input, weight, b, r, output, M, N, K, act, stream);
+    return;
+  case Served::KSplit: {
+    double cost;
+    const KSplitTile tile = gemmKSplitBest(M, N, K, act, &cost);
+    gemmKSplit(dt, input, weight, b, r, output, M, N, K, act, tile, weightKMajor, stream);
     return;
   }
+  case Served::F32Small:
+    gemmF32Small(static_cast<const float *>(input), static_cast<const float *>(weight), static_cast<const float *>(b),
+                 static_cast<const float *>(r), static_cast<float *>(output), M, N, K, act, stream);
+    return;
+  case Served::Library:
+    break;
+  }
+  std::lock_guard<std::mutex> lock(planMutex);
+  const Plan &p = getPlan(dt, M, N, K, hasBias, act, hasResidual, weightKMajor);
   if (hasBias)
     MGPU_CHECK_BLAS(hipblasLtMatmulDescSetAttribute(p.op, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &bias,
                                                     sizeof(bias)));

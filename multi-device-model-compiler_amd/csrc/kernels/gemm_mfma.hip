@@ -69,12 +69,14 @@ __host__ __device__ constexpr int wSwz(int row) { return (row & 3) << 2; } // 16
 
 // T: element type; ACT: epilogue activation; BK: reduction step (32 or 64);
 // NB: tile width in 32-column blocks (4 or 3).
-template <typename T, int ACT, int BK, int NB, bool PAIRED, bool SPLIT>
+// RAGGED: M is no multiple of 128 or N none of the tile width.  The tiles cover the shape; rows and
+// columns past the end are loaded from the last ones and not stored.
+template <typename T, int ACT, int BK, int NB, bool PAIRED, bool SPLIT, bool RAGGED>
 __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma_kernel(const uint16_t *__restrict__ in,
                                                                         const uint16_t *__restrict__ weight,
                                                                         const uint16_t *__restrict__ bias,
                                                                         const uint16_t *residual, uint16_t *out, int N,
-                                                                        int K, int tilesN, int tilesM) {
+                                                                        int K, int tilesN, int tilesM, int M_) {
   using M = Mma<T>;
   using v8 = typename M::v8;
   using v4 = typename M::v4;
@@ -139,14 +141,17 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
   // where its scalar operands are no longer scalar to the compiler.)
   const char *abase = reinterpret_cast<const char *>(in) + (size_t)m0 * K * 2;
   const char *wbase = reinterpret_cast<const char *>(weight) + (size_t)n0 * 2;
+  const int rowsLeft = RAGGED ? M_ - m0 : kBM; // rows of the tile that exist
+  auto memRow = [&](int row) { return RAGGED && row >= rowsLeft ? rowsLeft - 1 : row; };
   uint32_t aoff[NL], woff[NL];
 #pragma unroll
   for (int i = 0; i < NL; i++) {
     const int arow = RPI * (NL * mover + i) + lane / CPR;
-    aoff[i] = (uint32_t)arow * (uint32_t)K * 2u + (uint32_t)(((lane % CPR) ^ aSwz<BK>(arow)) * 16);
+    aoff[i] = (uint32_t)memRow(arow) * (uint32_t)K * 2u + (uint32_t)(((lane % CPR) ^ aSwz<BK>(arow)) * 16);
     const int wrow = 4 * (NL * mover + i) + lane / 16;
     int wchunk = (lane % 16) ^ wSwz(wrow);
     if (wchunk >= 4 * NB) wchunk -= 4;
+    if (RAGGED && n0 + 8 * wchunk >= N) wchunk = (N - 8 - n0) / 8;
     woff[i] = (uint32_t)wrow * (uint32_t)N * 2u + (uint32_t)(wchunk * 16);
   }
   // PAIRED: the input rows of two steps at once, 8 rows of 128 bytes per load
@@ -155,7 +160,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int arow = 8 * (4 * wave + i) + lane / 8;
-    aoffP[i] = (uint32_t)arow * (uint32_t)K * 2u + (uint32_t)(((lane % 8) ^ aSwz<64>(arow)) * 16);
+    aoffP[i] = (uint32_t)memRow(arow) * (uint32_t)K * 2u + (uint32_t)(((lane % 8) ^ aSwz<64>(arow)) * 16);
   }
   // Inline assembly keeps these loads out of the compiler's wait-count
   // bookkeeping, which would otherwise wait for every load in flight before
@@ -355,7 +360,10 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
 #pragma unroll
     for (int nb = 0; nb < NBW; nb++)
 #pragma unroll
-      for (int g = 0; g < 4; g++) braw[nb][g] = *reinterpret_cast<const v4 *>(bias + nw + 32 * nb + 8 * g + 4 * hl);
+      for (int g = 0; g < 4; g++) {
+        const int n = nw + 32 * nb + 8 * g + 4 * hl;
+        braw[nb][g] = *reinterpret_cast<const v4 *>(bias + (RAGGED && n >= N ? N - 4 : n));
+      }
   }
 #pragma unroll
   for (int nb = 0; nb < NBW; nb++) {
@@ -370,9 +378,11 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
 #pragma unroll
       for (int g = 0; g < 4; g++)
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-          rraw[g][mb] = *reinterpret_cast<const v4 *>(residual + (size_t)(mw + 32 * mb + l32) * N + nw + 32 * nb +
-                                                      8 * g + 4 * hl);
+        for (int mb = 0; mb < MB; mb++) {
+          const int n = nw + 32 * nb + 8 * g + 4 * hl;
+          rraw[g][mb] = *reinterpret_cast<const v4 *>(residual + (size_t)(m0 + memRow(mw - m0 + 32 * mb + l32)) * N +
+                                                      (RAGGED && n >= N ? N - 4 : n));
+        }
     }
 #pragma unroll
     for (int g = 0; g < 4; g++) {
@@ -410,21 +420,28 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
     const u32x2 lo = *reinterpret_cast<const u32x2 *>(&stage[r * kOutStride + cidx * 8]);
     const u32x2 hi = *reinterpret_cast<const u32x2 *>(&stage[r * kOutStride + cidx * 8 + 4]);
     const u32x4 val = {lo[0], lo[1], hi[0], hi[1]};
+    if (RAGGED && (mw + r >= M_ || nw + cidx * 8 >= N)) continue;
     *reinterpret_cast<u32x4 *>(out + (size_t)(mw + r) * N + nw + cidx * 8) = val;
   }
 }
 
+template <typename T, int BK, int NB, bool PAIRED, bool SPLIT, bool RAGGED>
+void launchAct(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint16_t *r, uint16_t *o, int64_t M,
+               int64_t N, int64_t K, int act, hipStream_t stream) {
+  const int tilesN = (int)((N + 32 * NB - 1) / (32 * NB)), tilesM = (int)((M + kBM - 1) / kBM);
+  const dim3 grid((unsigned)(tilesM * tilesN)), block(SPLIT ? 512 : 256);
+  if (act == ACT_GELU)
+    gemm_mfma_kernel<T, ACT_GELU, BK, NB, PAIRED, SPLIT, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_RELU)
+    gemm_mfma_kernel<T, ACT_RELU, BK, NB, PAIRED, SPLIT, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else
+    gemm_mfma_kernel<T, ACT_NONE, BK, NB, PAIRED, SPLIT, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+}
 template <typename T, int BK, int NB, bool PAIRED, bool SPLIT = false>
 void launchTile(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint16_t *r, uint16_t *o, int64_t M,
                 int64_t N, int64_t K, int act, hipStream_t stream) {
-  const int tilesN = (int)(N / (32 * NB));
-  const dim3 grid((unsigned)((M / kBM) * tilesN)), block(SPLIT ? 512 : 256);
-  if (act == ACT_GELU)
-    gemm_mfma_kernel<T, ACT_GELU, BK, NB, PAIRED, SPLIT><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, (int)(M / kBM));
-  else if (act == ACT_RELU)
-    gemm_mfma_kernel<T, ACT_RELU, BK, NB, PAIRED, SPLIT><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, (int)(M / kBM));
-  else
-    gemm_mfma_kernel<T, ACT_NONE, BK, NB, PAIRED, SPLIT><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, (int)(M / kBM));
+  if (M % kBM || N % (32 * NB)) launchAct<T, BK, NB, PAIRED, SPLIT, true>(a, w, b, r, o, M, N, K, act, stream);
+  else launchAct<T, BK, NB, PAIRED, SPLIT, false>(a, w, b, r, o, M, N, K, act, stream);
 }
 
 // Tile width: the one under which the busiest CU carries the fewest columns
@@ -435,13 +452,10 @@ template <typename T>
 void launch(const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M,
             int64_t N, int64_t K, int act, hipStream_t stream) {
   const int64_t cus = numComputeUnits();
-  auto load = [&](int64_t width) -> int64_t {
-    if (N % width) return INT64_MAX;
-    const int64_t tiles = (M / kBM) * (N / width);
-    return (tiles + cus - 1) / cus * width;
-  };
+  auto tilesAt = [&](int64_t width) { return (M + kBM - 1) / kBM * ((N + width - 1) / width); };
+  auto load = [&](int64_t width) { return (tilesAt(width) + cus - 1) / cus * width; };
   const bool narrow = load(96) < load(128);
-  const int64_t tiles = (M / kBM) * (N / (narrow ? 96 : 128));
+  const int64_t tiles = tilesAt(narrow ? 96 : 128);
   const bool deep = tiles <= cus && K % 64 == 0;
   const auto *a = static_cast<const uint16_t *>(in);
   const auto *w = static_cast<const uint16_t *>(weight);
@@ -473,6 +487,36 @@ bool gemmMfmaSupports(DType dt, const void *in, const void *weight, const void *
   if (bias && (reinterpret_cast<uintptr_t>(bias) & 7u)) return false;
   if (residual && !aligned16(residual)) return false;
   return true;
+}
+
+bool gemmMfmaSupportsRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual,
+                            const void *out, int64_t M, int64_t N, int64_t K) {
+  if (N % 8) return false;
+  const int64_t m = (M + kBM - 1) / kBM * kBM, n = (N + 127) / 128 * 128; // the tiles that cover the shape
+  return gemmMfmaSupports(dt, in, weight, bias, residual, out, m, n, K);
+}
+
+// One tile per CU (eight wavefronts, steps of 64): a fixed part and the operand bytes at what a CU pulls;
+// several: what overlaps of them at 52 GB/s behind 5 us of start and end.  (600 x 3072 x 768 + GELU 11.7 us,
+// 1200 x 1024 x 4096 31.7, 2500 x 2304 x 768 16.7.)
+double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act) {
+  const int64_t cus = numComputeUnits();
+  auto tilesAt = [&](int64_t width) { return (M + kBM - 1) / kBM * ((N + width - 1) / width); };
+  auto load = [&](int64_t width) { return (tilesAt(width) + cus - 1) / cus * width; };
+  const int64_t width = load(96) < load(128) ? 96 : 128, tiles = tilesAt(width);
+  const double bytes = (double)(kBM + width) * 2.0 * (double)K;
+  if (tiles <= cus) return (act == ACT_GELU ? 5.0 : 2.0) + bytes / 57e3;
+  return 5.0 + (double)tiles / (double)cus * bytes / 52e3;
+}
+
+void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,
+                    int64_t M, int64_t N, int64_t K, int act, hipStream_t stream) {
+  if (!gemmMfmaSupportsRagged(dt, in, weight, bias, residual, out, M, N, K))
+    fail("gemmMfma: shape, type or alignment not supported by the hand-written kernel");
+  if (dt == DType::F16)
+    launch<_Float16>(in, weight, bias, residual, out, M, N, K, act, stream);
+  else
+    launch<bf16_t>(in, weight, bias, residual, out, M, N, K, act, stream);
 }
 
 void gemmMfma(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,

@@ -69,6 +69,26 @@ bool gemmMfmaSupports(DType dt, const void *in, const void *weight, const void *
 void gemmMfma(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,
               int64_t M, int64_t N, int64_t K, int act, hipStream_t stream);
 
+// The same kernel where its tiles overhang the shape: any M, N a multiple of 8, K of 32.
+bool gemmMfmaSupportsRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual,
+                            const void *out, int64_t M, int64_t N, int64_t K);
+// gemmMfmaCost: its estimated us on a shape, on the scale of gemmKSplitBest.
+double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act);
+void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,
+                    int64_t M, int64_t N, int64_t K, int act, hipStream_t stream);
+
+// Small tiles, the reduction split over a block's wavefronts (gemm_ksplit.hip): fp16 / bf16, any M, N and K
+// multiples of 8.  gemmKSplitBest: the tile for a shape and its estimated us, to compare with the others.
+enum class KSplitTile { T32x32, T32x64, T64x64 };
+KSplitTile gemmKSplitBest(int64_t M, int64_t N, int64_t K, int act, double *cost);
+bool gemmKSplitSupports(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
+                        int64_t N, int64_t K);
+void gemmKSplit(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
+                int64_t K, int act, KSplitTile tile, bool weightKMajor, hipStream_t stream);
+// fp32, any shape, for few tiles (gemm_f32_small.hip).
+void gemmF32Small(const float *in, const float *weight, const float *bias, const float *residual, float *out, int64_t M, int64_t N, int64_t K,
+                  int act, hipStream_t stream);
+
 void conv2d(const float *input, const float *weight, const float *bias, float *output, const float *postAdd,
             int64_t N, int64_t IC, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW, int64_t OH,
             int64_t OW, int64_t PHL, int64_t PWL, int64_t PHR, int64_t PWR, int64_t SH, int64_t SW, int64_t DH,
