@@ -282,6 +282,13 @@ bool gemmPrefersKMajor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, 
   return !(mfmaShape(dt, M, N, K) && ruleSaysHandWritten(M, N, K, act));
 }
 
+bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual) {
+  // Wherever the [K, N] weight would be the library's: its kernels for the other layout are ahead.
+  alignas(16) static const char aligned[16] = {};
+  return chooseKernel(dt, aligned, aligned, aligned, nullptr, aligned, M, N, K, hasBias, act, hasResidual, false) == Served::Library &&
+         chooseKernel(dt, aligned, aligned, aligned, nullptr, aligned, M, N, K, hasBias, act, hasResidual, true) == Served::Library;
+}
+
 void matmulEx(DType dt, const void *input, const void *weight, const void *bias, void *output,
               const void *residual, int64_t M, int64_t N, int64_t K, bool hasBias, int act,
               bool hasResidual, hipStream_t stream, bool weightKMajor) {

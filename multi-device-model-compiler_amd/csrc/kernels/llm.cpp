@@ -20,16 +20,16 @@
 //    capture, so the graph owns its temporaries and a later eager call that
 //    grows (frees and replaces) the stream's arena cannot pull memory from
 //    under a graph that is still replayed;
-//  * the side stream casts all the weights as soon as the call starts (one
-//    event behind the first GEMM's weight, one behind the rest), while the
-//    input cast and the first LayerNorm run on the
-//    caller's stream (the reference interleaves cast and wait per GEMM, input
-//    cast included, so the first GEMM starts two casts late); the gamma = 1 /
+//  * one kernel casts all seven weight and bias arrays, on the caller's stream
+//    (the reference casts each on a side stream; here the casts are bound by
+//    memory, so beside a GEMM they only slow it, and their launches and events
+//    were half of the host time of a small layer: 4096 x 2048 321 -> 289 us,
+//    240 x 768 112 -> 47 us); it writes K-major the weights whose GEMM is the
+//    library's, which has faster kernels for that layout.  The gamma = 1 /
 //    beta = 0 vectors are written once per model width, not per call;
-//  * the side stream first waits for work already queued on the caller's
-//    stream, and the final fp16 -> fp32 cast runs after the last GEMM on the
-//    caller's stream (the reference issues it on the side stream without
-//    waiting for that GEMM: LLM.cu:136-141).
+//  * the final fp16 -> fp32 cast runs after the last GEMM on the caller's
+//    stream (the reference issues it on the side stream without waiting for
+//    that GEMM: LLM.cu:136-141).
 //
 // bertEncoderLayerF16 is the post-LN BERT encoder layer on fp16 tensors (GELU,
 // learned LayerNorm affine, optional key-padding lengths); the reference has
@@ -47,7 +47,7 @@ namespace mgpu {
 namespace {
 
 bool initialised = false;
-constexpr int kCopyEvents = 4; // one per GEMM whose operands the side stream prepares
+constexpr int kGemms = 4; // of a layer
 
 // What the layers keep per caller stream between calls: the arena, and the
 // side stream with its events (two caller streams in flight at once must not
@@ -56,7 +56,6 @@ struct StreamState {
   void *base = nullptr; // arena
   size_t bytes = 0;
   hipStream_t side = nullptr;
-  hipEvent_t copyEvent[kCopyEvents] = {nullptr, nullptr, nullptr, nullptr};
   hipEvent_t forkEvent = nullptr;
 };
 std::mutex scratchMutex;
@@ -67,13 +66,12 @@ bool isCapturing(hipStream_t s) {
   return hipStreamIsCapturing(s, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
 }
 
-// The caller stream's state, with its side stream and events in place.  They
+// The caller stream's state, with its side stream and event in place.  They
 // are created on the stream's first layer call; scratchMutex must be held.
 StreamState &sideOf(hipStream_t s) {
   StreamState &st = stateOf[s];
   if (!st.side) {
     MGPU_CHECK_HIP(hipStreamCreateWithFlags(&st.side, hipStreamNonBlocking));
-    for (hipEvent_t &e : st.copyEvent) MGPU_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     MGPU_CHECK_HIP(hipEventCreateWithFlags(&st.forkEvent, hipEventDisableTiming));
   }
   return st;
@@ -133,6 +131,11 @@ CachedWeight &cachedWeight(const void *src, bool srcIsF32, int64_t rows, int64_t
     throw;
   }
   return weightCache.emplace(key, fresh).first->second;
+}
+
+bool cacheIsOn() {
+  std::lock_guard<std::mutex> lock(scratchMutex);
+  return weightCacheOn;
 }
 
 void dropWeightCache() { // scratchMutex held; the device idle or the copies no longer in use
@@ -220,8 +223,6 @@ void llmDeinit() {
     StreamState &st = kv.second;
     if (st.base) (void)hipFreeAsync(st.base, nullptr);
     if (st.side) (void)hipStreamDestroy(st.side);
-    for (hipEvent_t e : st.copyEvent)
-      if (e) (void)hipEventDestroy(e);
     if (st.forkEvent) (void)hipEventDestroy(st.forkEvent);
   }
   if (!stateOf.empty()) (void)hipStreamSynchronize(nullptr);
@@ -274,83 +275,58 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
   const size_t oW2 = arena.reserve(ffn * d * h), oB2 = arena.reserve(d * h);
   const size_t oOut = arena.reserve(M * d * h);
 
-  // Fork: the side stream may not run ahead of what already sits on `stream`,
-  // the arena's allocation included.  It then casts the weights and biases of
-  // the four GEMMs, in the order the GEMMs run, and marks each group with an
-  // event; `stream` waits for a group just before the GEMM that reads it, so the
-  // casts run under the input cast, the LayerNorms, the attention and the
-  // earlier GEMMs.
   arena.allocate(stream);
-  hipStream_t copyStream = nullptr;
-  hipEvent_t forkEvent = nullptr, copyEvent[kCopyEvents];
-  {
-    // This caller stream's own side stream and events (created on its first
-    // call; under a capture that forbids creating them this fails with the
-    // runtime's message: run the layer once on the stream before capturing).
-    std::lock_guard<std::mutex> lock(scratchMutex);
-    const StreamState &st = sideOf(stream);
-    copyStream = st.side;
-    forkEvent = st.forkEvent;
-    for (int i = 0; i < kCopyEvents; i++) copyEvent[i] = st.copyEvent[i];
-  }
-  // The seven weight and bias arrays in fp16: cast by the side stream now, or - with the weight
-  // cache on - taken from the cache (cast once, when first seen, on the side stream as well).
+  // The seven weight and bias arrays in fp16: cast now, all in one launch, or - with the weight cache
+  // on - taken from the cache (cast once, when first seen, on a side stream).
   struct Operand {
     const float *src;
     int64_t rows, cols; // [K, N] of a weight; a bias is rows elements and cols = 0
     size_t slot;        // where the per-call copy goes in the arena
     int group;          // the GEMM (0..3) that reads it
     void *half;         // the fp16 copy the GEMM is given
-    int64_t elems() const { return cols ? rows * cols : rows; }
   };
   Operand ops[7] = {{qkv, d, 3 * d, oWqkv, 0, nullptr},      {gemm_weight, d, d, oWo, 1, nullptr},
                     {gemm_bias, d, 0, oBo, 1, nullptr},      {ffn1_weight, d, ffn, oW1, 2, nullptr},
                     {ffn1_bias, ffn, 0, oB1, 2, nullptr},    {ffn2_weight, ffn, d, oW2, 3, nullptr},
                     {ffn2_bias, d, 0, oB2, 3, nullptr}};
-  bool forked = false, sideWork[kCopyEvents] = {false, false, false, false};
   hipEvent_t cachedReady[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  auto fork = [&] {
-    if (forked) return;
-    MGPU_CHECK_HIP(hipEventRecord(forkEvent, stream));
-    MGPU_CHECK_HIP(hipStreamWaitEvent(copyStream, forkEvent, 0));
-    forked = true;
-  };
-  bool kMajor[kCopyEvents] = {false, false, false, false}; // GEMM g gets the cache's transposed copy of its weight
+  bool kMajor[kGemms]; // GEMM g gets a transposed copy of its weight
+  const int act = relu ? ACT_RELU : ACT_GELU;
+  const bool useCache = cacheIsOn() && !isCapturing(stream); // a capture neither allocates nor reads the cache's events
   {
+    auto *prefers = useCache ? gemmPrefersKMajor : gemmWantsKMajorCast;
+    kMajor[0] = prefers(DType::F16, M, 3 * d, d, false, ACT_NONE, false);
+    kMajor[1] = prefers(DType::F16, M, d, d, true, ACT_NONE, false);
+    kMajor[2] = prefers(DType::F16, M, ffn, d, true, act, false);
+    kMajor[3] = prefers(DType::F16, M, d, ffn, true, ACT_NONE, norm_first);
+  }
+  if (useCache) {
+    // (an array's first conversion runs on the side stream, behind what already sits on `stream`)
     std::lock_guard<std::mutex> lock(scratchMutex);
-    const bool useCache = weightCacheOn && !isCapturing(stream); // a capture neither allocates nor reads the cache's events
-    if (useCache) {
-      const int act = relu ? ACT_RELU : ACT_GELU;
-      kMajor[0] = gemmPrefersKMajor(DType::F16, M, 3 * d, d, false, ACT_NONE, false);
-      kMajor[1] = gemmPrefersKMajor(DType::F16, M, d, d, true, ACT_NONE, false);
-      kMajor[2] = gemmPrefersKMajor(DType::F16, M, ffn, d, true, act, false);
-      kMajor[3] = gemmPrefersKMajor(DType::F16, M, d, ffn, true, ACT_NONE, norm_first);
-    }
+    const StreamState &st = sideOf(stream);
+    bool forked = false;
     for (int i = 0; i < 7; i++) {
       Operand &op = ops[i];
-      if (useCache) {
-        const bool transposed = op.cols && kMajor[op.group];
-        if (!weightCache.count(WeightKey{op.src, op.rows, op.cols, transposed})) fork(); // the conversion runs on the side stream
-        CachedWeight &cw = cachedWeight(op.src, true, op.rows, op.cols, transposed, copyStream);
-        op.half = cw.half;
-        cachedReady[i] = cw.pending();
-      } else {
-        fork();
-        op.half = arena.at(op.slot);
-        castF32ToF16(op.half, op.src, op.elems(), copyStream);
-        sideWork[op.group] = true;
+      const bool transposed = op.cols && kMajor[op.group];
+      if (!forked && !weightCache.count(WeightKey{op.src, op.rows, op.cols, transposed})) {
+        MGPU_CHECK_HIP(hipEventRecord(st.forkEvent, stream));
+        MGPU_CHECK_HIP(hipStreamWaitEvent(st.side, st.forkEvent, 0));
+        forked = true;
       }
-      // The casts go out in the order the GEMMs run.  Two events: one right behind the first GEMM's
-      // weight, one behind everything else - the later casts are long done when the second GEMM
-      // starts (they run under the first, the longest), and every wait the caller's stream does
-      // not make is a barrier packet it does not stall on.
-      if ((i == 0 || i == 6) && sideWork[op.group])
-        MGPU_CHECK_HIP(hipEventRecord(copyEvent[i == 0 ? 0 : 1], copyStream));
+      CachedWeight &cw = cachedWeight(op.src, true, op.rows, op.cols, transposed, st.side);
+      op.half = cw.half;
+      cachedReady[i] = cw.pending();
     }
+  } else {
+    CastJob jobs[7];
+    for (int i = 0; i < 7; i++) {
+      Operand &op = ops[i];
+      op.half = arena.at(op.slot);
+      jobs[i] = CastJob{op.src, op.half, op.rows, op.cols ? op.cols : 1, op.cols && kMajor[op.group], false};
+    }
+    castWeightsF32ToF16(jobs, 7, stream);
   }
   auto join = [&](int group) {
-    if (group <= 1 && (sideWork[group] || (group == 1 && (sideWork[2] || sideWork[3]))))
-      MGPU_CHECK_HIP(hipStreamWaitEvent(stream, copyEvent[group], 0));
     for (int i = 0; i < 7; i++)
       if (ops[i].group == group && cachedReady[i]) MGPU_CHECK_HIP(hipStreamWaitEvent(stream, cachedReady[i], 0));
   };
@@ -394,7 +370,7 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
     matmulEx(DType::F16, arena.at(oLn), w1H, b1H, arena.at(oF), nullptr, M, ffn,
              d, true, relu ? ACT_RELU : ACT_GELU, false, stream, kMajor[2]);
 
-    join(3); // also the join of the fork: nothing of this call is left on the side stream after it
+    join(3);
     matmulEx(DType::F16, arena.at(oF), w2H, b2H, arena.at(oOut), arena.at(oY), M,
              d, ffn, true, ACT_NONE, true, stream, kMajor[3]);
   } else {

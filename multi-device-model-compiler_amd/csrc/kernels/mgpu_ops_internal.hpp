@@ -41,6 +41,16 @@ void castBF16ToF32(float *dst, const void *src, size_t size, hipStream_t stream)
 // dst[c][r] = src[r][c] of a row-major rows x cols matrix (fp32 -> fp16; any 16-bit type, bit for bit)
 void transposeCastF32ToF16(void *dst, const float *src, int64_t rows, int64_t cols, hipStream_t stream);
 void transpose16(void *dst, const void *src, int64_t rows, int64_t cols, hipStream_t stream);
+// fp32 arrays to fp16, up to kMaxCastJobs of them in one launch; kMajor: dst[c][r] = src[r][c].
+struct CastJob {
+  const float *src;
+  void *dst;
+  int64_t rows, cols;
+  bool kMajor;
+  bool vector; // (set by the call: 16-byte accesses allowed)
+};
+constexpr int kMaxCastJobs = 8;
+void castWeightsF32ToF16(CastJob *jobs, int count, hipStream_t stream);
 void fillF16(void *dst, size_t count, float value, hipStream_t stream);
 void fillI32(int32_t *dst, size_t count, int32_t value, hipStream_t stream);
 
@@ -61,6 +71,9 @@ void matmulEx(DType dt, const void *input, const void *weight, const void *bias,
 // Should a caller that can keep a K-major copy of the weight hand that one to matmulEx for this
 // problem?  (The committed table, else: wherever the library would serve the shape.)
 bool gemmPrefersKMajor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual);
+// Would a caller that makes its fp16 weight anew on every call, in either layout at the same price, rather
+// have it K-major?
+bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual);
 
 // Hand-written MFMA GEMM (gemm_mfma.hip): fp16 / bf16, M a multiple of 128, N of
 // 128 or 96, K of 32, 16-byte aligned operands; bias and residual may be null.
