@@ -9,9 +9,8 @@
 //   lane-exchange sums, one 128-bit non-temporal store per vector (plain loads
 //   + non-temporal stores measured fastest on MI355X).  One pass over HBM.
 // Rows wider than a wavefront can hold live in the registers of a whole block
-// (layernorm_block_kernel); rows whose length is not a multiple of the vector
-// width, rows beyond 256 x 16 vectors and unaligned pointers take the general
-// block-per-row kernel.
+// (layernorm_block_kernel); rows beyond 256 x 16 vectors and rows shorter than one vector
+// take the general block-per-row kernel.
 #include "common.hpp"
 #include "mgpu_ops_internal.hpp"
 #include "types.hpp"
@@ -22,11 +21,46 @@ namespace {
 
 constexpr int kMaxVPL = 8; // vectors per lane the register kernel is built for
 
+// How a row is cut into 16-byte vectors.  kFull: the row is all of an instantiation's vectors; kVectors: whole
+// vectors, some lanes without one; kRagged: any length of at least one vector, any alignment.  A ragged
+// row's last vector ends with the row, so that it overlaps the one before it: its first elements are left out of the
+// statistics and stored twice, with the same bits.  Vectors that are off the 16-byte grid still move
+// as one dwordx4 each, across two cache lines where they straddle.
+enum class RowShape { kFull, kVectors, kRagged };
+
+typedef u32x4 Loose32 __attribute__((aligned(2)));
+
+template <typename T, RowShape SHAPE>
+struct RowVectors {
+  static constexpr bool kRagged = SHAPE == RowShape::kRagged;
+  static constexpr int VEC = ElemTraits<T>::kVec;
+  static __device__ int count(int n) { return kRagged ? (n + VEC - 1) / VEC : n / VEC; }
+  // (mayBeLast, here and below: vector v can be the row's last one)
+  static __device__ int offset(bool mayBeLast, int v, int n) { return kRagged && mayBeLast && v * VEC > n - VEC ? n - VEC : v * VEC; }
+  static __device__ u32x4 load(const T *row, bool mayBeLast, int v, int n) {
+    if constexpr (kRagged) {
+      u32x4 x;
+      __builtin_memcpy(&x, row + offset(mayBeLast, v, n), sizeof(x));
+      return x;
+    } else {
+      return reinterpret_cast<const u32x4 *>(row)[v];
+    }
+  }
+  static __device__ void store(u32x4 x, T *row, bool mayBeLast, int v, int n) {
+    if constexpr (kRagged)
+      __builtin_nontemporal_store(x, reinterpret_cast<Loose32 *>(row + offset(mayBeLast, v, n)));
+    else
+      __builtin_nontemporal_store(x, reinterpret_cast<u32x4 *>(row) + v);
+  }
+  // element e of vector v belongs to the statistics
+  static __device__ bool counts(bool mayBeLast, int v, int e, int n) { return !kRagged || !mayBeLast || offset(true, v, n) + e >= v * VEC; }
+};
+
 // One group of LANES lanes owns one row: lane l holds vectors l, l+LANES, ...
-// (VPL of them, the last ones predicated off when the row is shorter; FULL
+// (VPL of them, the last ones predicated off when the row is shorter; kFull
 // says that the row fills all of them, which removes every predicate and with
 // it the branches that would sit between the loads).
-template <typename T, int LANES, int VPL, bool RESIDUAL, bool FULL>
+template <typename T, int LANES, int VPL, bool RESIDUAL, RowShape SHAPE>
 __global__ __launch_bounds__(256) void layernorm_rows_kernel(
     const T *__restrict__ input, const T *__restrict__ gamma, const T *__restrict__ beta, T *__restrict__ normed,
     int m, int nArg, int rowStep, float eps, const T *__restrict__ residual, T *__restrict__ sumOut) {
@@ -35,12 +69,14 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
   // gridDim, which would be a load from the kernarg segment.  A FULL row has a length the
   // instantiation knows.
   using Tr = ElemTraits<T>;
+  using Rows = RowVectors<T, SHAPE>;
+  constexpr bool FULL = SHAPE == RowShape::kFull;
   constexpr int VEC = Tr::kVec; // elements per 16-byte vector
   constexpr int GROUPS = 256 / LANES;
   const int n = FULL ? LANES * VPL * VEC : nArg;
   const int lane = threadIdx.x % LANES;
   const int group = threadIdx.x / LANES;
-  const int nvec = n / VEC;
+  const int nvec = Rows::count(n);
   const float inv_n = 1.0f / (float)n;
 
   // gamma and beta do not depend on the row: fetch them once, at the top, so that
@@ -48,19 +84,17 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
   // usually owns a single row and its run time is one chain of latencies) - but
   // behind the loads of the first row: loads return in order, and the row is what
   // the chain waits for first (fp32 (4096, 768): 4.46 -> 4.27 us).
-  const u32x4 *gv = reinterpret_cast<const u32x4 *>(gamma);
-  const u32x4 *bv = reinterpret_cast<const u32x4 *>(beta);
   u32x4 graw[VPL], braw[VPL];
   u32x4 raw[VPL], rawr[VPL];
   auto loadRow = [&](int row) {
-    const u32x4 *xv = reinterpret_cast<const u32x4 *>(input + (size_t)row * n);
-    const u32x4 *rv = RESIDUAL ? reinterpret_cast<const u32x4 *>(residual + (size_t)row * n) : nullptr;
+    const T *xr = input + (size_t)row * n;
+    const T *rr = RESIDUAL ? residual + (size_t)row * n : nullptr;
 #pragma unroll
     for (int k = 0; k < VPL; k++) {
       const int v = lane + k * LANES;
       if (FULL || v < nvec) {
-        raw[k] = xv[v];
-        if (RESIDUAL) rawr[k] = rv[v];
+        raw[k] = Rows::load(xr, k == VPL - 1, v, n);
+        if (RESIDUAL) rawr[k] = Rows::load(rr, k == VPL - 1, v, n);
       }
     }
   };
@@ -70,8 +104,8 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
   for (int k = 0; k < VPL; k++) {
     const int v = lane + k * LANES;
     if (FULL || v < nvec) {
-      graw[k] = gv[v];
-      braw[k] = bv[v];
+      graw[k] = Rows::load(gamma, k == VPL - 1, v, n);
+      braw[k] = Rows::load(beta, k == VPL - 1, v, n);
     }
   }
 
@@ -92,7 +126,7 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
           for (int e = 0; e < VEC; e++) x[k][e] += r[e];
         }
 #pragma unroll
-        for (int e = 0; e < VEC; e++) sum += x[k][e];
+        for (int e = 0; e < VEC; e++) sum += Rows::counts(k == VPL - 1, v, e, n) ? x[k][e] : 0.0f;
       } else {
 #pragma unroll
         for (int e = 0; e < VEC; e++) x[k][e] = 0.0f;
@@ -107,7 +141,7 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
       if (FULL || v < nvec) {
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
-          const float d = x[k][e] - mean;
+          const float d = Rows::counts(k == VPL - 1, v, e, n) ? x[k][e] - mean : 0.0f;
           sq += d * d;
         }
       }
@@ -118,8 +152,8 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
     // (4096, 768) 3.93 -> 3.80 us, (262144, 768) fp32 266 -> 263.5 us, the fp32 headline unchanged.
     const float rstd = __builtin_amdgcn_rsqf(var + eps);
 
-    u32x4 *yv = reinterpret_cast<u32x4 *>(normed + (size_t)row * n);
-    u32x4 *sv = (RESIDUAL && sumOut) ? reinterpret_cast<u32x4 *>(sumOut + (size_t)row * n) : nullptr;
+    T *yr = normed + (size_t)row * n;
+    T *sr = (RESIDUAL && sumOut) ? sumOut + (size_t)row * n : nullptr;
 #pragma unroll
     for (int k = 0; k < VPL; k++) {
       const int v = lane + k * LANES;
@@ -133,12 +167,12 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
           // un-rounded fp32 sums (reference dataflow, LayerNorm.cu:203-233).
           // (a caller that has no use for the sum passes no buffer for it)
           const u32x4 packed = Tr::pack(x[k]);
-          if (sv) __builtin_nontemporal_store(packed, sv + v);
+          if (sr) Rows::store(packed, sr, k == VPL - 1, v, n);
           Tr::unpack(packed, x[k]);
         }
 #pragma unroll
         for (int e = 0; e < VEC; e++) y[e] = (x[k][e] - mean) * rstd * g[e] + b[e];
-        __builtin_nontemporal_store(Tr::pack(y), yv + v);
+        Rows::store(Tr::pack(y), yr, k == VPL - 1, v, n);
       }
     }
   }
@@ -257,19 +291,19 @@ __global__ __launch_bounds__(256) void layernorm_cast_rows_kernel(const float *_
 // are used (holding them would double the registers of a wide row); with
 // ROWS = 2 a block works on two rows at a time, which halves that re-reading
 // and the barriers per row and keeps more loads in flight.
-template <typename T, int VPL, int ROWS, bool RESIDUAL, bool FULL>
+template <typename T, int VPL, int ROWS, bool RESIDUAL, RowShape SHAPE>
 __global__ __launch_bounds__(256) void layernorm_block_kernel(
     const T *__restrict__ input, const T *__restrict__ gamma, const T *__restrict__ beta, T *__restrict__ normed,
     int m, int nArg, int rowStep, float eps, const T *__restrict__ residual, T *__restrict__ sumOut) {
   using Tr = ElemTraits<T>;
+  using Rows = RowVectors<T, SHAPE>;
+  constexpr bool FULL = SHAPE == RowShape::kFull;
   constexpr int VEC = Tr::kVec;
   const int n = FULL ? 256 * VPL * VEC : nArg; // (arguments: as in layernorm_rows_kernel)
   __shared__ float partial[2][ROWS][4];
   const int t = threadIdx.x, wave = t / 64;
-  const int nvec = n / VEC;
+  const int nvec = Rows::count(n);
   const float inv_n = 1.0f / (float)n;
-  const u32x4 *gv = reinterpret_cast<const u32x4 *>(gamma);
-  const u32x4 *bv = reinterpret_cast<const u32x4 *>(beta);
 
   for (int row0 = blockIdx.x * ROWS; row0 < m; row0 += rowStep) {
     float x[ROWS][VPL][VEC];
@@ -280,14 +314,14 @@ __global__ __launch_bounds__(256) void layernorm_block_kernel(
       for (int r = 0; r < ROWS; r++) {
         // a row past the end re-reads the last row; its results are not stored
         const int row = row0 + r < m ? row0 + r : m - 1;
-        const u32x4 *xv = reinterpret_cast<const u32x4 *>(input + (size_t)row * n);
-        const u32x4 *rv = RESIDUAL ? reinterpret_cast<const u32x4 *>(residual + (size_t)row * n) : nullptr;
+        const T *xr = input + (size_t)row * n;
+        const T *rr = RESIDUAL ? residual + (size_t)row * n : nullptr;
 #pragma unroll
         for (int k = 0; k < VPL; k++) {
           const int v = t + k * 256;
           if (FULL || v < nvec) {
-            raw[r][k] = xv[v];
-            if (RESIDUAL) rawr[r][k] = rv[v];
+            raw[r][k] = Rows::load(xr, true, v, n);
+            if (RESIDUAL) rawr[r][k] = Rows::load(rr, true, v, n);
           }
         }
       }
@@ -306,7 +340,7 @@ __global__ __launch_bounds__(256) void layernorm_block_kernel(
               for (int e = 0; e < VEC; e++) x[r][k][e] += rr[e];
             }
 #pragma unroll
-            for (int e = 0; e < VEC; e++) sum[r] += x[r][k][e];
+            for (int e = 0; e < VEC; e++) sum[r] += Rows::counts(true, v, e, n) ? x[r][k][e] : 0.0f;
           } else {
 #pragma unroll
             for (int e = 0; e < VEC; e++) x[r][k][e] = 0.0f;
@@ -335,7 +369,7 @@ __global__ __launch_bounds__(256) void layernorm_block_kernel(
         if (FULL || v < nvec) {
 #pragma unroll
           for (int e = 0; e < VEC; e++) {
-            const float d = x[r][k][e] - mean[r];
+            const float d = Rows::counts(true, v, e, n) ? x[r][k][e] - mean[r] : 0.0f;
             sq[r] += d * d;
           }
         }
@@ -356,21 +390,20 @@ __global__ __launch_bounds__(256) void layernorm_block_kernel(
       const int v = t + k * 256;
       if (FULL || v < nvec) {
         float g[VEC], b[VEC];
-        Tr::unpack(gv[v], g);
-        Tr::unpack(bv[v], b);
+        Tr::unpack(Rows::load(gamma, true, v, n), g);
+        Tr::unpack(Rows::load(beta, true, v, n), b);
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
           if (row0 + r >= m) continue;
-          u32x4 *yv = reinterpret_cast<u32x4 *>(normed + (size_t)(row0 + r) * n);
           float y[VEC];
           if (RESIDUAL) { // rounded sum out, normalised value from the rounded sum (see above)
             const u32x4 packed = Tr::pack(x[r][k]);
-            if (sumOut) __builtin_nontemporal_store(packed, reinterpret_cast<u32x4 *>(sumOut + (size_t)(row0 + r) * n) + v);
+            if (sumOut) Rows::store(packed, sumOut + (size_t)(row0 + r) * n, true, v, n);
             Tr::unpack(packed, x[r][k]);
           }
 #pragma unroll
           for (int e = 0; e < VEC; e++) y[e] = (x[r][k][e] - mean[r]) * rstd[r] * g[e] + b[e];
-          __builtin_nontemporal_store(Tr::pack(y), yv + v);
+          Rows::store(Tr::pack(y), normed + (size_t)(row0 + r) * n, true, v, n);
         }
       }
     }
@@ -427,28 +460,29 @@ __global__ __launch_bounds__(256) void layernorm_general_kernel(
 }
 
 template <typename T, int LANES, int VPL, bool RESIDUAL>
-void launchRows(const T *input, const T *residual, const T *gamma, const T *beta, T *sumOut,
+void launchRows(bool ragged, const T *input, const T *residual, const T *gamma, const T *beta, T *sumOut,
                 T *normed, float eps, int m, int n, hipStream_t stream) {
   constexpr int GROUPS = 256 / LANES;
   int64_t blocks = ((int64_t)m + GROUPS - 1) / GROUPS;
   const int64_t cap = kMaxStreamBlocks;
   if (blocks > cap) blocks = cap;
-  if (n / ElemTraits<T>::kVec == LANES * VPL)
-    layernorm_rows_kernel<T, LANES, VPL, RESIDUAL, true><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(
-        input, gamma, beta, normed, m, n, (int)(blocks * GROUPS), eps, residual, sumOut);
-  else
-    layernorm_rows_kernel<T, LANES, VPL, RESIDUAL, false><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(
-        input, gamma, beta, normed, m, n, (int)(blocks * GROUPS), eps, residual, sumOut);
+#define MGPU_LN_ROWS(S)                                                                                                      \
+  layernorm_rows_kernel<T, LANES, VPL, RESIDUAL, RowShape::S><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>( \
+      input, gamma, beta, normed, m, n, (int)(blocks * GROUPS), eps, residual, sumOut)
+  if (ragged) MGPU_LN_ROWS(kRagged);
+  else if (n / ElemTraits<T>::kVec == LANES * VPL) MGPU_LN_ROWS(kFull);
+  else MGPU_LN_ROWS(kVectors);
+#undef MGPU_LN_ROWS
   MGPU_CHECK_LAUNCH("layernorm_rows_kernel");
 }
 
 template <typename T, int LANES, bool RESIDUAL>
-void dispatchVPL(int vpl, const T *input, const T *residual, const T *gamma, const T *beta,
+void dispatchVPL(int vpl, bool ragged, const T *input, const T *residual, const T *gamma, const T *beta,
                  T *sumOut, T *normed, float eps, int m, int n, hipStream_t stream) {
   switch (vpl) {
 #define MGPU_LN_CASE(V)                                                                          \
   case V:                                                                                        \
-    launchRows<T, LANES, V, RESIDUAL>(input, residual, gamma, beta, sumOut, normed, eps, m, n,   \
+    launchRows<T, LANES, V, RESIDUAL>(ragged, input, residual, gamma, beta, sumOut, normed, eps, m, n, \
                                       stream);                                                   \
     break;
     MGPU_LN_CASE(1)
@@ -469,20 +503,24 @@ template <typename T, bool RESIDUAL>
 void layerNormTyped(const T *input, const T *residual, const T *gamma, const T *beta, T *sumOut,
                     T *normed, float eps, int m, int n, hipStream_t stream) {
   constexpr int VEC = ElemTraits<T>::kVec;
-  const bool vectorOk = n % VEC == 0 && aligned16(input) && aligned16(gamma) && aligned16(beta) &&
-                        aligned16(normed) && (!RESIDUAL || (aligned16(residual) && aligned16(sumOut)));
-  const int nvec = n / VEC;
+  // Rows that are not whole aligned vectors go through the same kernels, ragged: fp16 (2051, 770) with
+  // residual 4.35 us against 7.0 in three scalar sweeps, fp32 (16384, 65) 3.0 against 10.4, (500, 8190) with
+  // residual 14.4 against 38.8.
+  const bool ragged = !(n % VEC == 0 && aligned16(input) && aligned16(gamma) && aligned16(beta) && aligned16(normed) &&
+                        (!RESIDUAL || (aligned16(residual) && aligned16(sumOut))));
+  const bool vectorOk = n >= VEC;
+  const int nvec = (n + VEC - 1) / VEC;
   if (vectorOk && nvec <= 64 * kMaxVPL) {
     // Smallest lane group that keeps at most 4 vectors per lane; wider rows
     // use the whole wavefront with up to kMaxVPL vectors per lane.
     if (nvec <= 16 * 4)
-      dispatchVPL<T, 16, RESIDUAL>((nvec + 15) / 16, input, residual, gamma, beta, sumOut, normed,
+      dispatchVPL<T, 16, RESIDUAL>((nvec + 15) / 16, ragged, input, residual, gamma, beta, sumOut, normed,
                                    eps, m, n, stream);
     else if (nvec <= 32 * 4)
-      dispatchVPL<T, 32, RESIDUAL>((nvec + 31) / 32, input, residual, gamma, beta, sumOut, normed,
+      dispatchVPL<T, 32, RESIDUAL>((nvec + 31) / 32, ragged, input, residual, gamma, beta, sumOut, normed,
                                    eps, m, n, stream);
     else
-      dispatchVPL<T, 64, RESIDUAL>((nvec + 63) / 64, input, residual, gamma, beta, sumOut, normed,
+      dispatchVPL<T, 64, RESIDUAL>((nvec + 63) / 64, ragged, input, residual, gamma, beta, sumOut, normed,
                                    eps, m, n, stream);
     return;
   }
@@ -498,21 +536,26 @@ void layerNormTyped(const T *input, const T *residual, const T *gamma, const T *
     const bool pairRows = m >= 2 && vpl * ElemTraits<T>::kVec <= 32;
     if (pairRows) blocks = (blocks + 1) / 2;
 #define MGPU_LN_BLOCK(V, R, F)                                                                    \
-  layernorm_block_kernel<T, V, R, RESIDUAL, F><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>( \
+  layernorm_block_kernel<T, V, R, RESIDUAL, RowShape::F><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>( \
       input, gamma, beta, normed, m, n, (int)(blocks * R), eps, residual, sumOut)
+#define MGPU_LN_SHAPES(V, R)                 \
+  if (ragged) MGPU_LN_BLOCK(V, R, kRagged);  \
+  else if (full) MGPU_LN_BLOCK(V, R, kFull); \
+  else MGPU_LN_BLOCK(V, R, kVectors)
     if (vpl == 4 && pairRows) {
-      if (full) MGPU_LN_BLOCK(4, 2, true); else MGPU_LN_BLOCK(4, 2, false);
+      MGPU_LN_SHAPES(4, 2);
     } else if (vpl == 4) {
-      if (full) MGPU_LN_BLOCK(4, 1, true); else MGPU_LN_BLOCK(4, 1, false);
+      MGPU_LN_SHAPES(4, 1);
     } else if (vpl == 8 && pairRows) {
-      if (full) MGPU_LN_BLOCK(8, 2, true); else MGPU_LN_BLOCK(8, 2, false);
+      MGPU_LN_SHAPES(8, 2);
     } else if (vpl == 8) {
-      if (full) MGPU_LN_BLOCK(8, 1, true); else MGPU_LN_BLOCK(8, 1, false);
+      MGPU_LN_SHAPES(8, 1);
     } else if (vpl == 12) {
-      if (full) MGPU_LN_BLOCK(12, 1, true); else MGPU_LN_BLOCK(12, 1, false);
+      MGPU_LN_SHAPES(12, 1);
     } else {
-      if (full) MGPU_LN_BLOCK(16, 1, true); else MGPU_LN_BLOCK(16, 1, false);
+      MGPU_LN_SHAPES(16, 1);
     }
+#undef MGPU_LN_SHAPES
 #undef MGPU_LN_BLOCK
     MGPU_CHECK_LAUNCH("layernorm_block_kernel");
     return;

@@ -178,3 +178,31 @@ def test_cast_layer_norm_refuses_other_widths(pkg, gpu):
         g = torch.zeros(n, device=gpu, dtype=torch.float16)
         with pytest.raises(pkg.MgpuError):
             pkg.cast_layer_norm(x, g, g)
+
+
+# ragged rows: the last vector overlaps the one before it by 0 .. VEC - 1 elements; lengths around one vector, around
+# what a lane group, a wavefront and a block hold, and rows and outputs that start off the 16-byte grid
+@pytest.mark.parametrize("m,n,shift", [(5, 8, 1), (6, 9, 0), (7, 15, 3), (300, 127, 0), (9, 128, 1), (9, 511, 0), (9, 513, 5),
+                                       (9, 1025, 0), (67, 770, 0), (5, 4095, 0), (4, 4096, 1), (4, 4097, 0), (3, 16383, 0),
+                                       (3, 16385, 0), (2, 32767, 0), (2, 32768, 7)])
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+def test_layernorm_ragged_rows(pkg, gpu, oracle, rng, dtype, m, n, shift):
+    import torch
+
+    def place(a):  # `a` on the device, `shift` elements into an allocation
+        flat = torch.full((a.size + shift,), 7.0, dtype=getattr(torch, dtype), device=gpu)
+        flat[shift:] = torch.from_numpy(a.ravel()).to(gpu)
+        return flat[shift:].view(*a.shape)
+
+    x, r = (rng.standard_normal((m, n)).astype(dtype) for _ in range(2))
+    g, b = params(rng, n, np.dtype(dtype).type)
+    dx, dr, dg, db = map(place, (x, r, g, b))
+    y = pkg.layer_norm(dx, dg, db).cpu().numpy().astype(np.float32)
+    s, z = (t.cpu().numpy().astype(np.float32) for t in pkg.add_residual_layer_norm(dx, dr, dg, db))
+    ry = oracle.layernorm(x, g, b)
+    rs, rz = oracle.add_residual_layernorm(x, r, g, b)
+    tol = ulp16 if dtype == "float16" else lambda ref: 1e-5 * np.abs(ref) + 4e-6
+    assert np.all(np.abs(y - ry) <= tol(ry))
+    assert np.all(np.abs(z - rz) <= tol(rz))
+    assert np.array_equal(s, rs)
+    assert np.array_equal(dx.cpu().numpy(), x) and np.array_equal(dr.cpu().numpy(), r)  # (the inputs are whole)
