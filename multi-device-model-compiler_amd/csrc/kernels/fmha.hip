@@ -1,5 +1,6 @@
 // Launcher of the fused multi-head attention kernel (fmha_kernel.hpp): picks the tile
-// geometry and the instantiation for a head size and a mask, checks the operands.
+// geometry and the instantiation for a head size and a mask, checks the operands.  Launches that would leave most of
+// the chip idle go to fmha_split.hip.
 //
 // Replaces the dispatcher of the reference's cubin kernels, FusedMHARunnerFP16v2
 // (3rdparty/trt_fused_multihead_attention/qkvToContext.cu:162-199,306-315;
@@ -97,9 +98,10 @@ void fusedMHAChecked(DType dt, const void *qkv, const int32_t *seqlens, const in
   if (!aligned16(qkv) || !aligned16(out)) fail("fusedMHA: qkv and out must be 16-byte aligned");
   if (!(scale > 0.0f) || !(scale < INFINITY)) fail("fusedMHA: softmax scale must be positive and finite");
   if ((int64_t)S * 3 * H * D * 2 > 0x7fffffffLL) fail("fusedMHA: one sequence of QKV must stay below 2 GiB");
+  if (dt != DType::F16 && dt != DType::BF16) fail("fusedMHA: element type must be fp16 or bf16");
+  if (fusedMHASplitKeys(dt, qkv, seqlens, cuSeqlens, out, B, S, H, D, scale, causal, stream)) return;
   if (dt == DType::F16) launchForHeadDim<_Float16>(qkv, seqlens, cuSeqlens, out, B, S, H, D, scale, causal, stream);
-  else if (dt == DType::BF16) launchForHeadDim<bf16_t>(qkv, seqlens, cuSeqlens, out, B, S, H, D, scale, causal, stream);
-  else fail("fusedMHA: element type must be fp16 or bf16");
+  else launchForHeadDim<bf16_t>(qkv, seqlens, cuSeqlens, out, B, S, H, D, scale, causal, stream);
 }
 } // namespace
 

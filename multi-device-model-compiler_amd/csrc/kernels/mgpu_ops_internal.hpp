@@ -33,6 +33,10 @@ void fusedMHA(DType dt, const void *qkv, const int32_t *seqlens, void *out, int 
 // bounds the longest sequence.
 void fusedMHACuSeqlens(DType dt, const void *qkv, const int32_t *cuSeqlens, void *out, int B, int maxS, int H,
                        int D, float scale, bool causal, hipStream_t stream);
+// The kernel whose wavefronts split the keys (fmha_split.hip), on operands that fusedMHA has checked; false, and nothing
+// launched, where its rule leaves the call to the 128-query kernel.
+bool fusedMHASplitKeys(DType dt, const void *qkv, const int32_t *seqlens, const int32_t *cuSeqlens, void *out, int B, int S,
+                       int H, int D, float scale, bool causal, hipStream_t stream);
 
 void castF32ToF16(void *dst, const float *src, size_t size, hipStream_t stream);
 void castF16ToF32(float *dst, const void *src, size_t size, hipStream_t stream);
