@@ -289,6 +289,44 @@ bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias
          chooseKernel(dt, aligned, aligned, aligned, nullptr, aligned, M, N, K, hasBias, act, hasResidual, true) == Served::Library;
 }
 
+// Splitting pays where a product has so few tiles that most CUs idle behind a long reduction: the layers' projection and
+// second FFN product at a few to some 2000 tokens.  Estimates as in chooseKernel, plus 2 us and the planes' way through
+// the caches (written and read at about 5 TB/s) in place of the product's: 77 x 768 x 3072 9.3 us whole, 6.1 in three
+// parts; 1368 x 768 x 3072 26 against 15.5, its LayerNorm 4.0 against 4.7.  Where the estimates differ by less than a
+// tenth the product stays whole: 20 x 256 x 1024 (layer 23.2 us against 24.3 split) and 2048 x 768 x 3072 (80.6 / 81.7).
+PartialPlan gemmPartialPlan(const void *in, const void *weight, int64_t M, int64_t N, int64_t K, bool weightKMajor) {
+  PartialPlan best;
+  if (forcedKernel() || weightKMajor || K < 512) return best;
+  const Served whole = chooseKernel(DType::F16, in, weight, weight, nullptr, weight, M, N, K, true, ACT_NONE, false, false);
+  double bestCost;
+  if (whole == Served::Mfma) bestCost = gemmMfmaCost(M, N, K, ACT_NONE);
+  else if (whole == Served::KSplit) (void)gemmKSplitBest(M, N, K, ACT_NONE, &bestCost);
+  else return best;
+  bestCost = 0.9 * bestCost;
+  const bool mfmaOk = gemmMfmaSupportsRagged(DType::F16, in, weight, nullptr, nullptr, weight, M, N, K);
+  const bool kSplitOk = gemmKSplitSupports(DType::F16, in, weight, nullptr, nullptr, weight, M, N, K);
+  for (int parts = 2; parts <= 4 && K / parts >= 256; parts++) {
+    const double planes = 2.0 + (double)M * (double)N * (8.0 * parts - 4.0) / 5e6;
+    if (mfmaOk && gemmMfmaPartialCost(M, N, K, parts) + planes < bestCost) {
+      bestCost = gemmMfmaPartialCost(M, N, K, parts) + planes;
+      best = PartialPlan{parts, true, KSplitTile::T32x32};
+    }
+    double cost;
+    const KSplitTile tile = gemmKSplitBest(M, N, K, ACT_NONE, &cost, parts);
+    if (kSplitOk && cost + planes < bestCost) {
+      bestCost = cost + planes;
+      best = PartialPlan{parts, false, tile};
+    }
+  }
+  return best;
+}
+
+void gemmPartialF16(const PartialPlan &plan, const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K,
+                    hipStream_t stream) {
+  if (plan.mfma) gemmMfmaPartialF16(in, weight, planes, M, N, K, plan.parts, stream);
+  else gemmKSplitPartialF16(in, weight, planes, M, N, K, plan.tile, plan.parts, stream);
+}
+
 void matmulEx(DType dt, const void *input, const void *weight, const void *bias, void *output,
               const void *residual, int64_t M, int64_t N, int64_t K, bool hasBias, int act,
               bool hasResidual, hipStream_t stream, bool weightKMajor) {

@@ -12,6 +12,9 @@
 //
 // MFMA formulation and operand reads are those of gemm_mfma.hip: the transposed product
 // out^T[n, m] = W^T[n, k] . in^T[k, m] with W^T through the transposing LDS read.
+//
+// PARTIAL: the blocks of grid row y take the y-th share of the reduction and write their fp32 sums to plane y of `out`
+// (float [gridDim.y][M][N]; partial_sums.hip adds the planes up and has the epilogue).
 #include "common.hpp"
 #include "mfma.hpp"
 #include "mgpu_ops_internal.hpp"
@@ -25,7 +28,7 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 
 constexpr int kSplit = 8; // wavefronts of a block
 
-template <typename T, int ACT, int MB, int NB, int RING, bool KMAJOR>
+template <typename T, int ACT, int MB, int NB, int RING, bool KMAJOR, bool PARTIAL = false>
 __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
                                                                  const uint16_t *__restrict__ bias, const uint16_t *residual, uint16_t *out,
                                                                  int M, int N, int K, int tilesM, int nblk) {
@@ -50,8 +53,12 @@ __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint1
   const int ks = __builtin_amdgcn_readfirstlane(tid / 64);
   const int l32 = lane % 32, hl = lane / 32;
 
-  const int chunks = (K + 31) / 32;
-  const int c0 = chunks * ks / KS, c1 = chunks * (ks + 1) / KS;
+  int chunks = (K + 31) / 32, firstChunk = 0;
+  if (PARTIAL) {
+    firstChunk = chunks * (int)blockIdx.y / (int)gridDim.y;
+    chunks = chunks * ((int)blockIdx.y + 1) / (int)gridDim.y - firstChunk;
+  }
+  const int c0 = firstChunk + chunks * ks / KS, c1 = firstChunk + chunks * (ks + 1) / KS;
 
   // ---- movers: per instruction 16 input rows of 64 bytes, or 1 KiB of weight rows.  Rows and columns past
   // the end are clamped to the last ones (their products are not stored), k past the end likewise (those
@@ -220,6 +227,10 @@ __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint1
     float4v x = *reinterpret_cast<const float4v *>(part);
 #pragma unroll
     for (int s = 1; s < KS; s++) x += *reinterpret_cast<const float4v *>(part + s * kWave);
+    if (PARTIAL) {
+      *reinterpret_cast<float4v *>(reinterpret_cast<float *>(out) + ((size_t)blockIdx.y * M + m) * N + n) = x;
+      continue;
+    }
     if (bias) {
       const v4 b = *reinterpret_cast<const v4 *>(bias + n);
 #pragma unroll
@@ -275,11 +286,11 @@ void launch(const void *in, const void *weight, const void *bias, const void *re
 // us of the variant on a shape, up to a constant all hand-written variants share: one tile per CU and round,
 // a fixed part (first loads, partial sums, epilogue) and the tile's operand bytes at the 55 GB/s a CU pulls.
 // (77 x 2304 x 768 32 x 32: 4.5 us; 77 x 3072 x 768 + GELU 32 x 64: 5.3; 300 x 3072 x 768 + GELU 64 x 64: 8.2.)
-KSplitTile gemmKSplitBest(int64_t M, int64_t N, int64_t K, int act, double *cost) {
+KSplitTile gemmKSplitBest(int64_t M, int64_t N, int64_t K, int act, double *cost, int parts) {
   auto costOf = [&](int bm, int bn, double fixed) {
-    const int64_t tiles = (M + bm - 1) / bm * ((N + bn - 1) / bn);
+    const int64_t tiles = (M + bm - 1) / bm * ((N + bn - 1) / bn) * parts;
     const int64_t rounds = (tiles + numComputeUnits() - 1) / numComputeUnits();
-    return (double)rounds * (fixed + (double)(bm + bn) * 2.0 * (double)K / 55e3);
+    return (double)rounds * (fixed + (double)(bm + bn) * 2.0 * (double)K / parts / 55e3);
   };
   const double c[3] = {costOf(32, 32, 1.8), costOf(32, 64, 1.9), costOf(64, 64, act == ACT_GELU ? 3.6 : 2.4)};
   const int best = c[0] <= c[1] && c[0] <= c[2] ? 0 : c[1] <= c[2] ? 1 : 2;
@@ -307,6 +318,25 @@ void gemmKSplit(DType dt, const void *in, const void *weight, const void *bias, 
     if (weightKMajor) launch<bf16_t, true>(in, weight, bias, residual, out, M, N, K, act, tile, stream);
     else launch<bf16_t, false>(in, weight, bias, residual, out, M, N, K, act, tile, stream);
   }
+}
+
+void gemmKSplitPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, KSplitTile tile, int parts,
+                          hipStream_t stream) {
+  if (!gemmKSplitSupports(DType::F16, in, weight, nullptr, nullptr, planes, M, N, K)) fail("gemmKSplitPartial: internal dispatch error");
+  const auto *a = static_cast<const uint16_t *>(in);
+  const auto *w = static_cast<const uint16_t *>(weight);
+  auto *o = reinterpret_cast<uint16_t *>(planes);
+  const int bm = tile == KSplitTile::T64x64 ? 64 : 32, bn = tile == KSplitTile::T32x32 ? 32 : 64;
+  const int tilesM = (int)((M + bm - 1) / bm), nblk = tilesM * (int)((N + bn - 1) / bn);
+  const dim3 grid((unsigned)nblk, (unsigned)parts), block(64 * kSplit);
+  const int m = (int)M, n = (int)N, k = (int)K;
+  if (tile == KSplitTile::T32x32)
+    gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 1, 4, false, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+  else if (tile == KSplitTile::T32x64)
+    gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 2, 3, false, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+  else
+    gemm_ksplit_kernel<_Float16, ACT_NONE, 2, 2, 2, false, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+  MGPU_CHECK_LAUNCH("gemm_ksplit_kernel");
 }
 
 } // namespace mgpu

@@ -69,9 +69,12 @@ __host__ __device__ constexpr int wSwz(int row) { return (row & 3) << 2; } // 16
 
 // T: element type; ACT: epilogue activation; BK: reduction step (32 or 64);
 // NB: tile width in 32-column blocks (4 or 3).
+// PARTIAL: the blocks of grid row y take the y-th share of the reduction and write their fp32 sums to plane y of `out`
+// (float [gridDim.y][M][N]; partial_sums.hip adds the planes up and has the epilogue).
+//
 // RAGGED: M is no multiple of 128 or N none of the tile width.  The tiles cover the shape; rows and
 // columns past the end are loaded from the last ones and not stored.
-template <typename T, int ACT, int BK, int NB, bool PAIRED, bool SPLIT, bool RAGGED>
+template <typename T, int ACT, int BK, int NB, bool PAIRED, bool SPLIT, bool RAGGED, bool PARTIAL = false>
 __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma_kernel(const uint16_t *__restrict__ in,
                                                                         const uint16_t *__restrict__ weight,
                                                                         const uint16_t *__restrict__ bias,
@@ -80,6 +83,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
   using M = Mma<T>;
   using v8 = typename M::v8;
   using v4 = typename M::v4;
+  static_assert(!PARTIAL || (SPLIT && RAGGED && ACT == ACT_NONE), "partial sums");
   static_assert((BK == 32 || BK == 64) && (NB == 4 || NB == 3) && (!PAIRED || BK == 32) && (!SPLIT || BK == 64),
                 "tile geometry");
   constexpr int kBN = 32 * NB;
@@ -141,6 +145,13 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
   // where its scalar operands are no longer scalar to the compiler.)
   const char *abase = reinterpret_cast<const char *>(in) + (size_t)m0 * K * 2;
   const char *wbase = reinterpret_cast<const char *>(weight) + (size_t)n0 * 2;
+  int nk = K / BK; // reduction steps
+  if (PARTIAL) {
+    const int first = nk * (int)blockIdx.y / (int)gridDim.y;
+    nk = nk * ((int)blockIdx.y + 1) / (int)gridDim.y - first;
+    abase += (size_t)first * kARow;
+    wbase += (size_t)first * BK * N * 2;
+  }
   const int rowsLeft = RAGGED ? M_ - m0 : kBM; // rows of the tile that exist
   auto memRow = [&](int row) { return RAGGED && row >= rowsLeft ? rowsLeft - 1 : row; };
   uint32_t aoff[NL], woff[NL];
@@ -204,7 +215,6 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
     for (int i = 0; i < 4; i++) dma16(aoffP[i], ag, adst + i * 1024);
   };
 
-  const int nk = K / BK;
   if (PAIRED) {
     issueWeights(0);
     issuePair(0);
@@ -344,6 +354,21 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
     }
     __syncthreads(); // the staging area below overlaps what the other wavefronts have just read
     if (khalf == 1) return;
+  }
+  if constexpr (PARTIAL) {
+    float *plane = reinterpret_cast<float *>(out) + (size_t)blockIdx.y * M_ * N;
+#pragma unroll
+    for (int nb = 0; nb < NBW; nb++)
+#pragma unroll
+      for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const int m = m0 + wm * (32 * MB) + 32 * mb + l32, n = n0 + wn * (32 * NBW) + 32 * nb + 8 * g + 4 * hl;
+          if (m < M_ && n < N)
+            *reinterpret_cast<float4v *>(plane + (size_t)m * N + n) = float4v{acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1],
+                                                                              acc[nb][mb][4 * g + 2], acc[nb][mb][4 * g + 3]};
+        }
+    return;
   }
   uint16_t *stage = reinterpret_cast<uint16_t *>(smem) + wave * (32 * MB * kOutStride);
   const int mw = m0 + wm * (32 * MB), nw = n0 + wn * (32 * NBW); // origin of the wavefront's part
@@ -507,6 +532,35 @@ double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act) {
   const double bytes = (double)(kBM + width) * 2.0 * (double)K;
   if (tiles <= cus) return (act == ACT_GELU ? 5.0 : 2.0) + bytes / 57e3;
   return 5.0 + (double)tiles / (double)cus * bytes / 52e3;
+}
+
+// The tile width and estimated us of gemmMfmaPartialF16; no width where its blocks are more than one round of the CUs.
+// (4 us dearer than a whole product of that length: more CUs pull at once, and the sums leave in fp32.  640 x 768 x 768
+// of 3072 in four parts 11.6 us, 1368 x 768 x 1024 in three 15.5.)
+static int partialWidth(int64_t M, int64_t N, int parts) {
+  const int64_t tilesM = (M + kBM - 1) / kBM * parts;
+  return tilesM * ((N + 95) / 96) <= numComputeUnits() ? 96 : tilesM * ((N + 127) / 128) <= numComputeUnits() ? 128 : 0;
+}
+
+double gemmMfmaPartialCost(int64_t M, int64_t N, int64_t K, int parts) {
+  const int width = partialWidth(M, N, parts);
+  return width && K % 64 == 0 ? 6.0 + (double)(kBM + width) * 2.0 * (double)K / parts / 57e3 : 1e30;
+}
+
+void gemmMfmaPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, int parts, hipStream_t stream) {
+  const int width = partialWidth(M, N, parts);
+  if (!gemmMfmaSupportsRagged(DType::F16, in, weight, nullptr, nullptr, planes, M, N, K) || !width || K % 64 || K / 64 < parts)
+    fail("gemmMfmaPartial: internal dispatch error");
+  const int tilesN = (int)((N + width - 1) / width), tilesM = (int)((M + kBM - 1) / kBM);
+  const dim3 grid((unsigned)(tilesM * tilesN), (unsigned)parts), block(512);
+  const auto *a = static_cast<const uint16_t *>(in);
+  const auto *w = static_cast<const uint16_t *>(weight);
+  auto *o = reinterpret_cast<uint16_t *>(planes);
+  if (width == 96)
+    gemm_mfma_kernel<_Float16, ACT_NONE, 64, 3, false, true, true, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else
+    gemm_mfma_kernel<_Float16, ACT_NONE, 64, 4, false, true, true, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  MGPU_CHECK_LAUNCH("gemm_mfma_kernel");
 }
 
 void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,

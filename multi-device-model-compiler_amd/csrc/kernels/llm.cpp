@@ -36,6 +36,7 @@
 // no such entry point.
 #include "common.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <mutex>
@@ -274,6 +275,21 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
   const size_t oF = arena.reserve(M * ffn * h);
   const size_t oW2 = arena.reserve(ffn * d * h), oB2 = arena.reserve(d * h);
   const size_t oOut = arena.reserve(M * d * h);
+  const int act = relu ? ACT_RELU : ACT_GELU;
+  const bool useCache = cacheIsOn() && !isCapturing(stream); // a capture neither allocates nor reads the cache's events
+  bool kMajor[kGemms]; // GEMM g gets a transposed copy of its weight
+  {
+    auto *prefers = useCache ? gemmPrefersKMajor : gemmWantsKMajorCast;
+    kMajor[0] = prefers(DType::F16, M, 3 * d, d, false, ACT_NONE, false);
+    kMajor[1] = prefers(DType::F16, M, d, d, true, ACT_NONE, false);
+    kMajor[2] = prefers(DType::F16, M, ffn, d, true, act, false);
+    kMajor[3] = prefers(DType::F16, M, d, ffn, true, ACT_NONE, norm_first);
+  }
+  // (the operands of both split products are slices of the arena: aligned)
+  const bool sumsOk = partialSumsSupports(nullptr, nullptr, nullptr, nullptr, output, M, d);
+  const PartialPlan projPlan = sumsOk ? gemmPartialPlan(nullptr, nullptr, M, d, d, kMajor[1]) : PartialPlan{};
+  const PartialPlan ffn2Plan = sumsOk ? gemmPartialPlan(nullptr, nullptr, M, d, ffn, kMajor[3]) : PartialPlan{};
+  const size_t oPlanes = arena.reserve((size_t)std::max(projPlan.parts, ffn2Plan.parts) * M * d * 4);
 
   arena.allocate(stream);
   // The seven weight and bias arrays in fp16: cast now, all in one launch, or - with the weight cache
@@ -290,16 +306,6 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
                     {ffn1_bias, ffn, 0, oB1, 2, nullptr},    {ffn2_weight, ffn, d, oW2, 3, nullptr},
                     {ffn2_bias, d, 0, oB2, 3, nullptr}};
   hipEvent_t cachedReady[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  bool kMajor[kGemms]; // GEMM g gets a transposed copy of its weight
-  const int act = relu ? ACT_RELU : ACT_GELU;
-  const bool useCache = cacheIsOn() && !isCapturing(stream); // a capture neither allocates nor reads the cache's events
-  {
-    auto *prefers = useCache ? gemmPrefersKMajor : gemmWantsKMajorCast;
-    kMajor[0] = prefers(DType::F16, M, 3 * d, d, false, ACT_NONE, false);
-    kMajor[1] = prefers(DType::F16, M, d, d, true, ACT_NONE, false);
-    kMajor[2] = prefers(DType::F16, M, ffn, d, true, act, false);
-    kMajor[3] = prefers(DType::F16, M, d, ffn, true, ACT_NONE, norm_first);
-  }
   if (useCache) {
     // (an array's first conversion runs on the side stream, behind what already sits on `stream`)
     std::lock_guard<std::mutex> lock(scratchMutex);
@@ -342,6 +348,18 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
     fillF16(arena.at(oBeta), d, 0.0f, stream);
   }
 
+  // LN(in . w + bias + residual), the rounded sum to sumOut when it is not null
+  auto productAddNorm = [&](const PartialPlan &plan, const void *in, const void *w, const void *bias, int64_t K, bool transposed,
+                            const void *residual, void *sumOut, void *out) {
+    if (plan.parts) {
+      gemmPartialF16(plan, in, w, arena.at<float>(oPlanes), M, d, K, stream);
+      partialSumsLayerNormF16(arena.at<float>(oPlanes), plan.parts, bias, residual, gamma, beta, sumOut, out, 1e-5f, M, d, stream);
+      return;
+    }
+    matmulEx(DType::F16, in, w, bias, arena.at(oProj), nullptr, M, d, K, true, ACT_NONE, false, stream, transposed);
+    layerNorm(DType::F16, arena.at(oProj), residual, gamma, beta, sumOut, out, 1e-5f, (int)M, (int)d, stream);
+  };
+
   if (norm_first) {
     // y = x + proj(attention(LN(x))), out = y + ffn(LN(y))
     // fp16 copy of the input (the residual of the second LayerNorm) and its
@@ -360,17 +378,19 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
              (int)heads, (int)(d_model / heads), 1.0f / sqrtf((float)(d_model / heads)), causal, stream);
 
     join(1);
-    matmulEx(DType::F16, arena.at(oLn), woH, boH, arena.at(oProj), nullptr, M, d,
-             d, true, ACT_NONE, false, stream, kMajor[1]);
-
-    layerNorm(DType::F16, arena.at(oProj), arena.at(oX), gamma, beta, arena.at(oY), arena.at(oLn), 1e-5f, (int)M,
-              (int)d, stream);
+    productAddNorm(projPlan, arena.at(oLn), woH, boH, d, kMajor[1], arena.at(oX), arena.at(oY), arena.at(oLn));
 
     join(2);
     matmulEx(DType::F16, arena.at(oLn), w1H, b1H, arena.at(oF), nullptr, M, ffn,
              d, true, relu ? ACT_RELU : ACT_GELU, false, stream, kMajor[2]);
 
     join(3);
+    if (ffn2Plan.parts) { // the fp32 result straight from the sums
+      gemmPartialF16(ffn2Plan, arena.at(oF), w2H, arena.at<float>(oPlanes), M, d, ffn, stream);
+      partialSumsF32(arena.at<float>(oPlanes), ffn2Plan.parts, b2H, arena.at(oY), output, M, d, stream);
+      arena.release(stream);
+      return;
+    }
     matmulEx(DType::F16, arena.at(oF), w2H, b2H, arena.at(oOut), arena.at(oY), M,
              d, ffn, true, ACT_NONE, true, stream, kMajor[3]);
   } else {
@@ -385,19 +405,13 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
     fusedMHA(DType::F16, arena.at(oQkv), nullptr, arena.at(oLn), (int)batch, (int)seq_len,
              (int)heads, (int)(d_model / heads), 1.0f / sqrtf((float)(d_model / heads)), causal, stream);
     join(1);
-    matmulEx(DType::F16, arena.at(oLn), woH, boH, arena.at(oProj), nullptr, M, d,
-             d, true, ACT_NONE, false, stream, kMajor[1]);
     // h (in oY) = LN(proj + x); the rounded sum is not needed again
-    layerNorm(DType::F16, arena.at(oProj), arena.at(oX), gamma, beta, nullptr, arena.at(oY), 1e-5f, (int)M,
-              (int)d, stream);
+    productAddNorm(projPlan, arena.at(oLn), woH, boH, d, kMajor[1], arena.at(oX), nullptr, arena.at(oY));
     join(2);
     matmulEx(DType::F16, arena.at(oY), w1H, b1H, arena.at(oF), nullptr, M, ffn,
              d, true, relu ? ACT_RELU : ACT_GELU, false, stream, kMajor[2]);
     join(3);
-    matmulEx(DType::F16, arena.at(oF), w2H, b2H, arena.at(oProj), nullptr, M,
-             d, ffn, true, ACT_NONE, false, stream, kMajor[3]);
-    layerNorm(DType::F16, arena.at(oProj), arena.at(oY), gamma, beta, nullptr, arena.at(oOut), 1e-5f, (int)M,
-              (int)d, stream);
+    productAddNorm(ffn2Plan, arena.at(oF), w2H, b2H, ffn, kMajor[3], arena.at(oY), nullptr, arena.at(oOut));
   }
 
   castF16ToF32(output, arena.at(oOut), M * d, stream);
@@ -425,6 +439,15 @@ void bertEncoderLayerF16(const void *x, const void *wqkv, const void *bqkv, cons
   const size_t oQkv = arena.reserve(M * 3 * d * h), oCtx = arena.reserve(M * d * h);
   const size_t oProj = arena.reserve(M * d * h);
   const size_t oH1 = arena.reserve(M * d * h), oF = arena.reserve(M * ffn * h);
+  // The products before the two LayerNorms, split over blocks where few tiles leave CUs idle.  (The weight cache's K-major
+  // copies are for the library: such a product stays whole.  The inputs are slices of the arena: aligned.)
+  const bool cached = cacheIsOn() && !isCapturing(stream);
+  auto planOf = [&](const void *w, const void *bias, const void *residual, const void *gamma, const void *beta, const void *to, int64_t K) {
+    if (!partialSumsSupports(bias, residual, gamma, beta, to, M, d)) return PartialPlan{};
+    return gemmPartialPlan(nullptr, w, M, d, K, cached && gemmPrefersKMajor(DType::F16, M, d, K, true, ACT_NONE, false));
+  };
+  const PartialPlan projPlan = planOf(wo, bo, x, gamma1, beta1, nullptr, d), ffn2Plan = planOf(w2, b2, nullptr, gamma2, beta2, out, ffn);
+  const size_t oPlanes = arena.reserve((size_t)std::max(projPlan.parts, ffn2Plan.parts) * M * d * 4);
   arena.allocate(stream);
 
   // With the weight cache on, a GEMM for which the library on a K-major weight is the fastest
@@ -453,17 +476,21 @@ void bertEncoderLayerF16(const void *x, const void *wqkv, const void *bqkv, cons
   matmulEx(DType::F16, x, wq.w, bqkv, arena.at(oQkv), nullptr, M, 3 * d, d, true, ACT_NONE, false, stream, wq.kMajor);
   fusedMHA(DType::F16, arena.at(oQkv), seqlens, arena.at(oCtx), (int)B, (int)S, (int)H, (int)(d / H),
            1.0f / sqrtf((float)(d / H)), false, stream);
-  matmulEx(DType::F16, arena.at(oCtx), wp.w, bo, arena.at(oProj), nullptr, M, d, d, true, ACT_NONE, false, stream,
-           wp.kMajor);
   // (nobody reads the rounded sums of this layer: they are not written)
-  layerNorm(DType::F16, arena.at(oProj), x, gamma1, beta1, nullptr, arena.at(oH1), eps,
-            (int)M, (int)d, stream);
+  auto productAddNorm = [&](const PartialPlan &plan, const void *in, const Weight &w, const void *bias, int64_t K, const void *residual,
+                            const void *gamma, const void *beta, void *to) {
+    if (plan.parts && !w.kMajor) {
+      gemmPartialF16(plan, in, w.w, arena.at<float>(oPlanes), M, d, K, stream);
+      partialSumsLayerNormF16(arena.at<float>(oPlanes), plan.parts, bias, residual, gamma, beta, nullptr, to, eps, M, d, stream);
+      return;
+    }
+    matmulEx(DType::F16, in, w.w, bias, arena.at(oProj), nullptr, M, d, K, true, ACT_NONE, false, stream, w.kMajor);
+    layerNorm(DType::F16, arena.at(oProj), residual, gamma, beta, nullptr, to, eps, (int)M, (int)d, stream);
+  };
+  productAddNorm(projPlan, arena.at(oCtx), wp, bo, d, x, gamma1, beta1, arena.at(oH1));
   matmulEx(DType::F16, arena.at(oH1), wf1.w, b1, arena.at(oF), nullptr, M, ffn, d, true, ACT_GELU, false, stream,
            wf1.kMajor);
-  matmulEx(DType::F16, arena.at(oF), wf2.w, b2, arena.at(oProj), nullptr, M, d, ffn, true, ACT_NONE, false, stream,
-           wf2.kMajor);
-  layerNorm(DType::F16, arena.at(oProj), arena.at(oH1), gamma2, beta2, nullptr, out, eps,
-            (int)M, (int)d, stream);
+  productAddNorm(ffn2Plan, arena.at(oF), wf2, b2, ffn, arena.at(oH1), gamma2, beta2, out);
   arena.release(stream);
 }
 

@@ -97,11 +97,31 @@ void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bi
 // Small tiles, the reduction split over a block's wavefronts (gemm_ksplit.hip): fp16 / bf16, any M, N and K
 // multiples of 8.  gemmKSplitBest: the tile for a shape and its estimated us, to compare with the others.
 enum class KSplitTile { T32x32, T32x64, T64x64 };
-KSplitTile gemmKSplitBest(int64_t M, int64_t N, int64_t K, int act, double *cost);
+KSplitTile gemmKSplitBest(int64_t M, int64_t N, int64_t K, int act, double *cost, int parts = 1);
 bool gemmKSplitSupports(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
                         int64_t N, int64_t K);
 void gemmKSplit(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
                 int64_t K, int act, KSplitTile tile, bool weightKMajor, hipStream_t stream);
+// A GEMM whose reduction is split over blocks: `parts` fp32 planes [M, N] of partial sums (16-byte aligned), added up by
+// one of the kernels of partial_sums.hip.  gemmPartialPlan: parts = 0 where the shape is better served whole.
+struct PartialPlan {
+  int parts = 0;
+  bool mfma = false; // gemm_mfma, else gemm_ksplit on `tile`
+  KSplitTile tile = KSplitTile::T32x32;
+};
+PartialPlan gemmPartialPlan(const void *in, const void *weight, int64_t M, int64_t N, int64_t K, bool weightKMajor);
+void gemmPartialF16(const PartialPlan &plan, const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, hipStream_t stream);
+double gemmMfmaPartialCost(int64_t M, int64_t N, int64_t K, int parts);
+void gemmMfmaPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, int parts, hipStream_t stream);
+void gemmKSplitPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, KSplitTile tile, int parts,
+                          hipStream_t stream);
+// The sum of the planes + bias + residual: through a LayerNorm (fp16; the rounded sum to sumOut when not null), or as it
+// is, in fp32.  partialSumsSupports: widths and alignment.
+bool partialSumsSupports(const void *bias, const void *residual, const void *gamma, const void *beta, const void *out, int64_t M, int64_t N);
+void partialSumsLayerNormF16(const float *planes, int parts, const void *bias, const void *residual, const void *gamma, const void *beta,
+                             void *sumOut, void *out, float eps, int64_t M, int64_t N, hipStream_t stream);
+void partialSumsF32(const float *planes, int parts, const void *bias, const void *residual, float *out, int64_t M, int64_t N,
+                    hipStream_t stream);
 // fp32, any shape, for few tiles (gemm_f32_small.hip).
 void gemmF32Small(const float *in, const float *weight, const float *bias, const float *residual, float *out, int64_t M, int64_t N, int64_t K,
                   int act, hipStream_t stream);
