@@ -129,8 +129,11 @@ enum class Served { Library, Mfma, KSplit, F32Small };
 
 // The kernel for a call, decided without a lookup of the library's plans (a library call costs 6-7 us of
 // host time, a hand-written one a launch).
-//  * fp32: the small kernel up to 131072 tile-k (256 tiles of 32 x 32, 512 deep: 6.1 us against 6.7; 240 tiles
-//    768 deep 9.1 against 7.9; 1024 tiles 300 deep 17.9 against 14.9).
+//  * fp32: the small kernel by tiles of 32 x 32 times k, as its calls cross those of the library (us a call, library /
+//    small): 256 x 512 10.9 / 6.0, 768 x 256 10.9 / 8.6, 3072 x 64 12.3 / 11.0, 2160 x 129 17.3 / 13.3, 768 x 400 10.6 / 11.9, 3072 x
+//    129 16.9 / 17.5, 12288 x 32 20.3 / 28.2.  With a GELU, which is a pass of its own behind the library, further the shorter
+//    the reduction: 23500 x 64 95 / 76, 12288 x 129 64 / 60, 3072 x 256 31.4 / 27.5, 2160 x 400 33.8 / 30.8, 768 x 512 14.2 / 13.7, but
+//    23500 x 129 115 / 119, 3072 x 400 38.6 / 39.7, 2160 x 512 34.7 / 37.2.
 //  * fp16 / bf16: the aligned shapes of the table as it says; otherwise the cheaper of gemm_mfma and
 //    gemm_ksplit by their estimates, as long as it is no large problem, where the library is ahead: more than
 //    400 tiles of 128 x 128 without a GELU to fuse (5000 x 2304 x 768 24.5 us against 27, 2000 x 6144 x 2048
@@ -143,7 +146,8 @@ Served chooseKernel(DType dt, const void *in, const void *weight, const void *bi
   if (forcedKernel() == 1) return Served::Library;
   if (dt == DType::F32) {
     const int64_t tiles = (M + 31) / 32 * ((N + 31) / 32);
-    return !forcedKernel() && !weightKMajor && K <= 512 && tiles <= 131072 / K ? Served::F32Small : Served::Library;
+    const int64_t most = act != ACT_GELU ? 200000 : K <= 128 ? 1500000 : K <= 400 ? 800000 : 300000;
+    return !forcedKernel() && !weightKMajor && K <= 512 && tiles <= most / K ? Served::F32Small : Served::Library;
   }
   const bool kSplitOk = gemmKSplitSupports(dt, in, weight, bias, residual, out, M, N, K);
   double kSplitCost = 0.0;

@@ -77,3 +77,19 @@ def test_rows_and_columns_outside_the_shape_are_neither_read_nor_written(pkg, gp
         ref = x.double() @ w.double() + r.double()
         assert torch.all((out.double() - ref).abs() <= 2e-3 * ref.abs() + 0.03 if dt == torch.float16 else (out.double() - ref).abs() < 1e-4)
         assert torch.isnan(big[:2048]).all() and torch.isnan(big[2048 + M * N:]).all()
+
+
+@pytest.mark.parametrize("M,K,N,act,residual", [
+    (1000, 250, 768, 0, True),      # 768 tiles, just short of the line without a GELU, K no multiple of a step
+    (2301, 33, 2600, 1, False),     # many tiles of a short reduction, cut on both sides
+    (6000, 127, 1990, 2, False),    # 11 844 tiles in front of a GELU
+    (1136, 400, 1700, 2, False),
+])
+def test_matmul_ex_f32_up_to_the_library(pkg, gpu, M, K, N, act, residual):
+    import torch
+    g = torch.Generator(device=gpu).manual_seed(K)
+    x, w, b, r = [torch.randn(*s, device=gpu, generator=g) for s in ((M, K), (K, N), (N,), (M, N))]
+    ref = x.double() @ w.double() + b
+    ref = ref + r if residual else ref.relu() if act == 1 else torch.nn.functional.gelu(ref) if act == 2 else ref
+    err = (pkg.matmul_ex(x, w, b, r if residual else None, act=act).double() - ref).abs().max().item()
+    assert err <= 2e-7 * K + 2e-6 * K ** 0.5, err  # the bound of the small shapes above
