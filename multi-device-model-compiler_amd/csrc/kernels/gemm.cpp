@@ -130,8 +130,8 @@ enum class Served { Library, Mfma, KSplit, F32Small };
 // The kernel for a call, decided without a lookup of the library's plans (a library call costs 6-7 us of
 // host time, a hand-written one a launch).
 //  * fp32: the small kernel by tiles of 32 x 32 times k, as its calls cross those of the library (us a call, library /
-//    small): 256 x 512 10.9 / 6.0, 768 x 256 10.9 / 8.6, 3072 x 64 12.3 / 11.0, 2160 x 129 17.3 / 13.3, 768 x 400 10.6 / 11.9, 3072 x
-//    129 16.9 / 17.5, 12288 x 32 20.3 / 28.2.  With a GELU, which is a pass of its own behind the library, further the shorter
+//    small: 256 x 512 10.9 / 6.0, 768 x 256 10.9 / 8.6, 3072 x 64 12.3 / 11.0, 2160 x 129 17.3 / 13.3, 768 x 400 10.6 / 11.9, 3072 x
+//    129 16.9 / 17.5, 12288 x 32 20.3 / 28.2; 7 x 768 23.9 / 6.6, 256 x 768 14.5 / 7.8, 128 x 1024 10.1 / 8.7, 7 x 1536 10.0 / 11.0).  With a GELU, which is a pass of its own behind the library, further the shorter
 //    the reduction: 23500 x 64 95 / 76, 12288 x 129 64 / 60, 3072 x 256 31.4 / 27.5, 2160 x 400 33.8 / 30.8, 768 x 512 14.2 / 13.7, but
 //    23500 x 129 115 / 119, 3072 x 400 38.6 / 39.7, 2160 x 512 34.7 / 37.2.
 //  * fp16 / bf16: the aligned shapes of the table as it says; otherwise the cheaper of gemm_mfma and
@@ -139,22 +139,25 @@ enum class Served { Library, Mfma, KSplit, F32Small };
 //    400 tiles of 128 x 128 without a GELU to fuse (5000 x 2304 x 768 24.5 us against 27, 2000 x 6144 x 2048
 //    53.5 against 59; below, 2500 x 2304 x 768 16.9 against 16.7, 1200 x 1024 x 4096 36.6 against 31.7, 600 x 768 x
 //    768 7.5 against 5.4) - except for aligned shapes that the rule above gives to gemm_mfma.
-//  * K-major weights: gemm_ksplit while its tiles are at most one round of the CUs (beyond, the library, for
-//    which the layout was made).
+//  * K-major weights: gemm_ksplit while its tiles are at most one round of the CUs, two of a reduction up to 512
+//    deep (us a call, library / gemm_ksplit, tiles of 64 x 64 times k: 414 x 80 10.7 / 6.9, 512 x 256 11.1 / 8.0, 512 x 384
+//    10.6 / 9.9, 414 x 512 11.1 / 10.6, but 414 x 768 10.5 / 12.8 and 1424 x 64 11.2 / 17.9); beyond, the library, for
+//    which the layout was made.
 Served chooseKernel(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
                     int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor) {
   if (forcedKernel() == 1) return Served::Library;
   if (dt == DType::F32) {
     const int64_t tiles = (M + 31) / 32 * ((N + 31) / 32);
-    const int64_t most = act != ACT_GELU ? 200000 : K <= 128 ? 1500000 : K <= 400 ? 800000 : 300000;
-    return !forcedKernel() && !weightKMajor && K <= 512 && tiles <= most / K ? Served::F32Small : Served::Library;
+    const int64_t most = act != ACT_GELU || K > 512 ? 200000 : K <= 128 ? 1500000 : K <= 400 ? 800000 : 300000;
+    return !forcedKernel() && !weightKMajor && K <= 1024 && tiles <= most / K ? Served::F32Small : Served::Library;
   }
   const bool kSplitOk = gemmKSplitSupports(dt, in, weight, bias, residual, out, M, N, K);
   double kSplitCost = 0.0;
   const KSplitTile tile = gemmKSplitBest(M, N, K, act, &kSplitCost);
   if (weightKMajor) {
     const int64_t bm = tile == KSplitTile::T64x64 ? 64 : 32, bn = tile == KSplitTile::T32x32 ? 32 : 64;
-    return kSplitOk && !forcedKernel() && (M + bm - 1) / bm * ((N + bn - 1) / bn) <= numComputeUnits() ? Served::KSplit : Served::Library;
+    const int64_t most = (K <= 512 ? 2 : 1) * (int64_t)numComputeUnits();
+    return kSplitOk && !forcedKernel() && (M + bm - 1) / bm * ((N + bn - 1) / bn) <= most ? Served::KSplit : Served::Library;
   }
   const bool mfmaOk = gemmMfmaSupportsRagged(dt, in, weight, bias, residual, out, M, N, K);
   if (forcedKernel() == 2) return mfmaShape(dt, M, N, K) && mfmaOk ? Served::Mfma : Served::Library;
@@ -287,10 +290,11 @@ bool gemmPrefersKMajor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, 
 }
 
 bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual) {
-  // Wherever the [K, N] weight would be the library's: its kernels for the other layout are ahead.
+  // Wherever the [K, N] weight would be the library's: its kernels for the other layout are ahead, and gemm_ksplit
+  // where it takes that layout of a short reduction.
   alignas(16) static const char aligned[16] = {};
   return chooseKernel(dt, aligned, aligned, aligned, nullptr, aligned, M, N, K, hasBias, act, hasResidual, false) == Served::Library &&
-         chooseKernel(dt, aligned, aligned, aligned, nullptr, aligned, M, N, K, hasBias, act, hasResidual, true) == Served::Library;
+         (K <= 512 || chooseKernel(dt, aligned, aligned, aligned, nullptr, aligned, M, N, K, hasBias, act, hasResidual, true) == Served::Library);
 }
 
 // Splitting pays where a product has so few tiles that most CUs idle behind a long reduction: the layers' projection and

@@ -84,6 +84,7 @@ def test_rows_and_columns_outside_the_shape_are_neither_read_nor_written(pkg, gp
     (2301, 33, 2600, 1, False),     # many tiles of a short reduction, cut on both sides
     (6000, 127, 1990, 2, False),    # 11 844 tiles in front of a GELU
     (1136, 400, 1700, 2, False),
+    (100, 1021, 1500, 2, False),    # the deepest reduction
 ])
 def test_matmul_ex_f32_up_to_the_library(pkg, gpu, M, K, N, act, residual):
     import torch
@@ -93,3 +94,16 @@ def test_matmul_ex_f32_up_to_the_library(pkg, gpu, M, K, N, act, residual):
     ref = ref + r if residual else ref.relu() if act == 1 else torch.nn.functional.gelu(ref) if act == 2 else ref
     err = (pkg.matmul_ex(x, w, b, r if residual else None, act=act).double() - ref).abs().max().item()
     assert err <= 2e-7 * K + 2e-6 * K ** 0.5, err  # the bound of the small shapes above
+
+
+@pytest.mark.parametrize("M,K,N", [(1145, 80, 1472), (1000, 504, 2040), (2048, 168, 1000)])
+def test_packed_weight_two_rounds_of_tiles(pkg, gpu, oracle, rng, M, K, N):
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    w = (rng.standard_normal((K, N)) / np.sqrt(K)).astype(np.float16)
+    b, r = rng.standard_normal(N).astype(np.float16), rng.standard_normal((M, N)).astype(np.float16)
+    tx, tw, tb, tr = [to_dev(t, gpu) for t in (x, w, b, r)]
+    packed = pkg.pack_weight(tw)
+    for kw, okw in epilogues(pkg, oracle, tb, b, tr, r):
+        ref = oracle.gemm(x, w, **okw)
+        got = pkg.matmul_ex(tx, packed, kernel="packed", **kw).cpu().numpy().astype(np.float32)
+        assert np.all(np.abs(got - ref) <= spacing_tol(ref, 10, 1e-3)), (sorted(kw), np.abs(got - ref).max())
