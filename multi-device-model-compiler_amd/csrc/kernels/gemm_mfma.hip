@@ -1,9 +1,8 @@
 // fp16 / bf16 GEMM with the bias, activation and residual epilogue fused, on
 // gfx950 MFMA: out[M,N] = act(in[M,K] . W[K,N] + bias[N]) (+ residual[M,N]).
 //
-// One of the two ways mgpuMatmulEx<half> (lib/Kernels/GPU/Ops.cu:134-234) is
-// served; the other is the library GEMM in gemm.cpp, and gemm.cpp times both
-// on the first use of a shape.  This kernel exists for the shapes of a
+// One of the ways mgpuMatmulEx<half> (lib/Kernels/GPU/Ops.cu:134-234) is
+// served; gemm.cpp has the others and the rule that chooses.  This kernel exists for the shapes of a
 // transformer layer at a few thousand tokens (M = 4096, N and K between 768
 // and 3072), where a GEMM is a few hundred 128x128 tiles - one to three per
 // CU - and the time goes to ramp-up, tail and the epilogue rather than to a
