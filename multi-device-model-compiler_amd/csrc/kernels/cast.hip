@@ -343,6 +343,9 @@ namespace mgpu {
 
 namespace {
 
+// As in the epilogues of the 16-bit GEMMs (Mma<T>::gelu).
+template <typename T> __device__ __forceinline__ float gelu16(float x) { return std::is_same<T, _Float16>::value ? gelu_poly(x) : gelu_erfc(x); }
+
 template <typename T>
 __global__ __launch_bounds__(256) void gelu_h_vec8_kernel(u32x4 *__restrict__ data, size_t n8) {
   const size_t stride = (size_t)gridDim.x * 256;
@@ -350,7 +353,7 @@ __global__ __launch_bounds__(256) void gelu_h_vec8_kernel(u32x4 *__restrict__ da
     float v[8];
     ElemTraits<T>::unpack(data[i], v);
 #pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = gelu_erfc(v[e]);
+    for (int e = 0; e < 8; e++) v[e] = gelu16<T>(v[e]);
     data[i] = ElemTraits<T>::pack(v);
   }
 }
@@ -363,7 +366,7 @@ __global__ __launch_bounds__(256) void gelu_scalar_kernel(T *__restrict__ data, 
   {
     const float x = ElemTraits<T>::toFloat(data[i]);
     // fp32 results keep the library erf; the 16-bit types take the same formula as their vector kernel
-    data[i] = ElemTraits<T>::fromFloat(sizeof(T) == 4 ? gelu_erf(x) : gelu_erfc(x));
+    data[i] = ElemTraits<T>::fromFloat(sizeof(T) == 4 ? gelu_erf(x) : gelu16<T>(x));
   }
 }
 

@@ -74,6 +74,29 @@ __device__ __forceinline__ float gelu_erfc(float x) {
   return x * (x > 0.0f ? 1.0f - halfErfc : halfErfc);
 }
 
+// The same function for fp16 results in fewer instructions: x * Phi(x) = max(x, 0) - |x| * Phi(-|x|), with log2 Phi(-a) as a
+// polynomial of degree 10 in a, fitted (weighted least squares, weights iterated towards the largest error) to erfc in double
+// over 0 .. 6: no reciprocal, no square, one exp2 - 17 issue slots where the form above takes 28, of which a whole tile's
+// worth stands exposed behind a GEMM (BERT-base layer of 4096 tokens 100.5 -> 99.6 us).  Beyond 6 the
+// second term is under half of the smallest fp16 number and is held there.  In fp32, before the rounding: largest relative
+// error over normal fp16 results 1.4e-6 (2.4e-6 above), root mean square over |x| < 3 1.05e-7 (1.5e-7); results that differ
+// from the correctly rounded one 0.007 % (0.010 %).  x + |x| rather than max, so that a NaN stays one.
+__device__ __forceinline__ float gelu_poly(float x) {
+  const float a = fminf(fabsf(x), 6.0f);
+  float p = -2.723218451e-08f;
+  p = fmaf(p, a, 7.944807976e-07f);
+  p = fmaf(p, a, -1.004298701e-05f);
+  p = fmaf(p, a, 6.978801684e-05f);
+  p = fmaf(p, a, -2.525362070e-04f);
+  p = fmaf(p, a, -6.444904284e-05f);
+  p = fmaf(p, a, 7.035285234e-03f);
+  p = fmaf(p, a, -5.250751600e-02f);
+  p = fmaf(p, a, -4.591967463e-01f);
+  p = fmaf(p, a, -1.151107430e+00f);
+  p = fmaf(p, a, -9.999999404e-01f);
+  return fmaf(-a, __builtin_amdgcn_exp2f(p), 0.5f * (x + fabsf(x)));
+}
+
 // ... and for fp32 results, by the library's erf.
 __device__ __forceinline__ float gelu_erf(float x) {
   return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));

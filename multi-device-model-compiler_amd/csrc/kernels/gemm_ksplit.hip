@@ -239,7 +239,7 @@ __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint1
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       if (ACT == ACT_RELU) x[i] = x[i] > 0.0f ? x[i] : 0.0f;
-      if (ACT == ACT_GELU) x[i] = gelu_erfc(x[i]);
+      if (ACT == ACT_GELU) x[i] = Mm::gelu(x[i]);
     }
     if (residual) {
       const v4 r = *reinterpret_cast<const v4 *>(residual + (size_t)m * N + n);

@@ -423,7 +423,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
           for (int i = 0; i < 4; i++) x[i] = x[i] > 0.0f ? x[i] : 0.0f;
         } else if (ACT == ACT_GELU) {
 #pragma unroll
-          for (int i = 0; i < 4; i++) x[i] = gelu_erfc(x[i]);
+          for (int i = 0; i < 4; i++) x[i] = M::gelu(x[i]);
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) x[i] += M::widen(rraw[g][mb][i]);

@@ -7,6 +7,7 @@
 // lane l column l % 32 and rows 8 * (i / 4) + 4 * (l / 32) + i % 4 for register i.
 #pragma once
 
+#include "common.hpp"
 #include "types.hpp"
 
 namespace mgpu {
@@ -30,6 +31,7 @@ template <> struct Mma<_Float16> {
   }
   __device__ static __forceinline__ _Float16 narrow(float f) { return (_Float16)f; }
   __device__ static __forceinline__ float widen(_Float16 h) { return (float)h; }
+  __device__ static __forceinline__ float gelu(float x) { return gelu_poly(x); }
   __device__ static __forceinline__ v4 readTr(const lds_u8 *p) {
     return __builtin_bit_cast(v4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((i16x4 __attribute__((address_space(3))) *)p));
   }
@@ -42,6 +44,7 @@ template <> struct Mma<bf16_t> {
   }
   __device__ static __forceinline__ __bf16 narrow(float f) { return (__bf16)f; }
   __device__ static __forceinline__ float widen(__bf16 h) { return (float)h; }
+  __device__ static __forceinline__ float gelu(float x) { return gelu_erfc(x); } // (bf16 has fp32's range: the tail counts)
   __device__ static __forceinline__ v4 readTr(const lds_u8 *p) {
     return __builtin_bit_cast(v4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((i16x4 __attribute__((address_space(3))) *)p));
   }

@@ -134,6 +134,28 @@ def test_gelu_erfc_form_tail(pkg, gpu, oracle):
     assert ulps.max() <= 1, ulps.max()
 
 
+@pytest.mark.parametrize("rows,kernel", [(128, "mfma"), (1, "auto")])
+def test_fused_gelu_over_every_fp16_value(pkg, gpu, rows, kernel):
+    """Every fp16 bit pattern as a bias: finite results within one unit in the last place of x * Phi(x) from erfc in
+    double; +inf stays, NaN stays NaN (-inf gives NaN or -0)."""
+    import math
+    import torch
+    bits = np.arange(65536, dtype=np.uint16)
+    vals = bits.view(np.float16)
+    x = torch.zeros((rows, 32), dtype=torch.float16, device=gpu)
+    w = torch.zeros((32, 65536), dtype=torch.float16, device=gpu)
+    got = pkg.matmul_ex(x, w, bias=to_dev(vals, gpu), act=pkg.ACT_GELU, kernel=kernel).cpu().numpy()[-1]
+    finite = np.isfinite(vals)
+    v = vals[finite].astype(np.float64)
+    want = (0.5 * v * np.array([math.erfc(-e / math.sqrt(2.0)) for e in v])).astype(np.float16)
+    ulps = np.abs(got[finite].view(np.int16).astype(np.int32) - want.view(np.int16).astype(np.int32))
+    # (+-0 for an underflowed result: one value, two patterns)
+    assert ulps[(got[finite] != 0) | (want != 0)].max() <= 1
+    assert np.isnan(got[np.isnan(vals)]).all() and np.isposinf(got[vals == np.inf]).all()
+    low = got[vals == -np.inf]
+    assert (np.isnan(low) | (low == 0)).all()
+
+
 def test_forced_kernel_choice_in_a_fresh_process(gpu):
     """MGPU_GEMM_KERNEL=mfma / =library fix the path behind mgpuMatmulExF16; both give
     the same matrix up to one fp16 spacing."""
