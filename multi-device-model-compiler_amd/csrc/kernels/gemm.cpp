@@ -11,10 +11,11 @@
 //  * GELU is applied by an exact-erf kernel after a bias-only epilogue, because
 //    the library's fused GELU is the tanh approximation;
 //  * a call only enqueues: which of the kernels serves a shape - the library or
-//    a hand-written one (gemm_mfma.hip, gemm_ksplit.hip, gemm_f32_small.hip) - comes
-//    from a table decided offline (gemm_table.inc, written by `bench.py --tune-gemm`
+//    a hand-written one (gemm_wide.hip, gemm_mfma.hip, gemm_ksplit.hip, gemm_f32_small.hip) -
+//    is a fixed rule: gemm_wide first, where it applies (wideWidth); for the rest a
+//    table decided offline (gemm_table.inc, written by `bench.py --tune-gemm`
 //    from measurements on an MI355X) and, for shapes the table does not hold,
-//    from a fixed rule; the library runs the heuristic's first algorithm.
+//    lines on the shape; the library runs the heuristic's first algorithm.
 //    MGPU_GEMM_KERNEL=library or =mfma in the environment overrides both.
 //    Nothing in this library measures anything: the tuner that writes the
 //    table lives with the benchmark's launch loops;
@@ -183,6 +184,23 @@ GemmKernel chooseKernel(DType dt, const void *in, const void *weight, const void
   return kSplitOk && kSplitCost < 1.2 * mfmaCost ? GemmKernel::KSplit : GemmKernel::Library;
 }
 
+// The width at which gemm_wide serves a call, 0 where it does not.  Beyond one round of 128 x 128 tiles it is ahead of
+// everything else - over 550 such shapes the library takes 1.19 to 1.38 times as long (by the number of tiles; never less
+// than 0.96), gemm_mfma 1.19 to 1.31 (us, library / gemm_mfma / gemm_wide: 4096 x 3072 x 768 + GELU 37 / 28.2 / 24.6, 4096 x
+// 6144 x 2048 107 / 109 / 88.5, 3000 x 2304 x 2048 36.6 / 36.6 / 27.4); up to one round by the estimates, all three of which
+// stand for tiles of their own shape (200 to 256 tiles: ahead of gemm_mfma on short reductions, whose loads it keeps deeper
+// in flight).  Fewer than 128 rows would leave more than half of every tile empty.
+int wideWidth(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M, int64_t N,
+              int64_t K, int act) {
+  if (forcedKernel() || M < 128 || !gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) return 0;
+  double cost, other = gemmMfmaCost(M, N, K, act);
+  const int width = gemmWideBest(M, N, K, act, residual != nullptr, &cost);
+  if (tiles128(M, N) > numComputeUnits()) return width;
+  double kSplitCost;
+  (void)gemmKSplitBest(M, N, K, act, &kSplitCost);
+  return cost < std::min(other, kSplitCost) ? width : 0;
+}
+
 using Key = std::tuple<int64_t, int64_t, int64_t, int, int, int, int, int>;
 std::map<Key, Plan> plans;
 
@@ -290,11 +308,17 @@ void gemmDeinit() {
 
 bool gemmPrefersKMajor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual) {
   if (forcedKernel()) return forcedKernel() == 1;
+  if (gemmWideWidth(dt, M, N, K, act, hasResidual)) return false;
   if (const TableEntry *e = tableRow(dt, M, N, K, hasBias, act, hasResidual)) return e->kMajorLibrary != 0;
   // Nobody measured the shape: the library's kernels for K-major weights were ahead of its
   // kernels for [K, N] weights at every shape measured, so the copy pays wherever the library
   // would serve the shape anyway.
   return !mfmaShape(dt, M, N, K) || (tiles128(M, N) > numComputeUnits() && (act == ACT_GELU ? libraryAhead(M, N, K, act, true) : K > 1024));
+}
+
+int gemmWideWidth(DType dt, int64_t M, int64_t N, int64_t K, int act, bool hasResidual) {
+  alignas(16) static const char aligned[16] = {};
+  return wideWidth(dt, aligned, aligned, aligned, hasResidual ? aligned : nullptr, aligned, M, N, K, act);
 }
 
 GemmKernel gemmKernelFor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor) {
@@ -322,7 +346,8 @@ PartialPlan gemmPartialPlan(const void *in, const void *weight, int64_t M, int64
   if (forcedKernel() || weightKMajor || K < 512) return best;
   const GemmKernel whole = chooseKernel(DType::F16, in, weight, weight, nullptr, weight, M, N, K, true, ACT_NONE, false, false);
   double bestCost;
-  if (whole == GemmKernel::Mfma) bestCost = gemmMfmaCost(M, N, K, ACT_NONE);
+  if (wideWidth(DType::F16, in, weight, weight, nullptr, weight, M, N, K, ACT_NONE)) (void)gemmWideBest(M, N, K, ACT_NONE, false, &bestCost);
+  else if (whole == GemmKernel::Mfma) bestCost = gemmMfmaCost(M, N, K, ACT_NONE);
   else if (whole == GemmKernel::KSplit) (void)gemmKSplitBest(M, N, K, ACT_NONE, &bestCost);
   else return best;
   bestCost = 0.9 * bestCost;
@@ -365,6 +390,11 @@ void matmulEx(DType dt, const void *input, const void *weight, const void *bias,
     fail("matmul: an activation cannot be combined with a residual");
 
   const void *b = hasBias ? bias : nullptr, *r = hasResidual ? residual : nullptr;
+  if (!weightKMajor)
+    if (const int width = wideWidth(dt, input, weight, b, r, output, M, N, K, act)) {
+      gemmWide(dt, input, weight, b, r, output, M, N, K, act, width, stream);
+      return;
+    }
   switch (chooseKernel(dt, input, weight, b, r, output, M, N, K, hasBias, act, hasResidual, weightKMajor)) {
   case GemmKernel::Mfma:
     gemmMfmaRagged(dt, input, weight, b, r, output, M, N, K, act, stream);

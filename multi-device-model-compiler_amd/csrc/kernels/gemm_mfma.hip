@@ -6,7 +6,8 @@
 // transformer layer at a few thousand tokens (M = 4096, N and K between 768
 // and 3072), where a GEMM is a few hundred 128x128 tiles - one to three per
 // CU - and the time goes to ramp-up, tail and the epilogue rather than to a
-// long steady state; and for the exact-erf GELU, which the library cannot fuse.
+// long steady state.  Beyond one tile per CU gemm_wide.hip has taken over wherever its
+// reduction steps of 64 fit; what is left here is one tile per CU and other depths.
 //
 // Work decomposition.  A 256-thread block (4 wavefronts) owns a 128 x 128 output
 // tile (wavefronts 2 x 2, each 64 x 64 as 2 x 2 accumulators of 32 x 32) or a
@@ -23,12 +24,7 @@
 // latency of a step behind other blocks, so it takes half as many, longer
 // steps, and wavefronts 4-7 cover the tile like 0-3 but take the upper half of
 // every step (all eight share the loads); the two sets of accumulators meet in
-// LDS before the epilogue (4096 x 768 x 3072: 35.2 -> 30.2 us).  With several tiles per CU
-// and K a multiple of 64 the input rows are fetched for two steps at a time
-// (two buffers of 128 rows x 128 bytes, the weight slices in a ring of two):
-// a 64-byte piece of a row is half a cache line, and fetched on its own it
-// costs the whole line on the way from L2 (loads alone: 18.3 us against 21.7
-// at 4096 x 3072 x 768).
+// LDS before the epilogue (4096 x 768 x 3072: 35.2 -> 30.2 us).
 //
 // MFMA formulation: the transposed product out^T[n, m] = W^T[n, k] . in^T[k, m],
 //   A operand = W^T: the weight slice sits in LDS row-major as in memory
@@ -74,7 +70,7 @@ __host__ __device__ constexpr int wSwz(int row) { return (row & 3) << 2; } // 16
 //
 // RAGGED: M is no multiple of 128 or N none of the tile width.  The tiles cover the shape; rows and
 // columns past the end are loaded from the last ones and not stored.
-template <typename T, int ACT, int BK, int NB, bool PAIRED, bool SPLIT, bool RAGGED, bool PARTIAL = false>
+template <typename T, int ACT, int BK, int NB, bool SPLIT, bool RAGGED, bool PARTIAL = false>
 __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma_kernel(const uint16_t *__restrict__ in,
                                                                         const uint16_t *__restrict__ weight,
                                                                         const uint16_t *__restrict__ bias,
@@ -84,8 +80,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
   using v8 = typename M::v8;
   using v4 = typename M::v4;
   static_assert(!PARTIAL || (SPLIT && RAGGED && ACT == ACT_NONE), "partial sums");
-  static_assert((BK == 32 || BK == 64) && (NB == 4 || NB == 3) && (!PAIRED || BK == 32) && (!SPLIT || BK == 64),
-                "tile geometry");
+  static_assert((BK == 32 || BK == 64) && (NB == 4 || NB == 3) && SPLIT == (BK == 64), "tile geometry");
   constexpr int kBN = 32 * NB;
   constexpr int kSlice = 256 * BK;                   // bytes of an input slice, and of a weight slice at full pitch
   constexpr int kARow = BK * 2;                      // bytes per row of the input slice: 64 / 128
@@ -99,10 +94,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
 
   // Ring of kRing stages, each an input slice followed by a weight slice;
   // reused as the output staging area at the end.
-  // PAIRED: two buffers of 16 KiB, each the input rows of two steps (128 rows of
-  // 128 bytes), then two weight slices of 8 KiB.
-  constexpr int kPairBytes = 16384, kWBase = 2 * kPairBytes;
-  constexpr int kLds = PAIRED ? kWBase + 2 * 8192 : kRing * 2 * kSlice;
+  constexpr int kLds = kRing * 2 * kSlice;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[kLds];
   static_assert(4 * 32 * MB * kOutStride * 2 <= kLds, "output staging must fit in the ring");
 
@@ -165,14 +157,6 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
     if (RAGGED && n0 + 8 * wchunk >= N) wchunk = (N - 8 - n0) / 8;
     woff[i] = (uint32_t)wrow * (uint32_t)N * 2u + (uint32_t)(wchunk * 16);
   }
-  // PAIRED: the input rows of two steps at once, 8 rows of 128 bytes per load
-  // instruction, four instructions per wavefront.
-  uint32_t aoffP[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int arow = 8 * (4 * wave + i) + lane / 8;
-    aoffP[i] = (uint32_t)memRow(arow) * (uint32_t)K * 2u + (uint32_t)(((lane % 8) ^ aSwz<64>(arow)) * 16);
-  }
   // Inline assembly keeps these loads out of the compiler's wait-count
   // bookkeeping, which would otherwise wait for every load in flight before
   // any later LDS read; completion is tracked by hand (2 * NL loads per stage
@@ -202,27 +186,9 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
     }
   };
 
-  auto issueWeights = [&](int kt) { // PAIRED: the weight slice of step kt
-    const uint32_t wdst = ldsBase + (uint32_t)(kWBase + (kt % 2) * 8192 + (2 * wave) * 1024);
-    const char *wg = wbase + (size_t)kt * 32 * N * 2;
 #pragma unroll
-    for (int i = 0; i < 2; i++) dma16(woff[i], wg, wdst + i * 1024);
-  };
-  auto issuePair = [&](int p) { // PAIRED: the input rows of steps 2p and 2p + 1
-    const uint32_t adst = ldsBase + (uint32_t)((p % 2) * kPairBytes + (4 * wave) * 1024);
-    const char *ag = abase + (size_t)p * 128;
-#pragma unroll
-    for (int i = 0; i < 4; i++) dma16(aoffP[i], ag, adst + i * 1024);
-  };
-
-  if (PAIRED) {
-    issueWeights(0);
-    issuePair(0);
-  } else {
-#pragma unroll
-    for (int t = 0; t < kRing - 1; t++)
-      if (t < nk) issueStage(t);
-  }
+  for (int t = 0; t < kRing - 1; t++)
+    if (t < nk) issueStage(t);
 
   // ---- operand addresses inside a stage ---------------------------------------
   // in^T: lane (row 32*MB*wm + 32mb + l32, k chunk 2c + hl) reads 16 bytes.
@@ -237,17 +203,6 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
   // W^T: as a source of the transposing read, lane L of a 16-lane group g points
   // at k row 8*hl + L/4 (+ 16c, + 4 for the upper k-slots) and the four columns
   // n = 32nb + 16*(g%2) + 4*(L%4) .. +3.
-  // PAIRED: row of a 128-byte pitch, k chunk 4 * (kt % 2) + 2c + hl of the pair's 8;
-  // the step's half is bit 2 of the chunk, i.e. bit 6 of the address, and passes
-  // through the XOR swizzle unchanged.
-  uint32_t afragP[MB][2];
-#pragma unroll
-  for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      const int row = wm * (32 * MB) + 32 * mb + l32;
-      afragP[mb][c] = (uint32_t)(row * 128 + (((2 * c + hl) ^ aSwz<64>(row)) * 16));
-    }
   uint32_t wfrag[NBW]; // relative to the weight slice
   {
     const int g = lane / 16, L = lane % 16, r = L % 4, j = L / 4;
@@ -267,34 +222,15 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
       for (int i = 0; i < 16; i++) acc[nb][mb][i] = 0.0f;
 
   for (int kt = 0; kt < nk; kt++) {
-    uint32_t aBase, wBase; // LDS addresses of this step's input rows and weight slice
-    if (PAIRED) {
-      // Issue order is: weights of step 1, pair 1, weights of step 2, weights of
-      // step 3, pair 2, ...  An even step needs its pair (issued two steps ago)
-      // and its weights (issued one step ago): everything in flight.  An odd step
-      // needs its weights only, issued just before the next pair: 4 loads may fly.
-      if ((kt & 1) == 0 || kt + 1 >= nk) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      __syncthreads();
-      if (kt + 1 < nk) issueWeights(kt + 1);
-      if ((kt & 1) == 0 && kt + 2 < nk) issuePair(kt / 2 + 1);
-      aBase = ldsBase + (uint32_t)(((kt / 2) % 2) * kPairBytes);
-      wBase = ldsBase + (uint32_t)(kWBase + (kt % 2) * 8192);
-    } else {
-      // The loads of stage kt (and of nothing later) must have landed; the barrier
-      // makes every wavefront's share visible and says that everybody is done
-      // with stage kt-1, which the next load overwrites.
-      if (kt + 1 < nk) {
-        if (NL == 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-      } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
-      __syncthreads();
-      if (kt + kRing - 1 < nk) issueStage(kt + kRing - 1);
-      aBase = ldsBase + (uint32_t)((kt % kRing) * (2 * kSlice));
-      wBase = aBase + kSlice;
-    }
+    // The loads of stage kt (and of nothing later) must have landed; the barrier
+    // makes every wavefront's share visible and says that everybody is done
+    // with stage kt-1, which the next load overwrites.
+    if (kt + 1 < nk) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (kt + kRing - 1 < nk) issueStage(kt + kRing - 1);
+    const uint32_t aBase = ldsBase + (uint32_t)((kt % kRing) * (2 * kSlice)); // LDS addresses of this step's input rows and weight slice
+    uint32_t wBase = aBase + kSlice;
 
     if (SPLIT) wBase += (uint32_t)khalf * (16 * NCW * kWRow); // this half's k-steps: 32 rows further down the weight slice
 #pragma unroll
@@ -303,8 +239,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
 #pragma unroll
       for (int mb = 0; mb < MB; mb++) {
         // SPLIT: the upper half's k-steps are chunk bit 2 of the input rows, which passes through the swizzle
-        const uint32_t off = PAIRED ? (afragP[mb][c & 1] ^ ((uint32_t)(kt & 1) << 6))
-                                    : SPLIT ? (afrag[mb][c] ^ ((uint32_t)khalf << 6)) : afrag[mb][c];
+        const uint32_t off = SPLIT ? (afrag[mb][c] ^ ((uint32_t)khalf << 6)) : afrag[mb][c];
         b[mb] = *reinterpret_cast<const v8 __attribute__((address_space(3))) *>((const lds_u8 *)(uintptr_t)(aBase + off));
       }
 #pragma unroll
@@ -450,29 +385,29 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
   }
 }
 
-template <typename T, int BK, int NB, bool PAIRED, bool SPLIT, bool RAGGED>
+template <typename T, int BK, int NB, bool RAGGED>
 void launchAct(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint16_t *r, uint16_t *o, int64_t M,
                int64_t N, int64_t K, int act, hipStream_t stream) {
   const int tilesN = (int)((N + 32 * NB - 1) / (32 * NB)), tilesM = (int)((M + kBM - 1) / kBM);
-  const dim3 grid((unsigned)(tilesM * tilesN)), block(SPLIT ? 512 : 256);
+  const dim3 grid((unsigned)(tilesM * tilesN)), block(BK == 64 ? 512 : 256);
   if (act == ACT_GELU)
-    gemm_mfma_kernel<T, ACT_GELU, BK, NB, PAIRED, SPLIT, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    gemm_mfma_kernel<T, ACT_GELU, BK, NB, BK == 64, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   else if (act == ACT_RELU)
-    gemm_mfma_kernel<T, ACT_RELU, BK, NB, PAIRED, SPLIT, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    gemm_mfma_kernel<T, ACT_RELU, BK, NB, BK == 64, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   else
-    gemm_mfma_kernel<T, ACT_NONE, BK, NB, PAIRED, SPLIT, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    gemm_mfma_kernel<T, ACT_NONE, BK, NB, BK == 64, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
 }
-template <typename T, int BK, int NB, bool PAIRED, bool SPLIT = false>
+template <typename T, int BK, int NB>
 void launchTile(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint16_t *r, uint16_t *o, int64_t M,
                 int64_t N, int64_t K, int act, hipStream_t stream) {
-  if (M % kBM || N % (32 * NB)) launchAct<T, BK, NB, PAIRED, SPLIT, true>(a, w, b, r, o, M, N, K, act, stream);
-  else launchAct<T, BK, NB, PAIRED, SPLIT, false>(a, w, b, r, o, M, N, K, act, stream);
+  if (M % kBM || N % (32 * NB)) launchAct<T, BK, NB, true>(a, w, b, r, o, M, N, K, act, stream);
+  else launchAct<T, BK, NB, false>(a, w, b, r, o, M, N, K, act, stream);
 }
 
 // Tile width: the one under which the busiest CU carries the fewest columns
 // (tiles are dealt evenly, so that CU holds ceil(tiles / CUs) of them); 128 on
-// a tie.  Reduction step: 64 when no CU gets a second tile; otherwise 32, with
-// the input rows fetched in pairs of steps when K allows.
+// a tie.  Reduction step: 64 when no CU gets a second tile; otherwise gemm_wide
+// where it goes, and steps of 32 where it does not.
 template <typename T>
 void launch(const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M,
             int64_t N, int64_t K, int act, hipStream_t stream) {
@@ -487,15 +422,17 @@ void launch(const void *in, const void *weight, const void *bias, const void *re
   const auto *b = static_cast<const uint16_t *>(bias);
   const auto *r = static_cast<const uint16_t *>(residual);
   auto *o = static_cast<uint16_t *>(out);
-  const bool paired = !deep && K % 64 == 0;
+  const DType dt = std::is_same<T, _Float16>::value ? DType::F16 : DType::BF16;
+  if (!deep && gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) {
+    double cost;
+    return gemmWide(dt, in, weight, bias, residual, out, M, N, K, act, gemmWideBest(M, N, K, act, residual != nullptr, &cost), stream);
+  }
   if (narrow) {
-    if (deep) launchTile<T, 64, 3, false, true>(a, w, b, r, o, M, N, K, act, stream);
-    else if (paired) launchTile<T, 32, 3, true>(a, w, b, r, o, M, N, K, act, stream);
-    else launchTile<T, 32, 3, false>(a, w, b, r, o, M, N, K, act, stream);
+    if (deep) launchTile<T, 64, 3>(a, w, b, r, o, M, N, K, act, stream);
+    else launchTile<T, 32, 3>(a, w, b, r, o, M, N, K, act, stream);
   } else {
-    if (deep) launchTile<T, 64, 4, false, true>(a, w, b, r, o, M, N, K, act, stream);
-    else if (paired) launchTile<T, 32, 4, true>(a, w, b, r, o, M, N, K, act, stream);
-    else launchTile<T, 32, 4, false>(a, w, b, r, o, M, N, K, act, stream);
+    if (deep) launchTile<T, 64, 4>(a, w, b, r, o, M, N, K, act, stream);
+    else launchTile<T, 32, 4>(a, w, b, r, o, M, N, K, act, stream);
   }
   MGPU_CHECK_LAUNCH("gemm_mfma_kernel");
 }
@@ -558,9 +495,9 @@ void gemmMfmaPartialF16(const void *in, const void *weight, float *planes, int64
   const auto *w = static_cast<const uint16_t *>(weight);
   auto *o = reinterpret_cast<uint16_t *>(planes);
   if (width == 96)
-    gemm_mfma_kernel<_Float16, ACT_NONE, 64, 3, false, true, true, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    gemm_mfma_kernel<_Float16, ACT_NONE, 64, 3, true, true, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   else
-    gemm_mfma_kernel<_Float16, ACT_NONE, 64, 4, false, true, true, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    gemm_mfma_kernel<_Float16, ACT_NONE, 64, 4, true, true, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_mfma_kernel");
 }
 

@@ -278,7 +278,10 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
   const bool useCache = cacheIsOn() && !isCapturing(stream); // a capture neither allocates nor reads the cache's events
   bool kMajor[kGemms]; // GEMM g gets a transposed copy of its weight
   {
-    auto *prefers = useCache ? gemmPrefersKMajor : gemmWantsKMajorCast;
+    auto prefers = [&](DType dt, int64_t m, int64_t n, int64_t k, bool bias, int activation, bool residual) {
+      if (useCache) return gemmPrefersKMajor(dt, m, n, k, bias, activation, residual);
+      return !gemmWideWidth(dt, m, n, k, activation, residual) && gemmWantsKMajorCast(dt, m, n, k, bias, activation, residual);
+    };
     kMajor[0] = prefers(DType::F16, M, 3 * d, d, false, ACT_NONE, false);
     kMajor[1] = prefers(DType::F16, M, d, d, true, ACT_NONE, false);
     kMajor[2] = prefers(DType::F16, M, ffn, d, true, act, false);

@@ -72,14 +72,16 @@ void gemmDeinit();
 void matmulEx(DType dt, const void *input, const void *weight, const void *bias, void *output,
               const void *residual, int64_t M, int64_t N, int64_t K, bool hasBias, int act,
               bool hasResidual, hipStream_t stream, bool weightKMajor = false);
-// Which kernel serves a product (K, N > 0; 16-byte aligned operands).
+// The width at which gemm_wide serves a product (K, N > 0; 16-byte aligned operands), 0 where it does not; and which of the
+// others serves it then.
+int gemmWideWidth(DType dt, int64_t M, int64_t N, int64_t K, int act, bool hasResidual);
 enum class GemmKernel { Library, Mfma, KSplit, F32Small };
 GemmKernel gemmKernelFor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor);
 // Should a caller that can keep a K-major copy of the weight hand that one to matmulEx for this
 // problem?  (The committed table, else: wherever the library would serve the shape.)
 bool gemmPrefersKMajor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual);
 // Would a caller that makes its fp16 weight anew on every call, in either layout at the same price, rather
-// have it K-major?
+// have it K-major (for a product that gemm_wide does not serve)?
 bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual);
 
 // Hand-written MFMA GEMM (gemm_mfma.hip): fp16 / bf16, M a multiple of 128, N of
@@ -96,6 +98,14 @@ bool gemmMfmaSupportsRagged(DType dt, const void *in, const void *weight, const 
 double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act);
 void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,
                     int64_t M, int64_t N, int64_t K, int act, hipStream_t stream);
+
+// Tiles of 256 rows, one block per CU (gemm_wide.hip): fp16 / bf16, any M, N a multiple of 8, K of 64 from 128 on.
+// width: 128, 192 or 256 columns; gemmWideBest: the width for a shape and its estimated us, on the scale of gemmKSplitBest.
+int gemmWideBest(int64_t M, int64_t N, int64_t K, int act, bool hasResidual, double *cost);
+bool gemmWideSupports(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
+                      int64_t N, int64_t K);
+void gemmWide(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
+              int64_t K, int act, int width, hipStream_t stream);
 
 // Small tiles, the reduction split over a block's wavefronts (gemm_ksplit.hip): fp16 / bf16, any M, N and K
 // multiples of 8.  gemmKSplitBest: the tile for a shape and its estimated us, to compare with the others.

@@ -1,0 +1,82 @@
+"""gemm_wide (csrc/kernels/gemm_wide.hip): every tile width, where tiles end inside the shape and where they fit, from the
+fewest reduction steps on, each epilogue, both types; nothing stored outside the output."""
+import ctypes
+
+import pytest
+
+from test_index_bounds import internal
+
+WIDE = "_ZN4mgpu8gemmWideENS_5DTypeEPKvS2_S2_S2_PvllliiP12ihipStream_t"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("width", [128, 192, 256])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8, 128),       # one row, one chunk of columns, no pass of the loop
+    (256, 768, 192),   # whole tiles of every width, one pass
+    (257, 520, 256),
+    (300, 1000, 320),  # two passes of the loop
+    (511, 248, 1088),
+    (2300, 136, 704),  # more tile rows than a group
+])
+def test_against_float64(pkg, gpu, dtype, width, M, N, K):
+    import torch
+    t, code, ulp = (torch.float16, 1, 2.0**-11) if dtype == "f16" else (torch.bfloat16, 2, 2.0**-8)
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    r = lambda *s: torch.randn(s, generator=g, device=gpu)
+    x, w, b, res = r(M, K).to(t), (r(K, N) / K**0.5).to(t), r(N).to(t), r(M, N).to(t)
+    wide = internal(pkg, WIDE, None, ctypes.c_int, *[ctypes.c_void_p] * 5, *[ctypes.c_int64] * 3, ctypes.c_int, ctypes.c_int, ctypes.c_void_p)
+    X, W = x.double().cpu(), w.double().cpu()
+    prod, size = X @ W, X.abs() @ W.abs()
+    B, R = b.double().cpu(), res.double().cpu()
+    for bias, act, residual in ((None, 0, None), (b, 1, None), (b, 2, None), (b, 0, res)):
+        out = torch.full((M + 2, N), 7.0, dtype=t, device=gpu)  # a row before and one behind
+        wide(code, x.data_ptr(), w.data_ptr(), bias.data_ptr() if bias is not None else None, residual.data_ptr() if residual is not None else None,
+             out[1:].data_ptr(), M, N, K, act, width, torch.cuda.current_stream().cuda_stream)
+        got = out.double().cpu()
+        ref = prod + (B if bias is not None else 0)
+        ref = ref.relu() if act == 1 else 0.5 * ref * torch.erfc(-ref / 2**0.5) if act == 2 else ref
+        ref = ref + R if residual is not None else ref
+        # one rounding of the result (and the smallest number), K + 2 fp32 roundings of partial sums no larger than |x||w| + |b|,
+        # through a GELU whose slope stays below 1.13 and whose own error is below 3e-6
+        bound = 1.05 * ulp * ref.abs() + 2.0**-25 + 1.13 * (K + 2) * 2.0**-24 * (size + B.abs()) + 3e-6 * ref.abs()
+        assert ((got[1:-1] - ref).abs() <= bound).all(), (act, ((got[1:-1] - ref).abs() / bound).max())
+        assert (got[0] == 7).all() and (got[-1] == 7).all()
+
+
+@pytest.mark.parametrize("M,N,K,act,residual,width", [
+    (4096, 3072, 768, 2, False, 192),    # a round of tiles of 192
+    (4096, 6144, 2048, 0, False, 192),
+    (8192, 8192, 8192, 0, False, 256),
+    (4096, 2048, 2048, 0, True, 128),
+    (2304, 2048, 2560, 0, False, 128),   # beyond one round of 128 x 128 tiles, however deep
+    (2049, 2048, 128, 0, False, None),   # ... whatever the width
+    (4096, 2048, 96, 0, False, 0),       # fewer steps than its loop is built for
+    (4096, 2048, 1056, 0, False, 0),     # not whole steps
+    (4096, 2044, 1024, 0, False, 0),
+    (127, 40000, 1024, 0, False, 0),
+    (4096, 768, 3072, 0, False, 0),      # up to one round: the estimates
+    (77, 768, 768, 0, False, 0),
+])
+def test_what_it_serves(pkg, M, N, K, act, residual, width):
+    served = internal(pkg, "_ZN4mgpu13gemmWideWidthENS_5DTypeElllib", ctypes.c_int, ctypes.c_int, *[ctypes.c_int64] * 3, ctypes.c_int, ctypes.c_bool)
+    for dtype in (1, 2):
+        got = served(dtype, M, N, K, act, residual)
+        assert got == width if width is not None else got in (128, 192, 256)
+    assert served(0, M, N, K, act, residual) == 0  # fp32
+
+
+def test_tiles_stay_inside_a_grid_and_rows_inside_an_int(pkg):
+    supports = internal(pkg, "_ZN4mgpu16gemmWideSupportsENS_5DTypeEPKvS2_S2_S2_S2_lll", ctypes.c_bool, ctypes.c_int,
+                        *[ctypes.c_void_p] * 5, *[ctypes.c_int64] * 3)
+
+    def ask(M, N, K, out=4096):
+        return supports(1, 4096, 4096, 4096, None, out, M, N, K)
+
+    assert ask(300, 104, 128) and not ask(300, 104, 128, out=4104)
+    for N in (8, 128, 136, 1024, 2**20):
+        for M in (2**24, 2**30, 2**31 - 256, 2**31 - 255, 2**31, 2**33 + 5):
+            if ask(M, N, 128):
+                assert -(-M // 256) * 256 < 2**31 and -(-M // 256) * -(-N // 128) * 512 < 2**32, (M, N)
+    assert ask(2**31 - 256, 8, 128) and not ask(2**31 - 255, 8, 128)
