@@ -186,19 +186,15 @@ GemmKernel chooseKernel(DType dt, const void *in, const void *weight, const void
 
 // The width at which gemm_wide serves a call, 0 where it does not.  Beyond one round of 128 x 128 tiles it is ahead of
 // everything else - over 550 such shapes the library takes 1.19 to 1.38 times as long (by the number of tiles; never less
-// than 0.96), gemm_mfma 1.19 to 1.31 (us, library / gemm_mfma / gemm_wide: 4096 x 3072 x 768 + GELU 37 / 28.2 / 24.6, 4096 x
-// 6144 x 2048 107 / 109 / 88.5, 3000 x 2304 x 2048 36.6 / 36.6 / 27.4); up to one round by the estimates, all three of which
-// stand for tiles of their own shape (200 to 256 tiles: ahead of gemm_mfma on short reductions, whose loads it keeps deeper
-// in flight).  Fewer than 128 rows would leave more than half of every tile empty.
+// than 0.96), gemm_mfma's paired schedule before it 1.19 to 1.31 (us, library / gemm_mfma / gemm_wide: 4096 x 3072 x 768 + GELU
+// 37 / 28.2 / 24.6, 4096 x 6144 x 2048 107 / 109 / 88.5, 3000 x 2304 x 2048 36.6 / 36.6 / 27.4).  Up to one round gemm_round's
+// smaller tiles are (609 shapes: gemm_wide the best of all in 14, by 8 % at most).  Fewer than 128 rows would leave more
+// than half of every tile empty.
 int wideWidth(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M, int64_t N,
               int64_t K, int act) {
-  if (forcedKernel() || M < 128 || !gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) return 0;
-  double cost, other = gemmMfmaCost(M, N, K, act);
-  const int width = gemmWideBest(M, N, K, act, residual != nullptr, &cost);
-  if (tiles128(M, N) > numComputeUnits()) return width;
-  double kSplitCost;
-  (void)gemmKSplitBest(M, N, K, act, &kSplitCost);
-  return cost < std::min(other, kSplitCost) ? width : 0;
+  if (forcedKernel() || M < 128 || tiles128(M, N) <= numComputeUnits() || !gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) return 0;
+  double cost;
+  return gemmWideBest(M, N, K, act, residual != nullptr, &cost);
 }
 
 using Key = std::tuple<int64_t, int64_t, int64_t, int, int, int, int, int>;
@@ -337,10 +333,11 @@ bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias
 }
 
 // Splitting pays where a product has so few tiles that most CUs idle behind a long reduction: the layers' projection and
-// second FFN product at a few to some 2000 tokens.  Estimates as in chooseKernel, plus 2 us and the planes' way through
-// the caches (written and read at about 5 TB/s) in place of the product's: 77 x 768 x 3072 9.3 us whole, 6.1 in three
-// parts; 1368 x 768 x 3072 26 against 15.5, its LayerNorm 4.0 against 4.7.  Where the estimates differ by less than a
-// tenth the product stays whole: 20 x 256 x 1024 (layer 23.2 us against 24.3 split) and 2048 x 768 x 3072 (80.6 / 81.7).
+// second FFN product at a few to some 2000 tokens.  Estimates as in chooseKernel, plus what writing the planes and reading
+// them in the LayerNorm behind costs over a product and its LayerNorm, fitted to 330 splits (7 % rms for gemm_mfma's, 12 % for
+// gemm_ksplit's; us, product + LayerNorm whole / split: 77 x 768 x 3072 11.6 / 8.7, 1024 x 768 x 3072 19.9 / 17.1, 1368 x 768 x
+// 3072 23.1 / 18.8, 2048 x 512 x 2048 18.7 / 15.5).  Where the estimates differ by less than a tenth the product stays whole
+// (1024 x 1024 x 2048 16.0 / 15.6): the choice is 1.7 % behind the best over 110 shapes, at worst 8 % behind the whole product.
 PartialPlan gemmPartialPlan(const void *in, const void *weight, int64_t M, int64_t N, int64_t K, bool weightKMajor) {
   PartialPlan best;
   if (forcedKernel() || weightKMajor || K < 512) return best;
@@ -354,15 +351,15 @@ PartialPlan gemmPartialPlan(const void *in, const void *weight, int64_t M, int64
   const bool mfmaOk = gemmMfmaSupportsRagged(DType::F16, in, weight, nullptr, nullptr, weight, M, N, K);
   const bool kSplitOk = gemmKSplitSupports(DType::F16, in, weight, nullptr, nullptr, weight, M, N, K);
   for (int parts = 2; parts <= 4 && K / parts >= 256; parts++) {
-    const double planes = 2.0 + (double)M * (double)N * (8.0 * parts - 4.0) / 5e6;
-    if (mfmaOk && gemmMfmaPartialCost(M, N, K, parts) + planes < bestCost) {
-      bestCost = gemmMfmaPartialCost(M, N, K, parts) + planes;
+    const double elements = (double)M * (double)N * parts, mfmaPlanes = 2.6e-6 * elements, kSplitPlanes = 0.6 + 1.2e-6 * elements;
+    if (mfmaOk && gemmMfmaPartialCost(M, N, K, parts) + mfmaPlanes < bestCost) {
+      bestCost = gemmMfmaPartialCost(M, N, K, parts) + mfmaPlanes;
       best = PartialPlan{parts, true, KSplitTile::T32x32};
     }
     double cost;
     const KSplitTile tile = gemmKSplitBest(M, N, K, ACT_NONE, &cost, parts);
-    if (kSplitOk && cost + planes < bestCost) {
-      bestCost = cost + planes;
+    if (kSplitOk && cost + kSplitPlanes < bestCost) {
+      bestCost = cost + kSplitPlanes;
       best = PartialPlan{parts, false, tile};
     }
   }

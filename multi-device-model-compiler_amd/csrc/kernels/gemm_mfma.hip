@@ -2,12 +2,9 @@
 // gfx950 MFMA: out[M,N] = act(in[M,K] . W[K,N] + bias[N]) (+ residual[M,N]).
 //
 // One of the ways mgpuMatmulEx<half> (lib/Kernels/GPU/Ops.cu:134-234) is
-// served; gemm.cpp has the others and the rule that chooses.  This kernel exists for the shapes of a
-// transformer layer at a few thousand tokens (M = 4096, N and K between 768
-// and 3072), where a GEMM is a few hundred 128x128 tiles - one to three per
-// CU - and the time goes to ramp-up, tail and the epilogue rather than to a
-// long steady state.  Beyond one tile per CU gemm_wide.hip has taken over wherever its
-// reduction steps of 64 fit; what is left here is one tile per CU and other depths.
+// served; gemm.cpp has the others and the rule that chooses.  This file has the launcher for 128-row tiles: at most one a
+// CU and a depth that is a multiple of 64 go to gemm_round.hip, more of them to gemm_wide.hip, and the kernel below is what
+// is left, depths that are an odd multiple of 32 (and one step of 64 over several tiles a CU).
 //
 // Work decomposition.  A 256-thread block (4 wavefronts) owns a 128 x 128 output
 // tile (wavefronts 2 x 2, each 64 x 64 as 2 x 2 accumulators of 32 x 32) or a
@@ -18,13 +15,7 @@
 // slice of the input (128 rows of 64 bytes) and a slice of the weight (32 rows
 // at a 256-byte pitch) travel HBM -> LDS directly (global_load_lds, 16 bytes per
 // lane) into a ring of three stages, two steps in flight behind the one
-// consumed; three blocks share a CU (48 KiB of LDS, < 128 VGPRs).  When there
-// is at most one tile per CU the step is 64 instead (96 KiB of LDS) and the
-// block has eight wavefronts: a lone block cannot hide the barrier and the LDS
-// latency of a step behind other blocks, so it takes half as many, longer
-// steps, and wavefronts 4-7 cover the tile like 0-3 but take the upper half of
-// every step (all eight share the loads); the two sets of accumulators meet in
-// LDS before the epilogue (4096 x 768 x 3072: 35.2 -> 30.2 us).
+// consumed; three blocks share a CU (48 KiB of LDS, < 128 VGPRs).
 //
 // MFMA formulation: the transposed product out^T[n, m] = W^T[n, k] . in^T[k, m],
 //   A operand = W^T: the weight slice sits in LDS row-major as in memory
@@ -51,27 +42,21 @@ namespace mgpu {
 
 namespace {
 
-typedef float float4v __attribute__((ext_vector_type(4)));
-
 constexpr int kBM = 128;       // rows of an output tile
+constexpr int kBK = 32;        // reduction step
 constexpr int kRing = 3;       // LDS ring depth
 constexpr int kWRow = 256;     // LDS pitch of a weight-slice row, bytes (128 columns, of which NB * 32 are loaded)
 
 // Chunk swizzles: the 16-byte chunk c of a row is kept at chunk c ^ swz(row).
-template <int BK> __host__ __device__ constexpr int aSwz(int row) {
-  return BK == 32 ? (row >> 2) & 3 : (row >> 1) & 7; // 4 or 8 chunks per row
-}
+__host__ __device__ constexpr int aSwz(int row) { return (row >> 2) & 3; }        // 4 chunks per row
 __host__ __device__ constexpr int wSwz(int row) { return (row & 3) << 2; } // 16 chunks per row
 
-// T: element type; ACT: epilogue activation; BK: reduction step (32 or 64);
-// NB: tile width in 32-column blocks (4 or 3).
-// PARTIAL: the blocks of grid row y take the y-th share of the reduction and write their fp32 sums to plane y of `out`
-// (float [gridDim.y][M][N]; partial_sums.hip adds the planes up and has the epilogue).
+// T: element type; ACT: epilogue activation; NB: tile width in 32-column blocks (4 or 3).
 //
 // RAGGED: M is no multiple of 128 or N none of the tile width.  The tiles cover the shape; rows and
 // columns past the end are loaded from the last ones and not stored.
-template <typename T, int ACT, int BK, int NB, bool SPLIT, bool RAGGED, bool PARTIAL = false>
-__global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma_kernel(const uint16_t *__restrict__ in,
+template <typename T, int ACT, int NB, bool RAGGED>
+__global__ __launch_bounds__(256, 3) void gemm_mfma_kernel(const uint16_t *__restrict__ in,
                                                                         const uint16_t *__restrict__ weight,
                                                                         const uint16_t *__restrict__ bias,
                                                                         const uint16_t *residual, uint16_t *out, int N,
@@ -79,15 +64,12 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
   using M = Mma<T>;
   using v8 = typename M::v8;
   using v4 = typename M::v4;
-  static_assert(!PARTIAL || (SPLIT && RAGGED && ACT == ACT_NONE), "partial sums");
-  static_assert((BK == 32 || BK == 64) && (NB == 4 || NB == 3) && SPLIT == (BK == 64), "tile geometry");
+  static_assert(NB == 4 || NB == 3, "tile geometry");
   constexpr int kBN = 32 * NB;
-  constexpr int kSlice = 256 * BK;                   // bytes of an input slice, and of a weight slice at full pitch
-  constexpr int kARow = BK * 2;                      // bytes per row of the input slice: 64 / 128
-  constexpr int NC = BK / 16;                        // MFMA k-steps per reduction step: 2 / 4
-  constexpr int NL = BK / 16 / (SPLIT ? 2 : 1);      // load instructions per wavefront and slice: 2 / 4 (2 when 8 wavefronts share them)
-  constexpr int NCW = NC / (SPLIT ? 2 : 1);          // MFMA k-steps a wavefront takes per reduction step
-  constexpr int CPR = BK / 8, RPI = 64 / CPR;        // input slice: chunks per row, rows per load instruction
+  constexpr int kSlice = 256 * kBK;                  // bytes of an input slice, and of a weight slice at full pitch
+  constexpr int kARow = kBK * 2;                     // bytes per row of the input slice
+  constexpr int NC = 2, NL = 2;                      // per reduction step: MFMA k-steps; load instructions a wavefront and slice
+  constexpr int CPR = kBK / 8, RPI = 64 / CPR;       // input slice: chunks per row, rows per load instruction
   constexpr int WN = NB == 4 ? 2 : 1, WM = 4 / WN;   // wavefront grid over the tile: 2 x 2 or 4 x 1
   constexpr int MB = 4 / WM, NBW = NB / WN;          // 32 x 32 accumulators per wavefront: MB x NBW = 2 x 2 or 1 x 3
   constexpr int kOutStride = 32 * NBW + 4;           // staging row stride of a wavefront's part, in elements
@@ -119,11 +101,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
 
   const int tid = threadIdx.x;
   const int lane = tid % 64;
-  // SPLIT: eight wavefronts; 0-3 and 4-7 cover the tile in the same way and take the
-  // lower and the upper half of every reduction step, all eight share the loads.
-  const int mover = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int khalf = SPLIT ? mover / 4 : 0;
-  const int wave = SPLIT ? mover % 4 : mover;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int l32 = lane % 32;
   const int hl = lane / 32;
   const int wm = wave / WN, wn = wave % WN; // the wavefront's part of the tile
@@ -137,52 +115,31 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
   // where its scalar operands are no longer scalar to the compiler.)
   const char *abase = reinterpret_cast<const char *>(in) + (size_t)m0 * K * 2;
   const char *wbase = reinterpret_cast<const char *>(weight) + (size_t)n0 * 2;
-  int nk = K / BK; // reduction steps
-  if (PARTIAL) {
-    const int first = nk * (int)blockIdx.y / (int)gridDim.y;
-    nk = nk * ((int)blockIdx.y + 1) / (int)gridDim.y - first;
-    abase += (size_t)first * kARow;
-    wbase += (size_t)first * BK * N * 2;
-  }
+  const int nk = K / kBK; // reduction steps
   const int rowsLeft = RAGGED ? M_ - m0 : kBM; // rows of the tile that exist
   auto memRow = [&](int row) { return RAGGED && row >= rowsLeft ? rowsLeft - 1 : row; };
   uint32_t aoff[NL], woff[NL];
 #pragma unroll
   for (int i = 0; i < NL; i++) {
-    const int arow = RPI * (NL * mover + i) + lane / CPR;
-    aoff[i] = (uint32_t)memRow(arow) * (uint32_t)K * 2u + (uint32_t)(((lane % CPR) ^ aSwz<BK>(arow)) * 16);
-    const int wrow = 4 * (NL * mover + i) + lane / 16;
+    const int arow = RPI * (NL * wave + i) + lane / CPR;
+    aoff[i] = (uint32_t)memRow(arow) * (uint32_t)K * 2u + (uint32_t)(((lane % CPR) ^ aSwz(arow)) * 16);
+    const int wrow = 4 * (NL * wave + i) + lane / 16;
     int wchunk = (lane % 16) ^ wSwz(wrow);
     if (wchunk >= 4 * NB) wchunk -= 4;
     if (RAGGED && n0 + 8 * wchunk >= N) wchunk = (N - 8 - n0) / 8;
     woff[i] = (uint32_t)wrow * (uint32_t)N * 2u + (uint32_t)(wchunk * 16);
   }
-  // Inline assembly keeps these loads out of the compiler's wait-count
-  // bookkeeping, which would otherwise wait for every load in flight before
-  // any later LDS read; completion is tracked by hand (2 * NL loads per stage
-  // and wavefront).
+  // (2 * NL loads per stage and wavefront, counted by hand)
   const uint32_t ldsBase = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) unsigned char *)smem);
-  // M0 is on the clobber list so that the statement counts as a definition of it
-  // (the compiler reserves M0 and notes that such a clobber is not saved and restored:
-  // nothing here needs it preserved).
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-  auto dma16 = [&](uint32_t voffset, const char *sbase, uint32_t ldsAddr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voffset), "s"(sbase), "s"(ldsAddr)
-                 : "memory", "m0");
-  };
-#pragma clang diagnostic pop
   auto issueStage = [&](int kt) {
-    const uint32_t adst = ldsBase + (uint32_t)((kt % kRing) * (2 * kSlice) + (NL * mover) * 1024);
+    const uint32_t adst = ldsBase + (uint32_t)((kt % kRing) * (2 * kSlice) + (NL * wave) * 1024);
     const uint32_t wdst = adst + kSlice;
     const char *ag = abase + (size_t)kt * kARow;
-    const char *wg = wbase + (size_t)kt * BK * N * 2;
+    const char *wg = wbase + (size_t)kt * kBK * N * 2;
 #pragma unroll
     for (int i = 0; i < NL; i++) {
-      dma16(aoff[i], ag, adst + i * 1024);
-      dma16(woff[i], wg, wdst + i * 1024);
+      ldsLoad16(aoff[i], ag, adst + i * 1024);
+      ldsLoad16(woff[i], wg, wdst + i * 1024);
     }
   };
 
@@ -198,7 +155,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
 #pragma unroll
     for (int c = 0; c < NC; c++) {
       const int row = wm * (32 * MB) + 32 * mb + l32;
-      afrag[mb][c] = (uint32_t)(row * kARow + (((2 * c + hl) ^ aSwz<BK>(row)) * 16));
+      afrag[mb][c] = (uint32_t)(row * kARow + (((2 * c + hl) ^ aSwz(row)) * 16));
     }
   // W^T: as a source of the transposing read, lane L of a 16-lane group g points
   // at k row 8*hl + L/4 (+ 16c, + 4 for the upper k-slots) and the four columns
@@ -230,18 +187,14 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
     __syncthreads();
     if (kt + kRing - 1 < nk) issueStage(kt + kRing - 1);
     const uint32_t aBase = ldsBase + (uint32_t)((kt % kRing) * (2 * kSlice)); // LDS addresses of this step's input rows and weight slice
-    uint32_t wBase = aBase + kSlice;
+    const uint32_t wBase = aBase + kSlice;
 
-    if (SPLIT) wBase += (uint32_t)khalf * (16 * NCW * kWRow); // this half's k-steps: 32 rows further down the weight slice
 #pragma unroll
-    for (int c = 0; c < NCW; c++) {
+    for (int c = 0; c < NC; c++) {
       v8 b[MB], a[NBW];
 #pragma unroll
-      for (int mb = 0; mb < MB; mb++) {
-        // SPLIT: the upper half's k-steps are chunk bit 2 of the input rows, which passes through the swizzle
-        const uint32_t off = SPLIT ? (afrag[mb][c] ^ ((uint32_t)khalf << 6)) : afrag[mb][c];
-        b[mb] = *reinterpret_cast<const v8 __attribute__((address_space(3))) *>((const lds_u8 *)(uintptr_t)(aBase + off));
-      }
+      for (int mb = 0; mb < MB; mb++)
+        b[mb] = *reinterpret_cast<const v8 __attribute__((address_space(3))) *>((const lds_u8 *)(uintptr_t)(aBase + afrag[mb][c]));
 #pragma unroll
       for (int nb = 0; nb < NBW; nb++) {
         const lds_u8 *p = (const lds_u8 *)(uintptr_t)(wBase + wfrag[nb]) + 16 * c * kWRow;
@@ -258,53 +211,6 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
 
   // ---- epilogue: bias, activation, residual; transpose through LDS; store ------
   __syncthreads(); // every wavefront is done reading the slices
-  if (SPLIT) {
-    // the upper half hands its accumulators to the lower half through LDS: 16
-    // bytes per lane and register group, consecutive lanes consecutive
-    float4v *red = reinterpret_cast<float4v *>(smem) + wave * (NBW * MB * 4 * 64);
-    if (khalf == 1) {
-#pragma unroll
-      for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-          for (int g = 0; g < 4; g++)
-            red[((nb * MB + mb) * 4 + g) * 64 + lane] = float4v{acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1],
-                                                               acc[nb][mb][4 * g + 2], acc[nb][mb][4 * g + 3]};
-    }
-    __syncthreads();
-    if (khalf == 0) {
-#pragma unroll
-      for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-          for (int g = 0; g < 4; g++) {
-            const float4v other = red[((nb * MB + mb) * 4 + g) * 64 + lane];
-            acc[nb][mb][4 * g] += other[0];
-            acc[nb][mb][4 * g + 1] += other[1];
-            acc[nb][mb][4 * g + 2] += other[2];
-            acc[nb][mb][4 * g + 3] += other[3];
-          }
-    }
-    __syncthreads(); // the staging area below overlaps what the other wavefronts have just read
-    if (khalf == 1) return;
-  }
-  if constexpr (PARTIAL) {
-    float *plane = reinterpret_cast<float *>(out) + (size_t)blockIdx.y * M_ * N;
-#pragma unroll
-    for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-      for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-          const int m = m0 + wm * (32 * MB) + 32 * mb + l32, n = n0 + wn * (32 * NBW) + 32 * nb + 8 * g + 4 * hl;
-          if (m < M_ && n < N)
-            *reinterpret_cast<float4v *>(plane + (size_t)m * N + n) = float4v{acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1],
-                                                                              acc[nb][mb][4 * g + 2], acc[nb][mb][4 * g + 3]};
-        }
-    return;
-  }
   uint16_t *stage = reinterpret_cast<uint16_t *>(smem) + wave * (32 * MB * kOutStride);
   const int mw = m0 + wm * (32 * MB), nw = n0 + wn * (32 * NBW); // origin of the wavefront's part
   // All bias pieces of the part first, then per 32-column block all of its
@@ -385,29 +291,29 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, BK == 32 ? 3 : 1) void gemm_mfma
   }
 }
 
-template <typename T, int BK, int NB, bool RAGGED>
+template <typename T, int NB, bool RAGGED>
 void launchAct(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint16_t *r, uint16_t *o, int64_t M,
                int64_t N, int64_t K, int act, hipStream_t stream) {
   const int tilesN = (int)((N + 32 * NB - 1) / (32 * NB)), tilesM = (int)((M + kBM - 1) / kBM);
-  const dim3 grid((unsigned)(tilesM * tilesN)), block(BK == 64 ? 512 : 256);
+  const dim3 grid((unsigned)(tilesM * tilesN)), block(256);
   if (act == ACT_GELU)
-    gemm_mfma_kernel<T, ACT_GELU, BK, NB, BK == 64, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    gemm_mfma_kernel<T, ACT_GELU, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   else if (act == ACT_RELU)
-    gemm_mfma_kernel<T, ACT_RELU, BK, NB, BK == 64, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    gemm_mfma_kernel<T, ACT_RELU, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   else
-    gemm_mfma_kernel<T, ACT_NONE, BK, NB, BK == 64, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    gemm_mfma_kernel<T, ACT_NONE, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
 }
-template <typename T, int BK, int NB>
+template <typename T, int NB>
 void launchTile(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint16_t *r, uint16_t *o, int64_t M,
                 int64_t N, int64_t K, int act, hipStream_t stream) {
-  if (M % kBM || N % (32 * NB)) launchAct<T, BK, NB, true>(a, w, b, r, o, M, N, K, act, stream);
-  else launchAct<T, BK, NB, false>(a, w, b, r, o, M, N, K, act, stream);
+  if (M % kBM || N % (32 * NB)) launchAct<T, NB, true>(a, w, b, r, o, M, N, K, act, stream);
+  else launchAct<T, NB, false>(a, w, b, r, o, M, N, K, act, stream);
 }
 
 // Tile width: the one under which the busiest CU carries the fewest columns
 // (tiles are dealt evenly, so that CU holds ceil(tiles / CUs) of them); 128 on
-// a tie.  Reduction step: 64 when no CU gets a second tile; otherwise gemm_wide
-// where it goes, and steps of 32 where it does not.
+// a tie.  gemm_round when no CU gets a second tile, otherwise gemm_wide, each
+// where it goes; the kernel above where neither does.
 template <typename T>
 void launch(const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M,
             int64_t N, int64_t K, int act, hipStream_t stream) {
@@ -423,17 +329,13 @@ void launch(const void *in, const void *weight, const void *bias, const void *re
   const auto *r = static_cast<const uint16_t *>(residual);
   auto *o = static_cast<uint16_t *>(out);
   const DType dt = std::is_same<T, _Float16>::value ? DType::F16 : DType::BF16;
-  if (!deep && gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) {
+  if (deep) return gemmRound(dt, in, weight, bias, residual, out, M, N, K, act, narrow ? 96 : 128, stream);
+  if (gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) {
     double cost;
     return gemmWide(dt, in, weight, bias, residual, out, M, N, K, act, gemmWideBest(M, N, K, act, residual != nullptr, &cost), stream);
   }
-  if (narrow) {
-    if (deep) launchTile<T, 64, 3>(a, w, b, r, o, M, N, K, act, stream);
-    else launchTile<T, 32, 3>(a, w, b, r, o, M, N, K, act, stream);
-  } else {
-    if (deep) launchTile<T, 64, 4>(a, w, b, r, o, M, N, K, act, stream);
-    else launchTile<T, 32, 4>(a, w, b, r, o, M, N, K, act, stream);
-  }
+  if (narrow) launchTile<T, 3>(a, w, b, r, o, M, N, K, act, stream);
+  else launchTile<T, 4>(a, w, b, r, o, M, N, K, act, stream);
   MGPU_CHECK_LAUNCH("gemm_mfma_kernel");
 }
 
@@ -459,22 +361,21 @@ bool gemmMfmaSupportsRagged(DType dt, const void *in, const void *weight, const 
   return gemmMfmaSupports(dt, in, weight, bias, residual, out, m, n, K);
 }
 
-// One tile per CU (eight wavefronts, steps of 64): a fixed part and the operand bytes at what a CU pulls;
-// several: what overlaps of them at 52 GB/s behind 5 us of start and end.  (600 x 3072 x 768 + GELU 11.7 us,
-// 1200 x 1024 x 4096 31.7, 2500 x 2304 x 768 16.7.)
+// One tile per CU: gemm_round, fitted to 600 shapes (4 % rms, 14 % at worst; with it and gemm_ksplit's estimate the choice
+// between the two is 0.3 % behind the best of them, the library and gemm_wide, whose tiles it never pays to have less than one
+// round of).  Several: what overlaps of the operand bytes at 52 GB/s a CU behind 5 us of start and end.
 double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act) {
   const int64_t cus = numComputeUnits();
   auto tilesAt = [&](int64_t width) { return (M + kBM - 1) / kBM * ((N + width - 1) / width); };
   auto load = [&](int64_t width) { return (tilesAt(width) + cus - 1) / cus * width; };
   const int64_t width = load(96) < load(128) ? 96 : 128, tiles = tilesAt(width);
-  const double bytes = (double)(kBM + width) * 2.0 * (double)K;
-  if (tiles <= cus) return (act == ACT_GELU ? 5.0 : 2.0) + bytes / 57e3;
-  return 5.0 + (double)tiles / (double)cus * bytes / 52e3;
+  const double bytes = (double)(kBM + width) * 2.0 * (double)K, full = (double)tiles / (double)cus;
+  if (tiles <= cus) return 3.2 + 1.14 * full + bytes * (11.4e-6 + 2e-6 * full) + (act == ACT_GELU ? 1.4 : 0.0);
+  return 5.0 + full * bytes / 52e3;
 }
 
-// The tile width and estimated us of gemmMfmaPartialF16; no width where its blocks are more than one round of the CUs.
-// (4 us dearer than a whole product of that length: more CUs pull at once, and the sums leave in fp32.  640 x 768 x 768
-// of 3072 in four parts 11.6 us, 1368 x 768 x 1024 in three 15.5.)
+// The tile width and estimated us of gemmMfmaPartialF16 without what its planes cost (gemmPartialPlan has that); no width where
+// its blocks are more than one round of the CUs.
 static int partialWidth(int64_t M, int64_t N, int parts) {
   const int64_t tilesM = (M + kBM - 1) / kBM * parts;
   return tilesM * ((N + 95) / 96) <= numComputeUnits() ? 96 : tilesM * ((N + 127) / 128) <= numComputeUnits() ? 128 : 0;
@@ -482,23 +383,14 @@ static int partialWidth(int64_t M, int64_t N, int parts) {
 
 double gemmMfmaPartialCost(int64_t M, int64_t N, int64_t K, int parts) {
   const int width = partialWidth(M, N, parts);
-  return width && K % 64 == 0 ? 6.0 + (double)(kBM + width) * 2.0 * (double)K / parts / 57e3 : 1e30;
+  return width && K % 64 == 0 ? 3.05 + (double)(kBM + width) * 2.0 * (double)K / parts * 11.3e-6 : 1e30;
 }
 
 void gemmMfmaPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, int parts, hipStream_t stream) {
   const int width = partialWidth(M, N, parts);
   if (!gemmMfmaSupportsRagged(DType::F16, in, weight, nullptr, nullptr, planes, M, N, K) || !width || K % 64 || K / 64 < parts)
     fail("gemmMfmaPartial: internal dispatch error");
-  const int tilesN = (int)((N + width - 1) / width), tilesM = (int)((M + kBM - 1) / kBM);
-  const dim3 grid((unsigned)(tilesM * tilesN), (unsigned)parts), block(512);
-  const auto *a = static_cast<const uint16_t *>(in);
-  const auto *w = static_cast<const uint16_t *>(weight);
-  auto *o = reinterpret_cast<uint16_t *>(planes);
-  if (width == 96)
-    gemm_mfma_kernel<_Float16, ACT_NONE, 64, 3, true, true, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else
-    gemm_mfma_kernel<_Float16, ACT_NONE, 64, 4, true, true, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  MGPU_CHECK_LAUNCH("gemm_mfma_kernel");
+  gemmRoundPartialF16(in, weight, planes, M, N, K, width, parts, stream);
 }
 
 void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,

@@ -98,40 +98,17 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const uint16_t *
     if (n0 + 8 * chunk >= N) chunk = (N - 8 - n0) / 8;
     woff[i] = (uint32_t)row * (uint32_t)N * 2u + (uint32_t)(chunk * 16);
   }
-  // Inline assembly keeps the loads out of the compiler's wait counts, which would have every LDS read wait for all of
-  // them; the waits below count by hand.  (M0 is on the clobber list so that the statement counts as a definition of it.)
   const uint32_t ldsBase = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) unsigned char *)smem);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-  auto dma16 = [&](uint32_t voffset, const char *sbase, uint32_t ldsAddr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voffset), "s"(sbase), "s"(ldsAddr)
-                 : "memory", "m0");
-  };
-  auto dma4 = [&](uint32_t voffset, const char *sbase, uint32_t ldsAddr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-                 :
-                 : "v"(voffset), "s"(sbase), "s"(ldsAddr)
-                 : "memory", "m0");
-  };
-  auto dma16LowerLanes = [&](uint32_t voffset, const char *sbase, uint32_t ldsAddr) { // (all lanes are on around it)
-    asm volatile("s_mov_b32 m0, %2\n\ts_mov_b32 exec_hi, 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b32 exec_hi, -1"
-                 :
-                 : "v"(voffset), "s"(sbase), "s"(ldsAddr)
-                 : "memory", "m0");
-  };
-#pragma clang diagnostic pop
   int aSlot = 0, wSlot = 0; // ring slots filled next
-  auto issueA = [&](int i) { dma16(aoff[i], ag, ldsBase + (uint32_t)(aSlot * kABuf + wave * 4096 + i * 1024)); };
+  auto issueA = [&](int i) { ldsLoad16(aoff[i], ag, ldsBase + (uint32_t)(aSlot * kABuf + wave * 4096 + i * 1024)); };
   auto nextIssueA = [&]() {
     ag += 128;
     aSlot = aSlot == kARing - 1 ? 0 : aSlot + 1;
   };
   auto issueW = [&](int i) {
     const uint32_t dst = ldsBase + (uint32_t)(kWBase + wSlot * kWSlice + wave * (kWSlice / 8) + i * 1024);
-    if (kHalf && i == WI - 1) dma16LowerLanes(woff[i], wg, dst);
-    else dma16(woff[i], wg, dst);
+    if (kHalf && i == WI - 1) ldsLoad16LowerLanes(woff[i], wg, dst);
+    else ldsLoad16(woff[i], wg, dst);
   };
   auto nextIssueW = [&]() {
     wg += (size_t)N * 64;
@@ -221,7 +198,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const uint16_t *
   const uint32_t biasAt = ldsBase + (uint32_t)(2 * kABuf + wave * 256);
   if (bias) {
     const int n = n0 + wn * (32 * NBW) + 2 * lane;
-    dma4((uint32_t)(n < N ? n : N - 2) * 2u, reinterpret_cast<const char *>(bias), biasAt);
+    ldsLoad4((uint32_t)(n < N ? n : N - 2) * 2u, reinterpret_cast<const char *>(bias), biasAt);
   }
   if (kAhead == 4) issueSlice();
   issueA(0), issueA(1);

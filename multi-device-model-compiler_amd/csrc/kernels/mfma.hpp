@@ -50,6 +50,25 @@ template <> struct Mma<bf16_t> {
   }
 };
 
+// Loads from memory into LDS, 16 (4) bytes a lane to ldsAddr + 16 (4) * lane; a scalar base and a 32-bit offset a lane.
+// Inline assembly keeps them out of the compiler's wait counts, which would have every LDS read wait for all of them: the
+// kernels count by hand.  M0 is on the clobber list so that the statement counts as a definition of it (nothing here needs it
+// preserved).  LowerLanes: lanes 32-63 load nothing; all lanes must be on around it.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void ldsLoad16(uint32_t offset, const char *base, uint32_t ldsAddr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(ldsAddr) : "memory", "m0");
+}
+__device__ __forceinline__ void ldsLoad16LowerLanes(uint32_t offset, const char *base, uint32_t ldsAddr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b32 exec_hi, 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b32 exec_hi, -1" ::"v"(offset), "s"(base),
+               "s"(ldsAddr)
+               : "memory", "m0");
+}
+__device__ __forceinline__ void ldsLoad4(uint32_t offset, const char *base, uint32_t ldsAddr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(offset), "s"(base), "s"(ldsAddr) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 // Exchange with lane l ^ 32: v_permlane32_swap hands every lane the value of
 // the lower half in r[0] and of the upper half in r[1].
 __device__ __forceinline__ float halves_max(float v) {

@@ -107,6 +107,12 @@ bool gemmWideSupports(DType dt, const void *in, const void *weight, const void *
 void gemmWide(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
               int64_t K, int act, int width, hipStream_t stream);
 
+// At most one tile of 128 x 96 or 128 x 128 per CU (gemm_round.hip), for gemm_mfma.hip's launchers: N a multiple of 8, K of 64.
+void gemmRound(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
+               int64_t K, int act, int width, hipStream_t stream);
+void gemmRoundPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, int width, int parts,
+                         hipStream_t stream);
+
 // Small tiles, the reduction split over a block's wavefronts (gemm_ksplit.hip): fp16 / bf16, any M, N and K
 // multiples of 8.  gemmKSplitBest: the tile for a shape and its estimated us, to compare with the others.
 enum class KSplitTile { T32x32, T32x64, T64x64 };

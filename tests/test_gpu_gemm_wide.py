@@ -1,4 +1,4 @@
-"""gemm_wide (csrc/kernels/gemm_wide.hip): every tile width, where tiles end inside the shape and where they fit, from the
+"""gemm_wide and gemm_round (csrc/kernels): every tile width, where tiles end inside the shape and where they fit, from the
 fewest reduction steps on, each epilogue, both types; nothing stored outside the output."""
 import ctypes
 
@@ -6,33 +6,33 @@ import pytest
 
 from test_index_bounds import internal
 
-WIDE = "_ZN4mgpu8gemmWideENS_5DTypeEPKvS2_S2_S2_PvllliiP12ihipStream_t"
+SHAPES = [
+    (1, 8, 128),       # one row, one chunk of columns; gemm_wide: no pass of the loop
+    (256, 768, 192),   # whole tiles of every width; gemm_wide: one pass
+    (257, 520, 256),   # gemm_round: as many steps as are kept ahead
+    (300, 1000, 320),
+    (511, 248, 1088),
+    (2300, 136, 704),  # more tile rows than a group
+]
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
-@pytest.mark.parametrize("width", [128, 192, 256])
-@pytest.mark.parametrize("M,N,K", [
-    (1, 8, 128),       # one row, one chunk of columns, no pass of the loop
-    (256, 768, 192),   # whole tiles of every width, one pass
-    (257, 520, 256),
-    (300, 1000, 320),  # two passes of the loop
-    (511, 248, 1088),
-    (2300, 136, 704),  # more tile rows than a group
-])
-def test_against_float64(pkg, gpu, dtype, width, M, N, K):
+@pytest.mark.parametrize("name,width,M,N,K", [("8gemmWide", w, *s) for w in (128, 192, 256) for s in SHAPES] +
+                         [("9gemmRound", w, *s) for w in (96, 128) for s in SHAPES + [(130, 104, 64)]])
+def test_against_float64(pkg, gpu, dtype, name, width, M, N, K):
     import torch
     t, code, ulp = (torch.float16, 1, 2.0**-11) if dtype == "f16" else (torch.bfloat16, 2, 2.0**-8)
     g = torch.Generator(device=gpu).manual_seed(M + N + K)
     r = lambda *s: torch.randn(s, generator=g, device=gpu)
     x, w, b, res = r(M, K).to(t), (r(K, N) / K**0.5).to(t), r(N).to(t), r(M, N).to(t)
-    wide = internal(pkg, WIDE, None, ctypes.c_int, *[ctypes.c_void_p] * 5, *[ctypes.c_int64] * 3, ctypes.c_int, ctypes.c_int, ctypes.c_void_p)
+    gemm = internal(pkg, "_ZN4mgpu" + name + "ENS_5DTypeEPKvS2_S2_S2_PvllliiP12ihipStream_t", None, ctypes.c_int, *[ctypes.c_void_p] * 5, *[ctypes.c_int64] * 3, ctypes.c_int, ctypes.c_int, ctypes.c_void_p)
     X, W = x.double().cpu(), w.double().cpu()
     prod, size = X @ W, X.abs() @ W.abs()
     B, R = b.double().cpu(), res.double().cpu()
     for bias, act, residual in ((None, 0, None), (b, 1, None), (b, 2, None), (b, 0, res)):
         out = torch.full((M + 2, N), 7.0, dtype=t, device=gpu)  # a row before and one behind
-        wide(code, x.data_ptr(), w.data_ptr(), bias.data_ptr() if bias is not None else None, residual.data_ptr() if residual is not None else None,
+        gemm(code, x.data_ptr(), w.data_ptr(), bias.data_ptr() if bias is not None else None, residual.data_ptr() if residual is not None else None,
              out[1:].data_ptr(), M, N, K, act, width, torch.cuda.current_stream().cuda_stream)
         got = out.double().cpu()
         ref = prod + (B if bias is not None else 0)
@@ -45,18 +45,35 @@ def test_against_float64(pkg, gpu, dtype, width, M, N, K):
         assert (got[0] == 7).all() and (got[-1] == 7).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,M,N,K,parts", [(96, 300, 200, 512, 2), (128, 131, 264, 1088, 4), (96, 128, 96, 832, 3)])
+def test_planes_of_partial_sums(pkg, gpu, width, M, N, K, parts):
+    """Shares of unequal length; the planes add up to the product."""
+    import torch
+    g = torch.Generator(device=gpu).manual_seed(K)
+    x, w = torch.randn((M, K), generator=g, device=gpu).half(), torch.randn((K, N), generator=g, device=gpu).half()
+    gemm = internal(pkg, "_ZN4mgpu19gemmRoundPartialF16EPKvS1_PfllliiP12ihipStream_t", None, *[ctypes.c_void_p] * 3, *[ctypes.c_int64] * 3,
+                    ctypes.c_int, ctypes.c_int, ctypes.c_void_p)
+    planes = torch.full((parts + 1, M, N), 7.0, device=gpu)
+    gemm(x.data_ptr(), w.data_ptr(), planes.data_ptr(), M, N, K, width, parts, torch.cuda.current_stream().cuda_stream)
+    X, W = x.double().cpu(), w.double().cpu()
+    got = planes[:parts].double().cpu().sum(0)
+    assert ((got - X @ W).abs() <= (K + parts) * 2.0**-24 * (X.abs() @ W.abs())).all()
+    assert (planes[parts] == 7).all()
+
+
 @pytest.mark.parametrize("M,N,K,act,residual,width", [
     (4096, 3072, 768, 2, False, 192),    # a round of tiles of 192
     (4096, 6144, 2048, 0, False, 192),
     (8192, 8192, 8192, 0, False, 256),
     (4096, 2048, 2048, 0, True, 128),
     (2304, 2048, 2560, 0, False, 128),   # beyond one round of 128 x 128 tiles, however deep
-    (2049, 2048, 128, 0, False, None),   # ... whatever the width
+    (2049, 2048, 128, 0, False, None),   # (whatever the width)
     (4096, 2048, 96, 0, False, 0),       # fewer steps than its loop is built for
     (4096, 2048, 1056, 0, False, 0),     # not whole steps
     (4096, 2044, 1024, 0, False, 0),
     (127, 40000, 1024, 0, False, 0),
-    (4096, 768, 3072, 0, False, 0),      # up to one round: the estimates
+    (4096, 768, 3072, 0, False, 0),      # up to one round of 128 x 128 tiles
     (77, 768, 768, 0, False, 0),
 ])
 def test_what_it_serves(pkg, M, N, K, act, residual, width):
