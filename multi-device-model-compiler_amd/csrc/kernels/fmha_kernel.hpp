@@ -398,6 +398,11 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
 #pragma unroll
       for (int c = 0; c < G::DC; c++) asm volatile("" ::"v"(qf[qi][c]));
   }
+  // Where the loads of the next tile go out: right behind the barrier they keep a wavefront from its score MFMAs until the
+  // address path has taken all of them (16 cycles an instruction, 8 of every wavefront at head_dim 128); behind the scores the wait falls under MFMAs that are still running.  At head_dim 128 (b2 s4096 h32 606 -> 555 us, b4
+  // s2048 h32 333 -> 318, b8 s1024 h32 186 -> 178, b8 s700 h12 d96 45.3 -> 40.9, causal b4 s2048 h32 188 -> 186; b16 s256 h16 16.0
+  // -> 16.4); at 64, four loads a wavefront and three wavefronts a SIMD, the causal kernel loses 3-5 %, and at 256 it spills.
+  constexpr bool kLoadsBehindScores = D == 128;
   for (int kt = 0; kt < nkt; kt++) {
     if (TRACE) tMark = clock64();
     // The loads of tile kt (and of nothing later) must have landed; the barrier
@@ -408,7 +413,7 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (TRACE && kt == 0) tFirstTile = clock64();
-    if (kt + kStages - 1 < nkt) issueTile(kt + kStages - 1);
+    if (!kLoadsBehindScores && kt + kStages - 1 < nkt) issueTile(kt + kStages - 1);
 
     const uint32_t stageOff = (uint32_t)((kt % kStages) * kStageBytes);
     const int key0 = kt * kBN;
@@ -427,7 +432,8 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
     }
 
     // Causal: a wavefront whose queries all precede this tile has nothing to add.
-    if (CAUSAL && key0 > q0 + NQ * 32 - 1) continue;
+    const bool nothing = CAUSAL && key0 > q0 + NQ * 32 - 1;
+    if (!kLoadsBehindScores && nothing) continue;
 
     // Operand pointers in the LDS address space: one add per tile, the rest
     // of every address is an instruction immediate.
@@ -448,25 +454,31 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
     }
     // ---- S^T = K Q^T -------------------------------------------------------
     f32x16 accS[NQ][G::KB];
-    __builtin_amdgcn_s_setprio(2); // MFMA phases outrank the softmax phases of the SIMD's other wavefronts
+    if (!kLoadsBehindScores || !nothing) {
+      __builtin_amdgcn_s_setprio(2); // MFMA phases outrank the softmax phases of the SIMD's other wavefronts
 #pragma unroll
-    for (int kb = 0; kb < G::KB; kb++) {
+      for (int kb = 0; kb < G::KB; kb++) {
 #pragma unroll
-      for (int c = 0; c < G::DC; c++) {
-        const v8 a = *reinterpret_cast<const v8 __attribute__((address_space(3))) *>(kp[c % G::KF] + (c / G::KF) * 256 +
-                                                                                      kb * 32 * G::rowBytes);
+        for (int c = 0; c < G::DC; c++) {
+          const v8 a = *reinterpret_cast<const v8 __attribute__((address_space(3))) *>(kp[c % G::KF] + (c / G::KF) * 256 +
+                                                                                        kb * 32 * G::rowBytes);
 #pragma unroll
-        for (int qi = 0; qi < NQ; qi++) {
-          if (c == 0) {
+          for (int qi = 0; qi < NQ; qi++) {
+            if (c == 0) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) accS[qi][kb][i] = 0.0f;
+              for (int i = 0; i < 16; i++) accS[qi][kb][i] = 0.0f;
+            }
+            accS[qi][kb] = M::run(a, qf[qi][c], accS[qi][kb]);
           }
-          accS[qi][kb] = M::run(a, qf[qi][c], accS[qi][kb]);
         }
       }
-    }
 
-    __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_s_setprio(0);
+    }
+    if (kLoadsBehindScores) {
+      if (kt + kStages - 1 < nkt) issueTile(kt + kStages - 1);
+      if (nothing) continue;
+    }
     if (TRACE) {
       // a use of the last accumulator makes the stamp wait for the MFMAs
       asm volatile("" ::"v"(accS[NQ - 1][G::KB - 1][15]));
