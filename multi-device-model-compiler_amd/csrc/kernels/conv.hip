@@ -13,16 +13,17 @@
 // columns, so that a register of an accumulator is 32 consecutive pixels of a channel: whole
 // 128-byte runs of the NCHW output.  The tap matrix is never written to memory.  Taps come
 // through buffer loads, whose bounds check answers 0 for an offset outside the image: padding costs
-// no branch and no second instruction.  Four kernels share the work (conv2d below has the rule and
+// no branch and no second instruction.  Five kernels share the work (conv2d below has the rule and
 // the measurements behind it):
 //   few taps  (K <= 32, a network's stem)  filter in registers, wavefronts walk over pixel tiles
+//   quads     (the same, many tiles, rows of whole quads, stride 1 across)  four pixels a lane
 //   window    (1, 3, 5 or 7 square, few tiles)  operands straight from L1 / L2 into registers,
 //             four wavefronts per tile
 //   tile      (the same windows, many tiles)    operands shared through LDS by 64 x 64 tiles
 //   table     (every other window, and images beyond 2 GiB)  tap offsets from a table in LDS
 // What bounds them: one 32x32x2 MFMA takes 64 cycles of a SIMD (157 TFLOP/s on the chip) and the
 // vector instructions of the same wavefront do not overlap with it, so the loops are built to have
-// none; the stem is bound by its output (268 MB at 16 x 3 x 256 x 256 -> 64: 116 -> 70 us, a plain fill
+// none; the stem is bound by its output (268 MB at 16 x 3 x 256 x 256 -> 64: 65 us, a plain fill
 // of as many bytes takes 39).  Unlike the reference, asymmetric padding is honoured (it passes only
 // PHL / PWL to cuDNN).
 #include "common.hpp"
@@ -42,6 +43,7 @@ struct ConvGeo {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kChunk = 16;     // taps per step of the reduction: 8 a lane half
 constexpr int kSegment = 2048; // taps the tap table holds at a time
@@ -531,10 +533,11 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
     // (opaque, or the compiler keeps their multiples and comparisons in scalar registers across the loop)
     int row = P * 4, channels = OC;
     asm volatile("" : "+s"(row), "+s"(channels));
+    // (written through to memory: 8 x 3 x 224 x 224 -> 64 33.2 -> 31.8 us, 4 x 3 x 224 x 224 -> 32 of stride 2 7.40 -> 6.86)
     auto store = [&](int ocl, float v, int voffset, int soffset) {
       if (add) v += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(post, voffset, soffset, 0));
       // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, relu ? fmaxf(v, 0.0f) : v), out, voffset, soffset, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, relu ? fmaxf(v, 0.0f) : v), out, voffset, soffset, 16);
     };
     if (fullOc) {
 #pragma unroll
@@ -553,6 +556,137 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
           if (oc0 + ocl < channels) // (a scalar offset past the resource would wrap the check)
             store(ocl, acc[t][r], oc0 + ocl + 4 * hl < channels ? at : kOutside, ocl * row);
         }
+    }
+  };
+  Tile even, odd;
+  int tile = (int)blockIdx.x * 4 + wave;
+  if (tile < tiles) fetch(even, tile);
+  for (; tile < tiles; tile += 2 * tileStep) {
+    if (tile + tileStep < tiles) fetch(odd, tile + tileStep);
+    finish(even);
+    if (tile + tileStep >= tiles) break;
+    if (tile + 2 * tileStep < tiles) fetch(even, tile + 2 * tileStep);
+    finish(odd);
+  }
+}
+
+// ---- few taps, four pixels a lane ------------------------------------------------------------
+// The same reduction where output rows are whole quads of pixels and the window's columns are neighbours.  Column l of
+// accumulator j is pixel 4 l + j of a tile of 128, so that a lane holds four consecutive pixels of every channel of its
+// registers: a store writes 16 bytes a lane, 512 of each of two channels, where pixel l of every accumulator gave 4 and
+// 128.  And the taps of four neighbours overlap: a lane half takes whole window rows - NR of the IC * KH, the lower half the
+// first - and per row one 16-byte load of the quad's own columns and KW - 1 single ones beside it serve 4 KW taps.
+// What bounds it: the output and, not wholly hidden behind it, the matrix cores (15 steps of 64 clocks a 32 x 32 tile).  16 x 3 x
+// 256 x 256 -> 64, 268 MB: 76.9 -> 65.5 us (1 x 1 from the same: 68.0 -> 49.2; a fill of as many bytes takes 39); 8 x 3 x 224 x
+// 224 -> 64 with a postAdd 87 -> 49; 8 x 3 x 128 x 128 -> 16 11.0 -> 6.7.  Stores of one tile dealt out between the matrix
+// instructions of the next measured the same, an order of tiles by XCD too, runs of tiles a wavefront 90.
+// STREAM: an output beyond what the Infinity Cache keeps leaves by non-temporal stores (72 against 65.5 us above), a smaller
+// one is written through (4 x 3 x 256 x 256 -> 64 20.6 non-temporal, 21.4 plain, 19.2 so).
+template <int KW, int NR, bool STREAM>
+__global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                            const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
+                                                            int P, int N, FastDiv byP, FastDiv byOW, const float *__restrict__ add,
+                                                            int relu, int tiles, int tileStep) {
+  constexpr int SIDE = KW - 1; // columns beside the quad's own
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int l32 = lane % 32, hl = lane / 32;
+  const int oc0 = blockIdx.y * 32;
+  const int pixels = N * P, rows = g.IC * g.KH;
+
+  float a[NR][KW];
+  int toff[NR], tkh[NR]; // a row's byte offset from the quad's first tap, and its window row (31: past the end, always outside)
+#pragma unroll
+  for (int i = 0; i < NR; i++) {
+    const int r = hl * NR + i, ic = r / g.KH, kh = r - ic * g.KH;
+    const bool in = r < rows;
+    toff[i] = in ? (ic * g.H + kh * g.DH) * g.W * 4 : 0;
+    tkh[i] = in ? kh : 31;
+    const int oc = oc0 + l32 < OC ? oc0 + l32 : OC - 1;
+#pragma unroll
+    for (int k = 0; k < KW; k++) a[i][k] = in ? w[((int64_t)oc * rows + r) * KW + k] : 0.0f;
+  }
+  float bv[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int oc = oc0 + 8 * (r / 4) + r % 4 + 4 * hl;
+    bv[r] = bias[oc < OC ? oc : OC - 1];
+  }
+  struct Tile {
+    int pix, img, nFirst; // the lane's first pixel (-1: past the end), its image less the tile's first, that image
+    f32x4 own[NR];        // of a row: the quad's own columns, those left of them, those right
+    float side[NR][SIDE > 0 ? SIDE : 1];
+  };
+  const int64_t imageElems = (int64_t)g.IC * g.H * g.W;
+  auto fetch = [&](Tile &o, int tile) {
+    const int q0 = tile * 128, q = q0 + 4 * l32;
+    const bool live = q < pixels;
+    o.nFirst = __builtin_amdgcn_readfirstlane(divide(q0, byP));
+    const int n = live ? divide(q, byP) : o.nFirst;
+    const int p = live ? q - n * P : 0;
+    const int oh = divide(p, byOW), ow = p - oh * g.OW;
+    o.img = n - o.nFirst;
+    o.pix = live ? p : -1;
+    const int ih0 = oh * g.SH - g.PHL;
+    const unsigned rowOut = live ? outsideBits(ih0, g.H, g.KH, g.DH) | 0x80000000u : ~0u;
+    const int base = (o.img * (int)imageElems + ih0 * g.W + ow) * 4; // of the quad's own columns
+    const auto rsrc = resource(x + o.nFirst * imageElems, (N - o.nFirst) * imageElems);
+    int sideOut[SIDE > 0 ? SIDE : 1], sideOff[SIDE > 0 ? SIDE : 1]; // column e of the window's KW + 3 is ow - PWL + e
+#pragma unroll
+    for (int e = 0; e < SIDE; e++) {
+      const int d = e < g.PWL ? e - g.PWL : e - g.PWL + 4;
+      sideOff[e] = d * 4;
+      sideOut[e] = (unsigned)(ow + d) < (unsigned)g.W ? 0 : kOutside;
+    }
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+      const int out = __builtin_amdgcn_sbfe(rowOut, tkh[i], 1) & kOutside; // (not all ones: 16 bytes from there would wrap)
+      o.own[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (base + toff[i]) | out, 0, 0));
+#pragma unroll
+      for (int e = 0; e < SIDE; e++)
+        o.side[i][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (base + toff[i] + sideOff[e]) | out | sideOut[e], 0, 0));
+    }
+  };
+  const int64_t outElems = (int64_t)OC * P;
+  auto finish = [&](Tile &o) {
+    f32x16 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[j][i] = bv[i];
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+      // the window's KW + 3 columns in order (uniform selects: PWL of them lie left of the quad)
+      float c[KW + 3];
+#pragma unroll
+      for (int e = 0; e < KW + 3; e++) {
+        float v = e < SIDE ? o.side[i][e] : 0.0f; // e < PWL
+#pragma unroll
+        for (int own = 0; own < 4; own++)
+          if (e - own >= 0 && e - own <= SIDE && e - own == g.PWL) v = o.own[i][own];
+        if (e >= 4 && e - 4 >= 0 && e - 4 < SIDE && e >= g.PWL + 4) v = o.side[i][e - 4];
+        c[e] = v;
+      }
+#pragma unroll
+      for (int k = 0; k < KW; k++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][k], c[k + j], acc[j], 0, 0, 0);
+    }
+    const auto out = resource(y + o.nFirst * outElems, (N - o.nFirst) * outElems);
+    const auto post = resource(add + (add ? o.nFirst * outElems : 0), (N - o.nFirst) * outElems);
+    const int at = o.pix < 0 ? kOutside : ((o.img * OC + oc0 + 4 * hl) * P + o.pix) * 4;
+    int row = P * 4, channels = OC;
+    asm volatile("" : "+s"(row), "+s"(channels));
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int ocl = 8 * (r / 4) + r % 4;
+      if (oc0 + ocl >= channels) break; // (uniform; a scalar offset past the resource would wrap the check)
+      const int voffset = oc0 + ocl + 4 * hl < channels ? at : kOutside;
+      f32x4 v = {acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
+      if (add) v += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(post, voffset, ocl * row, 0));
+      // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
+      if (relu) v = f32x4{fmaxf(v[0], 0.0f), fmaxf(v[1], 0.0f), fmaxf(v[2], 0.0f), fmaxf(v[3], 0.0f)};
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, voffset, ocl * row, STREAM ? 2 : 16);
     }
   };
   Tile even, odd;
@@ -846,6 +980,17 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     conv_few_taps_kernel<OCT, NS><<<gridOf(blocks, 32 * OCT, 256), dim3(256), 0, stream>>>(
         input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu, (int)K, (int)pix32, (int)(4 * blocks));
   };
+  const int64_t tiles128 = (pixels + 127) / 128;
+  const bool streams = N * OC * P * 4 > int64_t(128) << 20;
+  auto quads = [&](auto kw, auto nr) {
+    constexpr int KWC = decltype(kw)::value, NR = decltype(nr)::value;
+    // two blocks per CU and channel tile
+    const int64_t most = std::max<int64_t>(1, (int64_t)numComputeUnits() * 2 / ((OC + 31) / 32));
+    const int64_t blocks = std::min((tiles128 + 3) / 4, most);
+    auto *kernel = streams ? conv_quads_kernel<KWC, NR, true> : conv_quads_kernel<KWC, NR, false>;
+    kernel<<<gridOf(blocks, 32, 256), dim3(256), 0, stream>>>(input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu,
+                                                              (int)tiles128, (int)(4 * blocks));
+  };
   auto window = [&](auto win, auto pts, auto kss) {
     constexpr int WIN = decltype(win)::value, PT = decltype(pts)::value, KS = decltype(kss)::value;
     const int64_t perBlock = 4 / KS * 32 * PT;
@@ -878,6 +1023,23 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
   if (!narrow) {
     table(std::true_type());
   } else if (K <= 32) {
+    // Four pixels a lane from two tiles of 32 x 128 a CU on (us, pixel by pixel / quads, 3 x 3 from 3 channels: 256 tiles 5.2 / 6.9,
+    // 512 6.9 / 7.2 and 6.8 / 6.4, 768 10.2 / 7.8, 1024 11.2 / 7.9, 2048 15.5 / 12.8); not from more than 16 window rows, whose
+    // taps leave no registers to prefetch into (1 x 1 from 32 channels, 2048 tiles: 18.8 / 23.0).
+    const int64_t rows = IC * KH;
+    const bool wholeQuads = OW % 4 == 0 && OW <= W && SW == 1 && PWL < KW && (KW == 1 || ((KW == 3 || KW == 5) && DW == 1));
+    if (wholeQuads && rows <= 16 && tiles128 * ((OC + 31) / 32) >= 2 * numComputeUnits() &&
+        fitsInt((127 / P + 2) * IC * H * W * 4) && fitsInt((127 / P + 2) * OC * P * 4)) {
+      if (KW == 1 && rows <= 4) quads(c1, c2);
+      else if (KW == 1 && rows <= 8) quads(c1, c4);
+      else if (KW == 1) quads(c1, integral_constant<int, 8>());
+      else if (KW == 3 && rows <= 4) quads(integral_constant<int, 3>(), c2);
+      else if (KW == 3 && rows <= 6) quads(integral_constant<int, 3>(), integral_constant<int, 3>());
+      else if (KW == 3) quads(integral_constant<int, 3>(), integral_constant<int, 5>());
+      else quads(integral_constant<int, 5>(), integral_constant<int, 3>());
+      MGPU_CHECK_LAUNCH("mgpuConv2d");
+      return;
+    }
     auto steps = [&](auto octs) {
       if (K <= 10) few(octs, integral_constant<int, 5>());
       else if (K <= 16) few(octs, integral_constant<int, 8>());

@@ -43,6 +43,22 @@ def test_conv2d(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation
     conv_case(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add)
 
 
+@pytest.mark.parametrize("N,IC,H,W,OC,K,pad,stride,dilation,relu,add", [
+    (2, 3, 64, 64, 256, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, True),       # nine window rows, whole tiles
+    (64, 3, 8, 16, 250, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True),      # an image a tile, channels past the end
+    (130, 3, 6, 12, 225, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False),     # tiles over several images, the last one cut
+    (40, 1, 16, 20, 249, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), False, False),    # five rows of five
+    (40, 1, 16, 20, 249, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, False),    # three rows
+    (20, 2, 20, 24, 256, (3, 3), (0, 2, 2, 0), (1, 1), (1, 1), False, False),    # both columns left of the pixel
+    (20, 3, 40, 26, 256, (3, 3), (1, 0, 1, 0), (2, 1), (1, 1), True, False),     # none, stride down
+    (30, 3, 20, 20, 256, (2, 1), (0, 0, 0, 0), (1, 1), (1, 1), False, True),     # six rows of one column
+    (30, 1, 24, 20, 256, (3, 1), (2, 0, 2, 0), (1, 1), (2, 3), False, False),    # dilated down (across, one column: nothing to dilate)
+    (24, 16, 20, 24, 256, (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), False, False),   # sixteen rows
+])
+def test_conv2d_of_few_taps_four_pixels_a_lane(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add):
+    conv_case(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add)
+
+
 @pytest.mark.parametrize("C,H,W,K,pad,stride", [
     (3, 8, 8, (2, 2), (0, 0, 0, 0), (2, 2)), (2, 9, 7, (3, 3), (1, 1, 1, 1), (2, 2)),
     (64, 112, 112, (3, 3), (1, 1, 1, 1), (2, 2)),  # ResNet stem pool
