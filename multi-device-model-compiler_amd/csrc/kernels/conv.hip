@@ -13,12 +13,13 @@
 // columns, so that a register of an accumulator is 32 consecutive pixels of a channel: whole
 // 128-byte runs of the NCHW output.  The tap matrix is never written to memory.  Taps come
 // through buffer loads, whose bounds check answers 0 for an offset outside the image: padding costs
-// no branch and no second instruction.  Five kernels share the work (conv2d below has the rule and
+// no branch and no second instruction.  Six kernels share the work (conv2d below has the rule and
 // the measurements behind it):
 //   few taps  (K <= 32, a network's stem)  filter in registers, wavefronts walk over pixel tiles
 //   quads     (the same, many tiles, rows of whole quads, stride 1 across)  four pixels a lane
 //   window    (1, 3, 5 or 7 square, few tiles)  operands straight from L1 / L2 into registers,
 //             four wavefronts per tile
+//   staged    (3 or 5 square, even channels, few tiles)  the same with the filter through LDS
 //   tile      (the same windows, many tiles)    operands shared through LDS by 64 x 64 tiles
 //   table     (every other window, and images beyond 2 GiB)  tap offsets from a table in LDS
 // What bounds them: one 32x32x2 MFMA takes 64 cycles of a SIMD (157 TFLOP/s on the chip) and the
@@ -443,6 +444,125 @@ __global__ __launch_bounds__(256, 2) void conv_window_kernel(const float *__rest
     tail(tail, std::integral_constant<int, 0>());
   }
   finishTile<PT, KS, uint32_t>(acc, partial, tile * KS, ks, bias, add, y, OC, P, oc0, nFirst, img, pix, lane, relu);
+}
+
+// The same for few tiles, one of 32 x 32 a block: the filter through LDS.  A matrix instruction wants one value of each of 32
+// channels, whose rows lie IC * KK floats apart: loaded straight into registers every instruction touches 32 lines, and the CU's
+// one L1, not its four SIMDs, set the pace (8 x 256 x 7 x 7 -> 512, 3 x 3: 20.8 us, 14 with the filter loads of all
+// channels on one line, 7.7 by the matrix cores; now 16.8).  Here a wavefront loads its channels' rows along the rows - CG channel groups
+// at a time, 16 bytes a lane, under the matrix instructions of the groups before -, keeps them in an LDS area of its own (no
+// barrier) and reads an operand a step from there.
+template <int WIN> struct Staged {
+  static constexpr int CG = WIN == 5 ? 2 : 4;                          // channel groups staged at a time
+  static constexpr int ROW = CG * 2 * Window<WIN>::HALF * WIN * WIN;   // floats of a channel's row among them: a multiple of 4
+  static constexpr int PIECES = ROW / 4, LOADS = (32 * PIECES + 63) / 64;
+  static constexpr int PITCH = ROW % 16 == 0 ? ROW + 4 : ROW + (ROW % 8 == 0 ? 4 : 0); // 4 or 12 modulo 16 words: 16 rows on different banks
+};
+template <int WIN, int KS>
+__global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                                 const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
+                                                                 int P, int N, FastDiv byP, FastDiv byOW, const float *__restrict__ add,
+                                                                 int relu) {
+  using Win = Window<WIN>;
+  using St = Staged<WIN>;
+  constexpr int KK = Win::KK, UNITS = Win::UNITS, STEPS = Win::STEPS, HALF = Win::HALF;
+  constexpr int kRows = 32 * St::PITCH;
+  __shared__ __attribute__((aligned(16))) float smem[KS * (kRows > 16 * 64 ? kRows : 16 * 64)];
+
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int ks = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int l32 = lane % 32, hl = lane / 32;
+  const int oc0 = blockIdx.y * 32, q0 = pixelBlock<64 * KS>() * 32;
+  const int HW4 = g.H * g.W * 4, pixels = N * P;
+
+  const int nFirst = __builtin_amdgcn_readfirstlane(divide(q0 < pixels ? q0 : pixels - 1, byP));
+  int pix[1], img[1], voff[KK];
+  {
+    const int q = q0 + l32;
+    const bool live = q < pixels;
+    const int n = live ? divide(q, byP) : nFirst;
+    const int p = live ? q - n * P : 0;
+    const int oh = divide(p, byOW), ow = p - oh * g.OW;
+    img[0] = n - nFirst;
+    pix[0] = live ? p : -1;
+    const int ih0 = live ? oh * g.SH - g.PHL : -kNever, iw0 = ow * g.SW - g.PWL;
+    const int base = (img[0] * g.IC + hl * HALF) * HW4 + ((oh * g.SH - g.PHL) * g.W + iw0) * 4;
+#pragma unroll
+    for (int kh = 0; kh < WIN; kh++)
+#pragma unroll
+      for (int kw = 0; kw < WIN; kw++) {
+        const bool in = (unsigned)(ih0 + kh * g.DH) < (unsigned)g.H && (unsigned)(iw0 + kw * g.DW) < (unsigned)g.W;
+        voff[kh * WIN + kw] = in ? base + (kh * g.DH * g.W + kw * g.DW) * 4 : kOutside;
+      }
+  }
+  const int64_t imageElems = (int64_t)g.IC * g.H * g.W;
+  const auto image = resource(x + nFirst * imageElems, (N - nFirst) * imageElems);
+  const auto filter = resource(w + (int64_t)oc0 * g.IC * KK, (int64_t)(OC - oc0) * g.IC * KK);
+
+  f32x16 acc[1];
+#pragma unroll
+  for (int i = 0; i < 16; i++) acc[0][i] = 0.0f;
+
+  const int groups = g.IC / (2 * HALF); // (whole: the launcher sees to it)
+  const int g0 = groups * ks / KS, g1 = groups * (ks + 1) / KS; // this wavefront's share
+
+  // Filter rows: piece p of 16 bytes is piece p % PIECES of channel p / PIECES.  (A channel past the end reads the last one's
+  // row and is not stored; groups past the share are loaded and not used.)
+  float *mine = smem + ks * kRows;
+  int woff[St::LOADS];
+#pragma unroll
+  for (int i = 0; i < St::LOADS; i++) {
+    const int p = i * 64 + lane, oc = p / St::PIECES;
+    woff[i] = oc < 32 ? ((oc0 + oc < OC ? oc : OC - 1 - oc0) * g.IC * KK + 4 * (p - oc * St::PIECES)) * 4 : kOutside;
+  }
+  f32x4 stage[St::LOADS];
+  auto load = [&](int group) {
+#pragma unroll
+    for (int i = 0; i < St::LOADS; i++)
+      stage[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(filter, woff[i], group * (2 * HALF * KK * 4), 0));
+  };
+  auto keep = [&]() {
+#pragma unroll
+    for (int i = 0; i < St::LOADS; i++) {
+      const int p = i * 64 + lane, oc = p / St::PIECES;
+      if (64 * (i + 1) <= 32 * St::PIECES || oc < 32) *reinterpret_cast<f32x4 *>(mine + oc * St::PITCH + 4 * (p - oc * St::PIECES)) = stage[i];
+    }
+  };
+  // The reduction walks units - a group, or one of its window rows - in a pipeline two deep: a unit's taps fly under the
+  // matrix instructions of the one before.
+  auto fetch = [&](float (&b)[STEPS], int group, int unit) {
+#pragma unroll
+    for (int i = 0; i < STEPS; i++)
+      b[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(image, voff[WIN == 1 ? 0 : unit * STEPS + i],
+                                                                            (group * (2 * HALF) + (WIN == 1 ? i : 0)) * HW4, 0));
+  };
+  const float *ap = mine + l32 * St::PITCH + hl * (HALF * KK);
+  auto multiply = [&](const float (&b)[STEPS], int inChunk, int unit) {
+#pragma unroll
+    for (int i = 0; i < STEPS; i++)
+      acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(ap[inChunk * (2 * HALF * KK) + unit * STEPS + i], b[i], acc[0], 0, 0, 0);
+  };
+  constexpr int NU = St::CG * UNITS; // units of a chunk: an even number
+  float b[2][STEPS];
+  if (g0 < g1) {
+    load(g0);
+    fetch(b[0], g0, 0);
+  }
+  for (int chunk = g0; chunk < g1; chunk += St::CG) {
+    keep();
+    if (chunk + St::CG < g1) load(chunk + St::CG);
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      const int group = chunk + u / UNITS;
+      if (u % UNITS == 0 && group >= g1) break; // (uniform)
+      const int next = u + 1; // (fetched if it is still in the share)
+      if (chunk + next / UNITS < g1) fetch(b[next % 2], chunk + next / UNITS, next % UNITS);
+      multiply(b[u % 2], u / UNITS, u % UNITS);
+    }
+  }
+  if (KS > 1) __syncthreads(); // the partial sums take the filter rows' place
+  auto &partial = *reinterpret_cast<float(*)[KS][16 * 64]>(smem);
+  finishTile<1, KS, uint32_t>(acc, partial, 0, ks, bias, add, y, OC, P, oc0, nFirst, img, pix, lane, relu);
 }
 
 // ---- few taps -----------------------------------------------------------------------------
@@ -931,6 +1051,26 @@ FastDiv fastDiv(int d) {
   return {(unsigned)((((uint64_t)1 << 32) * (((uint64_t)1 << shift) - d)) / d + 1), shift};
 }
 
+// How many wavefronts share a tile of conv_staged_kernel; 0: one of the other kernels is faster.  Us, what ran before / four /
+// eight wavefronts, a 3 x 3 unless said otherwise:
+//  * from 32 channel groups, up to two tiles a CU: 196 tiles of 32 groups 6.81 / - / 5.98, 112 of 128 20.8 / - / 16.8, 248 of
+//    128 20.0 / 18.0 / 16.0, 496 of 128 45.1 / 27.9 / 27.0; 588 of 128 45.5 / 37.2 / 37.3.  Of 16 groups, 392 tiles, 8.68 / 7.50 / -,
+//    but nothing to gain below (294: 0.96 times as fast);
+//  * four beyond: 784 tiles of 64-channel tiles 15.5 / 14.9 and, of 128 groups, 45.7 / 44.4; 980 of them 48.2 / 48.5: the 64 x 64
+//    tiles are as good from three a CU on.  Window tiles (`paired` false) are not: 1176 tiles of 96 channels 1.3-1.6 times as
+//    fast, 1568 of 32 channels 33.2 / 24.9; beyond eight a CU their two accumulators are (3136 tiles 28.0 / 29.7);
+//  * 5 x 5, a block's LDS holds one a CU of eight: 248 tiles of 32 groups 16.5 / 13.5 / 12.0, 442 tiles 42.9 / 23.3 / 24.2; of 8
+//    groups 442 tiles 16.6 / 7.7, but 784, just over three a CU, 0.89 times as fast; 10125 tiles of 16 groups 268 / 211; 64-channel
+//    tiles as above (784 tiles 43.3 / 36.2, 980 43.6 / 44.9).
+// 1 x 1 gained nothing: sixteen channels of a row are one line already.
+int stagedWaves(int win, int64_t tiles, int64_t groups, bool paired, int64_t cus) {
+  const int64_t few = win == 3 ? 2 * cus : cus, few4 = 3 * cus;
+  if (tiles <= few && groups >= (win == 3 ? 32 : 16)) return 8;
+  if (win == 3 && groups >= 16 && tiles > cus * 3 / 2 && tiles <= (paired ? few4 : 8 * cus)) return 4;
+  if (win == 5 && tiles > cus && (tiles <= few4 ? groups >= 8 : !paired && groups >= 16)) return 4;
+  return 0;
+}
+
 } // namespace
 
 void conv2d(const float *input, const float *weight, const float *bias, float *output, const float *postAdd,
@@ -997,6 +1137,11 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     conv_window_kernel<WIN, PT, KS><<<gridOf((pixels + perBlock - 1) / perBlock, 32, 256), dim3(256), 0, stream>>>(
         input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu);
   };
+  auto staged = [&](auto win, auto kss) {
+    constexpr int WIN = decltype(win)::value, KS = decltype(kss)::value;
+    conv_staged_kernel<WIN, KS><<<gridOf(pix32, 32, 64 * KS), dim3(64 * KS), 0, stream>>>(
+        input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu);
+  };
   auto tile = [&](auto win, auto kss) {
     constexpr int WIN = decltype(win)::value, KS = decltype(kss)::value;
     conv_tile_kernel<WIN, KS><<<gridOf((pixels + 63) / 64, 64, 256 * KS), dim3(256 * KS), 0, stream>>>(
@@ -1019,6 +1164,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
   //  * 96 channels are two 64-channel tiles with a quarter of nothing: 12 x 32 x 100 x 90 -> 96 takes 87 in LDS
   //    tiles and 66-75 in window tiles of two accumulators.
   const int64_t tiles = pix32 * ((OC + 31) / 32);
+  //    (Squares of 3 and 5 come here only where stagedWaves leaves them.)
   const bool squareWindow = KH == KW && (KH == 1 || KH == 3 || KH == 5 || KH == 7);
   if (!narrow) {
     table(std::true_type());
@@ -1054,6 +1200,11 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
       constexpr int WIN = decltype(win)::value;
       const int64_t units = ((IC + 2 * Window<WIN>::HALF - 1) / (2 * Window<WIN>::HALF)) * Window<WIN>::UNITS;
       const int64_t blocks = (pixels + 63) / 64 * ((OC + 63) / 64);
+      if constexpr (WIN == 3 || WIN == 5) {
+        const int ks = IC % 2 ? 0 : stagedWaves(WIN, tiles, IC / 2, (OC - 1) % 64 >= 32, numComputeUnits());
+        if (ks == 8) return staged(win, integral_constant<int, 8>());
+        if (ks == 4) return staged(win, c4);
+      }
       if (tiles <= 400) window(win, c1, c4);
       else if ((OC - 1) % 64 >= 32) {
         if (blocks <= numComputeUnits() && units >= 64) tile(win, c4);

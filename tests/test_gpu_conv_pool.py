@@ -59,6 +59,19 @@ def test_conv2d_of_few_taps_four_pixels_a_lane(pkg, gpu, oracle, rng, N, IC, H, 
     conv_case(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add)
 
 
+@pytest.mark.parametrize("N,IC,H,W,OC,K,pad,stride,dilation,relu,add", [
+    # eight wavefronts a tile: 33 and 35 groups of channels (cut shares, cut chunks, a last piece half past the filter's end), a
+    # last channel tile of one, images smaller than a tile; the smallest that takes it
+    (5, 66, 7, 7, 33, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, True), (2, 70, 9, 31, 32, (3, 3), (0, 2, 1, 0), (2, 1), (1, 2), False, False),
+    (1, 64, 1, 1, 1, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (3, 34, 11, 13, 40, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), True, True),
+    # four: 17, 19 and 35 groups, one and several channel tiles, 64-channel tiles cut, the last pixel tile cut
+    (5, 34, 50, 51, 32, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (8, 38, 41, 40, 48, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False),
+    (3, 70, 61, 60, 96, (3, 3), (2, 2, 2, 2), (1, 1), (2, 2), False, False), (4, 18, 30, 91, 32, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), False, True),
+    (9, 32, 50, 61, 32, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), True, False)])
+def test_conv2d_with_the_filter_through_lds(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add):
+    conv_case(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add)
+
+
 @pytest.mark.parametrize("C,H,W,K,pad,stride", [
     (3, 8, 8, (2, 2), (0, 0, 0, 0), (2, 2)), (2, 9, 7, (3, 3), (1, 1, 1, 1), (2, 2)),
     (64, 112, 112, (3, 3), (1, 1, 1, 1), (2, 2)),  # ResNet stem pool
