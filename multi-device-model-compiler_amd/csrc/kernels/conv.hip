@@ -570,7 +570,8 @@ __global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__
 // filter of its OCT x 32 channels in registers, lane half hl the taps 2 s + hl of step s, and walks
 // over tiles of 32 pixels; the taps of the next tile are in flight while this one's are multiplied
 // and stored.
-template <int OCT, int NS>
+enum class Output { Cached, Through, Added }; // written through to memory or not; an addend, and not
+template <int OCT, int NS, Output OUT>
 __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                                const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
                                                                int P, int N, FastDiv byP, FastDiv byOW, const float *__restrict__ add,
@@ -637,6 +638,41 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
   const bool fullOc = oc0 + 32 * OCT <= OC;
   const int64_t outElems = (int64_t)OC * P;
   auto finish = [&](Tile &o) {
+    // (stores through the bounds check too: a pixel or a channel past the end is dropped by it)
+    const auto out = resource(y + o.nFirst * outElems, (N - o.nFirst) * outElems);
+    const int at = o.pix < 0 ? kOutside : ((o.img * OC + oc0 + 4 * hl) * P + o.pix) * 4;
+    // (opaque, or the compiler keeps their multiples and comparisons in scalar registers across the loop)
+    int row = P * 4, channels = OC;
+    asm volatile("" : "+s"(row), "+s"(channels));
+    auto everyChannel = [&](auto each) { // of the lane: its register, its byte offsets
+      if (fullOc) {
+#pragma unroll
+        for (int t = 0; t < OCT; t++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            const int ocl = 32 * t + 8 * (r / 4) + r % 4;
+            each(t, r, at, ocl * row);
+          }
+      } else {
+#pragma unroll
+        for (int t = 0; t < OCT; t++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            const int ocl = 32 * t + 8 * (r / 4) + r % 4;
+            if (oc0 + ocl < channels) // (a scalar offset past the resource would wrap the check)
+              each(t, r, oc0 + ocl + 4 * hl < channels ? at : kOutside, ocl * row);
+          }
+      }
+    };
+    // (the addend is in flight under the matrix instructions: loaded channel by channel between the stores, each load
+    // waited for the stores before it; 8 x 3 x 224 x 224 -> 64 of stride 2 32.1 -> 17.0 us, 6 x 1 x 12 x 91 -> 256 7.0 -> 5.3)
+    float addend[OCT][16];
+    if (OUT == Output::Added) {
+      const auto post = resource(add + o.nFirst * outElems, (N - o.nFirst) * outElems);
+      everyChannel([&](int t, int r, int voffset, int soffset) {
+        addend[t][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(post, voffset, soffset, 0));
+      });
+    }
     f32x16 acc[OCT];
 #pragma unroll
     for (int t = 0; t < OCT; t++)
@@ -646,37 +682,12 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
     for (int s = 0; s < NS; s++)
 #pragma unroll
       for (int t = 0; t < OCT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t][s], o.b[s], acc[t], 0, 0, 0);
-    // (stores through the bounds check too: a pixel or a channel past the end is dropped by it)
-    const auto out = resource(y + o.nFirst * outElems, (N - o.nFirst) * outElems);
-    const auto post = resource(add + (add ? o.nFirst * outElems : 0), (N - o.nFirst) * outElems);
-    const int at = o.pix < 0 ? kOutside : ((o.img * OC + oc0 + 4 * hl) * P + o.pix) * 4;
-    // (opaque, or the compiler keeps their multiples and comparisons in scalar registers across the loop)
-    int row = P * 4, channels = OC;
-    asm volatile("" : "+s"(row), "+s"(channels));
-    // (written through to memory: 8 x 3 x 224 x 224 -> 64 33.2 -> 31.8 us, 4 x 3 x 224 x 224 -> 32 of stride 2 7.40 -> 6.86)
-    auto store = [&](int ocl, float v, int voffset, int soffset) {
-      if (add) v += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(post, voffset, soffset, 0));
+    everyChannel([&](int t, int r, int voffset, int soffset) {
+      const float v = OUT == Output::Added ? acc[t][r] + addend[t][r] : acc[t][r];
       // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, relu ? fmaxf(v, 0.0f) : v), out, voffset, soffset, 16);
-    };
-    if (fullOc) {
-#pragma unroll
-      for (int t = 0; t < OCT; t++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int ocl = 32 * t + 8 * (r / 4) + r % 4;
-          store(ocl, acc[t][r], at, ocl * row);
-        }
-    } else {
-#pragma unroll
-      for (int t = 0; t < OCT; t++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int ocl = 32 * t + 8 * (r / 4) + r % 4;
-          if (oc0 + ocl < channels) // (a scalar offset past the resource would wrap the check)
-            store(ocl, acc[t][r], oc0 + ocl + 4 * hl < channels ? at : kOutside, ocl * row);
-        }
-    }
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, relu ? fmaxf(v, 0.0f) : v), out, voffset, soffset,
+                                            OUT == Output::Through ? 16 : 0);
+    });
   };
   Tile even, odd;
   int tile = (int)blockIdx.x * 4 + wave;
@@ -702,7 +713,7 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
 // instructions of the next measured the same, an order of tiles by XCD too, runs of tiles a wavefront 90.
 // STREAM: an output beyond what the Infinity Cache keeps leaves by non-temporal stores (72 against 65.5 us above), a smaller
 // one is written through (4 x 3 x 256 x 256 -> 64 20.6 non-temporal, 21.4 plain, 19.2 so).
-template <int KW, int NR, bool STREAM>
+template <int KW, int NR, bool STREAM, bool ADDED>
 __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                             const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
                                                             int P, int N, FastDiv byP, FastDiv byOW, const float *__restrict__ add,
@@ -769,6 +780,27 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
   };
   const int64_t outElems = (int64_t)OC * P;
   auto finish = [&](Tile &o) {
+    const auto out = resource(y + o.nFirst * outElems, (N - o.nFirst) * outElems);
+    const int at = o.pix < 0 ? kOutside : ((o.img * OC + oc0 + 4 * hl) * P + o.pix) * 4;
+    int row = P * 4, channels = OC;
+    asm volatile("" : "+s"(row), "+s"(channels));
+    auto everyChannel = [&](auto each) { // of the lane: its register, its byte offsets
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const int ocl = 8 * (r / 4) + r % 4;
+        if (oc0 + ocl >= channels) break; // (uniform; a scalar offset past the resource would wrap the check)
+        each(r, oc0 + ocl + 4 * hl < channels ? at : kOutside, ocl * row);
+      }
+    };
+    // The addend: in flight under the matrix instructions (16 x 3 x 256 x 256 -> 64 140 -> 126 us, 8 x 1 x 128 x 128 -> 96, 5 x 5,
+    // 27.1 -> 22.0), where the registers last: NR = 8 loads it a channel at a time (8 x 16 x 128 x 128 -> 64 15.8, so 21.6).
+    constexpr bool kEarly = NR < 8;
+    const auto post = resource(add + (ADDED ? o.nFirst * outElems : 0), (N - o.nFirst) * outElems);
+    auto fromPost = [&](int voffset, int soffset) {
+      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(post, voffset, soffset, 0));
+    };
+    f32x4 addend[16];
+    if (ADDED && kEarly) everyChannel([&](int r, int voffset, int soffset) { addend[r] = fromPost(voffset, soffset); });
     f32x16 acc[4];
 #pragma unroll
     for (int j = 0; j < 4; j++)
@@ -792,22 +824,13 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][k], c[k + j], acc[j], 0, 0, 0);
     }
-    const auto out = resource(y + o.nFirst * outElems, (N - o.nFirst) * outElems);
-    const auto post = resource(add + (add ? o.nFirst * outElems : 0), (N - o.nFirst) * outElems);
-    const int at = o.pix < 0 ? kOutside : ((o.img * OC + oc0 + 4 * hl) * P + o.pix) * 4;
-    int row = P * 4, channels = OC;
-    asm volatile("" : "+s"(row), "+s"(channels));
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int ocl = 8 * (r / 4) + r % 4;
-      if (oc0 + ocl >= channels) break; // (uniform; a scalar offset past the resource would wrap the check)
-      const int voffset = oc0 + ocl + 4 * hl < channels ? at : kOutside;
+    everyChannel([&](int r, int voffset, int soffset) {
       f32x4 v = {acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
-      if (add) v += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(post, voffset, ocl * row, 0));
+      if (ADDED) v += kEarly ? addend[r] : fromPost(voffset, soffset);
       // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
       if (relu) v = f32x4{fmaxf(v[0], 0.0f), fmaxf(v[1], 0.0f), fmaxf(v[2], 0.0f), fmaxf(v[3], 0.0f)};
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, voffset, ocl * row, STREAM ? 2 : 16);
-    }
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, voffset, soffset, STREAM ? 2 : 16);
+    });
   };
   Tile even, odd;
   int tile = (int)blockIdx.x * 4 + wave;
@@ -1112,12 +1135,19 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
   const int64_t images = 63 / P + 2;
   const bool narrow = fitsInt(pixels) && fitsInt(images * IC * H * W * 4) && fitsInt(images * OC * P * 4) &&
                       fitsInt(65 * K * 4) && KH <= 31 && KW <= 31;
+  // Few taps: stores written through to memory (us, not / written through: 12 x 1 x 12 x 91 -> 256 7.8 / 6.9, 8 x 3 x 224 x 224 ->
+  // 64 of stride 2 16.1 / 14.4, 8 x 3 x 224 x 224 -> 64 33.2 / 31.8), unless much is written and a tile's runs of 32 pixels are no whole
+  // lines, which then go to memory twice (4 x 3 x 223 x 225 -> 64, 51 MB, 20.1 / 20.6, 103 MB 40.9 / 47.1; 28 MB 10.3 / 9.1), and
+  // not beside an addend, whose loads wait for them (6 x 1 x 12 x 91 -> 256 7.0 / 9.7).
+  const bool through = P % 32 == 0 || N * OC * P * 4 <= int64_t(32) << 20;
   auto few = [&](auto octs, auto nss) {
     constexpr int OCT = decltype(octs)::value, NS = decltype(nss)::value;
     // two blocks per CU and channel tile at the registers of OCT = 2, four at those of OCT = 1
     const int64_t most = std::max<int64_t>(1, (int64_t)numComputeUnits() * (4 / OCT) / ((OC + 32 * OCT - 1) / (32 * OCT)));
     const int64_t blocks = std::min((pix32 + 3) / 4, most);
-    conv_few_taps_kernel<OCT, NS><<<gridOf(blocks, 32 * OCT, 256), dim3(256), 0, stream>>>(
+    auto *kernel = add ? conv_few_taps_kernel<OCT, NS, Output::Added>
+                       : through ? conv_few_taps_kernel<OCT, NS, Output::Through> : conv_few_taps_kernel<OCT, NS, Output::Cached>;
+    kernel<<<gridOf(blocks, 32 * OCT, 256), dim3(256), 0, stream>>>(
         input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu, (int)K, (int)pix32, (int)(4 * blocks));
   };
   const int64_t tiles128 = (pixels + 127) / 128;
@@ -1127,7 +1157,8 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     // two blocks per CU and channel tile
     const int64_t most = std::max<int64_t>(1, (int64_t)numComputeUnits() * 2 / ((OC + 31) / 32));
     const int64_t blocks = std::min((tiles128 + 3) / 4, most);
-    auto *kernel = streams ? conv_quads_kernel<KWC, NR, true> : conv_quads_kernel<KWC, NR, false>;
+    auto *kernel = add ? (streams ? conv_quads_kernel<KWC, NR, true, true> : conv_quads_kernel<KWC, NR, false, true>)
+                       : streams ? conv_quads_kernel<KWC, NR, true, false> : conv_quads_kernel<KWC, NR, false, false>;
     kernel<<<gridOf(blocks, 32, 256), dim3(256), 0, stream>>>(input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu,
                                                               (int)tiles128, (int)(4 * blocks));
   };
