@@ -39,11 +39,11 @@ constexpr int kThreads = 512;
 __host__ __device__ constexpr int aSwz(int row) { return (row >> 1) & 7; }
 template <int BN> __host__ __device__ constexpr int wSwz(int row) { return BN == 192 ? ((row >> 1) & 1) << 2 : (row & 3) << 2; }
 
-// ACT: the activation, or kResidual in its place.
+// ACT: the activation, or kResidual in its place.  Out: uint16_t for T's own type, or float.
 constexpr int kResidual = 3;
-template <typename T, int ACT, int BN>
+template <typename T, int ACT, int BN, typename Out>
 __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
-                                                                const uint16_t *__restrict__ bias, const uint16_t *residual, uint16_t *out,
+                                                                const uint16_t *__restrict__ bias, const uint16_t *residual, Out *out,
                                                                 int N, int K, int tilesN, int tilesM, int M_) {
   using M = Mma<T>;
   using v8 = typename M::v8;
@@ -285,8 +285,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const uint16_t *
   // Through a staging area of the wavefront's own (the LDS accesses of one wavefront are ordered), in the layout of the
   // output's rows: a residual, asked for before the last k-steps, comes in through it and the result goes out through it.
   // One 32-row half of the part after the other, so that the first one's stores drain under the second one's arithmetic.
+  // (fp32: the same area holds one half's rows, 16 * odd bytes apart.)
   __syncthreads(); // every wavefront is done reading the ring
-  const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(out + partAt, 0, partBytes, 0x00020000);
+  constexpr bool kWide = sizeof(Out) == 4;
+  constexpr int kOutSize = (int)sizeof(Out), kStoreChunks = kOutChunks * kOutSize / 2, kStoreCols = kStoreChunks == 12 || kStoreChunks == 24 ? 3 : 1,
+                kStoreRowStep = 64 * kStoreCols / kStoreChunks;
+  const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(out + partAt, 0, partBytes / 2 * kOutSize, 0x00020000);
+  float *wideStage = reinterpret_cast<float *>(stage);
+  uint32_t soff[kStoreCols];
+  int sat[kStoreCols];
+#pragma unroll
+  for (int i = 0; i < kStoreCols; i++) {
+    const int r = (64 * i + lane) / kStoreChunks, c = (64 * i + lane) % kStoreChunks;
+    soff[i] = nw + 16 / kOutSize * c < N ? (uint32_t)(r * N * kOutSize + c * 16) : 0x40000000u;
+    sat[i] = r * kOutStride + 16 / kOutSize * c;
+  }
 #pragma unroll
   for (int mb = 0; mb < 2; mb++) {
     uint16_t *pieces = &stage[(32 * mb + l32) * kOutStride + 4 * hl];
@@ -309,23 +322,32 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const uint16_t *
 #pragma unroll
       for (int g = 0; g < 4; g++) { // four consecutive columns
         v4 o;
+        f32x4 wide;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           float x = acc[nb][mb][4 * g + i];
           if (ACT == ACT_RELU) x = x > 0.0f ? x : 0.0f;
           if (ACT == ACT_GELU) x = M::gelu(x);
           if (ACT == kResidual) x += M::widen(r[nb][g][i]);
-          o[i] = M::narrow(x);
+          if (kWide) wide[i] = x;
+          else o[i] = M::narrow(x);
         }
-        *reinterpret_cast<v4 *>(pieces + 32 * nb + 8 * g) = o;
+        if (kWide) *reinterpret_cast<f32x4 *>(&wideStage[l32 * kOutStride + 4 * hl + 32 * nb + 8 * g]) = wide;
+        else *reinterpret_cast<v4 *>(pieces + 32 * nb + 8 * g) = o;
       }
 #pragma unroll
-    for (int it = 0; it < kOutChunks / 2; it++) {
-      const int row = 32 * mb + it / kCols * kRowStep;
-      const uint16_t *p = staged[it % kCols] + row * kOutStride;
-      const u32x2 lo = *reinterpret_cast<const u32x2 *>(p);
-      const u32x2 hi = *reinterpret_cast<const u32x2 *>(p + 4);
-      __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], lo[1], hi[0], hi[1]}, rows, goff[it % kCols] + (uint32_t)(row * N * 2), 0, 16);
+    for (int it = 0; it < kStoreChunks / 2; it++) {
+      const int row = it / kStoreCols * kStoreRowStep;
+      u32x4 v;
+      if (kWide) {
+        v = *reinterpret_cast<const u32x4 *>(&wideStage[row * kOutStride + sat[it % kStoreCols]]);
+      } else {
+        const uint16_t *p = &stage[(32 * mb + row) * kOutStride + sat[it % kStoreCols]];
+        const u32x2 lo = *reinterpret_cast<const u32x2 *>(p);
+        const u32x2 hi = *reinterpret_cast<const u32x2 *>(p + 4);
+        v = u32x4{lo[0], lo[1], hi[0], hi[1]};
+      }
+      __builtin_amdgcn_raw_buffer_store_b128(v, rows, soff[it % kStoreCols] + (uint32_t)((32 * mb + row) * N * kOutSize), 0, 16);
     }
   }
 }
@@ -335,10 +357,19 @@ void launch(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint1
             int act, hipStream_t stream) {
   const int tilesM = (int)((M + kBM - 1) / kBM), tilesN = (int)((N + BN - 1) / BN);
   const dim3 grid((unsigned)(tilesM * tilesN)), block(kThreads);
-  if (r) gemm_wide_kernel<T, kResidual, BN><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_GELU) gemm_wide_kernel<T, ACT_GELU, BN><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_RELU) gemm_wide_kernel<T, ACT_RELU, BN><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else gemm_wide_kernel<T, ACT_NONE, BN><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  if (r) gemm_wide_kernel<T, kResidual, BN, uint16_t><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_GELU) gemm_wide_kernel<T, ACT_GELU, BN, uint16_t><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_RELU) gemm_wide_kernel<T, ACT_RELU, BN, uint16_t><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else gemm_wide_kernel<T, ACT_NONE, BN, uint16_t><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  MGPU_CHECK_LAUNCH("gemm_wide_kernel");
+}
+
+template <int BN>
+void launchToF32(const void *a, const void *w, const void *b, const void *r, float *o, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
+  const int tilesM = (int)((M + kBM - 1) / kBM), tilesN = (int)((N + BN - 1) / BN);
+  gemm_wide_kernel<_Float16, kResidual, BN, float><<<dim3((unsigned)(tilesM * tilesN)), dim3(kThreads), 0, stream>>>(
+      static_cast<const uint16_t *>(a), static_cast<const uint16_t *>(w), static_cast<const uint16_t *>(b), static_cast<const uint16_t *>(r), o,
+      (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_wide_kernel");
 }
 
@@ -399,6 +430,14 @@ void gemmWide(DType dt, const void *in, const void *weight, const void *bias, co
     fail("gemmWide: internal dispatch error");
   if (dt == DType::F16) launchWidth<_Float16>(in, weight, bias, residual, out, M, N, K, act, width, stream);
   else launchWidth<bf16_t>(in, weight, bias, residual, out, M, N, K, act, width, stream);
+}
+
+void gemmWideResidualF32(const void *in, const void *weight, const void *bias, const void *residual, float *out, int64_t M, int64_t N, int64_t K,
+                         int width, hipStream_t stream) {
+  if (!gemmWideSupports(DType::F16, in, weight, bias, residual, out, M, N, K) || !residual) fail("gemmWide: internal dispatch error");
+  if (width == 256) launchToF32<256>(in, weight, bias, residual, out, M, N, K, stream);
+  else if (width == 192) launchToF32<192>(in, weight, bias, residual, out, M, N, K, stream);
+  else launchToF32<128>(in, weight, bias, residual, out, M, N, K, stream);
 }
 
 } // namespace mgpu

@@ -106,6 +106,9 @@ bool gemmWideSupports(DType dt, const void *in, const void *weight, const void *
                       int64_t N, int64_t K);
 void gemmWide(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
               int64_t K, int act, int width, hipStream_t stream);
+// fp16 operands, in . weight + bias + residual in fp32.
+void gemmWideResidualF32(const void *in, const void *weight, const void *bias, const void *residual, float *out, int64_t M, int64_t N, int64_t K,
+                         int width, hipStream_t stream);
 
 // At most one tile of 128 x 96 or 128 x 128 per CU (gemm_round.hip), for gemm_mfma.hip's launchers: N a multiple of 8, K of 64.
 void gemmRound(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,

@@ -46,6 +46,25 @@ def test_against_float64(pkg, gpu, dtype, name, width, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("width", [128, 192, 256])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_fp32_result_against_float64(pkg, gpu, width, M, N, K):
+    import torch
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    r = lambda *s: torch.randn(s, generator=g, device=gpu)
+    x, w, b, res = r(M, K).half(), (r(K, N) / K**0.5).half(), r(N).half(), r(M, N).half()
+    gemm = internal(pkg, "_ZN4mgpu19gemmWideResidualF32EPKvS1_S1_S1_PfllliP12ihipStream_t", None, *[ctypes.c_void_p] * 5,
+                    *[ctypes.c_int64] * 3, ctypes.c_int, ctypes.c_void_p)
+    out = torch.full((M + 2, N), 7.0, device=gpu)  # a row before and one behind
+    gemm(x.data_ptr(), w.data_ptr(), b.data_ptr(), res.data_ptr(), out[1:].data_ptr(), M, N, K, width, torch.cuda.current_stream().cuda_stream)
+    got, X, W, B, R = [t.double().cpu() for t in (out, x, w, b, res)]
+    # K + 2 fp32 roundings of partial sums no larger than |x||w| + |b| + |residual|
+    bound = (K + 2) * 2.0**-24 * (X.abs() @ W.abs() + B.abs() + R.abs())
+    assert ((got[1:-1] - (X @ W + B + R)).abs() <= bound).all()
+    assert (got[0] == 7).all() and (got[-1] == 7).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("width,M,N,K,parts", [(96, 300, 200, 512, 2), (128, 131, 264, 1088, 4), (96, 128, 96, 832, 3)])
 def test_planes_of_partial_sums(pkg, gpu, width, M, N, K, parts):
     """Shares of unequal length; the planes add up to the product."""
