@@ -19,7 +19,7 @@
 //   quads     (the same, many tiles, rows of whole quads, stride 1 across)  four pixels a lane
 //   window    (1, 3, 5 or 7 square, few tiles)  operands straight from L1 / L2 into registers,
 //             four wavefronts per tile
-//   staged    (3 or 5 square, even channels, few tiles)  the same with the filter through LDS
+//   staged    (3, 5 or 7 square, even channels, few tiles)  the same with the filter through LDS
 //   tile      (the same windows, many tiles)    operands shared through LDS by 64 x 64 tiles
 //   table     (every other window, and images beyond 2 GiB)  tap offsets from a table in LDS
 // What bounds them: one 32x32x2 MFMA takes 64 cycles of a SIMD (157 TFLOP/s on the chip) and the
@@ -453,9 +453,10 @@ __global__ __launch_bounds__(256, 2) void conv_window_kernel(const float *__rest
 // at a time, 16 bytes a lane, under the matrix instructions of the groups before -, keeps them in an LDS area of its own (no
 // barrier) and reads an operand a step from there.
 template <int WIN> struct Staged {
-  static constexpr int CG = WIN == 5 ? 2 : 4;                          // channel groups staged at a time
-  static constexpr int ROW = CG * 2 * Window<WIN>::HALF * WIN * WIN;   // floats of a channel's row among them: a multiple of 4
-  static constexpr int PIECES = ROW / 4, LOADS = (32 * PIECES + 63) / 64;
+  static constexpr int CG = WIN == 7 ? 1 : WIN == 5 ? 2 : 4;           // channel groups staged at a time
+  static constexpr int ROW = CG * 2 * Window<WIN>::HALF * WIN * WIN;   // floats of a channel's row among them
+  static constexpr int PIECE = ROW % 4 == 0 ? 4 : 2;                   // floats loaded at a time
+  static constexpr int PIECES = ROW / PIECE, LOADS = (32 * PIECES + 63) / 64;
   static constexpr int PITCH = ROW % 16 == 0 ? ROW + 4 : ROW + (ROW % 8 == 0 ? 4 : 0); // 4 or 12 modulo 16 words: 16 rows on different banks
 };
 template <int WIN, int KS>
@@ -476,7 +477,10 @@ __global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__
   const int HW4 = g.H * g.W * 4, pixels = N * P;
 
   const int nFirst = __builtin_amdgcn_readfirstlane(divide(q0 < pixels ? q0 : pixels - 1, byP));
-  int pix[1], img[1], voff[KK];
+  // A tap's byte offset, kOutside where it lies outside; 7 x 7, whose 49 would not leave the registers for the filter: the first
+  // window row's, and in bit 31 - kh of rowOut which rows lie outside.
+  int pix[1], img[1], voff[WIN == 7 ? WIN : KK];
+  unsigned rowOut = 0;
   {
     const int q = q0 + l32;
     const bool live = q < pixels;
@@ -487,13 +491,21 @@ __global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__
     pix[0] = live ? p : -1;
     const int ih0 = live ? oh * g.SH - g.PHL : -kNever, iw0 = ow * g.SW - g.PWL;
     const int base = (img[0] * g.IC + hl * HALF) * HW4 + ((oh * g.SH - g.PHL) * g.W + iw0) * 4;
+    if constexpr (WIN == 7) {
 #pragma unroll
-    for (int kh = 0; kh < WIN; kh++)
-#pragma unroll
-      for (int kw = 0; kw < WIN; kw++) {
-        const bool in = (unsigned)(ih0 + kh * g.DH) < (unsigned)g.H && (unsigned)(iw0 + kw * g.DW) < (unsigned)g.W;
-        voff[kh * WIN + kw] = in ? base + (kh * g.DH * g.W + kw * g.DW) * 4 : kOutside;
+      for (int k = 0; k < WIN; k++) {
+        voff[k] = (unsigned)(iw0 + k * g.DW) < (unsigned)g.W ? base + k * g.DW * 4 : kOutside;
+        rowOut |= (unsigned)(ih0 + k * g.DH) < (unsigned)g.H ? 0u : 0x80000000u >> k;
       }
+    } else {
+#pragma unroll
+      for (int kh = 0; kh < WIN; kh++)
+#pragma unroll
+        for (int kw = 0; kw < WIN; kw++) {
+          const bool in = (unsigned)(ih0 + kh * g.DH) < (unsigned)g.H && (unsigned)(iw0 + kw * g.DW) < (unsigned)g.W;
+          voff[kh * WIN + kw] = in ? base + (kh * g.DH * g.W + kw * g.DW) * 4 : kOutside;
+        }
+    }
   }
   const int64_t imageElems = (int64_t)g.IC * g.H * g.W;
   const auto image = resource(x + nFirst * imageElems, (N - nFirst) * imageElems);
@@ -513,28 +525,33 @@ __global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__
 #pragma unroll
   for (int i = 0; i < St::LOADS; i++) {
     const int p = i * 64 + lane, oc = p / St::PIECES;
-    woff[i] = oc < 32 ? ((oc0 + oc < OC ? oc : OC - 1 - oc0) * g.IC * KK + 4 * (p - oc * St::PIECES)) * 4 : kOutside;
+    woff[i] = oc < 32 ? ((oc0 + oc < OC ? oc : OC - 1 - oc0) * g.IC * KK + St::PIECE * (p - oc * St::PIECES)) * 4 : kOutside;
   }
-  f32x4 stage[St::LOADS];
+  typedef float Piece __attribute__((ext_vector_type(St::PIECE)));
+  Piece stage[St::LOADS];
   auto load = [&](int group) {
 #pragma unroll
     for (int i = 0; i < St::LOADS; i++)
-      stage[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(filter, woff[i], group * (2 * HALF * KK * 4), 0));
+      if constexpr (St::PIECE == 4) stage[i] = __builtin_bit_cast(Piece, __builtin_amdgcn_raw_buffer_load_b128(filter, woff[i], group * (2 * HALF * KK * 4), 0));
+      else stage[i] = __builtin_bit_cast(Piece, __builtin_amdgcn_raw_buffer_load_b64(filter, woff[i], group * (2 * HALF * KK * 4), 0));
   };
   auto keep = [&]() {
 #pragma unroll
     for (int i = 0; i < St::LOADS; i++) {
       const int p = i * 64 + lane, oc = p / St::PIECES;
-      if (64 * (i + 1) <= 32 * St::PIECES || oc < 32) *reinterpret_cast<f32x4 *>(mine + oc * St::PITCH + 4 * (p - oc * St::PIECES)) = stage[i];
+      if (64 * (i + 1) <= 32 * St::PIECES || oc < 32) *reinterpret_cast<Piece *>(mine + oc * St::PITCH + St::PIECE * (p - oc * St::PIECES)) = stage[i];
     }
   };
   // The reduction walks units - a group, or one of its window rows - in a pipeline two deep: a unit's taps fly under the
   // matrix instructions of the one before.
   auto fetch = [&](float (&b)[STEPS], int group, int unit) {
+    const unsigned out = (rowOut << unit) & 0x80000000u;
+    const int down = unit * g.DH * g.W * 4;
 #pragma unroll
-    for (int i = 0; i < STEPS; i++)
-      b[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(image, voff[WIN == 1 ? 0 : unit * STEPS + i],
-                                                                            (group * (2 * HALF) + (WIN == 1 ? i : 0)) * HW4, 0));
+    for (int i = 0; i < STEPS; i++) {
+      const int at = WIN == 7 ? (int)((unsigned)(voff[i] + down) | out) : voff[WIN == 1 ? 0 : unit * STEPS + i];
+      b[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(image, at, (group * (2 * HALF) + (WIN == 1 ? i : 0)) * HW4, 0));
+    }
   };
   const float *ap = mine + l32 * St::PITCH + hl * (HALF * KK);
   auto multiply = [&](const float (&b)[STEPS], int inChunk, int unit) {
@@ -542,22 +559,27 @@ __global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__
     for (int i = 0; i < STEPS; i++)
       acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(ap[inChunk * (2 * HALF * KK) + unit * STEPS + i], b[i], acc[0], 0, 0, 0);
   };
-  constexpr int NU = St::CG * UNITS; // units of a chunk: an even number
+  constexpr int NU = St::CG * UNITS, TURN = NU % 2 ? 2 : 1; // units of a chunk; chunks until a unit's buffer is the first again
   float b[2][STEPS];
   if (g0 < g1) {
     load(g0);
     fetch(b[0], g0, 0);
   }
-  for (int chunk = g0; chunk < g1; chunk += St::CG) {
-    keep();
-    if (chunk + St::CG < g1) load(chunk + St::CG);
+  for (int turn = g0; turn < g1; turn += TURN * St::CG) {
 #pragma unroll
-    for (int u = 0; u < NU; u++) {
-      const int group = chunk + u / UNITS;
-      if (u % UNITS == 0 && group >= g1) break; // (uniform)
-      const int next = u + 1; // (fetched if it is still in the share)
-      if (chunk + next / UNITS < g1) fetch(b[next % 2], chunk + next / UNITS, next % UNITS);
-      multiply(b[u % 2], u / UNITS, u % UNITS);
+    for (int h = 0; h < TURN; h++) {
+      const int chunk = turn + h * St::CG;
+      if (h && chunk >= g1) break; // (uniform)
+      keep();
+      if (chunk + St::CG < g1) load(chunk + St::CG);
+#pragma unroll
+      for (int u = 0; u < NU; u++) {
+        const int group = chunk + u / UNITS;
+        if (u % UNITS == 0 && group >= g1) break; // (uniform)
+        const int next = u + 1; // (fetched if it is still in the share)
+        if (chunk + next / UNITS < g1) fetch(b[(h * NU + next) % 2], chunk + next / UNITS, next % UNITS);
+        multiply(b[(h * NU + u) % 2], u / UNITS, u % UNITS);
+      }
     }
   }
   if (KS > 1) __syncthreads(); // the partial sums take the filter rows' place
@@ -1085,9 +1107,12 @@ FastDiv fastDiv(int d) {
 //  * 5 x 5, a block's LDS holds one a CU of eight: 248 tiles of 32 groups 16.5 / 13.5 / 12.0, 442 tiles 42.9 / 23.3 / 24.2; of 8
 //    groups 442 tiles 16.6 / 7.7, but 784, just over three a CU, 0.89 times as fast; 10125 tiles of 16 groups 268 / 211; 64-channel
 //    tiles as above (784 tiles 43.3 / 36.2, 980 43.6 / 44.9).
+//  * 7 x 7, the same: 196 tiles of 32 groups 35.5 / 22.3 / 21.0, 112 of 128 156 / 85 / 75, 324 of 64 165 / 81 / 80, 784 of 8 33.9 / 23.2 /
+//    28.1, 6272 of 16 427 / 250 / 290; 64-channel tiles 784 of 8 25.7 / 22.0 / 27.0, of 16 39.3 / 38.5 / 43.3, 980 of 32 81.9 / 82.4.
 // 1 x 1 gained nothing: sixteen channels of a row are one line already.
 int stagedWaves(int win, int64_t tiles, int64_t groups, bool paired, int64_t cus) {
   const int64_t few = win == 3 ? 2 * cus : cus, few4 = 3 * cus;
+  if (win == 7) return groups < 8 || (paired && tiles > few4) ? 0 : tiles <= cus ? 8 : 4;
   if (tiles <= few && groups >= (win == 3 ? 32 : 16)) return 8;
   if (win == 3 && groups >= 16 && tiles > cus * 3 / 2 && tiles <= (paired ? few4 : 8 * cus)) return 4;
   if (win == 5 && tiles > cus && (tiles <= few4 ? groups >= 8 : !paired && groups >= 16)) return 4;
@@ -1231,7 +1256,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
       constexpr int WIN = decltype(win)::value;
       const int64_t units = ((IC + 2 * Window<WIN>::HALF - 1) / (2 * Window<WIN>::HALF)) * Window<WIN>::UNITS;
       const int64_t blocks = (pixels + 63) / 64 * ((OC + 63) / 64);
-      if constexpr (WIN == 3 || WIN == 5) {
+      if constexpr (WIN >= 3) {
         const int ks = IC % 2 ? 0 : stagedWaves(WIN, tiles, IC / 2, (OC - 1) % 64 >= 32, numComputeUnits());
         if (ks == 8) return staged(win, integral_constant<int, 8>());
         if (ks == 4) return staged(win, c4);

@@ -67,7 +67,10 @@ def test_conv2d_of_few_taps_four_pixels_a_lane(pkg, gpu, oracle, rng, N, IC, H, 
     # four: 17, 19 and 35 groups, one and several channel tiles, 64-channel tiles cut, the last pixel tile cut
     (5, 34, 50, 51, 32, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (8, 38, 41, 40, 48, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False),
     (3, 70, 61, 60, 96, (3, 3), (2, 2, 2, 2), (1, 1), (2, 2), False, False), (4, 18, 30, 91, 32, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), False, True),
-    (9, 32, 50, 61, 32, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), True, False)])
+    (9, 32, 50, 61, 32, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), True, False),
+    # 7 x 7: rows and columns outside on every side, dilation, eight groups and an odd number; eight and four wavefronts
+    (2, 18, 5, 6, 33, (7, 7), (3, 3, 3, 3), (1, 1), (1, 1), True, True), (3, 16, 20, 23, 40, (7, 7), (4, 6, 5, 2), (2, 1), (1, 2), False, False),
+    (4, 22, 41, 60, 32, (7, 7), (3, 3, 3, 3), (1, 1), (1, 1), False, True), (3, 16, 50, 51, 64, (7, 7), (3, 3, 3, 3), (1, 1), (2, 1), True, False)])
 def test_conv2d_with_the_filter_through_lds(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add):
     conv_case(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add)
 
