@@ -13,10 +13,11 @@
 // columns, so that a register of an accumulator is 32 consecutive pixels of a channel: whole
 // 128-byte runs of the NCHW output.  The tap matrix is never written to memory.  Taps come
 // through buffer loads, whose bounds check answers 0 for an offset outside the image: padding costs
-// no branch and no second instruction.  Six kernels share the work (conv2d below has the rule and
+// no branch and no second instruction.  Seven kernels share the work (conv2d below has the rule and
 // the measurements behind it):
 //   few taps  (K <= 32, a network's stem)  filter in registers, wavefronts walk over pixel tiles
 //   quads     (the same, many tiles, rows of whole quads, stride 1 across)  four pixels a lane
+//   patch     (5 or 7 square from one channel or three)  input rows through LDS, once for all taps
 //   window    (1, 3, 5 or 7 square, few tiles)  operands straight from L1 / L2 into registers,
 //             four wavefronts per tile
 //   staged    (3, 5 or 7 square, even channels, few tiles)  the same with the filter through LDS
@@ -866,6 +867,155 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
   }
 }
 
+// ---- larger windows over few channels -----------------------------------------------------------
+// A stem: 5 x 5 or 7 x 7 from one channel or three, 49 to 147 taps.  The window kernel reads a tap a lane from memory for every
+// matrix instruction and pairs channels, of which one or three leave a quarter or half for nothing (8 x 3 x 224 x 224 -> 64, 7 x 7
+// of stride 2: 44 us, 13 by the matrix cores; now 30).  Here a tile is 32 neighbouring pixels of one output row, and the input under it
+// - IC * KH window rows of 31 SW + KW columns - comes in whole lines into an LDS patch of the wavefront's own, each element
+// once, with zeros where the window leaves the image, while the tile before is multiplied.  Lane half hl takes window rows
+// hl * NR and on, so that a step's taps lie at one immediate offset from the lane's place in the patch; the filter lies in LDS in the
+// order of the steps.  The loop is LDS reads and matrix instructions, nothing else.
+template <int KW, int NR, int SW, bool ADDED>
+__global__ __launch_bounds__(256, 2) void conv_patch_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                            const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC, int P,
+                                                            int N, FastDiv byAcross, FastDiv byOH, const float *__restrict__ add, int relu,
+                                                            int across, int tiles, int tileStep) {
+  constexpr int COLS = 31 * SW + KW, LOADS = (2 * NR * COLS + 63) / 64, STEPS = NR * KW;
+  constexpr int PITCH = 33;                // channels of a step, apart for the writes along the steps
+  __shared__ float filter[STEPS * 2 * PITCH]; // [step][lane half][channel]
+  __shared__ float patches[4][LOADS * 64];
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int l32 = lane % 32, hl = lane / 32;
+  const int oc0 = blockIdx.y * 32, rows = g.IC * g.KH;
+  constexpr int FILL = (STEPS * 2 * 32 + 255) / 256;
+  float fill[FILL]; // (all in flight at once)
+  const auto weights = resource(w + (int64_t)oc0 * (rows * KW), (int64_t)(OC - oc0) * (rows * KW));
+#pragma unroll
+  for (int i = 0; i < FILL; i++) {
+    const int e = i * 256 + tid, oc = e / (2 * STEPS), k = e - oc * (2 * STEPS);
+    fill[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(weights, k < rows * KW ? (oc * (rows * KW) + k) * 4 : kOutside, 0, 0));
+  }
+#pragma unroll
+  for (int i = 0; i < FILL; i++) {
+    const int e = i * 256 + tid, oc = e / (2 * STEPS), k = e - oc * (2 * STEPS), half = k / STEPS;
+    if (oc < 32) filter[((k - half * STEPS) * 2 + half) * PITCH + oc] = fill[i];
+  }
+  float bv[16]; // the accumulators start from the bias
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int oc = oc0 + 8 * (r / 4) + r % 4 + 4 * hl;
+    bv[r] = bias[oc < OC ? oc : OC - 1];
+  }
+  // Element i * 64 + lane of the patch: its byte offset from the tile's first tap (kOutside past the last window row), column and row
+  // in the window.
+  int poff[LOADS], pcol[LOADS], prow[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; i++) {
+    const int e = i * 64 + lane, r = e / COLS, c = e - r * COLS, ic = r / KW, kh = r - ic * KW;
+    poff[i] = r < rows ? ((ic * g.H + kh * g.DH) * g.W + c) * 4 : kOutside;
+    pcol[i] = r < rows ? c : 1 << 30; // (always outside: an offset from kOutside could wrap)
+    prow[i] = kh;
+  }
+  float *patch = patches[wave];
+  const int64_t imageElems = (int64_t)g.IC * g.H * g.W, outElems = (int64_t)OC * P;
+  float next[LOADS];
+  struct Place {
+    int n, oh, ow0;
+  };
+  auto place = [&](int tile) {
+    const int row = divide(tile, byAcross), n = divide(row, byOH);
+    return Place{n, row - n * g.OH, (tile - row * across) * 32};
+  };
+  auto fetch = [&](int tile) {
+    const Place o = place(tile);
+    const int ih0 = o.oh * g.SH - g.PHL, iw0 = o.ow0 * SW - g.PWL;
+    const unsigned rowOut = outsideBits(ih0, g.H, KW, g.DH) & ((1u << KW) - 1u);
+    const auto rsrc = resource(x + o.n * imageElems, (N - o.n) * imageElems);
+    const int first = (ih0 * g.W + iw0) * 4;
+    if (iw0 >= 0 && iw0 + COLS <= g.W && !rowOut) { // (uniform) nothing outside
+#pragma unroll
+      for (int i = 0; i < LOADS; i++) next[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, poff[i], first, 0));
+    } else {
+#pragma unroll
+      for (int i = 0; i < LOADS; i++) {
+        const bool in = (unsigned)(iw0 + pcol[i]) < (unsigned)g.W;
+        const int out = __builtin_amdgcn_sbfe(rowOut, prow[i], 1) & kOutside;
+        next[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, in ? (first + poff[i]) | out : kOutside, 0, 0));
+      }
+    }
+  };
+  auto keep = [&]() {
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) patch[i * 64 + lane] = next[i];
+  };
+  const bool fullOc = oc0 + 32 <= OC;
+  const float *ap = filter + hl * PITCH + l32, *bp = patch + hl * (NR * COLS) + l32 * SW;
+  int tile = (int)blockIdx.x * 4 + wave;
+  if (tile < tiles) {
+    fetch(tile);
+    keep();
+  }
+  __syncthreads(); // the filter
+  for (; tile < tiles; tile += tileStep) {
+    const bool more = tile + tileStep < tiles;
+    if (more) fetch(tile + tileStep);
+    const Place o = place(tile);
+    const auto out = resource(y + o.n * outElems, (N - o.n) * outElems);
+    const int at = o.ow0 + l32 < g.OW ? ((oc0 + 4 * hl) * P + o.oh * g.OW + o.ow0 + l32) * 4 : kOutside;
+    int row = P * 4, channels = OC;
+    asm volatile("" : "+s"(row), "+s"(channels));
+    auto everyChannel = [&](auto each) { // of the lane: its register, its byte offsets
+      if (fullOc) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) each(r, at, (8 * (r / 4) + r % 4) * row);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int ocl = 8 * (r / 4) + r % 4;
+          if (oc0 + ocl < channels) // (a scalar offset past the resource would wrap the check)
+            each(r, oc0 + ocl + 4 * hl < channels ? at : kOutside, ocl * row);
+        }
+      }
+    };
+    float addend[16]; // (in flight under the matrix instructions)
+    if (ADDED) {
+      const auto post = resource(add + o.n * outElems, (N - o.n) * outElems);
+      everyChannel([&](int r, int voffset, int soffset) {
+        addend[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(post, voffset, soffset, 0));
+      });
+    }
+    f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i] = bv[i];
+    // One window row's operands are read under the matrix instructions of the row before (the fences keep them there).
+    float av[2][KW], bw[2][KW];
+    auto read = [&](int i) {
+#pragma unroll
+      for (int k = 0; k < KW; k++) {
+        bw[i % 2][k] = bp[i * COLS + k];
+        av[i % 2][k] = ap[(i * KW + k) * (2 * PITCH)];
+      }
+    };
+    read(0);
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+      if (i + 1 < NR) read(i + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < KW; k++)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i % 2][k], bw[i % 2][k], acc, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    everyChannel([&](int r, int voffset, int soffset) {
+      const float v = ADDED ? acc[r] + addend[r] : acc[r];
+      // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, relu ? fmaxf(v, 0.0f) : v), out, voffset, soffset, 16);
+    });
+    if (more) keep();
+  }
+}
+
 // ---- square windows, operands shared through LDS ---------------------------------------------
 // A block owns 64 output channels x 64 output pixels: 2 x 2 wavefronts of a 32 x 32 tile each, KS
 // times over when KS groups of four wavefronts split the channel groups.  Per unit of a channel group
@@ -1144,7 +1294,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
                   (int)SH, (int)SW, (int)DH, (int)DW};
   const float *add = hasPostAdd ? postAdd : nullptr;
   const int64_t pixels = N * P, pix32 = (pixels + 31) / 32;
-  const FastDiv byP = fastDiv((int)P), byOW = fastDiv((int)OW);
+  const FastDiv byP = fastDiv((int)P), byOW = fastDiv((int)OW), byOH = fastDiv((int)OH);
   auto gridOf = [&](int64_t blocks, int64_t channels, int64_t threads) {
     const int64_t ocTiles = (OC + channels - 1) / channels;
     if (ocTiles > 65535) fail("mgpuConv2d: too many output channels for one launch");
@@ -1186,6 +1336,17 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
                        : streams ? conv_quads_kernel<KWC, NR, true, false> : conv_quads_kernel<KWC, NR, false, false>;
     kernel<<<gridOf(blocks, 32, 256), dim3(256), 0, stream>>>(input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu,
                                                               (int)tiles128, (int)(4 * blocks));
+  };
+  const int64_t across = (OW + 31) / 32;
+  auto patch = [&](auto kw, auto nr, auto sw) {
+    constexpr int KWC = decltype(kw)::value, NR = decltype(nr)::value, SWC = decltype(sw)::value;
+    const int64_t rowTiles = N * OH * across;
+    // two blocks per CU and channel tile
+    const int64_t most = std::max<int64_t>(1, (int64_t)numComputeUnits() * 2 / ((OC + 31) / 32));
+    const int64_t blocks = std::min((rowTiles + 3) / 4, most);
+    auto *kernel = add ? conv_patch_kernel<KWC, NR, SWC, true> : conv_patch_kernel<KWC, NR, SWC, false>;
+    kernel<<<gridOf(blocks, 32, 256), dim3(256), 0, stream>>>(input, weight, bias, output, g, (int)OC, (int)P, (int)N, fastDiv((int)across),
+                                                              byOH, add, relu, (int)across, (int)rowTiles, (int)(4 * blocks));
   };
   auto window = [&](auto win, auto pts, auto kss) {
     constexpr int WIN = decltype(win)::value, PT = decltype(pts)::value, KS = decltype(kss)::value;
@@ -1251,6 +1412,18 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     // (two accumulators share the gathered taps; few pixels are spread over more wavefronts instead)
     if (OC > 32 && pix32 >= 4 * numComputeUnits()) steps(c2);
     else steps(c1);
+  } else if (squareWindow && KH >= 5 && (IC == 1 || IC == 3) && DW == 1 && SW <= 2 && 2 * OW >= 32 * across && fitsInt(N * OH * across)) {
+    // From half of a row's tiles filled on (us, window tiles / patches, 7 x 7 from 3 channels unless said otherwise: 1 x 224 x 224 -> 64
+    // of stride 2 13.0 / 7.4, 16 x 256 x 256 94 / 57, 4 x 112 x 112 -> 32 14.2 / 10.3, 2 x 28 x 28 -> 96 7.5 / 6.9; 32 x 28 x 28 -> 64 from
+    // 1 12.3 / 5.7; 5 x 5 16 x 128 x 128 -> 64 55 / 33, rows of 17 19.3 / 18.8; but rows of 10 13.1 / 16.4;
+    // from 2 channels, whole pairs, 1 x 56 x 56 3.6 / 5.1).
+    auto go = [&](auto kw, auto nr) {
+      if (SW == 1) patch(kw, nr, c1);
+      else patch(kw, nr, c2);
+    };
+    if (KH == 5) go(integral_constant<int, 5>(), integral_constant<int, 8>());
+    else if (IC == 1) go(integral_constant<int, 7>(), c4);
+    else go(integral_constant<int, 7>(), integral_constant<int, 11>());
   } else if (squareWindow) {
     auto pick = [&](auto win) {
       constexpr int WIN = decltype(win)::value;
