@@ -1255,7 +1255,7 @@ FastDiv fastDiv(int d) {
 //    tiles are as good from three a CU on.  Window tiles (`paired` false) are not: 1176 tiles of 96 channels 1.3-1.6 times as
 //    fast, 1568 of 32 channels 33.2 / 24.9; beyond eight a CU their two accumulators are (3136 tiles 28.0 / 29.7);
 //  * 5 x 5, a block's LDS holds one a CU of eight: 248 tiles of 32 groups 16.5 / 13.5 / 12.0, 442 tiles 42.9 / 23.3 / 24.2; of 8
-//    groups 442 tiles 16.6 / 7.7, but 784, just over three a CU, 0.89 times as fast; 10125 tiles of 16 groups 268 / 211; 64-channel
+//    groups 442 tiles 16.6 / 7.7, but 784, just over three a CU, 0.89 times as fast, then 1689 26.8 / 21.7; 10125 of 16 groups 268 / 211; 64-channel
 //    tiles as above (784 tiles 43.3 / 36.2, 980 43.6 / 44.9).
 //  * 7 x 7, the same: 196 tiles of 32 groups 35.5 / 22.3 / 21.0, 112 of 128 156 / 85 / 75, 324 of 64 165 / 81 / 80, 784 of 8 33.9 / 23.2 /
 //    28.1, 6272 of 16 427 / 250 / 290; 64-channel tiles 784 of 8 25.7 / 22.0 / 27.0, of 16 39.3 / 38.5 / 43.3, 980 of 32 81.9 / 82.4.
@@ -1265,7 +1265,7 @@ int stagedWaves(int win, int64_t tiles, int64_t groups, bool paired, int64_t cus
   if (win == 7) return groups < 8 || (paired && tiles > few4) ? 0 : tiles <= cus ? 8 : 4;
   if (tiles <= few && groups >= (win == 3 ? 32 : 16)) return 8;
   if (win == 3 && groups >= 16 && tiles > cus * 3 / 2 && tiles <= (paired ? few4 : 8 * cus)) return 4;
-  if (win == 5 && tiles > cus && (tiles <= few4 ? groups >= 8 : !paired && groups >= 16)) return 4;
+  if (win == 5 && tiles > cus && (tiles <= few4 || !paired)) return groups >= (tiles > few4 && tiles <= 4 * cus ? 16 : 8) ? 4 : 0;
   return 0;
 }
 
