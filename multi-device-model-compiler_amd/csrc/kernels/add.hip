@@ -10,75 +10,50 @@
 #include "common.hpp"
 #include "mgpu_ops_internal.hpp"
 
+#include <algorithm>
+
 namespace mgpu {
 
 typedef float float4v __attribute__((ext_vector_type(4)));
 
-// Each block walks UNROLL * 256 float4 per array per trip; all 2*UNROLL loads
-// of a trip are issued before the first add.  Measured on MI355X at the
-// (3,640,640) shape: plain loads + non-temporal stores with one vector per lane
-// and one block per 256 vectors is the fastest combination (non-temporal LOADS
-// cost about 10 %, more vectors per lane do not help at this size).
+// One vector per lane, one block per 256 vectors.  Measured on MI355X at the (3,640,640) shape: plain loads + non-temporal
+// stores with one vector per lane is the fastest combination (non-temporal LOADS cost about 10 %, more vectors per lane do
+// not help at this size).  The last n % 4 elements are one lane's, element by element: as a launch of their own they took
+// as long as a small array (75850 elements 8.0 -> 4.1 us, 31136098 65 -> 63).
 //
 // Everything the kernel needs arrives as an explicit argument (the grid's stride included,
 // instead of gridDim): the explicit arguments are preloaded into SGPRs, the grid dimensions
 // would cost a load from the kernarg segment on the path to the first data load.
-template <int UNROLL>
-__global__ __launch_bounds__(256) void add_f32_vec4_kernel(const float4v *__restrict__ a,
-                                                           const float4v *__restrict__ b,
-                                                           float4v *__restrict__ c, int64_t n4, int64_t stride) {
-  for (int64_t base = (int64_t)blockIdx.x * 256 * UNROLL + threadIdx.x; base < n4; base += stride) {
-    float4v va[UNROLL], vb[UNROLL];
-#pragma unroll
-    for (int u = 0; u < UNROLL; u++) {
-      const int64_t i = base + (int64_t)u * 256;
-      if (i < n4) {
-        va[u] = a[i];
-        vb[u] = b[i];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < UNROLL; u++) {
-      const int64_t i = base + (int64_t)u * 256;
-      if (i < n4) __builtin_nontemporal_store(va[u] + vb[u], c + i);
+__global__ __launch_bounds__(256) void add_f32_vec4_kernel(const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c,
+                                                           int64_t n, int64_t stride) {
+  for (int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x * 4; i < n; i += stride) {
+    if (i + 4 <= n) {
+      const float4v va = *reinterpret_cast<const float4v *>(a + i), vb = *reinterpret_cast<const float4v *>(b + i);
+      __builtin_nontemporal_store(va + vb, reinterpret_cast<float4v *>(c + i));
+    } else {
+      for (int64_t j = i; j < n; j++) c[j] = a[j] + b[j];
     }
   }
 }
 
-// Tail (n % 4 elements) and the fallback for pointers that are not 16-byte
-// aligned.
-__global__ __launch_bounds__(256) void add_f32_scalar_kernel(const float *__restrict__ a,
-                                                             const float *__restrict__ b,
-                                                             float *__restrict__ c, int64_t begin,
+// Pointers that are not 16-byte aligned.
+__global__ __launch_bounds__(256) void add_f32_scalar_kernel(const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c,
                                                              int64_t n) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = begin + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-    c[i] = a[i] + b[i];
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) c[i] = a[i] + b[i];
 }
 
 void addF32(const float *a, const float *b, float *c, int64_t n, hipStream_t stream) {
   if (n < 0) fail("mgpuAddF32: negative element count");
   if (n == 0) return;
   if (!a || !b || !c) fail("mgpuAddF32: null pointer");
-  if (aligned16(a) && aligned16(b) && aligned16(c) && n >= 4) {
-    constexpr int UNROLL = 1;
-    const int64_t n4 = n / 4;
-    int64_t blocks = (n4 + 256 * UNROLL - 1) / (256 * UNROLL);
-    const int64_t cap = kMaxStreamBlocks;
-    if (blocks > cap) blocks = cap;
-    add_f32_vec4_kernel<UNROLL><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(
-        reinterpret_cast<const float4v *>(a), reinterpret_cast<const float4v *>(b),
-        reinterpret_cast<float4v *>(c), n4, blocks * 256 * UNROLL);
+  if (aligned16(a) && aligned16(b) && aligned16(c)) {
+    const int64_t blocks = std::min<int64_t>((n + 1023) / 1024, kMaxStreamBlocks);
+    add_f32_vec4_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(a, b, c, n, blocks * 1024);
     MGPU_CHECK_LAUNCH("add_f32_vec4_kernel");
-    if (n % 4) {
-      add_f32_scalar_kernel<<<dim3(1), dim3(64), 0, stream>>>(a, b, c, n4 * 4, n);
-      MGPU_CHECK_LAUNCH("add_f32_scalar_kernel");
-    }
   } else {
-    int64_t blocks = (n + 255) / 256;
-    const int64_t cap = kMaxStreamBlocks;
-    if (blocks > cap) blocks = cap;
-    add_f32_scalar_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(a, b, c, 0, n);
+    const int64_t blocks = std::min<int64_t>((n + 255) / 256, kMaxStreamBlocks);
+    add_f32_scalar_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(a, b, c, n);
     MGPU_CHECK_LAUNCH("add_f32_scalar_kernel");
   }
 }
