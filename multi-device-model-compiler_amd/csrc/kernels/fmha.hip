@@ -50,6 +50,23 @@ void launch(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqlens, v
   const auto *in = static_cast<const uint16_t *>(qkv);
   auto *o = static_cast<uint16_t *>(out);
   const dim3 grid((unsigned)blocks), block(256);
+  // Two sets of wavefronts a block where a launch leaves every CU about one block, one wavefront a SIMD, and each set still has a
+  // few tiles (us, one set / two, b x s x heads): 256 blocks 2 x 1024 x 16 of 64 16.9 / 14.5, 1 x 2048 x 16 of 128 46.0 / 41.4, of 256 103 / 91,
+  // 192 1 x 3072 x 8 of 128 61.9 / 49.5, 4 x 512 x 16 of 64 10.1 / 9.5; but 7 x 384 x 12 of 128 13.9 / 15.3, 3 x 600 x 12 of 256 37.1 / 38.1, and
+  // 264 blocks, a second round, 1 x 2697 x 12 of 128 74 / 93.  Causal launches end with a few long blocks: 352 2 x 1374 x 16 of 64 24.8 /
+  // 19.8, 384 1 x 3000 x 16 of 128 67 / 56, 3 x 1024 x 16 19.7 / 18.5, 512 1 x 4096 x 16 100 / 86, but 360 6 x 640 x 12 14.0 / 15.9, 448 4 x 1024 x 14
+  // 19.9 / 20.8, 640 1 x 4096 x 20 72 / 77.
+  if constexpr (NQ == 1) {
+    const int64_t cus = deviceComputeUnits();
+    const bool halves = causal ? S >= 512 && !pair && 2 * blocks <= cus * (nQB >= 12 ? 4 : nQB >= 8 ? 3 : 2)
+                               : S >= (D == 256 ? 768 : 512) && blocks <= cus;
+    if (halves) {
+      auto *kernel = causal ? fmha_fwd_kernel<T, D, 1, true, false, PAD, true> : fmha_fwd_kernel<T, D, 1, false, false, PAD, true>;
+      kernel<<<grid, dim3(512), 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
+      MGPU_CHECK_LAUNCH("fmha_fwd_kernel");
+      return;
+    }
+  }
   if (causal) {
     // (the causal kernel exists with one 32-query block per wavefront only)
     if constexpr (NQ == 1)

@@ -136,8 +136,8 @@ constexpr float kSumFloor = 0.015625f;
 // fetches chunk 0 of that row instead (in bounds, finite wherever the row is),
 // Q is zero there, so the scores do not see the K filler, and the O^T rows the V
 // filler feeds are never stored.
-template <typename T, int D, int NQ, bool CAUSAL, bool TRACE = false, bool PAD = false>
-__global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_kernel(const uint16_t *__restrict__ qkv,
+template <typename T, int D, int NQ, bool CAUSAL, bool TRACE = false, bool PAD = false, bool HALVES = false>
+__global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) ? 3 : 2) void fmha_fwd_kernel(const uint16_t *__restrict__ qkv,
                                                               const int32_t *__restrict__ seqlens,
                                                               const int32_t *__restrict__ cuSeqlens,
                                                               uint16_t *__restrict__ out, int S, int H,
@@ -167,7 +167,10 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
   // bank conflicts, need 1 KiB more than the ring).
   constexpr int kRingBytes = kStages * kStageBytes;
   constexpr int kStagingBytes = 4 * NQ * 32 * G::OS * 2;
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kRingBytes > kStagingBytes ? kRingBytes : kStagingBytes];
+  constexpr int kMergeBytes = 4 * 64 * (D / 2 + 2) * 4; // HALVES: a wavefront's O, reference and sum, a float a lane each
+  constexpr int kLdsBytes = HALVES ? (2 * kRingBytes > kMergeBytes ? 2 * kRingBytes : kMergeBytes) : kRingBytes > kStagingBytes ? kRingBytes : kStagingBytes;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kLdsBytes];
+  static_assert(!HALVES || (NQ == 1 && !TRACE && kStagingBytes <= kLdsBytes && kLdsBytes <= 160 * 1024), "HALVES: one query block a wavefront");
 
   // Work-item order: query blocks of one (batch, head) are consecutive, and a
   // contiguous run of work items goes to each of the 8 XCDs (consecutive block
@@ -184,7 +187,7 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
   // short one has just read (b32 s512 h12: 29.0 -> 27.6 us); at 128, with its ring
   // of two stages, the long block first measured faster (b8 s1024 h16: 46.5
   // against 49.6 us).
-  constexpr bool kCanPair = CAUSAL && D <= 128; // at 256 the second pass is compiled out
+  constexpr bool kCanPair = CAUSAL && D <= 128 && !HALVES; // at 256 the second pass is compiled out
   const bool paired = kCanPair && pairItems == 1;
   const int nItems = paired ? (nQB + 1) / 2 : nQB; // work items per (batch, head)
   int item = wid % nItems;
@@ -220,9 +223,15 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
   const int h = bh % H;
   const int b = bh / H;
 
-  const int tid = threadIdx.x;
+  // HALVES: wavefronts 4 to 7 are a second set over the same queries.  Set `half` takes key tiles half, half + 2, ... through a
+  // ring of its own; only the barriers are common, and a merge in fp32 at the end.  One block a CU is one wavefront a SIMD, whose
+  // scores, softmax and products wait for each other; of two, one's softmax runs beside the other's matrix instructions (b1
+  // s3072 h8 d128, 192 blocks: 61.9 -> 49.5 us).
+  const int tid = HALVES ? threadIdx.x % 256 : threadIdx.x;
   const int lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int half = HALVES ? __builtin_amdgcn_readfirstlane(threadIdx.x / 256) : 0;
+  unsigned char *const ring = smem + half * kRingBytes;
   const int l32 = lane % 32;
   const int hl = lane / 32;
 
@@ -266,7 +275,10 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
     lastq = lastq < S - 1 ? lastq : S - 1;
     kend = kend < lastq + 1 ? kend : lastq + 1;
   }
-  const int nkt = (kend + kBN - 1) / kBN;
+  const int nktAll = (kend + kBN - 1) / kBN;
+  const int nkt = HALVES ? (nktAll - half + 1) / 2 : nktAll; // this set's tiles
+  const int trips = HALVES ? (nktAll + 1) / 2 : nktAll;
+  auto tileAt = [&](int kt) { return HALVES ? 2 * kt + half : kt; }; // the kt-th of them
 
   // ---- tile movers: HBM -> LDS, 16 bytes per lane ---------------------------
   // One wavefront instruction fills 1 KiB = RPI tile rows; wavefront w moves
@@ -295,7 +307,7 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
   // bookkeeping does not see them: it would otherwise wait for every load in
   // flight, prefetches included, before any later LDS read.  Completion is
   // tracked by hand with s_waitcnt vmcnt(n) below (2 * LPW loads per tile and wave).
-  const uint32_t ldsBase = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) unsigned char *)smem);
+  const uint32_t ldsBase = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) unsigned char *)ring);
   // M0 is on the clobber list so that the statement counts as a definition of it
   // (the compiler reserves M0 and notes that such a clobber is not saved and restored:
   // nothing here needs it preserved).
@@ -311,9 +323,10 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
   auto issueTile = [&](int kt) {
     const uint32_t kdst = ldsBase + (uint32_t)((kt % kStages) * kStageBytes + (LPW * wave) * 1024);
     const uint32_t vdst = kdst + kTileBytes;
-    if (kt * kBN + kBN <= rows) { // whole tile inside the sequence
-      const char *kg = kbase + (size_t)kt * kBN * tokBytes;
-      const char *vg = vbase + (size_t)kt * kBN * tokBytes;
+    const int key0 = tileAt(kt) * kBN;
+    if (key0 + kBN <= rows) { // whole tile inside the sequence
+      const char *kg = kbase + (size_t)key0 * tokBytes;
+      const char *vg = vbase + (size_t)key0 * tokBytes;
 #pragma unroll
       for (int i = 0; i < LPW; i++) {
         dma16(kRecomputeOffsets ? tileOffset(i, false) : koff[i], kg, kdst + i * 1024);
@@ -323,7 +336,7 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
 #pragma unroll
       for (int i = 0; i < LPW; i++) {
         const int row = G::RPI * (LPW * wave + i) + mrow;
-        int key = kt * kBN + row;
+        int key = key0 + row;
         key = key < rows ? key : rows - 1;
         const uint32_t rowOff = (uint32_t)key * tokBytes;
         dma16(rowOff + srcChunk(mchunk ^ G::kSwz(row)) * 16, kbase, kdst + i * 1024);
@@ -403,7 +416,7 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
   // s2048 h32 333 -> 318, b8 s1024 h32 186 -> 178, b8 s700 h12 d96 45.3 -> 40.9, causal b4 s2048 h32 188 -> 186; b16 s256 h16 16.0
   // -> 16.4); at 64, four loads a wavefront and three wavefronts a SIMD, the causal kernel loses 3-5 %, and at 256 it spills.
   constexpr bool kLoadsBehindScores = D == 128;
-  for (int kt = 0; kt < nkt; kt++) {
+  for (int kt = 0; kt < trips; kt++) {
     if (TRACE) tMark = clock64();
     // The loads of tile kt (and of nothing later) must have landed; the barrier
     // makes every wavefront's share visible and also says that everybody is
@@ -416,12 +429,12 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
     if (!kLoadsBehindScores && kt + kStages - 1 < nkt) issueTile(kt + kStages - 1);
 
     const uint32_t stageOff = (uint32_t)((kt % kStages) * kStageBytes);
-    const int key0 = kt * kBN;
+    const int key0 = tileAt(kt) * kBN;
 
     // Rows of masked keys meet p = 0; zero them so that stray NaN/Inf bits in
     // padding cannot reach the accumulators.  Only the last tile can be partial.
-    if (key0 + kBN > kvlen) {
-      unsigned char *vst = smem + stageOff + kTileBytes;
+    if (HALVES ? kt == trips - 1 && nktAll * kBN > kvlen : key0 + kBN > kvlen) { // (uniform: both sets come to the barrier)
+      unsigned char *vst = ring + stageOff + kTileBytes;
 #pragma unroll
       for (int i = 0; i < kTileBytes / 4096; i++) {
         const int chunk = tid + 256 * i; // 16-byte chunk of the V tile
@@ -430,6 +443,7 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
       }
       __syncthreads();
     }
+    if (HALVES && kt >= nkt) break; // (the other set's last tile)
 
     // Causal: a wavefront whose queries all precede this tile has nothing to add.
     const bool nothing = CAUSAL && key0 > q0 + NQ * 32 - 1;
@@ -578,11 +592,36 @@ __global__ __launch_bounds__(256, (CAUSAL && D == 64) ? 3 : 2) void fmha_fwd_ker
   if (TRACE) tLoopEnd = clock64();
   // ---- normalise, transpose through LDS, store whole rows ------------------
   __syncthreads(); // every wavefront is done reading the K / V tiles
+  if constexpr (HALVES) { // the second set's sums to the first, both on the higher of the two references
+    float *mine = reinterpret_cast<float *>(smem) + wave * 64 * (D / 2 + 2) + lane;
+    l_run[0] = halves_sum(l_run[0]);
+    if (half == 1) {
+#pragma unroll
+      for (int db = 0; db < G::DB; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) mine[64 * (16 * db + i)] = accO[0][db][i];
+      mine[64 * (D / 2)] = m_run[0];
+      mine[64 * (D / 2 + 1)] = l_run[0];
+    }
+    __syncthreads();
+    if (half == 0) {
+      const float m1 = mine[64 * (D / 2)], l1 = mine[64 * (D / 2 + 1)], m0 = m_run[0];
+      const float m = l1 != 0.0f ? fmaxf(m0, m1) : m0; // (no tile in the second set: its reference means nothing; a NaN passes)
+      const float e0 = __builtin_amdgcn_exp2f((m0 - m) * scale_log2e), e1 = l1 != 0.0f ? __builtin_amdgcn_exp2f((m1 - m) * scale_log2e) : 0.0f;
+      l_run[0] = l_run[0] * e0 + l1 * e1;
+#pragma unroll
+      for (int db = 0; db < G::DB; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) accO[0][db][i] = accO[0][db][i] * e0 + mine[64 * (16 * db + i)] * e1;
+    }
+    __syncthreads(); // the output staging takes the sums' place
+    if (half == 1) return;
+  }
   constexpr int kOS = G::OS;
   uint16_t *stage = reinterpret_cast<uint16_t *>(smem) + wave * (NQ * 32 * kOS);
 #pragma unroll
   for (int qi = 0; qi < NQ; qi++) {
-    const float l = halves_sum(l_run[qi]);
+    const float l = HALVES ? l_run[qi] : halves_sum(l_run[qi]);
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
     for (int db = 0; db < G::DB; db++)

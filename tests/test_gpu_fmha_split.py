@@ -90,3 +90,47 @@ def test_split_keys_with_references_far_apart(pkg, gpu, oracle, D):
             got = pkg.fused_mha(to_dev(qkv, gpu), causal=causal).float().cpu().numpy()
             ref = oracle.fmha(qkv, causal=causal)
             assert np.isfinite(got).all() and (np.abs(got - ref) <= TOL["f16"] * np.maximum(1.0, np.abs(ref))).all()
+
+
+def two_sets(D, B, S, H, causal, cus):
+    """The launcher's rule for two sets of wavefronts over the same 128 queries, each with every other tile of keys."""
+    if groups(D, B, S, H, causal, cus):
+        return False
+    nqb = -(-S // 128)
+    if causal:
+        return S >= 512 and 2 * B * H * nqb <= cus * (4 if nqb >= 12 else 3 if nqb >= 8 else 2)
+    return S >= (768 if D > 128 else 512) and B * H * nqb <= cus
+
+
+@pytest.mark.parametrize("D,B,S,H,lens,causal,dtype", [
+    (64, 2, 520, 15, None, False, "f16"),           # nine tiles of 64 keys: the second set has one fewer, the last tile is cut
+    (64, 2, 577, 15, [577, 64], False, "bf16"),     # one tile: nothing for the second set
+    (40, 2, 640, 16, [640, 65], False, "f16"),      # ten whole tiles; two, the second of one key
+    (128, 3, 640, 10, [640, 0, 129], False, "f16"), # an empty sequence
+    (80, 2, 600, 14, [600, 1], True, "bf16"),
+    (64, 2, 1100, 16, None, True, "f16"),           # more than a round, longest blocks first
+    (64, 1, 1540, 20, None, True, "bf16"),
+    (256, 2, 800, 11, [800, 33], False, "f16"),     # tiles of 32
+    (144, 2, 520, 15, None, True, "f16"),
+])
+def test_two_sets(pkg, gpu, oracle, D, B, S, H, lens, causal, dtype):
+    import torch
+    assert two_sets(D, B, S, H, causal, torch.cuda.get_device_properties(gpu).multi_processor_count)
+    test_split_keys(pkg, gpu, oracle, D, B, S, H, lens, causal, dtype, 0)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_two_sets_with_references_far_apart(pkg, gpu, oracle, D):
+    """Logits that differ by 960 D^-1/2 between the sets' tiles, along the keys and alternating with them."""
+    rng = np.random.Generator(np.random.PCG64(D))
+    B, S, H = 2, 790, 11
+    tile = np.arange(S) // (32 if D == 256 else 64) % 2
+    qkv = (rng.standard_normal((B, S, 3, H, D)) * 0.5).astype(np.float16)
+    for ramp in (np.linspace(-60, 60, S), np.linspace(60, -60, S), 120.0 * tile - 60, 60 - 120.0 * tile, np.full(S, -60.0)):
+        qkv[:, :, 0, :, :] = 0
+        qkv[:, :, 0, :, 0] = 8.0
+        qkv[:, :, 1, :, 0] = ramp.astype(np.float16)[None, :, None]
+        for causal in (False, True):
+            got = pkg.fused_mha(to_dev(qkv, gpu), causal=causal).float().cpu().numpy()
+            ref = oracle.fmha(qkv, causal=causal)
+            assert np.isfinite(got).all() and (np.abs(got - ref) <= TOL["f16"] * np.maximum(1.0, np.abs(ref))).all()
