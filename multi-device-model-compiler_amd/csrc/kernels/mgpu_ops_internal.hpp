@@ -137,11 +137,13 @@ double gemmMfmaPartialCost(int64_t M, int64_t N, int64_t K, int parts);
 void gemmMfmaPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, int parts, hipStream_t stream);
 void gemmKSplitPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, KSplitTile tile, int parts,
                           hipStream_t stream);
-// The sum of the planes + bias + residual: through a LayerNorm (fp16; the rounded sum to sumOut when not null), or as it
+// The sum of the planes + bias + residual: through a LayerNorm (fp16; the rounded sum to sumOut when not null; or fp32), or as it
 // is, in fp32.  partialSumsSupports: widths and alignment.
 bool partialSumsSupports(const void *bias, const void *residual, const void *gamma, const void *beta, const void *out, int64_t M, int64_t N);
 void partialSumsLayerNormF16(const float *planes, int parts, const void *bias, const void *residual, const void *gamma, const void *beta,
                              void *sumOut, void *out, float eps, int64_t M, int64_t N, hipStream_t stream);
+void partialSumsLayerNormF32(const float *planes, int parts, const void *bias, const void *residual, const void *gamma, const void *beta,
+                             float *out, float eps, int64_t M, int64_t N, hipStream_t stream);
 void partialSumsF32(const float *planes, int parts, const void *bias, const void *residual, float *out, int64_t M, int64_t N,
                     hipStream_t stream);
 // fp32, any shape, for few tiles (gemm_f32_small.hip).

@@ -23,12 +23,14 @@ __device__ __forceinline__ float waveSum(float v) {
   return v;
 }
 
-// NORM: out = LayerNorm(sum) in fp16, and the rounded sum to sumOut when it is not null; else the fp32 sum to out.
-template <int V, int PARTS, bool NORM>
+// Sum: the fp32 sum to out.  Norm: LayerNorm(sum) in fp16, and the rounded sum to sumOut when it is not null.  NormF32: in fp32.
+enum class Result { Sum, Norm, NormF32 };
+template <int V, int PARTS, Result RESULT>
 __global__ __launch_bounds__(64) void partial_sums_kernel(const float *__restrict__ planes, const _Float16 *__restrict__ bias,
                                                           const _Float16 *__restrict__ residual, const _Float16 *__restrict__ gamma,
                                                           const _Float16 *__restrict__ beta, _Float16 *__restrict__ sumOut,
                                                           void *__restrict__ out, int M, int N, float eps) {
+  constexpr bool NORM = RESULT != Result::Sum;
   const int row = blockIdx.x, lane = threadIdx.x;
   // every load first, so that one trip to memory covers them all (columns past the row fetch its last vector)
   float4v p[V][PARTS][2];
@@ -89,30 +91,39 @@ __global__ __launch_bounds__(64) void partial_sums_kernel(const float *__restric
   for (int v = 0; v < V; v++) {
     const int n = (v * 64 + lane) * 8;
     if (n >= N) continue;
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) y[i] = (x[v][i] - mean) * inv * (float)g[v][i] + (float)be[v][i];
+    if (RESULT == Result::NormF32) {
+      float *o = static_cast<float *>(out) + (size_t)row * N + n;
+      *reinterpret_cast<float4v *>(o) = float4v{y[0], y[1], y[2], y[3]};
+      *reinterpret_cast<float4v *>(o + 4) = float4v{y[4], y[5], y[6], y[7]};
+      continue;
+    }
     half8 o;
 #pragma unroll
-    for (int i = 0; i < 8; i++) o[i] = (_Float16)((x[v][i] - mean) * inv * (float)g[v][i] + (float)be[v][i]);
+    for (int i = 0; i < 8; i++) o[i] = (_Float16)y[i];
     *reinterpret_cast<half8 *>(static_cast<_Float16 *>(out) + (size_t)row * N + n) = o;
   }
 }
 
-template <int PARTS, bool NORM>
+template <int PARTS, Result RESULT>
 void launch(const float *planes, const void *bias, const void *residual, const void *gamma, const void *beta, void *sumOut, void *out,
             float eps, int64_t M, int64_t N, hipStream_t stream) {
   const dim3 grid((unsigned)M), block(64);
   const auto *b = static_cast<const _Float16 *>(bias), *r = static_cast<const _Float16 *>(residual);
   const auto *g = static_cast<const _Float16 *>(gamma), *be = static_cast<const _Float16 *>(beta);
   auto *s = static_cast<_Float16 *>(sumOut);
-  const auto kernel = N <= 512 ? partial_sums_kernel<1, PARTS, NORM> : N <= 1024 ? partial_sums_kernel<2, PARTS, NORM>
-                                                                                 : partial_sums_kernel<4, PARTS, NORM>;
+  const auto kernel = N <= 512 ? partial_sums_kernel<1, PARTS, RESULT> : N <= 1024 ? partial_sums_kernel<2, PARTS, RESULT>
+                                                                                   : partial_sums_kernel<4, PARTS, RESULT>;
   kernel<<<grid, block, 0, stream>>>(planes, b, r, g, be, s, out, (int)M, (int)N, eps);
   MGPU_CHECK_LAUNCH("partial_sums_kernel");
 }
 
-template <bool NORM, typename... Args> void launchParts(int parts, Args... args) {
-  if (parts == 2) launch<2, NORM>(args...);
-  else if (parts == 3) launch<3, NORM>(args...);
-  else if (parts == 4) launch<4, NORM>(args...);
+template <Result RESULT, typename... Args> void launchParts(int parts, Args... args) {
+  if (parts == 2) launch<2, RESULT>(args...);
+  else if (parts == 3) launch<3, RESULT>(args...);
+  else if (parts == 4) launch<4, RESULT>(args...);
   else fail("partialSums: internal dispatch error");
 }
 
@@ -124,12 +135,17 @@ bool partialSumsSupports(const void *bias, const void *residual, const void *gam
 
 void partialSumsLayerNormF16(const float *planes, int parts, const void *bias, const void *residual, const void *gamma, const void *beta,
                              void *sumOut, void *out, float eps, int64_t M, int64_t N, hipStream_t stream) {
-  launchParts<true>(parts, planes, bias, residual, gamma, beta, sumOut, out, eps, M, N, stream);
+  launchParts<Result::Norm>(parts, planes, bias, residual, gamma, beta, sumOut, out, eps, M, N, stream);
+}
+
+void partialSumsLayerNormF32(const float *planes, int parts, const void *bias, const void *residual, const void *gamma, const void *beta,
+                             float *out, float eps, int64_t M, int64_t N, hipStream_t stream) {
+  launchParts<Result::NormF32>(parts, planes, bias, residual, gamma, beta, nullptr, out, eps, M, N, stream);
 }
 
 void partialSumsF32(const float *planes, int parts, const void *bias, const void *residual, float *out, int64_t M, int64_t N,
                     hipStream_t stream) {
-  launchParts<false>(parts, planes, bias, residual, nullptr, nullptr, nullptr, out, 0.0f, M, N, stream);
+  launchParts<Result::Sum>(parts, planes, bias, residual, nullptr, nullptr, nullptr, out, 0.0f, M, N, stream);
 }
 
 } // namespace mgpu
