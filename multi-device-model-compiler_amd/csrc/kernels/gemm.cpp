@@ -197,6 +197,20 @@ int wideWidth(DType dt, const void *in, const void *weight, const void *bias, co
   return gemmWideBest(M, N, K, act, residual != nullptr, &cost);
 }
 
+// And gemm_round's where the depth is no multiple of 64, which it fills up with zeros (us, what ran before - the library, or gemm_mfma at
+// multiples of 32 - / gemm_round: 512 x 3072 x 72 10.5 / 4.6, x 296 10.4 / 5.6, x 1000 16.1 / 10.5, x 3000 30.9 / 23.6; 3000 x 1000 x 520 15.6 /
+// 10.3; x 96 6.0 / 6.4, x 1376 18.3 / 17.0).  Where gemm_ksplit's estimate is lower it stays: 500 x 2000 x 1000 9.6 / 9.6.  gemm_wide, the
+// same: 4261 x 1064 x 1000 28.4 / 18.4, 6000 x 3000 x 520 49.9 / 31, 4096 x 3080 x 296 33.0 / 16.9, x 160 26.1 / 13.6.
+int raggedRoundWidth(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M, int64_t N,
+                     int64_t K, int act) {
+  if (forcedKernel() || K % 64 == 0 || dt == DType::F32) return 0;
+  const int width = gemmRoundWidth(dt, in, weight, bias, residual, out, M, N, K);
+  if (!width) return 0;
+  double kSplitCost;
+  (void)gemmKSplitBest(M, N, K, act, &kSplitCost);
+  return gemmMfmaCost(M, N, (K + 63) / 64 * 64, act) < kSplitCost ? width : 0;
+}
+
 using Key = std::tuple<int64_t, int64_t, int64_t, int, int, int, int, int>;
 std::map<Key, Plan> plans;
 
@@ -390,6 +404,11 @@ void matmulEx(DType dt, const void *input, const void *weight, const void *bias,
   if (!weightKMajor)
     if (const int width = wideWidth(dt, input, weight, b, r, output, M, N, K, act)) {
       gemmWide(dt, input, weight, b, r, output, M, N, K, act, width, stream);
+      return;
+    }
+  if (!weightKMajor)
+    if (const int width = raggedRoundWidth(dt, input, weight, b, r, output, M, N, K, act)) {
+      gemmRound(dt, input, weight, b, r, output, M, N, K, act, width, stream);
       return;
     }
   switch (chooseKernel(dt, input, weight, b, r, output, M, N, K, hasBias, act, hasResidual, weightKMajor)) {

@@ -322,7 +322,7 @@ void launch(const void *in, const void *weight, const void *bias, const void *re
   auto load = [&](int64_t width) { return (tilesAt(width) + cus - 1) / cus * width; };
   const bool narrow = load(96) < load(128);
   const int64_t tiles = tilesAt(narrow ? 96 : 128);
-  const bool deep = tiles <= cus && K % 64 == 0;
+  const bool deep = tiles <= cus && (K % 64 == 0 || K * N < int64_t(1) << 30);
   const auto *a = static_cast<const uint16_t *>(in);
   const auto *w = static_cast<const uint16_t *>(weight);
   const auto *b = static_cast<const uint16_t *>(bias);
@@ -372,6 +372,15 @@ double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act) {
   const double bytes = (double)(kBM + width) * 2.0 * (double)K, full = (double)tiles / (double)cus;
   if (tiles <= cus) return 3.2 + 1.14 * full + bytes * (11.4e-6 + 2e-6 * full) + (act == ACT_GELU ? 1.4 : 0.0);
   return 5.0 + full * bytes / 52e3;
+}
+
+int gemmRoundWidth(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M, int64_t N,
+                   int64_t K) {
+  if (K % 8 || K * N >= int64_t(1) << 30 || !gemmMfmaSupportsRagged(dt, in, weight, bias, residual, out, M, N, (K + 31) / 32 * 32)) return 0;
+  const int64_t cus = numComputeUnits(), tilesM = (M + kBM - 1) / kBM;
+  auto load = [&](int64_t width) { return (tilesM * ((N + width - 1) / width) + cus - 1) / cus * width; };
+  const int width = load(96) < load(128) ? 96 : 128;
+  return load(width) == width ? width : 0;
 }
 
 // The tile width and estimated us of gemmMfmaPartialF16 without what its planes cost (gemmPartialPlan has that); no width where

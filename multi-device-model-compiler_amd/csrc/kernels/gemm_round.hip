@@ -13,7 +13,7 @@
 // per matrix instruction); and both sets of wavefronts share the epilogue, each with half of every accumulator.
 //
 // Shapes: any M, N a multiple of 8 (tiles overhang the shape: rows and columns past the end are loaded from the last ones
-// and not stored), K a multiple of 64, 16-byte aligned operands.
+// and not stored), K a multiple of 8 (filled up to one of 64 with zeros; planes: of 64), 16-byte aligned operands.
 #include "common.hpp"
 #include "mfma.hpp"
 #include "mgpu_ops_internal.hpp"
@@ -36,7 +36,7 @@ template <int NB> __host__ __device__ constexpr int wSwz(int row) { return NB ==
 constexpr int kResidual = 3; // + residual in its place
 constexpr int kPartial = 4;  // the blocks of grid row y take the y-th share of the reduction and write their fp32 sums to
                              // plane y of `out` (float [gridDim.y][M][N]; partial_sums.hip adds them up and has the epilogue)
-template <typename T, int ACT, int NB>
+template <typename T, int ACT, int NB, bool RAGGED>
 __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
                                                                  const uint16_t *__restrict__ bias, const uint16_t *residual, uint16_t *out,
                                                                  int N, int K, int tilesN, int tilesM, int M_) {
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
   // ---- loads: two instructions of input rows and two (NB 3: one and a half) of the weight a wavefront and step ------
   const char *ag = reinterpret_cast<const char *>(in) + (size_t)m0 * K * 2;
   const char *wg = reinterpret_cast<const char *>(weight) + (size_t)n0 * 2;
-  int steps = K / 64;
+  int steps = RAGGED ? (K + 63) / 64 : K / 64;
   if (ACT == kPartial) {
     const int first = steps * (int)blockIdx.y / (int)gridDim.y;
     steps = steps * ((int)blockIdx.y + 1) / (int)gridDim.y - first;
@@ -94,13 +94,28 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
   }
   const uint32_t ldsBase = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) unsigned char *)smem);
   uint32_t fill = 0; // offset of the ring slot filled next
+  // RAGGED: K ends inside the last step, whose loads past it arrive as zeros (see gemm_wide.hip).
+  i32x4 abuf{}, wbuf{};
+  int k0 = 0; // first column and row of the step loaded next
+  if (RAGGED) {
+    abuf = ldsBuffer(ag, (uint32_t)(rowsLeft < kBM ? rowsLeft : kBM) * (uint32_t)K * 2u);
+    wbuf = ldsBuffer(wg, ((uint32_t)K * (uint32_t)N - (uint32_t)n0) * 2u);
+  }
   auto issueW = [&](int i) {
     const uint32_t dst = ldsBase + fill + (uint32_t)(kA + mover * (kW / 8) + i * 1024);
-    if (NB == 3 && i == 1) ldsLoad16LowerLanes(woff[i], wg, dst);
+    if (RAGGED && NB == 3 && i == 1) ldsLoad16LowerLanes(woff[i], wbuf, (uint32_t)k0 * (uint32_t)N * 2u, dst);
+    else if (RAGGED) ldsLoad16(woff[i], wbuf, (uint32_t)k0 * (uint32_t)N * 2u, dst);
+    else if (NB == 3 && i == 1) ldsLoad16LowerLanes(woff[i], wg, dst);
     else ldsLoad16(woff[i], wg, dst);
   };
-  auto issueA = [&](int i) { ldsLoad16(aoff[i], ag, ldsBase + fill + (uint32_t)((2 * mover + i) * 1024)); };
+  auto issueA = [&](int i) {
+    const uint32_t dst = ldsBase + fill + (uint32_t)((2 * mover + i) * 1024);
+    if (!RAGGED) return ldsLoad16(aoff[i], ag, dst);
+    const int column = ((lane % 8) ^ aSwz(8 * i + lane / 8)) * 8; // (rows 16 apart have the same swizzle)
+    ldsLoad16(column < K - k0 ? aoff[i] : kPastBuffer, abuf, (uint32_t)k0 * 2u, dst);
+  };
   auto nextIssue = [&]() {
+    k0 += 64;
     ag += 128;
     wg += (size_t)N * 128;
     fill = fill == (kRing - 1) * kStage ? 0 : fill + kStage;
@@ -327,19 +342,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
     const uint16_t *p = &stage[chunkRow(it) * kOutStride + 8 * chunkCol(it)];
     const u32x2 lo = *reinterpret_cast<const u32x2 *>(p);
     const u32x2 hi = *reinterpret_cast<const u32x2 *>(p + 4);
-    __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], lo[1], hi[0], hi[1]}, rows, chunkOffset(it), 0, 16);
+    // (as in gemm_wide.hip)
+    if (N % 64) __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], lo[1], hi[0], hi[1]}, rows, chunkOffset(it), 0, 0);
+      else __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], lo[1], hi[0], hi[1]}, rows, chunkOffset(it), 0, 16);
   }
 }
 
-template <typename T, int NB>
+template <typename T, int NB, bool RAGGED>
 void launch(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint16_t *r, uint16_t *o, int64_t M, int64_t N, int64_t K,
             int act, hipStream_t stream) {
   const int tilesM = (int)((M + kBM - 1) / kBM), tilesN = (int)((N + 32 * NB - 1) / (32 * NB));
   const dim3 grid((unsigned)(tilesM * tilesN)), block(kThreads);
-  if (r) gemm_round_kernel<T, kResidual, NB><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_GELU) gemm_round_kernel<T, ACT_GELU, NB><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_RELU) gemm_round_kernel<T, ACT_RELU, NB><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else gemm_round_kernel<T, ACT_NONE, NB><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  if (r) gemm_round_kernel<T, kResidual, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_GELU) gemm_round_kernel<T, ACT_GELU, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_RELU) gemm_round_kernel<T, ACT_RELU, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else gemm_round_kernel<T, ACT_NONE, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_round_kernel");
 }
 
@@ -349,8 +366,10 @@ void launchWidth(const void *in, const void *weight, const void *bias, const voi
   const auto *a = static_cast<const uint16_t *>(in), *w = static_cast<const uint16_t *>(weight), *b = static_cast<const uint16_t *>(bias),
              *r = static_cast<const uint16_t *>(residual);
   auto *o = static_cast<uint16_t *>(out);
-  if (width == 128) launch<T, 4>(a, w, b, r, o, M, N, K, act, stream);
-  else launch<T, 3>(a, w, b, r, o, M, N, K, act, stream);
+  if (width == 128 && K % 64) launch<T, 4, true>(a, w, b, r, o, M, N, K, act, stream);
+  else if (width == 128) launch<T, 4, false>(a, w, b, r, o, M, N, K, act, stream);
+  else if (K % 64) launch<T, 3, true>(a, w, b, r, o, M, N, K, act, stream);
+  else launch<T, 3, false>(a, w, b, r, o, M, N, K, act, stream);
 }
 
 } // namespace
@@ -358,7 +377,7 @@ void launchWidth(const void *in, const void *weight, const void *bias, const voi
 // (The callers, gemm_mfma.hip, have checked the shape and the operands.)
 void gemmRound(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
                int64_t K, int act, int width, hipStream_t stream) {
-  if (N % 8 || K % 64 || (act != ACT_NONE && residual) || (width != 96 && width != 128)) fail("gemmRound: internal dispatch error");
+  if (N % 8 || K % 8 || (K % 64 && K * N >= int64_t(1) << 30) || (act != ACT_NONE && residual) || (width != 96 && width != 128)) fail("gemmRound: internal dispatch error");
   if (dt == DType::F16) launchWidth<_Float16>(in, weight, bias, residual, out, M, N, K, act, width, stream);
   else launchWidth<bf16_t>(in, weight, bias, residual, out, M, N, K, act, width, stream);
 }
@@ -370,8 +389,8 @@ void gemmRoundPartialF16(const void *in, const void *weight, float *planes, int6
   const dim3 grid((unsigned)(tilesM * tilesN), (unsigned)parts), block(kThreads);
   const auto *a = static_cast<const uint16_t *>(in), *w = static_cast<const uint16_t *>(weight);
   auto *o = reinterpret_cast<uint16_t *>(planes);
-  if (width == 128) gemm_round_kernel<_Float16, kPartial, 4><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else gemm_round_kernel<_Float16, kPartial, 3><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  if (width == 128) gemm_round_kernel<_Float16, kPartial, 4, false><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else gemm_round_kernel<_Float16, kPartial, 3, false><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_round_kernel");
 }
 

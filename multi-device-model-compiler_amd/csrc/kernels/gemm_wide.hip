@@ -20,11 +20,13 @@
 //    the one before, across the barrier.
 //
 // Shapes: any M, N a multiple of 8 (tiles overhang the shape: rows and columns past the end are loaded from the last ones
-// and not stored), K a multiple of 64 from 128 on, 16-byte aligned operands.
+// and not stored), K a multiple of 8 from 72 on (filled up to a multiple of 64 with zeros), 16-byte aligned operands.
 #include "common.hpp"
 #include "mfma.hpp"
 #include "mgpu_ops_internal.hpp"
 #include "types.hpp"
+
+#include <type_traits>
 
 namespace mgpu {
 
@@ -41,7 +43,7 @@ template <int BN> __host__ __device__ constexpr int wSwz(int row) { return BN ==
 
 // ACT: the activation, or kResidual in its place.  Out: uint16_t for T's own type, or float.
 constexpr int kResidual = 3;
-template <typename T, int ACT, int BN, typename Out>
+template <typename T, int ACT, int BN, typename Out, bool RAGGED>
 __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
                                                                 const uint16_t *__restrict__ bias, const uint16_t *residual, Out *out,
                                                                 int N, int K, int tilesN, int tilesM, int M_) {
@@ -98,20 +100,40 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const uint16_t *
     if (n0 + 8 * chunk >= N) chunk = (N - 8 - n0) / 8;
     woff[i] = (uint32_t)row * (uint32_t)N * 2u + (uint32_t)(chunk * 16);
   }
+  // RAGGED: K ends inside a buffer.  There the loads go through the buffer check: weight rows past the end are past the weight's
+  // last, and the lanes whose chunk of an input row is past its end are pointed outside; both arrive as zeros.
+  i32x4 abuf{}, wbuf{};
+  int kA = 0, kW = 0; // first column of the buffer, first row of the slice filled next
+  if (RAGGED) {
+    abuf = ldsBuffer(ag, (uint32_t)(rowsLeft < kBM ? rowsLeft : kBM) * (uint32_t)K * 2u);
+    wbuf = ldsBuffer(wg, ((uint32_t)K * (uint32_t)N - (uint32_t)n0) * 2u);
+  }
   const uint32_t ldsBase = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) unsigned char *)smem);
   int aSlot = 0, wSlot = 0; // ring slots filled next
-  auto issueA = [&](int i) { ldsLoad16(aoff[i], ag, ldsBase + (uint32_t)(aSlot * kABuf + wave * 4096 + i * 1024)); };
+  auto issueA = [&](int i) {
+    const uint32_t dst = ldsBase + (uint32_t)(aSlot * kABuf + wave * 4096 + i * 1024);
+    if (!RAGGED) return ldsLoad16(aoff[i], ag, dst);
+    const int column = ((lane % 8) ^ aSwz(8 * i + lane / 8)) * 8;
+    ldsLoad16(column < K - kA ? aoff[i] : kPastBuffer, abuf, (uint32_t)kA * 2u, dst);
+  };
   auto nextIssueA = [&]() {
     ag += 128;
+    kA += 64;
     aSlot = aSlot == kARing - 1 ? 0 : aSlot + 1;
   };
   auto issueW = [&](int i) {
     const uint32_t dst = ldsBase + (uint32_t)(kWBase + wSlot * kWSlice + wave * (kWSlice / 8) + i * 1024);
-    if (kHalf && i == WI - 1) ldsLoad16LowerLanes(woff[i], wg, dst);
+    if (RAGGED) {
+      const bool past = kW >= K;
+      const uint32_t voff = past ? kPastBuffer : woff[i], soff = past ? 0u : (uint32_t)kW * (uint32_t)N * 2u;
+      if (kHalf && i == WI - 1) ldsLoad16LowerLanes(voff, wbuf, soff, dst);
+      else ldsLoad16(voff, wbuf, soff, dst);
+    } else if (kHalf && i == WI - 1) ldsLoad16LowerLanes(woff[i], wg, dst);
     else ldsLoad16(woff[i], wg, dst);
   };
   auto nextIssueW = [&]() {
     wg += (size_t)N * 64;
+    kW += 32;
     wSlot = wSlot == kWRing - 1 ? 0 : wSlot + 1;
   };
   auto issueSlice = [&]() {
@@ -192,7 +214,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const uint16_t *
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  const int steps = K / 32; // even, at least 4
+  const int steps = RAGGED ? (K + 63) / 64 * 2 : K / 32; // even, at least 4
   // The bias, two columns a lane, goes ahead of all other loads into a corner of the input buffer that is filled last, and
   // from there into the accumulators, while the first operands are on their way.
   const uint32_t biasAt = ldsBase + (uint32_t)(2 * kABuf + wave * 256);
@@ -347,27 +369,30 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const uint16_t *
         const u32x2 hi = *reinterpret_cast<const u32x2 *>(p + 4);
         v = u32x4{lo[0], lo[1], hi[0], hi[1]};
       }
-      __builtin_amdgcn_raw_buffer_store_b128(v, rows, soff[it % kStoreCols] + (uint32_t)((32 * mb + row) * N * kOutSize), 0, 16);
+      // (written through to memory; rows that are no whole lines are left to the caches, which put their pieces together: 6000 x 3000
+      // x 512 39.7 / 30.8 us, 4096 x 3080 x 160 18 / 13.6)
+      if (N % 64) __builtin_amdgcn_raw_buffer_store_b128(v, rows, soff[it % kStoreCols] + (uint32_t)((32 * mb + row) * N * kOutSize), 0, 0);
+      else __builtin_amdgcn_raw_buffer_store_b128(v, rows, soff[it % kStoreCols] + (uint32_t)((32 * mb + row) * N * kOutSize), 0, 16);
     }
   }
 }
 
-template <typename T, int BN>
+template <typename T, int BN, bool RAGGED>
 void launch(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint16_t *r, uint16_t *o, int64_t M, int64_t N, int64_t K,
             int act, hipStream_t stream) {
   const int tilesM = (int)((M + kBM - 1) / kBM), tilesN = (int)((N + BN - 1) / BN);
   const dim3 grid((unsigned)(tilesM * tilesN)), block(kThreads);
-  if (r) gemm_wide_kernel<T, kResidual, BN, uint16_t><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_GELU) gemm_wide_kernel<T, ACT_GELU, BN, uint16_t><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_RELU) gemm_wide_kernel<T, ACT_RELU, BN, uint16_t><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else gemm_wide_kernel<T, ACT_NONE, BN, uint16_t><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  if (r) gemm_wide_kernel<T, kResidual, BN, uint16_t, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_GELU) gemm_wide_kernel<T, ACT_GELU, BN, uint16_t, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_RELU) gemm_wide_kernel<T, ACT_RELU, BN, uint16_t, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else gemm_wide_kernel<T, ACT_NONE, BN, uint16_t, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_wide_kernel");
 }
 
 template <int BN>
 void launchToF32(const void *a, const void *w, const void *b, const void *r, float *o, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
   const int tilesM = (int)((M + kBM - 1) / kBM), tilesN = (int)((N + BN - 1) / BN);
-  gemm_wide_kernel<_Float16, kResidual, BN, float><<<dim3((unsigned)(tilesM * tilesN)), dim3(kThreads), 0, stream>>>(
+  gemm_wide_kernel<_Float16, kResidual, BN, float, false><<<dim3((unsigned)(tilesM * tilesN)), dim3(kThreads), 0, stream>>>(
       static_cast<const uint16_t *>(a), static_cast<const uint16_t *>(w), static_cast<const uint16_t *>(b), static_cast<const uint16_t *>(r), o,
       (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_wide_kernel");
@@ -379,9 +404,14 @@ void launchWidth(const void *in, const void *weight, const void *bias, const voi
   const auto *a = static_cast<const uint16_t *>(in), *w = static_cast<const uint16_t *>(weight), *b = static_cast<const uint16_t *>(bias),
              *r = static_cast<const uint16_t *>(residual);
   auto *o = static_cast<uint16_t *>(out);
-  if (width == 256) launch<T, 256>(a, w, b, r, o, M, N, K, act, stream);
-  else if (width == 192) launch<T, 192>(a, w, b, r, o, M, N, K, act, stream);
-  else launch<T, 128>(a, w, b, r, o, M, N, K, act, stream);
+  auto at = [&](auto ragged) {
+    constexpr bool RAGGED = decltype(ragged)::value;
+    if (width == 256) launch<T, 256, RAGGED>(a, w, b, r, o, M, N, K, act, stream);
+    else if (width == 192) launch<T, 192, RAGGED>(a, w, b, r, o, M, N, K, act, stream);
+    else launch<T, 128, RAGGED>(a, w, b, r, o, M, N, K, act, stream);
+  };
+  if (K % 64) at(std::true_type());
+  else at(std::false_type());
 }
 
 } // namespace
@@ -390,7 +420,8 @@ bool gemmWideSupports(DType dt, const void *in, const void *weight, const void *
                       int64_t N, int64_t K) {
   if (dt != DType::F16 && dt != DType::BF16) return false;
   // 32-bit lane offsets inside a buffer, a slice and a part; fewer than 2^23 tiles of 512 threads
-  if (M <= 0 || N <= 0 || N % 8 || K < 128 || K % 64 || K > (1 << 20) || N > (1 << 20)) return false;
+  if (M <= 0 || N <= 0 || N % 8 || K <= 64 || K % 8 || K > (1 << 20) || N > (1 << 20)) return false;
+  if (K % 64 && K * N >= int64_t(1) << 30) return false; // (a buffer holds the weight)
   if (M > 0x7fffff00 || (M + kBM - 1) / kBM > 0x7fffff / ((N + 127) / 128)) return false;
   if (!aligned16(in) || !aligned16(weight) || !aligned16(out)) return false;
   if (bias && (reinterpret_cast<uintptr_t>(bias) & 7u)) return false;
@@ -409,6 +440,7 @@ int gemmWideBest(int64_t M, int64_t N, int64_t K, int act, bool hasResidual, dou
   static const Width widths[3] = {
       {128, 4.0, 7.25e-3, 4.9e-3, 2.7, 1.95}, {192, 5.2, 10.1e-3, 7.2e-3, 4.0, 3.5}, {256, 6.0, 13.8e-3, 8.5e-3, 5.4, 5.4}};
   const int64_t cus = numComputeUnits();
+  K = (K + 63) / 64 * 64; // (what is multiplied)
   int best = 0;
   for (const Width &w : widths) {
     const int64_t tiles = (M + kBM - 1) / kBM * ((N + w.columns - 1) / w.columns), rounds = (tiles + cus - 1) / cus;
@@ -434,7 +466,7 @@ void gemmWide(DType dt, const void *in, const void *weight, const void *bias, co
 
 void gemmWideResidualF32(const void *in, const void *weight, const void *bias, const void *residual, float *out, int64_t M, int64_t N, int64_t K,
                          int width, hipStream_t stream) {
-  if (!gemmWideSupports(DType::F16, in, weight, bias, residual, out, M, N, K) || !residual) fail("gemmWide: internal dispatch error");
+  if (!gemmWideSupports(DType::F16, in, weight, bias, residual, out, M, N, K) || !residual || K % 64) fail("gemmWide: internal dispatch error");
   if (width == 256) launchToF32<256>(in, weight, bias, residual, out, M, N, K, stream);
   else if (width == 192) launchToF32<192>(in, weight, bias, residual, out, M, N, K, stream);
   else launchToF32<128>(in, weight, bias, residual, out, M, N, K, stream);

@@ -401,7 +401,7 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
       return;
     }
     // (or from gemm_wide's accumulators: 4096 x 2048 x 2048 42.2 + 11.2 for the cast behind it -> 40.5 us)
-    const int wide = kMajor[3] || reinterpret_cast<uintptr_t>(output) % 16 ? 0 : gemmWideWidth(DType::F16, M, d, ffn, ACT_NONE, true);
+    const int wide = kMajor[3] || ffn % 64 || reinterpret_cast<uintptr_t>(output) % 16 ? 0 : gemmWideWidth(DType::F16, M, d, ffn, ACT_NONE, true);
     if (wide) {
       gemmWideResidualF32(arena.at(oF), w2H, b2H, arena.at(oY), output, M, d, ffn, wide, stream);
       arena.release(stream);

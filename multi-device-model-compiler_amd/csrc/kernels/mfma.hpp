@@ -67,6 +67,22 @@ __device__ __forceinline__ void ldsLoad16LowerLanes(uint32_t offset, const char 
 __device__ __forceinline__ void ldsLoad4(uint32_t offset, const char *base, uint32_t ldsAddr) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(offset), "s"(base), "s"(ldsAddr) : "memory", "m0");
 }
+// The same through a buffer, whose bounds check answers zeros past the end (and must not be given a scalar offset past it).
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ i32x4 ldsBuffer(const void *base, uint32_t bytes) {
+  const uint64_t at = reinterpret_cast<uint64_t>(base);
+  return i32x4{(int)(uint32_t)at, (int)(uint32_t)(at >> 32) & 0xffff, (int)bytes, 0x00020000};
+}
+__device__ __forceinline__ void ldsLoad16(uint32_t offset, const i32x4 &buffer, uint32_t soffset, uint32_t ldsAddr) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(offset), "s"(buffer), "s"(soffset), "s"(ldsAddr)
+               : "memory", "m0");
+}
+__device__ __forceinline__ void ldsLoad16LowerLanes(uint32_t offset, const i32x4 &buffer, uint32_t soffset, uint32_t ldsAddr) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_mov_b32 exec_hi, 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds\n\ts_mov_b32 exec_hi, -1" ::"v"(offset),
+               "s"(buffer), "s"(soffset), "s"(ldsAddr)
+               : "memory", "m0");
+}
+constexpr uint32_t kPastBuffer = 0x80000000u; // an offset outside every buffer of less than 2 GiB
 #pragma clang diagnostic pop
 
 // Exchange with lane l ^ 32: v_permlane32_swap hands every lane the value of

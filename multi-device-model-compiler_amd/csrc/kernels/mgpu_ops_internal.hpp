@@ -99,7 +99,7 @@ double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act);
 void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,
                     int64_t M, int64_t N, int64_t K, int act, hipStream_t stream);
 
-// Tiles of 256 rows, one block per CU (gemm_wide.hip): fp16 / bf16, any M, N a multiple of 8, K of 64 from 128 on.
+// Tiles of 256 rows, one block per CU (gemm_wide.hip): fp16 / bf16, any M, N and K multiples of 8, K from 72 on.
 // width: 128, 192 or 256 columns; gemmWideBest: the width for a shape and its estimated us, on the scale of gemmKSplitBest.
 int gemmWideBest(int64_t M, int64_t N, int64_t K, int act, bool hasResidual, double *cost);
 bool gemmWideSupports(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
@@ -110,7 +110,10 @@ void gemmWide(DType dt, const void *in, const void *weight, const void *bias, co
 void gemmWideResidualF32(const void *in, const void *weight, const void *bias, const void *residual, float *out, int64_t M, int64_t N, int64_t K,
                          int width, hipStream_t stream);
 
-// At most one tile of 128 x 96 or 128 x 128 per CU (gemm_round.hip), for gemm_mfma.hip's launchers: N a multiple of 8, K of 64.
+// At most one tile of 128 x 96 or 128 x 128 per CU (gemm_round.hip): N and K multiples of 8; planes: K of 64.  gemmRoundWidth: the width
+// for a shape, 0 where it does not go.
+int gemmRoundWidth(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M, int64_t N,
+                   int64_t K);
 void gemmRound(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
                int64_t K, int act, int width, hipStream_t stream);
 void gemmRoundPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, int width, int parts,

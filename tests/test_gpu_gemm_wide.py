@@ -45,6 +45,34 @@ def test_against_float64(pkg, gpu, dtype, name, width, M, N, K):
         assert (got[0] == 7).all() and (got[-1] == 7).all()
 
 
+RAGGED = [
+    (3, 8, 72),        # the shortest of gemm_wide: a chunk of the second buffer, no pass of the loop
+    (256, 384, 136),
+    (257, 520, 184),   # the last slice of 32 all filler, and one chunk short of whole
+    (300, 1000, 232),
+    (513, 248, 1096),
+    (2300, 136, 680),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("name,width,M,N,K", [("8gemmWide", w, *s) for w in (128, 192, 256) for s in RAGGED] +
+                         [("9gemmRound", w, *s) for w in (96, 128) for s in RAGGED + [(130, 104, 8), (129, 200, 56), (64, 96, 296)]])
+def test_depths_that_are_no_multiple_of_64(pkg, gpu, dtype, name, width, M, N, K):
+    """As above; and what lies behind the end of a row or of the weight has no part in the result, whatever it is."""
+    import torch
+    test_against_float64(pkg, gpu, dtype, name, width, M, N, K)
+    t, code = (torch.float16, 1) if dtype == "f16" else (torch.bfloat16, 2)
+    x, w = torch.full((M + 1, K), float("inf"), dtype=t, device=gpu), torch.full((K + 64, N), float("nan"), dtype=t, device=gpu)
+    x[0:M:2], w[:K] = 1.0, 2.0**-4  # every other row is infinite
+    out = torch.zeros((M, N), dtype=t, device=gpu)
+    gemm = internal(pkg, "_ZN4mgpu" + name + "ENS_5DTypeEPKvS2_S2_S2_PvllliiP12ihipStream_t", None, ctypes.c_int, *[ctypes.c_void_p] * 5,
+                    *[ctypes.c_int64] * 3, ctypes.c_int, ctypes.c_int, ctypes.c_void_p)
+    gemm(code, x.data_ptr(), w.data_ptr(), None, None, out.data_ptr(), M, N, K, 0, width, torch.cuda.current_stream().cuda_stream)
+    assert (out[0::2].float() == torch.tensor(K / 16).to(t).float().item()).all() and (out[1::2] == float("inf")).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("width", [128, 192, 256])
 @pytest.mark.parametrize("M,N,K", SHAPES)
@@ -88,8 +116,10 @@ def test_planes_of_partial_sums(pkg, gpu, width, M, N, K, parts):
     (4096, 2048, 2048, 0, True, 128),
     (2304, 2048, 2560, 0, False, 128),   # beyond one round of 128 x 128 tiles, however deep
     (2049, 2048, 128, 0, False, None),   # (whatever the width)
-    (4096, 2048, 96, 0, False, 0),       # fewer steps than its loop is built for
-    (4096, 2048, 1056, 0, False, 0),     # not whole steps
+    (4096, 2048, 72, 0, False, None),    # filled up to the fewest steps its loop is built for
+    (4096, 2048, 64, 0, False, 0),
+    (4096, 2048, 1048, 0, False, None),
+    (4096, 2048, 1052, 0, False, 0),     # rows off the 16-byte grid
     (4096, 2044, 1024, 0, False, 0),
     (127, 40000, 1024, 0, False, 0),
     (4096, 768, 3072, 0, False, 0),      # up to one round of 128 x 128 tiles
