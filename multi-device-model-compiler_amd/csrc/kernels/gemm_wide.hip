@@ -445,8 +445,16 @@ int gemmWideBest(int64_t M, int64_t N, int64_t K, int act, bool hasResidual, dou
   for (const Width &w : widths) {
     const int64_t tiles = (M + kBM - 1) / kBM * ((N + w.columns - 1) / w.columns), rounds = (tiles + cus - 1) / cus;
     const double full = (double)tiles / (double)cus;
-    const double us = (double)rounds * (w.round + w.step * (double)K + (act == ACT_GELU ? w.gelu : 0.0)) +
-                      full * (w.shared * (double)K + (hasResidual ? w.residual : 0.0));
+    double us = (double)rounds * (w.round + w.step * (double)K + (act == ACT_GELU ? w.gelu : 0.0)) +
+                full * (w.shared * (double)K + (hasResidual ? w.residual : 0.0));
+    // Cards differ: on some, short products repeated back to back lose up to half of their rate once more than four fifths of the
+    // CUs pull tiles as narrow as these (the clock stays up), on others nothing.  The estimate takes a loss between the two, so that
+    // fewer, wider tiles win unless they are much slower (us on such a card / on another, tiles of 128 / 192 / 256 columns: 2048 x 4096 x
+    // 512 24 / 13.8 / 14.9 and 11.2 / 12.3 / 14.5, hipBLASLt 15 and 13; 4096 x 2048 x 1024 29 / 21.5 / 21.9 and 18.0 / 19.8 / 22.5, 23 and 21;
+    // 4096 x 3072 x 768 36 / 28 / 22.4, 26; not 4096 x 2048 x 2048 35.5 / 39.2 / 40.7, 39.7, nor 6144 x 3072 x 768 51 / 38.6 / 42.3, 42, nor 4096 x
+    // 1280 x 768, 160 tiles of 128, 11.8 / 14.0 / 16.7, 15.4).
+    const bool crowded = tiles * 5 > cus * 4 && (w.columns == 128 || (w.columns == 192 && rounds == 1));
+    if (crowded && K >= 192 && K <= 1408 && act != ACT_GELU) us += w.columns == 128 ? 9.0 : 7.0;
     if (!best || us < *cost) {
       best = w.columns;
       *cost = us;
