@@ -188,13 +188,19 @@ GemmKernel chooseKernel(DType dt, const void *in, const void *weight, const void
 // everything else - over 550 such shapes the library takes 1.19 to 1.38 times as long (by the number of tiles; never less
 // than 0.96), gemm_mfma's paired schedule before it 1.19 to 1.31 (us, library / gemm_mfma / gemm_wide: 4096 x 3072 x 768 + GELU
 // 37 / 28.2 / 24.6, 4096 x 6144 x 2048 107 / 109 / 88.5, 3000 x 2304 x 2048 36.6 / 36.6 / 27.4).  Up to one round gemm_round's
-// smaller tiles are (609 shapes: gemm_wide the best of all in 14, by 8 % at most).  Fewer than 128 rows would leave more
-// than half of every tile empty.
+// smaller tiles are (609 shapes: gemm_wide the best of all in 14, by 8 % at most) - but not where they would take more than four
+// fifths of the CUs on a product of middling depth, which some cards slow down (see gemmWideBest; us there, gemm_mfma before / gemm_round /
+// half as many tiles of 256 x 128: 2048 x 2048 x 512 10.7 / 12.0 / 8.2, x 1024 14.8 / 15.8 / 12.5, 4096 x 1024 x 512 9.7 / 11.7 / 8.0; x 256 6.8 / 5.9
+// and 2048 x 2048 x 2048 23.1 / 23.8 stay).  Fewer than 128 rows would leave more than half of every tile empty.
 int wideWidth(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M, int64_t N,
               int64_t K, int act) {
-  if (forcedKernel() || M < 128 || tiles128(M, N) <= numComputeUnits() || !gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) return 0;
+  if (forcedKernel() || M < 128 || !gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) return 0;
+  const int64_t cus = numComputeUnits(), tiles = tiles128(M, N);
+  const bool crowded = tiles <= cus && tiles * 5 > cus * 4 && K >= 384 && K <= 1408 && act != ACT_GELU;
+  if (tiles <= cus && !crowded) return 0;
   double cost;
-  return gemmWideBest(M, N, K, act, residual != nullptr, &cost);
+  const int width = gemmWideBest(M, N, K, act, residual != nullptr, &cost);
+  return !crowded || cost < gemmMfmaCost(M, N, K, act) + 3.0 ? width : 0;
 }
 
 // And gemm_round's where the depth is no multiple of 64, which it fills up with zeros (us, what ran before - the library, or gemm_mfma at
