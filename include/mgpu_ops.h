@@ -184,7 +184,7 @@ void mgpuMatmulExBF16(void *input, void *weight, void *bias, void *output, void 
                       int32_t hasResidual, mgpuStream_t stream);
 
 /* mgpuMatmulEx* only enqueue: which kernel serves a shape - the library's or one
- * of three hand-written ones, the MFMA kernel below, one for few tiles and one
+ * of the hand-written ones for many, about one round of and few 16-bit tiles and
  * for small fp32 products - comes from a table decided offline and a fixed rule,
  * never from a measurement inside this library; MGPU_GEMM_KERNEL = library |
  * mfma in the environment overrides both.  The first library GEMM on
@@ -196,10 +196,10 @@ void mgpuMatmulExBF16(void *input, void *weight, void *bias, void *output, void 
  * [K, N] row major in every call): mgpuPackWeight16 writes the K-major copy of a 16-bit weight,
  * packed[n * K + k] = weight[k * N + n], bit for bit (fp16 or bf16; a different array from
  * weight), and mgpuMatmulExPackedF16 / BF16 are mgpuMatmulExF16 / BF16 on such a copy.  The
- * GEMM library multiplies this layout 7-35 % faster at the shapes of the benchmark layers
- * (4096 x 2304 x 768: 19 against 29 us, against 22 on the hand-written kernel), so a caller
- * whose weights do not change packs them once.  The library's kernel, or for few tiles the
- * hand-written one for them; results may differ from mgpuMatmulEx* in the last bit (another
+ * GEMM library multiplies this layout faster than the other (4096 x 2304 x 768: 19 against 29
+ * us); the hand-written kernels behind mgpuMatmulEx*, which take [K, N], are ahead of both by
+ * now (18), so packing pays only where a shape is not theirs (N or K no multiple of 8).  The
+ * library's kernel, or for few tiles the hand-written one for them; results may differ from mgpuMatmulEx* in the last bit (another
  * summation order). */
 void mgpuPackWeight16(void *packed, void *weight, int64_t K, int64_t N, mgpuStream_t stream);
 void mgpuMatmulExPackedF16(void *input, void *packedWeight, void *bias, void *output, void *residual,
@@ -240,7 +240,7 @@ void mgpuLLMDecodingContextLayer(float *input, float *qkv, float *gemm_weight, f
  * mgpuLLMOpsCacheWeights(1) an array is converted the first time its (address, shape) is seen
  * and the copy is reused by every later call; the caller promises not to change a cached array
  * in place.  The copies are fp16, and a weight matrix is kept transposed ([N, K], K contiguous)
- * where the GEMM library multiplies that layout faster; mgpuBertEncoderLayerF16, whose weights
+ * where the GEMM library on that layout is the fastest; mgpuBertEncoderLayerF16, whose weights
  * are fp16 already, takes such transposed copies for the GEMMs that gain from them.  Results
  * stay within the layers' tolerances but are not bit-identical to the uncached path (another
  * GEMM kernel, another summation order).  mgpuLLMOpsCacheWeights(0) waits for the device, frees

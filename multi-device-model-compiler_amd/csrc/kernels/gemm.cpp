@@ -97,9 +97,10 @@ const TableEntry kTable[] = {
 // 128 x 128 tiles of a shape: up to one per CU every form of the hand-written kernels pays.
 int64_t tiles128(int64_t M, int64_t N) { return (M + 127) / 128 * ((N + 127) / 128); }
 
-// Where the library, on a [K, N] weight, is ahead of both hand-written 16-bit kernels: many tiles of a long reduction, its
-// steady state.  The lines lie where they cost least over 800 shapes timed on all three, aligned and ragged, 8 to 1200 tiles
-// by K 256 to 6144 (us, library / gemm_mfma or, small, gemm_ksplit):
+// Where the library, on a [K, N] weight, is ahead of both other hand-written 16-bit kernels, for products that gemm_wide and
+// gemm_round (wideWidth, raggedRoundWidth) do not take: many tiles of a long reduction, its steady state.  The lines lie where they cost least over 800 shapes timed on all three, aligned and ragged, 8 to 1200 tiles
+// by K 256 to 6144 (us, library / gemm_mfma, whose present schedule for K beyond 64 is gemm_wide's and
+// ahead, or, small, gemm_ksplit):
 //  * up to one round of the CUs its estimates choose within 0.3 % of the best of the three, the library alone 40 % behind
 //    (1536 x 2048 x 4096 37.6 / 36.6, 2048 x 2048 x 2048 25.8 / 22.1, 2000 x 2000 x 1024 17.7 / 13.7);
 //  * beyond, by tiles x K, as gemm_mfma's time grows with it: 288 tiles x 1024 22.4 / 18.5, x 2048 35.2 / 31.9, x 3072 37.1 /
