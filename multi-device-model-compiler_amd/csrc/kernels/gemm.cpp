@@ -420,6 +420,8 @@ void matmulEx(DType dt, const void *input, const void *weight, const void *bias,
     }
   switch (chooseKernel(dt, input, weight, b, r, output, M, N, K, hasBias, act, hasResidual, weightKMajor)) {
   case GemmKernel::Mfma:
+  case GemmKernel::Wide: // (gemmMfmaKernel's choice)
+  case GemmKernel::Round:
     gemmMfmaRagged(dt, input, weight, b, r, output, M, N, K, act, stream);
     return;
   case GemmKernel::KSplit: {

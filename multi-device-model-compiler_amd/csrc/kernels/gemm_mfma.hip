@@ -312,29 +312,27 @@ void launchTile(const uint16_t *a, const uint16_t *w, const uint16_t *b, const u
 
 // Tile width: the one under which the busiest CU carries the fewest columns
 // (tiles are dealt evenly, so that CU holds ceil(tiles / CUs) of them); 128 on
-// a tie.  gemm_round when no CU gets a second tile, otherwise gemm_wide, each
-// where it goes; the kernel above where neither does.
+// a tie.
+int tileWidth(int64_t M, int64_t N) {
+  const int64_t cus = numComputeUnits();
+  auto load = [&](int64_t width) { return ((M + kBM - 1) / kBM * ((N + width - 1) / width) + cus - 1) / cus * width; };
+  return load(96) < load(128) ? 96 : 128;
+}
+
 template <typename T>
 void launch(const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M,
             int64_t N, int64_t K, int act, hipStream_t stream) {
-  const int64_t cus = numComputeUnits();
-  auto tilesAt = [&](int64_t width) { return (M + kBM - 1) / kBM * ((N + width - 1) / width); };
-  auto load = [&](int64_t width) { return (tilesAt(width) + cus - 1) / cus * width; };
-  const bool narrow = load(96) < load(128);
-  const int64_t tiles = tilesAt(narrow ? 96 : 128);
-  const bool deep = tiles <= cus && (K % 64 == 0 || K * N < int64_t(1) << 30);
   const auto *a = static_cast<const uint16_t *>(in);
   const auto *w = static_cast<const uint16_t *>(weight);
   const auto *b = static_cast<const uint16_t *>(bias);
   const auto *r = static_cast<const uint16_t *>(residual);
   auto *o = static_cast<uint16_t *>(out);
   const DType dt = std::is_same<T, _Float16>::value ? DType::F16 : DType::BF16;
-  if (deep) return gemmRound(dt, in, weight, bias, residual, out, M, N, K, act, narrow ? 96 : 128, stream);
-  if (gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) {
-    double cost;
-    return gemmWide(dt, in, weight, bias, residual, out, M, N, K, act, gemmWideBest(M, N, K, act, residual != nullptr, &cost), stream);
-  }
-  if (narrow) launchTile<T, 3>(a, w, b, r, o, M, N, K, act, stream);
+  int width;
+  const GemmKernel kernel = gemmMfmaKernel(dt, in, weight, bias, residual, out, M, N, K, act, &width);
+  if (kernel == GemmKernel::Round) return gemmRound(dt, in, weight, bias, residual, out, M, N, K, act, width, stream);
+  if (kernel == GemmKernel::Wide) return gemmWide(dt, in, weight, bias, residual, out, M, N, K, act, width, stream);
+  if (width == 96) launchTile<T, 3>(a, w, b, r, o, M, N, K, act, stream);
   else launchTile<T, 4>(a, w, b, r, o, M, N, K, act, stream);
   MGPU_CHECK_LAUNCH("gemm_mfma_kernel");
 }
@@ -365,10 +363,7 @@ bool gemmMfmaSupportsRagged(DType dt, const void *in, const void *weight, const 
 // between the two is 0.3 % behind the best of them, the library and gemm_wide, whose tiles it never pays to have less than one
 // round of).  Several: what overlaps of the operand bytes at 52 GB/s a CU behind 5 us of start and end.
 double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act) {
-  const int64_t cus = numComputeUnits();
-  auto tilesAt = [&](int64_t width) { return (M + kBM - 1) / kBM * ((N + width - 1) / width); };
-  auto load = [&](int64_t width) { return (tilesAt(width) + cus - 1) / cus * width; };
-  const int64_t width = load(96) < load(128) ? 96 : 128, tiles = tilesAt(width);
+  const int64_t cus = numComputeUnits(), width = tileWidth(M, N), tiles = (M + kBM - 1) / kBM * ((N + width - 1) / width);
   const double bytes = (double)(kBM + width) * 2.0 * (double)K, full = (double)tiles / (double)cus;
   if (tiles <= cus) return 3.2 + 1.14 * full + bytes * (11.4e-6 + 2e-6 * full) + (act == ACT_GELU ? 1.4 : 0.0);
   return 5.0 + full * bytes / 52e3;
@@ -377,10 +372,8 @@ double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act) {
 int gemmRoundWidth(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M, int64_t N,
                    int64_t K) {
   if (K % 8 || K * N >= int64_t(1) << 30 || !gemmMfmaSupportsRagged(dt, in, weight, bias, residual, out, M, N, (K + 31) / 32 * 32)) return 0;
-  const int64_t cus = numComputeUnits(), tilesM = (M + kBM - 1) / kBM;
-  auto load = [&](int64_t width) { return (tilesM * ((N + width - 1) / width) + cus - 1) / cus * width; };
-  const int width = load(96) < load(128) ? 96 : 128;
-  return load(width) == width ? width : 0;
+  const int width = tileWidth(M, N);
+  return (M + kBM - 1) / kBM * ((N + width - 1) / width) <= numComputeUnits() ? width : 0;
 }
 
 // The tile width and estimated us of gemmMfmaPartialF16 without what its planes cost (gemmPartialPlan has that); no width where
@@ -400,6 +393,23 @@ void gemmMfmaPartialF16(const void *in, const void *weight, float *planes, int64
   if (!gemmMfmaSupportsRagged(DType::F16, in, weight, nullptr, nullptr, planes, M, N, K) || !width || K % 64 || K / 64 < parts)
     fail("gemmMfmaPartial: internal dispatch error");
   gemmRoundPartialF16(in, weight, planes, M, N, K, width, parts, stream);
+}
+
+// Which kernel runs a product here, and the width of its tiles: gemm_round when no CU gets a second tile, otherwise gemm_wide, each
+// where it goes, and the kernel above where neither does.  The kernel above also where gemm_wide's tiles of 256 rows would be three
+// quarters empty, or half and a GELU's wait exposed at one block a CU (us, gemm_wide / this kernel, with a GELU: 1 x 65536 x 256 16.9
+// / 11.4, 32 x 33024 x 512 15.8 / 12.1, 127 x 65536 x 512 23.7 / 19.0; without: 32 x 65536 x 128 6.7 / 6.0, 100 x 33024 x 96 6.1 / 5.7,
+// but 100 x 40000 x 128 6.0 / 6.8 and 127 x 33024 x 256 8.1 / 9.1).
+GemmKernel gemmMfmaKernel(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
+                          int64_t N, int64_t K, int act, int *width) {
+  *width = tileWidth(M, N);
+  if ((M + kBM - 1) / kBM * ((N + *width - 1) / *width) <= numComputeUnits() && (K % 64 == 0 || K * N < int64_t(1) << 30))
+    return GemmKernel::Round;
+  const bool tooFewRows = M < kBM && (act == ACT_GELU || M <= 64 || K < 128);
+  if (tooFewRows || !gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) return GemmKernel::Mfma;
+  double cost;
+  *width = gemmWideBest(M, N, K, act, residual != nullptr, &cost);
+  return GemmKernel::Wide;
 }
 
 void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,

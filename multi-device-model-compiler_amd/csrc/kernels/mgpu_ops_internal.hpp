@@ -75,7 +75,7 @@ void matmulEx(DType dt, const void *input, const void *weight, const void *bias,
 // The width at which gemm_wide serves a product (K, N > 0; 16-byte aligned operands), 0 where it does not; and which of the
 // others serves it then.
 int gemmWideWidth(DType dt, int64_t M, int64_t N, int64_t K, int act, bool hasResidual);
-enum class GemmKernel { Library, Mfma, KSplit, F32Small };
+enum class GemmKernel { Library, Mfma, KSplit, F32Small, Wide, Round };
 GemmKernel gemmKernelFor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor);
 // Should a caller that can keep a K-major copy of the weight hand that one to matmulEx for this
 // problem?  (The committed table, else: wherever the library would serve the shape.)
@@ -94,7 +94,10 @@ void gemmMfma(DType dt, const void *in, const void *weight, const void *bias, co
 // The same kernel where its tiles overhang the shape: any M, N a multiple of 8, K of 32.
 bool gemmMfmaSupportsRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual,
                             const void *out, int64_t M, int64_t N, int64_t K);
-// gemmMfmaCost: its estimated us on a shape, on the scale of gemmKSplitBest.
+// gemmMfmaKernel: which of gemm_round, gemm_wide and the kernel itself runs it there, and the width of the tiles; gemmMfmaCost:
+// the estimated us on a shape, on the scale of gemmKSplitBest.
+GemmKernel gemmMfmaKernel(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
+                          int64_t N, int64_t K, int act, int *width);
 double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act);
 void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,
                     int64_t M, int64_t N, int64_t K, int act, hipStream_t stream);

@@ -6,7 +6,7 @@ import pytest
 
 from test_index_bounds import internal
 
-LIBRARY, MFMA, KSPLIT, F32_SMALL = range(4)
+LIBRARY, MFMA, KSPLIT, F32_SMALL, WIDE, ROUND = range(6)
 NONE, RELU, GELU = range(3)
 
 
@@ -56,3 +56,24 @@ def test_layout_of_a_weight_that_is_cast_per_call(pkg, M, N, K, act, wanted):
     wants = internal(pkg, "_ZN4mgpu19gemmWantsKMajorCastENS_5DTypeElllbib", ctypes.c_bool, ctypes.c_int, *[ctypes.c_int64] * 3,
                      ctypes.c_bool, ctypes.c_int, ctypes.c_bool)
     assert wants(1, M, N, K, True, act, False) is wanted
+
+
+@pytest.mark.parametrize("M,N,K,act,kernel", [
+    (64, 40000, 128, NONE, MFMA),   # tiles of 256 rows three quarters empty
+    (65, 40000, 128, NONE, WIDE),
+    (100, 40000, 96, NONE, MFMA),
+    (127, 40000, 256, GELU, MFMA),
+    (128, 40000, 256, GELU, WIDE),
+    (128, 40000, 64, GELU, MFMA),   # too shallow for gemm_wide
+    (127, 32768, 256, GELU, ROUND),
+    (4096, 768, 768, NONE, ROUND),
+    (2000, 1024, 512, NONE, ROUND),
+])
+def test_kernel_behind_gemm_mfma(pkg, M, N, K, act, kernel):
+    """gemm_mfma's launcher hands products to gemm_round and gemm_wide; not those whose rows would leave their tiles empty."""
+    ask = internal(pkg, "_ZN4mgpu14gemmMfmaKernelENS_5DTypeEPKvS2_S2_S2_S2_llliPi", ctypes.c_int, ctypes.c_int, *[ctypes.c_void_p] * 5,
+                   *[ctypes.c_int64] * 3, ctypes.c_int, ctypes.POINTER(ctypes.c_int))
+    got = ctypes.c_int()
+    for dtype in (1, 2):
+        assert ask(dtype, 4096, 4096, 4096, None, 4096, M, N, K, act, got) == kernel
+        assert got.value in ((128, 192, 256) if kernel == WIDE else (96, 128))
