@@ -240,8 +240,8 @@ void mgpuLLMDecodingContextLayer(float *input, float *qkv, float *gemm_weight, f
  * mgpuLLMOpsCacheWeights(1) an array is converted the first time its (address, shape) is seen
  * and the copy is reused by every later call; the caller promises not to change a cached array
  * in place.  The copies are fp16, and a weight matrix is kept transposed ([N, K], K contiguous)
- * where the GEMM library on that layout is the fastest; mgpuBertEncoderLayerF16, whose weights
- * are fp16 already, takes such transposed copies for the GEMMs that gain from them.  Results
+ * for the GEMMs that the GEMM library serves (N or K no multiple of 8); mgpuBertEncoderLayerF16,
+ * whose weights are fp16 already, takes such transposed copies for the same GEMMs.  Results
  * stay within the layers' tolerances but are not bit-identical to the uncached path (another
  * GEMM kernel, another summation order).  mgpuLLMOpsCacheWeights(0) waits for the device, frees
  * the copies and returns to the default.  Calls under stream capture never use the cache.  The

@@ -92,7 +92,7 @@ struct TableEntry {
 };
 const TableEntry kTable[] = {
 #include "gemm_table.inc"
-};
+    {0, 0, 0, 0, 0, 0, 0, 0, 0}}; // (no product has no rows)
 
 // 128 x 128 tiles of a shape: up to one per CU every form of the hand-written kernels pays.
 int64_t tiles128(int64_t M, int64_t N) { return (M + 127) / 128 * ((N + 127) / 128); }
@@ -144,47 +144,6 @@ const TableEntry *tableRow(DType dt, int64_t M, int64_t N, int64_t K, bool hasBi
   return nullptr;
 }
 
-// The kernel for a call, decided without a lookup of the library's plans (a library call costs 6-7 us of
-// host time, a hand-written one a launch).
-//  * fp32: the small kernel by tiles of 32 x 32 times k, as its calls cross those of the library (us a call, library /
-//    small: 256 x 512 10.9 / 6.0, 768 x 256 10.9 / 8.6, 3072 x 64 12.3 / 11.0, 2160 x 129 17.3 / 13.3, 768 x 400 10.6 / 11.9, 3072 x
-//    129 16.9 / 17.5, 12288 x 32 20.3 / 28.2; 7 x 768 23.9 / 6.6, 256 x 768 14.5 / 7.8, 128 x 1024 10.1 / 8.7, 7 x 1536 10.0 / 11.0).  With a GELU, which is a pass of its own behind the library, further the shorter
-//    the reduction: 23500 x 64 95 / 76, 12288 x 129 64 / 60, 3072 x 256 31.4 / 27.5, 2160 x 400 33.8 / 30.8, 768 x 512 14.2 / 13.7, but
-//    23500 x 129 115 / 119, 3072 x 400 38.6 / 39.7, 2160 x 512 34.7 / 37.2.
-//  * fp16 / bf16: the aligned shapes of the table as it says; otherwise the library where libraryAhead says so, else the
-//    cheaper of gemm_mfma and gemm_ksplit by their estimates.
-//  * K-major weights: gemm_ksplit while its tiles are at most one round of the CUs, two of a reduction up to 512
-//    deep (us a call, library / gemm_ksplit, tiles of 64 x 64 times k: 414 x 80 10.7 / 6.9, 512 x 256 11.1 / 8.0, 512 x 384
-//    10.6 / 9.9, 414 x 512 11.1 / 10.6, but 414 x 768 10.5 / 12.8 and 1424 x 64 11.2 / 17.9); beyond, the library, for
-//    which the layout was made.
-GemmKernel chooseKernel(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
-                        int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor) {
-  if (forcedKernel() == 1) return GemmKernel::Library;
-  if (dt == DType::F32) {
-    const int64_t tiles = (M + 31) / 32 * ((N + 31) / 32);
-    const int64_t most = act != ACT_GELU || K > 512 ? 200000 : K <= 128 ? 1500000 : K <= 400 ? 800000 : 300000;
-    return !forcedKernel() && !weightKMajor && K <= 1024 && tiles <= most / K ? GemmKernel::F32Small : GemmKernel::Library;
-  }
-  const bool kSplitOk = gemmKSplitSupports(dt, in, weight, bias, residual, out, M, N, K);
-  double kSplitCost = 0.0;
-  const KSplitTile tile = gemmKSplitBest(M, N, K, act, &kSplitCost);
-  if (weightKMajor) {
-    const int64_t bm = tile == KSplitTile::T64x64 ? 64 : 32, bn = tile == KSplitTile::T32x32 ? 32 : 64;
-    const int64_t most = (K <= 512 ? 2 : 1) * (int64_t)numComputeUnits();
-    return kSplitOk && !forcedKernel() && (M + bm - 1) / bm * ((N + bn - 1) / bn) <= most ? GemmKernel::KSplit : GemmKernel::Library;
-  }
-  const bool mfmaOk = gemmMfmaSupportsRagged(dt, in, weight, bias, residual, out, M, N, K);
-  if (forcedKernel() == 2) return mfmaShape(dt, M, N, K) && mfmaOk ? GemmKernel::Mfma : GemmKernel::Library;
-  const bool aligned = mfmaOk && mfmaShape(dt, M, N, K);
-  if (aligned)
-    if (const TableEntry *e = tableRow(dt, M, N, K, hasBias, act, hasResidual)) return e->handWritten ? GemmKernel::Mfma : GemmKernel::Library;
-  if (libraryAhead(M, N, K, act, aligned)) return GemmKernel::Library;
-  const double mfmaCost = gemmMfmaCost(M, N, K, act);
-  if (mfmaOk && mfmaCost < kSplitCost) return GemmKernel::Mfma;
-  // (where gemm_mfma cannot go - K no multiple of 32 - its estimate stands for the library's time)
-  return kSplitOk && kSplitCost < 1.2 * mfmaCost ? GemmKernel::KSplit : GemmKernel::Library;
-}
-
 // The width at which gemm_wide serves a call, 0 where it does not.  Beyond one round of 128 x 128 tiles it is ahead of
 // everything else - over 550 such shapes the library takes 1.19 to 1.38 times as long (by the number of tiles; never less
 // than 0.96), gemm_mfma's paired schedule before it 1.19 to 1.31 (us, library / gemm_mfma / gemm_wide: 4096 x 3072 x 768 + GELU
@@ -216,6 +175,58 @@ int raggedRoundWidth(DType dt, const void *in, const void *weight, const void *b
   double kSplitCost;
   (void)gemmKSplitBest(M, N, K, act, &kSplitCost);
   return gemmMfmaCost(M, N, (K + 63) / 64 * 64, act) < kSplitCost ? width : 0;
+}
+
+// The kernel for a call, decided without a lookup of the library's plans (a library call costs 6-7 us of
+// host time, a hand-written one a launch).
+//  * fp32: the small kernel by tiles of 32 x 32 times k, as its calls cross those of the library (us a call, library /
+//    small: 256 x 512 10.9 / 6.0, 768 x 256 10.9 / 8.6, 3072 x 64 12.3 / 11.0, 2160 x 129 17.3 / 13.3, 768 x 400 10.6 / 11.9, 3072 x
+//    129 16.9 / 17.5, 12288 x 32 20.3 / 28.2; 7 x 768 23.9 / 6.6, 256 x 768 14.5 / 7.8, 128 x 1024 10.1 / 8.7, 7 x 1536 10.0 / 11.0).  With a GELU, which is a pass of its own behind the library, further the shorter
+//    the reduction: 23500 x 64 95 / 76, 12288 x 129 64 / 60, 3072 x 256 31.4 / 27.5, 2160 x 400 33.8 / 30.8, 768 x 512 14.2 / 13.7, but
+//    23500 x 129 115 / 119, 3072 x 400 38.6 / 39.7, 2160 x 512 34.7 / 37.2.
+//  * fp16 / bf16: the aligned shapes of the table as it says; otherwise the library where libraryAhead says so, else the
+//    cheaper of gemm_mfma and gemm_ksplit by their estimates.
+//  * K-major weights: gemm_ksplit while its tiles are at most one round of the CUs, two of a reduction up to 512
+//    deep (us a call, library / gemm_ksplit, tiles of 64 x 64 times k: 414 x 80 10.7 / 6.9, 512 x 256 11.1 / 8.0, 512 x 384
+//    10.6 / 9.9, 414 x 512 11.1 / 10.6, but 414 x 768 10.5 / 12.8 and 1424 x 64 11.2 / 17.9); beyond, the library, for
+//    which the layout was made.
+struct Choice {
+  GemmKernel kernel;
+  int width = 0; // of a tile of gemm_wide or gemm_round
+};
+Choice chooseKernel(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
+                    int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor) {
+  if (forcedKernel() == 1) return {GemmKernel::Library};
+  if (dt == DType::F32) {
+    const int64_t tiles = (M + 31) / 32 * ((N + 31) / 32);
+    const int64_t most = act != ACT_GELU || K > 512 ? 200000 : K <= 128 ? 1500000 : K <= 400 ? 800000 : 300000;
+    return !forcedKernel() && !weightKMajor && K <= 1024 && tiles <= most / K ? Choice{GemmKernel::F32Small} : Choice{GemmKernel::Library};
+  }
+  const bool kSplitOk = gemmKSplitSupports(dt, in, weight, bias, residual, out, M, N, K);
+  double kSplitCost = 0.0;
+  const KSplitTile tile = gemmKSplitBest(M, N, K, act, &kSplitCost);
+  if (weightKMajor) {
+    const int64_t bm = tile == KSplitTile::T64x64 ? 64 : 32, bn = tile == KSplitTile::T32x32 ? 32 : 64;
+    const int64_t most = (K <= 512 ? 2 : 1) * (int64_t)numComputeUnits();
+    return kSplitOk && !forcedKernel() && (M + bm - 1) / bm * ((N + bn - 1) / bn) <= most ? Choice{GemmKernel::KSplit} : Choice{GemmKernel::Library};
+  }
+  if (const int width = wideWidth(dt, in, weight, bias, residual, out, M, N, K, act)) return {GemmKernel::Wide, width};
+  if (const int width = raggedRoundWidth(dt, in, weight, bias, residual, out, M, N, K, act)) return {GemmKernel::Round, width};
+  const bool mfmaOk = gemmMfmaSupportsRagged(dt, in, weight, bias, residual, out, M, N, K);
+  auto mfma = [&] {
+    Choice c;
+    c.kernel = gemmMfmaKernel(dt, in, weight, bias, residual, out, M, N, K, act, &c.width);
+    return c;
+  };
+  if (forcedKernel() == 2) return mfmaShape(dt, M, N, K) && mfmaOk ? mfma() : Choice{GemmKernel::Library};
+  const bool aligned = mfmaOk && mfmaShape(dt, M, N, K);
+  if (aligned)
+    if (const TableEntry *e = tableRow(dt, M, N, K, hasBias, act, hasResidual)) return e->handWritten ? mfma() : Choice{GemmKernel::Library};
+  if (libraryAhead(M, N, K, act, aligned)) return {GemmKernel::Library};
+  const double mfmaCost = gemmMfmaCost(M, N, K, act);
+  if (mfmaOk && mfmaCost < kSplitCost) return mfma();
+  // (where gemm_mfma cannot go - K no multiple of 32 - its estimate stands for the library's time)
+  return kSplitOk && kSplitCost < 1.2 * mfmaCost ? Choice{GemmKernel::KSplit} : Choice{GemmKernel::Library};
 }
 
 using Key = std::tuple<int64_t, int64_t, int64_t, int, int, int, int, int>;
@@ -323,14 +334,18 @@ void gemmDeinit() {
   ltHandle = nullptr;
 }
 
-bool gemmPrefersKMajor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual) {
+bool gemmPrefersKMajor(DType dt, const void *weight, const void *bias, int64_t M, int64_t N, int64_t K, bool hasBias, int act,
+                       bool hasResidual) {
   if (forcedKernel()) return forcedKernel() == 1;
-  if (gemmWideWidth(dt, M, N, K, act, hasResidual)) return false;
   if (const TableEntry *e = tableRow(dt, M, N, K, hasBias, act, hasResidual)) return e->kMajorLibrary != 0;
-  // Nobody measured the shape: the library's kernels for K-major weights were ahead of its
-  // kernels for [K, N] weights at every shape measured, so the copy pays wherever the library
-  // would serve the shape anyway.
-  return !mfmaShape(dt, M, N, K) || (tiles128(M, N) > numComputeUnits() && (act == ACT_GELU ? libraryAhead(M, N, K, act, true) : K > 1024));
+  // The library's kernels for K-major weights were ahead of its kernels for [K, N] weights at every shape measured, so the copy
+  // pays wherever the library would serve the shape anyway.  Not where a kernel of ours does, which is ahead of the library on the copy
+  // too, and whose product may be split, the copy's not (us a layer, gemm_round's and gemm_ksplit's products from copies / as they
+  // are: BERT layer of 768 on 6 x 129 tokens 61.8 / 51.2, 32 x 128 95.0 / 92.3, of 512 on 10 x 136 58.9 / 47.4, 77 28.0 / 24.9; decoding
+  // layer of 2048, ffn 8192, on 500 123 / 99, of 512 on 2 x 750 67.2 / 59.0; never less than 0.98).
+  alignas(16) static const char aligned[16] = {};
+  return chooseKernel(dt, aligned, weight, hasBias ? bias : nullptr, hasResidual ? aligned : nullptr, aligned, M, N, K, hasBias, act,
+                      hasResidual, false).kernel == GemmKernel::Library;
 }
 
 int gemmWideWidth(DType dt, int64_t M, int64_t N, int64_t K, int act, bool hasResidual) {
@@ -340,16 +355,14 @@ int gemmWideWidth(DType dt, int64_t M, int64_t N, int64_t K, int act, bool hasRe
 
 GemmKernel gemmKernelFor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor) {
   alignas(16) static const char aligned[16] = {};
-  return chooseKernel(dt, aligned, aligned, aligned, nullptr, aligned, M, N, K, hasBias, act, hasResidual, weightKMajor);
+  return chooseKernel(dt, aligned, aligned, hasBias ? aligned : nullptr, hasResidual ? aligned : nullptr, aligned, M, N, K, hasBias, act,
+                      hasResidual, weightKMajor).kernel;
 }
 
 bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual) {
   // Wherever the [K, N] weight would be the library's, as its kernels for the other layout are ahead, and gemm_ksplit's
-  // where it takes that layout of a short reduction; and more than a round of tiles deeper than 1024, where those kernels
-  // are ahead of gemm_mfma too (us, gemm_mfma / library on a K-major copy: 288 tiles x 768 14.1 / 15.7, x 1024 18.5 / 15.4,
-  // x 2048 31.9 / 26.7; 384 x 1024 19.8 / 18.2, x 2048 35.1 / 28.9).
-  const bool deep = K > 1024 && act != ACT_GELU && tiles128(M, N) > numComputeUnits() && !tableRow(dt, M, N, K, hasBias, act, hasResidual);
-  if (!deep && gemmKernelFor(dt, M, N, K, hasBias, act, hasResidual, false) != GemmKernel::Library) return false;
+  // where it takes that layout of a short reduction.
+  if (gemmKernelFor(dt, M, N, K, hasBias, act, hasResidual, false) != GemmKernel::Library) return false;
   return K <= 512 || gemmKernelFor(dt, M, N, K, hasBias, act, hasResidual, true) == GemmKernel::Library;
 }
 
@@ -362,9 +375,10 @@ bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias
 PartialPlan gemmPartialPlan(const void *in, const void *weight, int64_t M, int64_t N, int64_t K, bool weightKMajor) {
   PartialPlan best;
   if (forcedKernel() || weightKMajor || K < 512) return best;
-  const GemmKernel whole = chooseKernel(DType::F16, in, weight, weight, nullptr, weight, M, N, K, true, ACT_NONE, false, false);
+  const GemmKernel whole = chooseKernel(DType::F16, in, weight, weight, nullptr, weight, M, N, K, true, ACT_NONE, false, false).kernel;
   double bestCost;
-  if (wideWidth(DType::F16, in, weight, weight, nullptr, weight, M, N, K, ACT_NONE)) (void)gemmWideBest(M, N, K, ACT_NONE, false, &bestCost);
+  if (whole == GemmKernel::Wide) (void)gemmWideBest(M, N, K, ACT_NONE, false, &bestCost);
+  else if (whole == GemmKernel::Round) bestCost = gemmMfmaCost(M, N, (K + 63) / 64 * 64, ACT_NONE);
   else if (whole == GemmKernel::Mfma) bestCost = gemmMfmaCost(M, N, K, ACT_NONE);
   else if (whole == GemmKernel::KSplit) (void)gemmKSplitBest(M, N, K, ACT_NONE, &bestCost);
   else return best;
@@ -408,20 +422,15 @@ void matmulEx(DType dt, const void *input, const void *weight, const void *bias,
     fail("matmul: an activation cannot be combined with a residual");
 
   const void *b = hasBias ? bias : nullptr, *r = hasResidual ? residual : nullptr;
-  if (!weightKMajor)
-    if (const int width = wideWidth(dt, input, weight, b, r, output, M, N, K, act)) {
-      gemmWide(dt, input, weight, b, r, output, M, N, K, act, width, stream);
-      return;
-    }
-  if (!weightKMajor)
-    if (const int width = raggedRoundWidth(dt, input, weight, b, r, output, M, N, K, act)) {
-      gemmRound(dt, input, weight, b, r, output, M, N, K, act, width, stream);
-      return;
-    }
-  switch (chooseKernel(dt, input, weight, b, r, output, M, N, K, hasBias, act, hasResidual, weightKMajor)) {
-  case GemmKernel::Mfma:
-  case GemmKernel::Wide: // (gemmMfmaKernel's choice)
+  const Choice choice = chooseKernel(dt, input, weight, b, r, output, M, N, K, hasBias, act, hasResidual, weightKMajor);
+  switch (choice.kernel) {
+  case GemmKernel::Wide:
+    gemmWide(dt, input, weight, b, r, output, M, N, K, act, choice.width, stream);
+    return;
   case GemmKernel::Round:
+    gemmRound(dt, input, weight, b, r, output, M, N, K, act, choice.width, stream);
+    return;
+  case GemmKernel::Mfma:
     gemmMfmaRagged(dt, input, weight, b, r, output, M, N, K, act, stream);
     return;
   case GemmKernel::KSplit: {

@@ -83,10 +83,10 @@ StreamState &sideOf(hipStream_t s) {
 // to the GEMMs.  With the cache on, an array is cast the first time its (address, shape) is seen
 // and the fp16 copy is kept until the cache is switched off or gpuLLMOpsDeinit; the caller
 // promises not to change a cached array in place.  The layout of a copy is the cache's own
-// business: where gemmPrefersKMajor says so for the GEMM that reads it, a weight matrix is stored
-// transposed, [N, K] with K contiguous, for which the library's kernels are 7-10 % faster at the
-// layer's shapes (4096 x 6144 x 2048: 87 against 95 us).  The BERT layer, whose weights arrive in
-// fp16, takes only such transposed copies from the cache.  Off by default: per-call casts, as in
+// business: where gemmPrefersKMajor says so for the GEMM that reads it - where the library would serve it, with N or K no multiple
+// of 8 - a weight matrix is stored transposed, [N, K] with K contiguous, for which the library's kernels are faster (4096 x 2304 x
+// 768: 19 against 29 us).  The BERT layer, whose weights arrive in fp16, takes only such transposed copies from the cache.  Off by
+// default: per-call casts, as in
 // the reference.  Guarded by scratchMutex.
 bool weightCacheOn = false;
 struct CachedWeight {
@@ -278,14 +278,15 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
   const bool useCache = cacheIsOn() && !isCapturing(stream); // a capture neither allocates nor reads the cache's events
   bool kMajor[kGemms]; // GEMM g gets a transposed copy of its weight
   {
-    auto prefers = [&](DType dt, int64_t m, int64_t n, int64_t k, bool bias, int activation, bool residual) {
-      if (useCache) return gemmPrefersKMajor(dt, m, n, k, bias, activation, residual);
-      return !gemmWideWidth(dt, m, n, k, activation, residual) && gemmWantsKMajorCast(dt, m, n, k, bias, activation, residual);
+    // (the copies, in the cache or in the arena, are aligned)
+    auto prefers = [&](int64_t n, int64_t k, bool bias, int activation, bool residual) {
+      return useCache ? gemmPrefersKMajor(DType::F16, nullptr, nullptr, M, n, k, bias, activation, residual)
+                      : gemmWantsKMajorCast(DType::F16, M, n, k, bias, activation, residual);
     };
-    kMajor[0] = prefers(DType::F16, M, 3 * d, d, false, ACT_NONE, false);
-    kMajor[1] = prefers(DType::F16, M, d, d, true, ACT_NONE, false);
-    kMajor[2] = prefers(DType::F16, M, ffn, d, true, act, false);
-    kMajor[3] = prefers(DType::F16, M, d, ffn, true, ACT_NONE, norm_first);
+    kMajor[0] = prefers(3 * d, d, false, ACT_NONE, false);
+    kMajor[1] = prefers(d, d, true, ACT_NONE, false);
+    kMajor[2] = prefers(ffn, d, true, act, false);
+    kMajor[3] = prefers(d, ffn, true, ACT_NONE, norm_first);
   }
   // (the operands of both split products are slices of the arena: aligned)
   const bool sumsOk = partialSumsSupports(nullptr, nullptr, nullptr, nullptr, output, M, d);
@@ -466,7 +467,7 @@ void bertEncoderLayerF16(const void *x, const void *wqkv, const void *bqkv, cons
   const bool cached = cacheIsOn() && !isCapturing(stream);
   auto planOf = [&](const void *w, const void *bias, const void *residual, const void *gamma, const void *beta, const void *to, int64_t K) {
     if (!partialSumsSupports(bias, residual, gamma, beta, to, M, d)) return PartialPlan{};
-    return gemmPartialPlan(nullptr, w, M, d, K, cached && gemmPrefersKMajor(DType::F16, M, d, K, true, ACT_NONE, false));
+    return gemmPartialPlan(nullptr, w, M, d, K, cached && gemmPrefersKMajor(DType::F16, w, bias, M, d, K, true, ACT_NONE, false));
   };
   const PartialPlan projPlan = planOf(wo, bo, x, gamma1, beta1, nullptr, d), ffn2Plan = planOf(w2, b2, nullptr, gamma2, beta2, out, ffn);
   const size_t oPlanes = arena.reserve((size_t)std::max(projPlan.parts, ffn2Plan.parts) * M * d * 4);
@@ -482,16 +483,16 @@ void bertEncoderLayerF16(const void *x, const void *wqkv, const void *bqkv, cons
   {
     std::lock_guard<std::mutex> lock(scratchMutex);
     if (weightCacheOn && !isCapturing(stream)) {
-      auto fromCache = [&](Weight &w, int64_t K, int64_t N, int act) {
-        if (!gemmPrefersKMajor(DType::F16, M, N, K, true, act, false)) return;
+      auto fromCache = [&](Weight &w, const void *bias, int64_t K, int64_t N, int act) {
+        if (!gemmPrefersKMajor(DType::F16, w.w, bias, M, N, K, true, act, false)) return;
         CachedWeight &cw = cachedWeight(w.w, false, K, N, true, stream);
         if (hipEvent_t e = cw.pending()) MGPU_CHECK_HIP(hipStreamWaitEvent(stream, e, 0)); // (filled by another stream, perhaps)
         w = Weight{cw.half, true};
       };
-      fromCache(wq, d, 3 * d, ACT_NONE);
-      fromCache(wp, d, d, ACT_NONE);
-      fromCache(wf1, d, ffn, ACT_GELU);
-      fromCache(wf2, ffn, d, ACT_NONE);
+      fromCache(wq, bqkv, d, 3 * d, ACT_NONE);
+      fromCache(wp, bo, d, d, ACT_NONE);
+      fromCache(wf1, b1, d, ffn, ACT_GELU);
+      fromCache(wf2, b2, ffn, d, ACT_NONE);
     }
   }
 

@@ -72,16 +72,17 @@ void gemmDeinit();
 void matmulEx(DType dt, const void *input, const void *weight, const void *bias, void *output,
               const void *residual, int64_t M, int64_t N, int64_t K, bool hasBias, int act,
               bool hasResidual, hipStream_t stream, bool weightKMajor = false);
-// The width at which gemm_wide serves a product (K, N > 0; 16-byte aligned operands), 0 where it does not; and which of the
-// others serves it then.
-int gemmWideWidth(DType dt, int64_t M, int64_t N, int64_t K, int act, bool hasResidual);
+// Which kernel matmulEx runs a product on (K, N > 0; 16-byte aligned operands), and the width at which gemm_wide serves it, 0 where
+// it does not.
 enum class GemmKernel { Library, Mfma, KSplit, F32Small, Wide, Round };
 GemmKernel gemmKernelFor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor);
+int gemmWideWidth(DType dt, int64_t M, int64_t N, int64_t K, int act, bool hasResidual);
 // Should a caller that can keep a K-major copy of the weight hand that one to matmulEx for this
-// problem?  (The committed table, else: wherever the library would serve the shape.)
-bool gemmPrefersKMajor(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual);
+// problem?  (The committed table, else: wherever the library would serve it as it is.)
+bool gemmPrefersKMajor(DType dt, const void *weight, const void *bias, int64_t M, int64_t N, int64_t K, bool hasBias, int act,
+                       bool hasResidual);
 // Would a caller that makes its fp16 weight anew on every call, in either layout at the same price, rather
-// have it K-major (for a product that gemm_wide does not serve)?
+// have it K-major?
 bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias, int act, bool hasResidual);
 
 // Hand-written MFMA GEMM (gemm_mfma.hip): fp16 / bf16, M a multiple of 128, N of

@@ -11,28 +11,28 @@ NONE, RELU, GELU = range(3)
 
 
 @pytest.mark.parametrize("M,N,K,act,kernel", [
-    (2048, 2048, 6144, NONE, MFMA),      # one round of tiles, however deep
-    (2000, 2000, 4096, RELU, MFMA),
-    (2304, 2048, 2048, NONE, MFMA),      # 288 tiles
-    (2304, 2048, 2560, NONE, LIBRARY),
-    (3072, 2048, 1536, RELU, MFMA),      # 384 tiles
-    (3072, 2048, 2048, NONE, LIBRARY),
-    (3000, 2048, 2048, RELU, LIBRARY),   # the same, ragged
-    (2500, 2304, 768, NONE, MFMA),
-    (5250, 1024, 4096, NONE, MFMA),      # 336 tiles, M at least twice N
-    (5250, 1024, 4192, RELU, LIBRARY),
-    (2047, 1024, 1536, NONE, MFMA),
-    (4096, 2048, 1024, NONE, MFMA),      # 512 whole tiles
-    (4096, 2048, 1056, NONE, LIBRARY),
-    (4000, 2048, 768, NONE, LIBRARY),    # 512 tiles that overhang
-    (3000, 2048, 3072, GELU, MFMA),      # a GELU to fuse
-    (3000, 2048, 4096, GELU, LIBRARY),
-    (4096, 3072, 1536, GELU, MFMA),
-    (5000, 3072, 1536, GELU, LIBRARY),
-    (32, 20000, 512, NONE, MFMA),        # few rows
+    (2048, 2048, 6144, NONE, ROUND),     # one round of tiles, however deep
+    (2000, 2000, 4096, RELU, ROUND),
+    (2000, 2000, 4104, NONE, ROUND),     # filled up to a multiple of 64
+    (2000, 2000, 4100, NONE, LIBRARY),   # rows off the 16-byte grid
+    (512, 3072, 72, NONE, ROUND),
+    (2304, 2048, 2560, NONE, WIDE),      # beyond one round
+    (4000, 2048, 768, RELU, WIDE),
+    (5250, 1024, 4192, NONE, WIDE),
+    (3000, 2048, 4096, GELU, WIDE),
+    (3200, 2048, 64, NONE, MFMA),        # 400 tiles, too shallow for gemm_wide
+    (3200, 2056, 64, NONE, LIBRARY),     # 425 that overhang
+    (3968, 2048, 64, NONE, MFMA),        # 496 whole ones
+    (4096, 3072, 64, GELU, MFMA),
+    (19200, 19200, 64, GELU, LIBRARY),
+    (32, 20000, 512, NONE, ROUND),       # few rows
     (32, 20000, 1024, NONE, LIBRARY),
+    (100, 40000, 256, NONE, WIDE),
+    (127, 40000, 1024, GELU, MFMA),
+    (127, 600000, 512, GELU, LIBRARY),
     (8, 16384, 1024, NONE, KSPLIT),
     (77, 2304, 768, NONE, KSPLIT),
+    (500, 2000, 1000, NONE, KSPLIT),
     (1024, 1024, 2048, NONE, KSPLIT),
 ])
 def test_kernel_of_a_product(pkg, M, N, K, act, kernel):
@@ -43,14 +43,15 @@ def test_kernel_of_a_product(pkg, M, N, K, act, kernel):
 
 
 @pytest.mark.parametrize("M,N,K,act,wanted", [
-    (3072, 2048, 2048, RELU, True),    # a decoding layer of 3072 tokens at d_model 2048
-    (3072, 6144, 2048, NONE, True),
-    (2304, 2048, 2048, NONE, True),    # although the [K, N] weight would be gemm_mfma's
+    (3072, 2048, 2048, RELU, False),   # gemm_wide's
     (2304, 2048, 768, NONE, False),
-    (2048, 2048, 2048, NONE, False),   # one round
-    (3072, 2048, 2048, GELU, False),
-    (4096, 2304, 768, NONE, False),    # a row of the table
-    (240, 768, 768, NONE, False),
+    (2048, 2048, 2048, NONE, False),   # gemm_round's
+    (512, 3000, 1000, NONE, False),    # ... of a depth that it fills up
+    (240, 768, 768, NONE, False),      # gemm_ksplit's
+    (240, 770, 768, NONE, True),       # the library's
+    (240, 770, 256, GELU, True),
+    (32, 20000, 1024, NONE, True),     # few rows: the library's either way
+    (64, 20000, 512, GELU, False),
 ])
 def test_layout_of_a_weight_that_is_cast_per_call(pkg, M, N, K, act, wanted):
     wants = internal(pkg, "_ZN4mgpu19gemmWantsKMajorCastENS_5DTypeElllbib", ctypes.c_bool, ctypes.c_int, *[ctypes.c_int64] * 3,
@@ -77,3 +78,25 @@ def test_kernel_behind_gemm_mfma(pkg, M, N, K, act, kernel):
     for dtype in (1, 2):
         assert ask(dtype, 4096, 4096, 4096, None, 4096, M, N, K, act, got) == kernel
         assert got.value in ((128, 192, 256) if kernel == WIDE else (96, 128))
+
+
+@pytest.mark.parametrize("M,N,K,act,prefers", [
+    (2000, 768, 3072, NONE, False),   # up to one round of tiles, ragged: gemm_round
+    (1368, 768, 3072, NONE, False),   # ... split over blocks
+    (774, 3072, 768, GELU, False),
+    (4096, 768, 3072, NONE, False),
+    (77, 768, 768, NONE, False),      # gemm_ksplit
+    (4096, 6144, 2048, NONE, False),  # gemm_wide
+    (774, 770, 768, NONE, True),      # no multiple of 8: the library
+    (774, 768, 3070, GELU, True),
+    (32, 20000, 1024, RELU, True),
+])
+def test_layout_of_a_weight_that_is_kept(pkg, M, N, K, act, prefers):
+    """K-major exactly where the [K, N] weight would be the library's, be it for where it lies."""
+    ask = internal(pkg, "_ZN4mgpu17gemmPrefersKMajorENS_5DTypeEPKvS2_lllbib", ctypes.c_bool, ctypes.c_int, *[ctypes.c_void_p] * 2,
+                   *[ctypes.c_int64] * 3, ctypes.c_bool, ctypes.c_int, ctypes.c_bool)
+    served = internal(pkg, "_ZN4mgpu13gemmKernelForENS_5DTypeElllbibb", ctypes.c_int, ctypes.c_int, *[ctypes.c_int64] * 3,
+                      ctypes.c_bool, ctypes.c_int, ctypes.c_bool, ctypes.c_bool)
+    assert ask(1, 4096, 4096, M, N, K, True, act, False) is prefers
+    assert (served(1, M, N, K, True, act, False, False) == LIBRARY) is prefers
+    assert ask(1, 4098, 4096, M, N, K, True, act, False) and ask(1, 4096, 4098, M, N, K, True, act, False)

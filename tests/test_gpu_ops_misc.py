@@ -220,13 +220,13 @@ def test_weight_cache_shared_by_two_streams(pkg, gpu, rng):
 
 
 def test_bert_encoder_layer_weight_cache(pkg, gpu, oracle):
-    """With mgpuLLMOpsCacheWeights(1) the BERT layer hands the GEMMs the committed table marks (QKV and FFN2 at
-    configs[4]) a transposed copy of their weight, kept by the cache: same layer against the oracle, the same
-    bits on the second call, and an odd shape (nothing in the table, library everywhere) as well."""
+    """With mgpuLLMOpsCacheWeights(1) the BERT layer hands the GEMMs that the library serves - both FFN products where ffn is
+    no multiple of 8 - a transposed copy of their weight, kept by the cache: same layer against the oracle, the same
+    bits on the second call, at the shapes that take none as well."""
     import torch
     rng = np.random.Generator(np.random.PCG64(20246))
     lib = pkg.ops()
-    for B, S, d, ffn, H in ((32, 128, 768, 3072, 12), (3, 50, 192, 200, 3)):
+    for B, S, d, ffn, H in ((32, 128, 768, 3072, 12), (3, 50, 192, 200, 3), (3, 50, 192, 204, 3)):
         h16 = lambda *s: (0.02 * rng.standard_normal(s)).astype(np.float16)
         gam = lambda: (1 + 0.02 * rng.standard_normal(d)).astype(np.float16)
         x = rng.standard_normal((B, S, d)).astype(np.float16)
@@ -266,13 +266,14 @@ def test_decoding_context_layer(pkg, gpu, oracle, rng, causal, relu, d, H):
     assert np.array_equal(got, got.astype(np.float16).astype(np.float32))
 
 
-def test_decoding_context_layer_weight_cache(pkg, gpu, oracle, rng):
-    """mgpuLLMOpsCacheWeights(1): the fp32 weights are cast once, when first seen (the matrices into a transposed
+@pytest.mark.parametrize("ffn", [1024, 1020])
+def test_decoding_context_layer_weight_cache(pkg, gpu, oracle, rng, ffn):
+    """mgpuLLMOpsCacheWeights(1): the fp32 weights are cast once, when first seen (1020: both FFN matrices into a transposed
     fp16 copy that a different library kernel multiplies, so the result is checked against the oracle, not against
     the bits of the per-call path), and later calls reuse the copies; switching the cache off and on again drops
     them, so weights changed in place in between are picked up."""
     import torch
-    B, S, d, ffn, H = 2, 128, 512, 1024, 8
+    B, S, d, H = 2, 128, 512, 8
     f = lambda *s, sc=0.03: (sc * rng.standard_normal(s)).astype(np.float32)
     x = rng.standard_normal((B, S, d)).astype(np.float32)
     Wh = [f(d, 3 * d), f(d, d), f(d), f(d, ffn), f(ffn), f(ffn, d), f(d)]
