@@ -458,7 +458,7 @@ template <int WIN> struct Staged {
   static constexpr int ROW = CG * 2 * Window<WIN>::HALF * WIN * WIN;   // floats of a channel's row among them
   static constexpr int PIECE = ROW % 4 == 0 ? 4 : 2;                   // floats loaded at a time
   static constexpr int PIECES = ROW / PIECE, LOADS = (32 * PIECES + 63) / 64;
-  static constexpr int PITCH = ROW % 16 == 0 ? ROW + 4 : ROW + (ROW % 8 == 0 ? 4 : 0); // 4 or 12 modulo 16 words: 16 rows on different banks
+  static constexpr int PITCH = ROW % 16 == 0 ? ROW + 4 : ROW + (ROW % 8 == 0 ? 4 : 0); // 4 or 12 modulo 16 words, or 98 of 7 x 7, 2 times an odd number: 16 rows on different banks
 };
 template <int WIN, int KS>
 __global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__restrict__ x, const float *__restrict__ w,
@@ -1246,30 +1246,52 @@ FastDiv fastDiv(int d) {
   return {(unsigned)((((uint64_t)1 << 32) * (((uint64_t)1 << shift) - d)) / d + 1), shift};
 }
 
-// How many wavefronts share a tile of conv_staged_kernel; 0: one of the other kernels is faster.  Us, what ran before / four /
-// eight wavefronts, a 3 x 3 unless said otherwise:
-//  * from 32 channel groups, up to two tiles a CU: 196 tiles of 32 groups 6.81 / - / 5.98, 112 of 128 20.8 / - / 16.8, 248 of
-//    128 20.0 / 18.0 / 16.0, 496 of 128 45.1 / 27.9 / 27.0; 588 of 128 45.5 / 37.2 / 37.3.  Of 16 groups, 392 tiles, 8.68 / 7.50 / -,
-//    but nothing to gain below (294: 0.96 times as fast);
-//  * four beyond: 784 tiles of 64-channel tiles 15.5 / 14.9 and, of 128 groups, 45.7 / 44.4; 980 of them 48.2 / 48.5: the 64 x 64
-//    tiles are as good from three a CU on.  Window tiles (`paired` false) are not: 1176 tiles of 96 channels 1.3-1.6 times as
-//    fast, 1568 of 32 channels 33.2 / 24.9; beyond eight a CU their two accumulators are (3136 tiles 28.0 / 29.7);
-//  * 5 x 5, a block's LDS holds one a CU of eight: 248 tiles of 32 groups 16.5 / 13.5 / 12.0, 442 tiles 42.9 / 23.3 / 24.2; of 8
-//    groups 442 tiles 16.6 / 7.7, but 784, just over three a CU, 0.89 times as fast, then 1689 26.8 / 21.7; 10125 of 16 groups 268 / 211; 64-channel
-//    tiles as above (784 tiles 43.3 / 36.2, 980 43.6 / 44.9).
-//  * 7 x 7, the same: 196 tiles of 32 groups 35.5 / 22.3 / 21.0, 112 of 128 156 / 85 / 75, 324 of 64 165 / 81 / 80, 784 of 8 33.9 / 23.2 /
-//    28.1, 6272 of 16 427 / 250 / 290; 64-channel tiles 784 of 8 25.7 / 22.0 / 27.0, of 16 39.3 / 38.5 / 43.3, 980 of 32 81.9 / 82.4.
-// 1 x 1 gained nothing: sixteen channels of a row are one line already.
-int stagedWaves(int win, int64_t tiles, int64_t groups, bool paired, int64_t cus) {
-  const int64_t few = win == 3 ? 2 * cus : cus, few4 = 3 * cus;
-  if (win == 7) return groups < 8 || (paired && tiles > few4) ? 0 : tiles <= cus ? 8 : 4;
-  if (tiles <= few && groups >= (win == 3 ? 32 : 16)) return 8;
-  if (win == 3 && groups >= 16 && tiles > cus * 3 / 2 && tiles <= (paired ? few4 : 8 * cus)) return 4;
-  if (win == 5 && tiles > cus && (tiles <= few4 || !paired)) return groups >= (tiles > few4 && tiles <= 4 * cus ? 16 : 8) ? 4 : 0;
-  return 0;
-}
-
 } // namespace
+
+// Two things beside the size decide (us, what ran before / staged, 3 x 3 unless said otherwise): whether a channel's row of the filter
+// is whole lines - IC a multiple of 32 -, since staged loads run along the rows (230 tiles from 64 channels 6.9 / 6.4, from 72 6.8 /
+// 8.1); and whether a tile has more than 16 channels, since with fewer the other kernels' filter loads touch half as many lines
+// (16 channels, 230 tiles from 128 9.1 / 9.7).  By rounds of the CUs (r, a tile each; window tiles take two beyond 400 tiles, so that
+// they waste most at r = 3):
+//  * r = 1, eight wavefronts: whole rows from 64 channels on (16 channels 14.5 / 14.8 from 256, ahead from there on where rows of the image are
+//    odd: 23 x 23 16.7 / 14.7);
+//  * r = 2: the same, 450 tiles from 32 channels 7.3 / 6.7 on four, other rows from 144 (505 from 160 22.4 / 19.1, but from 48 8.1 /
+//    8.9, 80 11.1 / 12.1), 16 channels from 192 (24.0 / 20.4; from 64 9.5 / 10.0).  The 64 x 64 tiles, from 1.5 a CU on, always (450 from
+//    40 13.3 / 8.6);
+//  * r = 3, four: all (750 from 40 channels 11.8 / 10.6; 64-channel tiles from 72 17.6 / 14.8; 16 channels from 64 15.2 / 13.0) but 16 channels from rows that are not whole;
+//  * beyond, four: whole rows, not 16 channels, not 64-channel tiles, which are as good from three a CU on (1020 from 32 11.4 / 10.5, 1500 17.1 / 15.0, but from 48 19.4 / 21.3
+//    and 16 channels from 32 13.1 / 14.8), up to eight a CU, where two accumulators are ahead (3136 tiles 28.0 / 29.7).
+//  * 5 x 5, a block's LDS holds one a CU of eight, half the channels suffice: r = 1 230 tiles from 32 9.5 / 8.0, from 40 10.2 / 10.3
+//    (16 channels 9.0 / 10.5); r = 2 330 from 20 9.8 / 9.4, 16 channels from 24 9.7 / 10.7; r = 3 750 from 24 18.1 / 14.2, 16 channels
+//    15.7 / 13.7; r = 4 1020 from 32 28.2 / 25.1, from 40 28.4 / 30.4; r = 5 1200 from 24 25.4 / 21.5; beyond 1500 from 32 40.1 / 31.4,
+//    1790 from 20 27.7 / 29.1, 16 channels 2000 from 32 37.6 / 41.0.
+//  * 7 x 7: 230 tiles from 20 11.9 / 11.7, from 64 35 / 21, 1020 from 24 43.9 / 30.4; 16 channels from 64 24.4 / 20.9, from 20 10.6 / 11.8,
+//    750 from 32 43.9 / 30.5.
+// 1 x 1 gained nothing: sixteen channels of a row are one line already.
+int convStagedWaves(int win, int64_t tiles, int64_t IC, int64_t OC, int64_t cus) {
+  const int64_t groups = IC / 2, r = (tiles + cus - 1) / cus;
+  if (IC % 2) return 0;
+  const bool whole = IC % 32 == 0, few = OC <= 16, paired = (OC - 1) % 64 >= 32; // (paired: the 64 x 64 tiles go beyond 400)
+  if (paired && r > 3) return 0;
+  if (win == 7) return groups < 8 || (few && !(whole && r <= 3)) ? 0 : r == 1 ? 8 : 4;
+  if (win == 5) {
+    if (groups < 8) return 0;
+    if (r == 1) return groups >= (few ? 64 : whole ? 16 : 24) && (whole || !few) ? 8 : 0;
+    if (r == 3) return 4;
+    if (r == 4) return whole && !few && groups >= 16 ? 4 : 0;
+    return !few && (whole || r == 2 || r == 5) ? 4 : 0;
+  }
+  if (win != 3 || groups < 16) return 0;
+  if (r == 1) return whole && groups >= (few ? 128 : 32) ? 8 : 0;
+  if (r == 2) {
+    const bool many = 2 * tiles > 3 * cus;
+    if (paired && many) return groups >= 32 ? 8 : 4;
+    if (groups < 32) return whole && !few && many ? 4 : 0;
+    return (few ? whole && groups >= 96 : whole || groups >= 72) ? 8 : 0;
+  }
+  if (r == 3) return !few || whole ? 4 : 0;
+  return whole && !few && tiles <= 8 * cus ? 4 : 0;
+}
 
 void conv2d(const float *input, const float *weight, const float *bias, float *output, const float *postAdd,
             int64_t N, int64_t IC, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW, int64_t OH,
@@ -1381,7 +1403,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
   //  * 96 channels are two 64-channel tiles with a quarter of nothing: 12 x 32 x 100 x 90 -> 96 takes 87 in LDS
   //    tiles and 66-75 in window tiles of two accumulators.
   const int64_t tiles = pix32 * ((OC + 31) / 32);
-  //    (Squares of 3 and 5 come here only where stagedWaves leaves them.)
+  //    (Squares of 3, 5 and 7 come here only where convStagedWaves leaves them.)
   const bool squareWindow = KH == KW && (KH == 1 || KH == 3 || KH == 5 || KH == 7);
   if (!narrow) {
     table(std::true_type());
@@ -1430,7 +1452,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
       const int64_t units = ((IC + 2 * Window<WIN>::HALF - 1) / (2 * Window<WIN>::HALF)) * Window<WIN>::UNITS;
       const int64_t blocks = (pixels + 63) / 64 * ((OC + 63) / 64);
       if constexpr (WIN >= 3) {
-        const int ks = IC % 2 ? 0 : stagedWaves(WIN, tiles, IC / 2, (OC - 1) % 64 >= 32, numComputeUnits());
+        const int ks = convStagedWaves(WIN, tiles, IC, OC, numComputeUnits());
         if (ks == 8) return staged(win, integral_constant<int, 8>());
         if (ks == 4) return staged(win, c4);
       }
