@@ -171,7 +171,7 @@ int raggedRoundWidth(DType dt, const void *in, const void *weight, const void *b
                      int64_t K, int act) {
   if (forcedKernel() || K % 64 == 0 || dt == DType::F32) return 0;
   const int width = gemmRoundWidth(dt, in, weight, bias, residual, out, M, N, K);
-  if (!width) return 0;
+  if (!width || gemmMfmaShallow(M, N, K, act, residual)) return 0;
   double kSplitCost;
   (void)gemmKSplitBest(M, N, K, act, &kSplitCost);
   return gemmMfmaCost(M, N, (K + 63) / 64 * 64, act) < kSplitCost ? width : 0;
@@ -210,20 +210,21 @@ Choice chooseKernel(DType dt, const void *in, const void *weight, const void *bi
     const int64_t most = (K <= 512 ? 2 : 1) * (int64_t)numComputeUnits();
     return kSplitOk && !forcedKernel() && (M + bm - 1) / bm * ((N + bn - 1) / bn) <= most ? Choice{GemmKernel::KSplit} : Choice{GemmKernel::Library};
   }
-  if (const int width = wideWidth(dt, in, weight, bias, residual, out, M, N, K, act)) return {GemmKernel::Wide, width};
-  if (const int width = raggedRoundWidth(dt, in, weight, bias, residual, out, M, N, K, act)) return {GemmKernel::Round, width};
   const bool mfmaOk = gemmMfmaSupportsRagged(dt, in, weight, bias, residual, out, M, N, K);
   auto mfma = [&] {
     Choice c;
     c.kernel = gemmMfmaKernel(dt, in, weight, bias, residual, out, M, N, K, act, &c.width);
     return c;
   };
+  if (const int width = wideWidth(dt, in, weight, bias, residual, out, M, N, K, act))
+    return mfmaOk && gemmMfmaShallow(M, N, K, act, residual) ? mfma() : Choice{GemmKernel::Wide, width};
+  if (const int width = raggedRoundWidth(dt, in, weight, bias, residual, out, M, N, K, act)) return {GemmKernel::Round, width};
   if (forcedKernel() == 2) return mfmaShape(dt, M, N, K) && mfmaOk ? mfma() : Choice{GemmKernel::Library};
   const bool aligned = mfmaOk && mfmaShape(dt, M, N, K);
   if (aligned)
     if (const TableEntry *e = tableRow(dt, M, N, K, hasBias, act, hasResidual)) return e->handWritten ? mfma() : Choice{GemmKernel::Library};
   if (libraryAhead(M, N, K, act, aligned)) return {GemmKernel::Library};
-  const double mfmaCost = gemmMfmaCost(M, N, K, act);
+  const double mfmaCost = gemmMfmaCost(M, N, K, act, hasResidual);
   if (mfmaOk && mfmaCost < kSplitCost) return mfma();
   // (where gemm_mfma cannot go - K no multiple of 32 - its estimate stands for the library's time)
   return kSplitOk && kSplitCost < 1.2 * mfmaCost ? Choice{GemmKernel::KSplit} : Choice{GemmKernel::Library};

@@ -362,9 +362,12 @@ bool gemmMfmaSupportsRagged(DType dt, const void *in, const void *weight, const 
 // One tile per CU: gemm_round, fitted to 600 shapes (4 % rms, 14 % at worst; with it and gemm_ksplit's estimate the choice
 // between the two is 0.3 % behind the best of them, the library and gemm_wide, whose tiles it never pays to have less than one
 // round of).  Several: what overlaps of the operand bytes at 52 GB/s a CU behind 5 us of start and end.
-double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act) {
+//  32 deep without a GELU, the kernel above: ahead of a second round of gemm_ksplit's tiles and of one of 64 x 64, not of smaller ones (768 x
+// 1152, gemm_ksplit / it, 3.85 / 3.39; 1.09 times as long on average), unless a residual comes in by whole lines (0.91).
+double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act, bool hasResidual) {
   const int64_t cus = numComputeUnits(), width = tileWidth(M, N), tiles = (M + kBM - 1) / kBM * ((N + width - 1) / width);
   const double bytes = (double)(kBM + width) * 2.0 * (double)K, full = (double)tiles / (double)cus;
+  if (tiles <= cus && K == 32 && act != ACT_GELU && !(hasResidual && N % 64 == 0)) return 2.3;
   if (tiles <= cus) return 3.2 + 1.14 * full + bytes * (11.4e-6 + 2e-6 * full) + (act == ACT_GELU ? 1.4 : 0.0);
   return 5.0 + full * bytes / 52e3;
 }
@@ -395,14 +398,34 @@ void gemmMfmaPartialF16(const void *in, const void *weight, float *planes, int64
   gemmRoundPartialF16(in, weight, planes, M, N, K, width, parts, stream);
 }
 
+// Where the kernel above is ahead of gemm_round and gemm_wide although they go (us, they / this kernel): a product so shallow that their
+// rings never fill, or that they fill up to a step of 64.  One round of tiles: rows that are no whole lines up to 64 deep, or 96 or 160
+// (1395 x 648 x 32 4.1 / 3.6; they take 1.13 times as long at 32 on average, 1.06 at 64, 1.09 at 96, 1.07 at 160, but 1.00 at 128 and 1.01 at
+// 224); whole lines at 32 and 96 (1.09, 1.03), not with a residual, which gemm_round asks for earlier (0.97, 0.93).  More rounds, up to
+// 256 deep: by the estimates, this kernel's fitted to 1500 products (7.5 % rms, so that it has to win by 4 %; by 10 with a GELU up to two
+// rounds, by nothing beyond, where gemm_wide's one block a CU exposes a GELU's wait each round): 5504 x 3552 x 96 15.0 / 12.7.  Of 1250
+// such products it takes 191, which become 9 % faster on average (27 slower by more than 3 %, the worst 1.14 times as long).
+bool gemmMfmaShallow(int64_t M, int64_t N, int64_t K, int act, bool hasResidual) {
+  const int64_t cus = numComputeUnits(), width = tileWidth(M, N), tiles = (M + kBM - 1) / kBM * ((N + width - 1) / width);
+  const bool wholeLines = N % 64 == 0, halfStep = K % 64 == 32;
+  if (K % 32 || K > 256 || (tiles > cus && M < kBM)) return false;
+  if (tiles <= cus) return wholeLines ? halfStep && K <= 96 && !hasResidual : K <= 64 || (halfStep && K <= 160);
+  const double each = 0.9 + 0.0107 * (double)K + (act == ACT_GELU ? 1.45 : 0.0) + (hasResidual ? (wholeLines ? 1.6 : 1.25) : 0.0) + (wholeLines ? 0.0 : 0.15);
+  double wide;
+  (void)gemmWideBest(M, N, K, act, hasResidual, &wide);
+  const double ahead = act != ACT_GELU ? 1.04 : tiles > 2 * cus ? 1.0 : 1.1;
+  return ahead * (3.6 + (double)tiles * (double)width / (128.0 * (double)cus) * each) < wide;
+}
+
 // Which kernel runs a product here, and the width of its tiles: gemm_round when no CU gets a second tile, otherwise gemm_wide, each
-// where it goes, and the kernel above where neither does.  The kernel above also where gemm_wide's tiles of 256 rows would be three
+// where it goes, and the kernel above where neither does or it is ahead.  The kernel above also where gemm_wide's tiles of 256 rows would be three
 // quarters empty, or half and a GELU's wait exposed at one block a CU (us, gemm_wide / this kernel, with a GELU: 1 x 65536 x 256 16.9
 // / 11.4, 32 x 33024 x 512 15.8 / 12.1, 127 x 65536 x 512 23.7 / 19.0; without: 32 x 65536 x 128 6.7 / 6.0, 100 x 33024 x 96 6.1 / 5.7,
 // but 100 x 40000 x 128 6.0 / 6.8 and 127 x 33024 x 256 8.1 / 9.1).
 GemmKernel gemmMfmaKernel(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
                           int64_t N, int64_t K, int act, int *width) {
   *width = tileWidth(M, N);
+  if (gemmMfmaShallow(M, N, K, act, residual != nullptr)) return GemmKernel::Mfma;
   if ((M + kBM - 1) / kBM * ((N + *width - 1) / *width) <= numComputeUnits() && (K % 64 == 0 || K * N < int64_t(1) << 30))
     return GemmKernel::Round;
   const bool tooFewRows = M < kBM && (act == ACT_GELU || M <= 64 || K < 128);

@@ -95,11 +95,13 @@ void gemmMfma(DType dt, const void *in, const void *weight, const void *bias, co
 // The same kernel where its tiles overhang the shape: any M, N a multiple of 8, K of 32.
 bool gemmMfmaSupportsRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual,
                             const void *out, int64_t M, int64_t N, int64_t K);
-// gemmMfmaKernel: which of gemm_round, gemm_wide and the kernel itself runs it there, and the width of the tiles; gemmMfmaCost:
-// the estimated us on a shape, on the scale of gemmKSplitBest.
+// gemmMfmaKernel: which of gemm_round, gemm_wide and the kernel itself runs it there, and the width of the tiles; gemmMfmaShallow:
+// is the product so shallow that the kernel itself is ahead of the other two; gemmMfmaCost: the estimated us on a shape, on the
+// scale of gemmKSplitBest.
+bool gemmMfmaShallow(int64_t M, int64_t N, int64_t K, int act, bool hasResidual);
 GemmKernel gemmMfmaKernel(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
                           int64_t N, int64_t K, int act, int *width);
-double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act);
+double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act, bool hasResidual = false);
 void gemmMfmaRagged(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out,
                     int64_t M, int64_t N, int64_t K, int act, hipStream_t stream);
 

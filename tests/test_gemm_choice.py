@@ -32,6 +32,12 @@ NONE, RELU, GELU = range(3)
     (127, 600000, 512, GELU, LIBRARY),
     (8, 16384, 1024, NONE, KSPLIT),
     (77, 2304, 768, NONE, KSPLIT),
+    (768, 1152, 32, NONE, MFMA),         # 54 tiles of 32 deep
+    (768, 1152, 32, GELU, KSPLIT),
+    (256, 1152, 32, NONE, KSPLIT),
+    (768, 1152, 64, NONE, KSPLIT),
+    (2209, 488, 96, NONE, MFMA),         # shallow
+    (5504, 3552, 96, RELU, MFMA),
     (500, 2000, 1000, NONE, KSPLIT),
     (1024, 1024, 2048, NONE, KSPLIT),
 ])
@@ -64,7 +70,21 @@ def test_layout_of_a_weight_that_is_cast_per_call(pkg, M, N, K, act, wanted):
     (65, 40000, 128, NONE, WIDE),
     (100, 40000, 96, NONE, MFMA),
     (127, 40000, 256, GELU, MFMA),
-    (128, 40000, 256, GELU, WIDE),
+    (128, 40000, 256, GELU, MFMA),  # shallow: 12.4 us on gemm_wide, 11.0 here
+    (128, 40000, 512, GELU, WIDE),
+    (1395, 648, 32, RELU, MFMA),    # one round, shallow, no whole lines
+    (2209, 488, 96, NONE, MFMA),
+    (2209, 488, 128, NONE, ROUND),
+    (300, 3000, 160, NONE, MFMA),
+    (300, 3000, 224, NONE, ROUND),
+    (2304, 576, 96, NONE, MFMA),    # whole lines
+    (2304, 576, 64, NONE, ROUND),
+    (2304, 576, 160, NONE, ROUND),
+    (5504, 3552, 96, NONE, MFMA),   # more rounds: by the estimates
+    (5504, 3552, 128, NONE, WIDE),
+    (14080, 2888, 96, GELU, MFMA),
+    (14080, 2888, 128, NONE, WIDE),
+    (5504, 3552, 320, GELU, WIDE),  # beyond 256 deep
     (128, 40000, 64, GELU, MFMA),   # too shallow for gemm_wide
     (127, 32768, 256, GELU, ROUND),
     (4096, 768, 768, NONE, ROUND),

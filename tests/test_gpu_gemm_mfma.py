@@ -2,10 +2,13 @@
 through the C ABI: every epilogue, both types, every tile geometry, shapes from
 one tile and one reduction step up to the BERT-base layer's, and the shapes it
 must refuse."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from conftest import to_dev
+from test_index_bounds import internal
 
 pytestmark = pytest.mark.gpu
 
@@ -253,3 +256,35 @@ def test_library_gemm_captured_on_a_stream_that_has_no_workspace(pkg, gpu, oracl
     call()                                      # eager, after the capture: may now allocate the workspace
     st.synchronize()
     assert np.abs(out.cpu().numpy() - ref).max() <= 1.2e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1395, 648, 32), (768, 1152, 32), (2209, 488, 96), (1100, 2000, 160), (2304, 1152, 96), (5504, 3552, 96), (2061, 8200, 224)])
+def test_shallow_products_stay_on_the_128_row_kernel(pkg, gpu, dtype, M, N, K):
+    """matmul_ex where gemm_round and gemm_wide would go too; against float64, nothing stored outside the output."""
+    import torch
+    t, code, ulp = (torch.float16, 1, 2.0**-11) if dtype == "f16" else (torch.bfloat16, 2, 2.0**-8)
+    served = internal(pkg, "_ZN4mgpu13gemmKernelForENS_5DTypeElllbibb", ctypes.c_int, ctypes.c_int, *[ctypes.c_int64] * 3, ctypes.c_bool, ctypes.c_int,
+                      ctypes.c_bool, ctypes.c_bool)
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    r = lambda *s: torch.randn(s, generator=g, device=gpu)
+    x, w, b, res = r(M, K).to(t), (r(K, N) / K**0.5).to(t), r(N).to(t), r(M, N).to(t)
+    X, W, B = x.double(), w.double(), b.double()
+    prod, size = X @ W + B, X.abs() @ W.abs() + B.abs()
+    own = 0
+    for act, residual in ((0, None), (1, None), (2, None), (0, res)):
+        own += served(code, M, N, K, True, act, residual is not None, False) == 1
+        out = torch.full((M + 2, N), 7.0, dtype=t, device=gpu)
+        run = pkg.ops().mgpuMatmulExF16 if dtype == "f16" else pkg.ops().mgpuMatmulExBF16
+        run(x.data_ptr(), w.data_ptr(), b.data_ptr(), out[1:].data_ptr(), residual.data_ptr() if residual is not None else None, M, N, K, 1, act,
+            int(residual is not None), torch.cuda.current_stream().cuda_stream)
+        got = out[1:-1].double()
+        ref = prod.relu() if act == 1 else 0.5 * prod * torch.erfc(-prod / 2**0.5) if act == 2 else prod
+        ref = ref if residual is None else ref + residual.double()
+        # one rounding of the result (and the smallest number), K + 2 fp32 roundings of partial sums no larger than |x||w| + |b|,
+        # through a GELU whose slope stays below 1.13 and whose own error is below 3e-6
+        bound = 1.05 * ulp * ref.abs() + 2.0**-25 + 1.13 * (K + 2) * 2.0**-24 * size + 3e-6 * ref.abs()
+        assert ((got - ref).abs() <= bound).all(), (act, ((got - ref).abs() / bound).max())
+        assert (out[0] == 7).all() and (out[-1] == 7).all()
+    assert own >= 1
