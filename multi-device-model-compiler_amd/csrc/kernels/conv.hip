@@ -593,7 +593,7 @@ __global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__
 // filter of its OCT x 32 channels in registers, lane half hl the taps 2 s + hl of step s, and walks
 // over tiles of 32 pixels; the taps of the next tile are in flight while this one's are multiplied
 // and stored.
-enum class Output { Cached, Through, Added }; // written through to memory or not; an addend, and not
+enum class Output { Cached, Through, Streamed, Added }; // plain stores, written through to memory, non-temporal; plain with an addend
 template <int OCT, int NS, Output OUT>
 __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                                const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
@@ -734,9 +734,7 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
 // 256 x 256 -> 64, 268 MB: 76.9 -> 65.5 us (1 x 1 from the same: 68.0 -> 49.2; a fill of as many bytes takes 39); 8 x 3 x 224 x
 // 224 -> 64 with a postAdd 87 -> 49; 8 x 3 x 128 x 128 -> 16 11.0 -> 6.7.  Stores of one tile dealt out between the matrix
 // instructions of the next measured the same, an order of tiles by XCD too, runs of tiles a wavefront 90.
-// STREAM: an output beyond what the Infinity Cache keeps leaves by non-temporal stores (72 against 65.5 us above), a smaller
-// one is written through (4 x 3 x 256 x 256 -> 64 20.6 non-temporal, 21.4 plain, 19.2 so).
-template <int KW, int NR, bool STREAM, bool ADDED>
+template <int KW, int NR, Output OUT, bool ADDED>
 __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                             const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
                                                             int P, int N, FastDiv byP, FastDiv byOW, const float *__restrict__ add,
@@ -852,7 +850,8 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
       if (ADDED) v += kEarly ? addend[r] : fromPost(voffset, soffset);
       // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
       if (relu) v = f32x4{fmaxf(v[0], 0.0f), fmaxf(v[1], 0.0f), fmaxf(v[2], 0.0f), fmaxf(v[3], 0.0f)};
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, voffset, soffset, STREAM ? 2 : 16);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, voffset, soffset,
+                                             OUT == Output::Streamed ? 2 : OUT == Output::Through ? 16 : 0);
     });
   };
   Tile even, odd;
@@ -1348,14 +1347,25 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
         input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu, (int)K, (int)pix32, (int)(4 * blocks));
   };
   const int64_t tiles128 = (pixels + 127) / 128;
-  const bool streams = N * OC * P * 4 > int64_t(128) << 20;
+  // Four pixels a lane: stores written through to memory, but (us, plain / written through / non-temporal, among passes on other inputs)
+  //  * non-temporal where the output fills the Infinity Cache by itself: 16 x 3 x 256 x 256 -> 64, 256 MiB, 65 / 63 / 57, 35 x 8 x 256 x 256 -> 32
+  //    76 / 72 / 56; of 135 MiB 30.9 / 26.7 / 31.3, and a pass that is waited for is slower so (216 MiB 49 / 46 / 55);
+  //  * plain where much is written and a tile's runs are no whole lines, of which non-temporal stores write each piece on its own: 14 x 4 x 193 x
+  //    188 -> 96, 186 MiB, 52 / 70 / 63, 17 x 1 x 101 x 68 -> 512 70 / 90 / 83; of 65 MiB 18.2 / 17.0 / 24.6, 86 18.1 / 17.0 / 27.2;
+  //    (where nothing of the output is in that cache from the pass before, plain stores are ahead of both from some 32 MiB on, by 10 % at 100 MiB);
+  //  * beside an addend non-temporal beyond 128 MiB (29 x 8 x 241 x 176 -> 32, 150 MiB, 73.6 / 71.1 / 68.3).
+  const int64_t written = N * OC * P * 4, MiB = int64_t(1) << 20;
+  const Output quadStores = add ? (written > 128 * MiB ? Output::Streamed : Output::Through)
+                            : P % 32 ? (written > 128 * MiB ? Output::Cached : Output::Through)
+                                     : written >= 256 * MiB ? Output::Streamed : Output::Through;
   auto quads = [&](auto kw, auto nr) {
     constexpr int KWC = decltype(kw)::value, NR = decltype(nr)::value;
     // two blocks per CU and channel tile
     const int64_t most = std::max<int64_t>(1, (int64_t)numComputeUnits() * 2 / ((OC + 31) / 32));
     const int64_t blocks = std::min((tiles128 + 3) / 4, most);
-    auto *kernel = add ? (streams ? conv_quads_kernel<KWC, NR, true, true> : conv_quads_kernel<KWC, NR, false, true>)
-                       : streams ? conv_quads_kernel<KWC, NR, true, false> : conv_quads_kernel<KWC, NR, false, false>;
+    auto *kernel = add ? (quadStores == Output::Streamed ? conv_quads_kernel<KWC, NR, Output::Streamed, true> : conv_quads_kernel<KWC, NR, Output::Through, true>)
+                   : quadStores == Output::Streamed ? conv_quads_kernel<KWC, NR, Output::Streamed, false>
+                   : quadStores == Output::Cached ? conv_quads_kernel<KWC, NR, Output::Cached, false> : conv_quads_kernel<KWC, NR, Output::Through, false>;
     kernel<<<gridOf(blocks, 32, 256), dim3(256), 0, stream>>>(input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu,
                                                               (int)tiles128, (int)(4 * blocks));
   };

@@ -182,3 +182,31 @@ def test_conv2d_of_large_images(pkg, gpu, N, H, W, K):
             for j in range(K[1]):
                 want += w[0, 0, i, j] * x[n, 0, i:i + y.shape[2], j:j + y.shape[3]]
         assert torch.equal(y[n, 0], want), n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,H,W,OC,add", [
+    (27, 219, 40, 256, False),   # 231 MiB of rows that are no whole lines: plain stores
+    (16, 256, 256, 64, False),   # 256 MiB of whole ones: non-temporal
+    (14, 200, 200, 64, False),   # 137 MiB: written through
+    (27, 219, 40, 250, True),    # beside an addend: non-temporal, channels past the end
+])
+def test_conv2d_of_few_taps_and_large_outputs(pkg, gpu, N, H, W, OC, add):
+    """Each way of storing; 1 x 1 from two channels, so that a reference is two products and sums in float64."""
+    import torch
+    g = torch.Generator(device=gpu).manual_seed(N + OC)
+    r = lambda *s: torch.randn(s, generator=g, device=gpu)
+    x, w, b = r(N, 2, H, W), r(OC, 2, 1, 1), r(OC)
+    post = r(N, OC, H, W) if add else None
+    count = N * OC * H * W
+    out = torch.full((count + 64,), 7.0, device=gpu)  # 32 elements before and behind
+    pkg.ops().mgpuConv2d(x.data_ptr(), w.data_ptr(), b.data_ptr(), out[32:].data_ptr(), post.data_ptr() if add else None, N, 2, H, W, OC, 1, 1,
+                         H, W, 0, 0, 0, 0, 1, 1, 1, 1, add, False, torch.cuda.current_stream().cuda_stream)
+    assert (out[:32] == 7).all() and (out[-32:] == 7).all()
+    got = out[32:-32].view(N, OC, H, W)
+    for n in range(N):
+        a, c = (w[:, i, :, :].double() * x[n, i].double() for i in (0, 1))
+        ref, size = a + c + b.double()[:, None, None], a.abs() + c.abs() + b.abs().double()[:, None, None]
+        if add:
+            ref, size = ref + post[n].double(), size + post[n].abs().double()
+        assert ((got[n].double() - ref).abs() <= 4 * 2.0**-24 * size).all()  # a rounding each of at most four partial sums
