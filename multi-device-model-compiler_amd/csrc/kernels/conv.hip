@@ -1292,6 +1292,24 @@ int convStagedWaves(int win, int64_t tiles, int64_t IC, int64_t OC, int64_t cus)
   return whole && !few && tiles <= 8 * cus ? 4 : 0;
 }
 
+// Do patches take a 5 x 5 or 7 x 7 from one channel or three?  From half of a row's tiles filled on (us, window tiles / patches, 7 x 7 from
+// 3 channels unless said otherwise: 1 x 224 x 224 -> 64 of stride 2 13.0 / 7.4, 16 x 256 x 256 94 / 57, 4 x 112 x 112 -> 32 14.2 / 10.3, 2 x
+// 28 x 28 -> 96 7.5 / 6.9; 32 x 28 x 28 -> 64 from 1 12.3 / 5.7; 5 x 5 16 x 128 x 128 -> 64 55 / 33; but rows of 10 13.1 / 16.4).  From one
+// channel always.  From three, not where
+//  * a 5 x 5 has few window tiles, whose start is shorter: up to one a CU (13 x 37 x 17 -> 24 5.5 / 6.0), at stride 2 up to 400, where they
+//    take four wavefronts each (4 x 26 x 57 -> 32 5.0 / 5.9, 2 x 50 x 116 -> 24 5.3 / 6.1);
+//  * half-filled rows cost patches another round of the SIMDs, a tile each, and the 64 x 64 tiles are no alternative: 8 x 95 x 146 -> 32, 5 x 5 of
+//    stride 2, 6.4 / 7.6, 4 x 90 x 82 -> 8 8.4 / 9.5.
+// Over 1500 shapes 0.82 of the time before, one more than 3 % slower, 1.06 times; without the last two lines 105 of 1300, up to 1.20 times.
+bool convByPatches(int win, int stride, int64_t tiles, int64_t rowTiles, int64_t IC, int64_t OC, int64_t OW, int64_t cus) {
+  if ((win != 5 && win != 7) || (IC != 1 && IC != 3) || stride > 2 || 2 * OW < (OW + 31) / 32 * 32) return false;
+  if (IC == 1) return true;
+  if (win == 5 && tiles <= (stride == 1 ? cus : 400)) return false;
+  const int64_t simds = 4 * cus, rounds = (rowTiles + simds - 1) / simds, before = (tiles + simds - 1) / simds;
+  const bool paired = (OC - 1) % 64 >= 32;
+  return paired || 2 * rounds < (win == 5 && stride == 2 ? 3 : 4) * before;
+}
+
 void conv2d(const float *input, const float *weight, const float *bias, float *output, const float *postAdd,
             int64_t N, int64_t IC, int64_t H, int64_t W, int64_t OC, int64_t KH, int64_t KW, int64_t OH,
             int64_t OW, int64_t PHL, int64_t PWL, int64_t PHR, int64_t PWR, int64_t SH, int64_t SW, int64_t DH,
@@ -1444,11 +1462,8 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     // (two accumulators share the gathered taps; few pixels are spread over more wavefronts instead)
     if (OC > 32 && pix32 >= 4 * numComputeUnits()) steps(c2);
     else steps(c1);
-  } else if (squareWindow && KH >= 5 && (IC == 1 || IC == 3) && DW == 1 && SW <= 2 && 2 * OW >= 32 * across && fitsInt(N * OH * across)) {
-    // From half of a row's tiles filled on (us, window tiles / patches, 7 x 7 from 3 channels unless said otherwise: 1 x 224 x 224 -> 64
-    // of stride 2 13.0 / 7.4, 16 x 256 x 256 94 / 57, 4 x 112 x 112 -> 32 14.2 / 10.3, 2 x 28 x 28 -> 96 7.5 / 6.9; 32 x 28 x 28 -> 64 from
-    // 1 12.3 / 5.7; 5 x 5 16 x 128 x 128 -> 64 55 / 33, rows of 17 19.3 / 18.8; but rows of 10 13.1 / 16.4;
-    // from 2 channels, whole pairs, 1 x 56 x 56 3.6 / 5.1).
+  } else if (squareWindow && DW == 1 && fitsInt(N * OH * across) &&
+             convByPatches((int)KH, (int)SW, tiles, N * OH * across * ((OC + 31) / 32), IC, OC, OW, numComputeUnits())) {
     auto go = [&](auto kw, auto nr) {
       if (SW == 1) patch(kw, nr, c1);
       else patch(kw, nr, c2);

@@ -53,3 +53,27 @@ from test_index_bounds import internal
 def test_wavefronts_a_tile(pkg, win, tiles, IC, OC, waves):
     ask = internal(pkg, "_ZN4mgpu15convStagedWavesEillll", ctypes.c_int, ctypes.c_int, *[ctypes.c_int64] * 4)
     assert ask(win, tiles, IC, OC, 256) == waves
+
+
+@pytest.mark.parametrize("win,stride,tiles,rowTiles,IC,OC,OW,patches", [
+    (5, 1, 1, 1, 1, 8, 16, True),         # from one channel, if half of a row's tiles are filled
+    (5, 1, 1, 1, 1, 8, 15, False),
+    (7, 2, 1, 2, 1, 8, 33, True),
+    (7, 1, 1, 1, 3, 8, 32, True),
+    (5, 1, 256, 300, 3, 64, 28, False),   # few tiles
+    (5, 1, 257, 300, 3, 64, 28, True),
+    (5, 2, 400, 500, 3, 96, 28, False),
+    (5, 2, 401, 500, 3, 96, 28, True),
+    (7, 2, 256, 300, 3, 96, 28, True),
+    (7, 1, 1024, 1025, 3, 96, 28, False), # another round of the SIMDs
+    (7, 1, 1025, 1026, 3, 96, 28, True),
+    (7, 1, 1024, 1025, 3, 64, 28, True),  # instead of 64 x 64 tiles
+    (5, 1, 2048, 3072, 3, 96, 28, True),  # three for two
+    (5, 2, 2048, 3072, 3, 96, 28, False),
+    (7, 3, 9000, 9000, 3, 96, 64, False),
+    (3, 1, 9000, 9000, 3, 96, 64, False),
+    (7, 1, 9000, 9000, 2, 96, 64, False),
+])
+def test_patches_of_input_rows(pkg, win, stride, tiles, rowTiles, IC, OC, OW, patches):
+    ask = internal(pkg, "_ZN4mgpu13convByPatchesEiillllll", ctypes.c_bool, ctypes.c_int, ctypes.c_int, *[ctypes.c_int64] * 6)
+    assert ask(win, stride, tiles, rowTiles, IC, OC, OW, 256) is patches

@@ -87,7 +87,9 @@ def test_conv2d_with_the_filter_through_lds(pkg, gpu, oracle, rng, N, IC, H, W, 
     (2, 1, 20, 100, 32, (7, 7), (0, 5, 6, 0), (1, 1), (2, 1), False, True),    # dilated down, padding on two sides
     (70, 1, 9, 22, 40, (7, 7), (3, 2, 3, 4), (3, 1), (1, 1), False, False),    # rows shorter than a tile, several tiles a wavefront
     (2, 3, 33, 96, 520, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), False, True),    # whole tiles, 17 channel tiles
-    (1, 3, 5, 39, 1, (5, 5), (0, 0, 0, 0), (1, 2), (1, 1), True, False),       # one output row
+    (1, 3, 5, 39, 1, (5, 5), (0, 0, 0, 0), (1, 2), (1, 1), True, False),       # one output row: few tiles, not by patches
+    (40, 3, 5, 299, 96, (5, 5), (0, 0, 0, 0), (1, 2), (1, 1), True, False),    # one output row an image
+    (40, 3, 5, 299, 64, (5, 5), (0, 0, 0, 0), (1, 2), (1, 1), True, True),     # ... of fewer tiles: not by patches
 ])
 def test_conv2d_of_few_channels_by_patches(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add):
     conv_case(pkg, gpu, oracle, rng, N, IC, H, W, OC, K, pad, stride, dilation, relu, add)
