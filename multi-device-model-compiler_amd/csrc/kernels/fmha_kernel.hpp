@@ -136,7 +136,8 @@ constexpr float kSumFloor = 0.015625f;
 // fetches chunk 0 of that row instead (in bounds, finite wherever the row is),
 // Q is zero there, so the scores do not see the K filler, and the O^T rows the V
 // filler feeds are never stored.
-template <typename T, int D, int NQ, bool CAUSAL, bool TRACE = false, bool PAD = false, bool HALVES = false>
+// SHORT: no sequence is longer than a tile of keys (kLoadsBehindScores has the reason).
+template <typename T, int D, int NQ, bool CAUSAL, bool TRACE = false, bool PAD = false, bool HALVES = false, bool SHORT = false>
 __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) ? 3 : 2) void fmha_fwd_kernel(const uint16_t *__restrict__ qkv,
                                                               const int32_t *__restrict__ seqlens,
                                                               const int32_t *__restrict__ cuSeqlens,
@@ -412,10 +413,13 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
       for (int c = 0; c < G::DC; c++) asm volatile("" ::"v"(qf[qi][c]));
   }
   // Where the loads of the next tile go out: right behind the barrier they keep a wavefront from its score MFMAs until the
-  // address path has taken all of them (16 cycles an instruction, 8 of every wavefront at head_dim 128); behind the scores the wait falls under MFMAs that are still running.  At head_dim 128 (b2 s4096 h32 606 -> 555 us, b4
-  // s2048 h32 333 -> 318, b8 s1024 h32 186 -> 178, b8 s700 h12 d96 45.3 -> 40.9, causal b4 s2048 h32 188 -> 186; b16 s256 h16 16.0
-  // -> 16.4); at 64, four loads a wavefront and three wavefronts a SIMD, the causal kernel loses 3-5 %, and at 256 it spills.
-  constexpr bool kLoadsBehindScores = D == 128;
+  // address path has taken all of them (16 cycles an instruction, 8 of every wavefront at head_dim 128); behind the scores the wait
+  // falls under MFMAs that are still running.  At head_dim 128 (b2 s4096 h32 606 -> 555 us, b4 s2048 h32 333 -> 318, b8 s1024 h32
+  // 186 -> 178, b8 s700 h12 d96 45.3 -> 40.9, causal b4 s2048 h32 171 -> 162; over 360 launches of 2 to 7 tiles 0.98 of the
+  // time); at 64, four loads a wavefront and three wavefronts a SIMD, the causal kernel loses 3-5 %, and at 256 it spills.  So
+  // written the compiler peels the first tile off the loop, 600 instructions that a launch of one unmasked tile fetches for nothing
+  // (b9 s8 h12 4.10 -> 4.28 us): such a launch has an instance with the loads in front (without a loop at all, 4.2).
+  constexpr bool kLoadsBehindScores = D == 128 && !SHORT;
   for (int kt = 0; kt < trips; kt++) {
     if (TRACE) tMark = clock64();
     // The loads of tile kt (and of nothing later) must have landed; the barrier
