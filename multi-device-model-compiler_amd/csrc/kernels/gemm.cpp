@@ -154,26 +154,27 @@ const TableEntry *tableRow(DType dt, int64_t M, int64_t N, int64_t K, bool hasBi
 // and 2048 x 2048 x 2048 23.1 / 23.8 stay).  Fewer than 128 rows would leave more than half of every tile empty.
 int wideWidth(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M, int64_t N,
               int64_t K, int act) {
-  if (forcedKernel() || M < 128 || !gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) return 0;
   const int64_t cus = numComputeUnits(), tiles = tiles128(M, N);
   const bool crowded = tiles <= cus && tiles * 5 > cus * 4 && K >= 384 && K <= 1408 && act != ACT_GELU;
-  if (tiles <= cus && !crowded) return 0;
+  if ((tiles <= cus && !crowded) || M < 128 || forcedKernel() || !gemmWideSupports(dt, in, weight, bias, residual, out, M, N, K)) return 0;
   double cost;
   const int width = gemmWideBest(M, N, K, act, residual != nullptr, &cost);
   return !crowded || cost < gemmMfmaCost(M, N, K, act) + 3.0 ? width : 0;
 }
+
+// What gemmMfmaCost answers at least, for gemm_round and for any of its kernels: a call of few tiles is decided without it (155 -> 65 ns of
+// the 2.8 us that a call takes the host).
+constexpr double kRoundLeast = 3.2, kMfmaLeast = 2.3;
 
 // And gemm_round's where the depth is no multiple of 64, which it fills up with zeros (us, what ran before - the library, or gemm_mfma at
 // multiples of 32 - / gemm_round: 512 x 3072 x 72 10.5 / 4.6, x 296 10.4 / 5.6, x 1000 16.1 / 10.5, x 3000 30.9 / 23.6; 3000 x 1000 x 520 15.6 /
 // 10.3; x 96 6.0 / 6.4, x 1376 18.3 / 17.0).  Where gemm_ksplit's estimate is lower it stays: 500 x 2000 x 1000 9.6 / 9.6.  gemm_wide, the
 // same: 4261 x 1064 x 1000 28.4 / 18.4, 6000 x 3000 x 520 49.9 / 31, 4096 x 3080 x 296 33.0 / 16.9, x 160 26.1 / 13.6.
 int raggedRoundWidth(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M, int64_t N,
-                     int64_t K, int act) {
-  if (forcedKernel() || K % 64 == 0 || dt == DType::F32) return 0;
+                     int64_t K, int act, double kSplitCost) {
+  if (K % 64 == 0 || dt == DType::F32 || kSplitCost <= kRoundLeast || forcedKernel()) return 0;
   const int width = gemmRoundWidth(dt, in, weight, bias, residual, out, M, N, K);
   if (!width || gemmMfmaShallow(M, N, K, act, residual)) return 0;
-  double kSplitCost;
-  (void)gemmKSplitBest(M, N, K, act, &kSplitCost);
   return gemmMfmaCost(M, N, (K + 63) / 64 * 64, act) < kSplitCost ? width : 0;
 }
 
@@ -193,6 +194,7 @@ int raggedRoundWidth(DType dt, const void *in, const void *weight, const void *b
 struct Choice {
   GemmKernel kernel;
   int width = 0; // of a tile of gemm_wide or gemm_round
+  KSplitTile tile = KSplitTile::T32x32; // of gemm_ksplit
 };
 Choice chooseKernel(DType dt, const void *in, const void *weight, const void *bias, const void *residual, const void *out, int64_t M,
                     int64_t N, int64_t K, bool hasBias, int act, bool hasResidual, bool weightKMajor) {
@@ -208,7 +210,7 @@ Choice chooseKernel(DType dt, const void *in, const void *weight, const void *bi
   if (weightKMajor) {
     const int64_t bm = tile == KSplitTile::T64x64 ? 64 : 32, bn = tile == KSplitTile::T32x32 ? 32 : 64;
     const int64_t most = (K <= 512 ? 2 : 1) * (int64_t)numComputeUnits();
-    return kSplitOk && !forcedKernel() && (M + bm - 1) / bm * ((N + bn - 1) / bn) <= most ? Choice{GemmKernel::KSplit} : Choice{GemmKernel::Library};
+    return kSplitOk && !forcedKernel() && (M + bm - 1) / bm * ((N + bn - 1) / bn) <= most ? Choice{GemmKernel::KSplit, 0, tile} : Choice{GemmKernel::Library};
   }
   const bool mfmaOk = gemmMfmaSupportsRagged(dt, in, weight, bias, residual, out, M, N, K);
   auto mfma = [&] {
@@ -218,16 +220,17 @@ Choice chooseKernel(DType dt, const void *in, const void *weight, const void *bi
   };
   if (const int width = wideWidth(dt, in, weight, bias, residual, out, M, N, K, act))
     return mfmaOk && gemmMfmaShallow(M, N, K, act, residual) ? mfma() : Choice{GemmKernel::Wide, width};
-  if (const int width = raggedRoundWidth(dt, in, weight, bias, residual, out, M, N, K, act)) return {GemmKernel::Round, width};
+  if (const int width = raggedRoundWidth(dt, in, weight, bias, residual, out, M, N, K, act, kSplitCost)) return {GemmKernel::Round, width};
   if (forcedKernel() == 2) return mfmaShape(dt, M, N, K) && mfmaOk ? mfma() : Choice{GemmKernel::Library};
   const bool aligned = mfmaOk && mfmaShape(dt, M, N, K);
   if (aligned)
     if (const TableEntry *e = tableRow(dt, M, N, K, hasBias, act, hasResidual)) return e->handWritten ? mfma() : Choice{GemmKernel::Library};
   if (libraryAhead(M, N, K, act, aligned)) return {GemmKernel::Library};
+  if (kSplitOk && kSplitCost <= kMfmaLeast) return {GemmKernel::KSplit, 0, tile};
   const double mfmaCost = gemmMfmaCost(M, N, K, act, hasResidual);
   if (mfmaOk && mfmaCost < kSplitCost) return mfma();
   // (where gemm_mfma cannot go - K no multiple of 32 - its estimate stands for the library's time)
-  return kSplitOk && kSplitCost < 1.2 * mfmaCost ? Choice{GemmKernel::KSplit} : Choice{GemmKernel::Library};
+  return kSplitOk && kSplitCost < 1.2 * mfmaCost ? Choice{GemmKernel::KSplit, 0, tile} : Choice{GemmKernel::Library};
 }
 
 using Key = std::tuple<int64_t, int64_t, int64_t, int, int, int, int, int>;
@@ -434,12 +437,9 @@ void matmulEx(DType dt, const void *input, const void *weight, const void *bias,
   case GemmKernel::Mfma:
     gemmMfmaRagged(dt, input, weight, b, r, output, M, N, K, act, stream);
     return;
-  case GemmKernel::KSplit: {
-    double cost;
-    const KSplitTile tile = gemmKSplitBest(M, N, K, act, &cost);
-    gemmKSplit(dt, input, weight, b, r, output, M, N, K, act, tile, weightKMajor, stream);
+  case GemmKernel::KSplit:
+    gemmKSplit(dt, input, weight, b, r, output, M, N, K, act, choice.tile, weightKMajor, stream);
     return;
-  }
   case GemmKernel::F32Small:
     gemmF32Small(static_cast<const float *>(input), static_cast<const float *>(weight), static_cast<const float *>(b),
                  static_cast<const float *>(r), static_cast<float *>(output), M, N, K, act, stream);
