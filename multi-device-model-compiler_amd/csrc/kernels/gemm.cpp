@@ -164,7 +164,7 @@ int wideWidth(DType dt, const void *in, const void *weight, const void *bias, co
 
 // What gemmMfmaCost answers at least, for gemm_round and for any of its kernels: a call of few tiles is decided without it (155 -> 65 ns of
 // the 2.8 us that a call takes the host).
-constexpr double kRoundLeast = 3.2, kMfmaLeast = 2.3;
+constexpr double kRoundLeast = 3.2, kMfmaLeast = 2.4;
 
 // And gemm_round's where the depth is no multiple of 64, which it fills up with zeros (us, what ran before - the library, or gemm_mfma at
 // multiples of 32 - / gemm_round: 512 x 3072 x 72 10.5 / 4.6, x 296 10.4 / 5.6, x 1000 16.1 / 10.5, x 3000 30.9 / 23.6; 3000 x 1000 x 520 15.6 /

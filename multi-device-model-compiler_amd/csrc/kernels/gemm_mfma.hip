@@ -359,15 +359,21 @@ bool gemmMfmaSupportsRagged(DType dt, const void *in, const void *weight, const 
   return gemmMfmaSupports(dt, in, weight, bias, residual, out, m, n, K);
 }
 
+// Is the kernel above ahead of gemm_round in one round (gemmMfmaShallow has the times)?
+static bool shallowRound(int64_t N, int64_t K, bool hasResidual) {
+  const bool halfStep = K % 64 == 32;
+  return K % 32 == 0 && (N % 64 == 0 ? halfStep && K <= 96 && !hasResidual : K <= 64 || (halfStep && K <= 160));
+}
+
 // One tile per CU: gemm_round, fitted to 600 shapes (4 % rms, 14 % at worst; with it and gemm_ksplit's estimate the choice
 // between the two is 0.3 % behind the best of them, the library and gemm_wide, whose tiles it never pays to have less than one
 // round of).  Several: what overlaps of the operand bytes at 52 GB/s a CU behind 5 us of start and end.
-//  32 deep without a GELU, the kernel above: ahead of a second round of gemm_ksplit's tiles and of one of 64 x 64, not of smaller ones (768 x
-// 1152, gemm_ksplit / it, 3.85 / 3.39; 1.09 times as long on average), unless a residual comes in by whole lines (0.91).
+// A shallow round without a GELU: the kernel above, ahead of a second round of gemm_ksplit's tiles and, 32 deep, of one of 64 x 64 (us,
+// gemm_ksplit / it: 768 x 1152 x 32 3.85 / 3.39, 26 x 18240 x 32 4.7 / 3.8, 1 x 23568 x 96 4.45 / 3.8).
 double gemmMfmaCost(int64_t M, int64_t N, int64_t K, int act, bool hasResidual) {
   const int64_t cus = numComputeUnits(), width = tileWidth(M, N), tiles = (M + kBM - 1) / kBM * ((N + width - 1) / width);
   const double bytes = (double)(kBM + width) * 2.0 * (double)K, full = (double)tiles / (double)cus;
-  if (tiles <= cus && K == 32 && act != ACT_GELU && !(hasResidual && N % 64 == 0)) return 2.3;
+  if (tiles <= cus && act != ACT_GELU && shallowRound(N, K, hasResidual)) return 2.0 + 0.0125 * (double)K;
   if (tiles <= cus) return 3.2 + 1.14 * full + bytes * (11.4e-6 + 2e-6 * full) + (act == ACT_GELU ? 1.4 : 0.0);
   return 5.0 + full * bytes / 52e3;
 }
@@ -407,9 +413,9 @@ void gemmMfmaPartialF16(const void *in, const void *weight, float *planes, int64
 // such products it takes 191, which become 9 % faster on average (27 slower by more than 3 %, the worst 1.14 times as long).
 bool gemmMfmaShallow(int64_t M, int64_t N, int64_t K, int act, bool hasResidual) {
   const int64_t cus = numComputeUnits(), width = tileWidth(M, N), tiles = (M + kBM - 1) / kBM * ((N + width - 1) / width);
-  const bool wholeLines = N % 64 == 0, halfStep = K % 64 == 32;
-  if (K % 32 || K > 256 || (tiles > cus && M < kBM)) return false;
-  if (tiles <= cus) return wholeLines ? halfStep && K <= 96 && !hasResidual : K <= 64 || (halfStep && K <= 160);
+  const bool wholeLines = N % 64 == 0;
+  if (tiles <= cus) return shallowRound(N, K, hasResidual);
+  if (K % 32 || K > 256 || M < kBM) return false;
   const double each = 0.9 + 0.0107 * (double)K + (act == ACT_GELU ? 1.45 : 0.0) + (hasResidual ? (wholeLines ? 1.6 : 1.25) : 0.0) + (wholeLines ? 0.0 : 0.15);
   double wide;
   (void)gemmWideBest(M, N, K, act, hasResidual, &wide);

@@ -36,6 +36,9 @@ NONE, RELU, GELU = range(3)
     (768, 1152, 32, GELU, KSPLIT),
     (256, 1152, 32, NONE, KSPLIT),
     (768, 1152, 64, NONE, KSPLIT),
+    (26, 18248, 32, NONE, MFMA),         # two rounds of gemm_ksplit's
+    (1, 23560, 96, NONE, MFMA),
+    (83, 6128, 96, NONE, KSPLIT),        # one
     (2209, 488, 96, NONE, MFMA),         # shallow
     (5504, 3552, 96, RELU, MFMA),
     (500, 2000, 1000, NONE, KSPLIT),

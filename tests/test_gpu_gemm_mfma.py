@@ -260,7 +260,7 @@ def test_library_gemm_captured_on_a_stream_that_has_no_workspace(pkg, gpu, oracl
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
-@pytest.mark.parametrize("M,N,K", [(1395, 648, 32), (768, 1152, 32), (2209, 488, 96), (1100, 2000, 160), (2304, 1152, 96), (5504, 3552, 96), (2061, 8200, 224)])
+@pytest.mark.parametrize("M,N,K", [(1395, 648, 32), (768, 1152, 32), (26, 18248, 32), (1, 23560, 96), (2209, 488, 96), (1100, 2000, 160), (2304, 1152, 96), (5504, 3552, 96), (2061, 8200, 224)])
 def test_shallow_products_stay_on_the_128_row_kernel(pkg, gpu, dtype, M, N, K):
     """matmul_ex where gemm_round and gemm_wide would go too; against float64, nothing stored outside the output."""
     import torch
