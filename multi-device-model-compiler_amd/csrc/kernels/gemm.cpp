@@ -97,27 +97,18 @@ const TableEntry kTable[] = {
 // 128 x 128 tiles of a shape: up to one per CU every form of the hand-written kernels pays.
 int64_t tiles128(int64_t M, int64_t N) { return (M + 127) / 128 * ((N + 127) / 128); }
 
-// Where the library, on a [K, N] weight, is ahead of both other hand-written 16-bit kernels, for products that gemm_wide and
-// gemm_round (wideWidth, raggedRoundWidth) do not take: many tiles of a long reduction, its steady state.  The lines lie where they cost least over 800 shapes timed on all three, aligned and ragged, 8 to 1200 tiles
-// by K 256 to 6144 (us, library / gemm_mfma, whose present schedule for K beyond 64 is gemm_wide's and
-// ahead, or, small, gemm_ksplit):
-//  * up to one round of the CUs its estimates choose within 0.3 % of the best of the three, the library alone 40 % behind
-//    (1536 x 2048 x 4096 37.6 / 36.6, 2048 x 2048 x 2048 25.8 / 22.1, 2000 x 2000 x 1024 17.7 / 13.7);
-//  * beyond, by tiles x K, as gemm_mfma's time grows with it: 288 tiles x 1024 22.4 / 18.5, x 2048 35.2 / 31.9, x 3072 37.1 /
-//    46.9; 336 x 2048 35.7 / 32.4, x 2560 36.2 / 39.9; 384 x 1024 19.1 / 19.7, x 2048 31.2 / 35.1, x 4096 54 / 64; where M is at
-//    least twice N, later (5226 x 840 x 2720 47.6 / 41.0, 5250 x 1024 x 4096 63 / 59, 7936 x 768 x 4352 56.9 / 68.0).  1.6 %
-//    behind the best on average, worst 38 %, at 640 x 8192 x 2048; without a line 6 % and 57 %;
-//  * a GELU, a pass of its own behind the library: 384 tiles x 3072 49.3 / 51.9, x 4096 61.0 / 65.4; 768 x 1536 54.4 / 47.8,
-//    x 4096 104 / 110; 960 x 1536 60.5 / 66.1, x 4096 119 / 153;
-//  * beyond 400 tiles: 5000 x 2304 x 768 24.5 / 27, 2000 x 6144 x 2048 53.5 / 59; whole tiles up to 1024 deep stay;
-//  * tiles of fewer than 128 rows read the weight no faster for it: 32 x 20000 x 512 8.8 / 7.9, x 1024 10.8 / 12.2, 8 x 16384 x
-//    2048 13.2 / 14.6, 1 x 33024 x 1024 13.8 / 16.8, but 8 x 16384 x 1024 8.6 / 5.7, 1 x 12288 x 4096 21.3 / 20.2.
+// Where the library, on a [K, N] weight, is ahead of gemm_ksplit and of what gemm_mfma's launcher has, for products that gemm_wide and
+// gemm_round (wideWidth, raggedRoundWidth) do not take (us, library / gemm_mfma or, small, gemm_ksplit):
+//  * up to one round of the CUs nowhere (2000 x 2000 x 1024 17.7 / 13.7), but for fewer than 128 rows: those tiles read the weight no
+//    faster for it: 32 x 20000 x 512 8.8 / 7.9, x 1024 10.8 / 12.2, 8 x 16384 x 2048 13.2 / 14.6, 1 x 33024 x 1024 13.8 / 16.8, but 8 x
+//    16384 x 1024 8.6 / 5.7, 1 x 12288 x 4096 21.3 / 20.2; with a GELU, a pass of its own behind the library, later;
+//  * beyond, 64 deep at most: from 400 tiles that overhang on; and what is too large for gemm_wide, which is deep or wide.
 bool libraryAhead(int64_t M, int64_t N, int64_t K, int act, bool aligned) {
   const int64_t tiles = tiles128(M, N);
   if (M < 128 && act != ACT_GELU) return tiles > 128 && tiles > 100000 / K;
   if (tiles <= numComputeUnits()) return false;
-  if (tiles > 400 && act != ACT_GELU) return !aligned || K > 1024;
-  return tiles > (act == ACT_GELU || M >= 2 * N ? 1400000 : 650000) / K;
+  if (act == ACT_GELU) return tiles > 1400000 / K;
+  return K > 1024 || (tiles > 400 && !aligned);
 }
 
 // 0: measure, 1: always the library, 2: the hand-written kernel wherever it applies
