@@ -226,7 +226,9 @@ void mgpuGemmMfmaBF16(void *input, void *weight, void *bias, void *output, void 
  * pre-LN dataflow, y = x + proj(attention(LN(x))), out = y + ffn(LN(y)); norm_first =
  * false (declared but never read by the reference's bodies) is the post-LN ordering of
  * the same blocks, h = LN(x + proj(attention(x))), out = LN(h + ffn(h)).  Both
- * LayerNorms have gamma = 1, beta = 0, eps = 1e-5, as in the reference. */
+ * LayerNorms have gamma = 1, beta = 0, eps = 1e-5, as in the reference.  The reference's last
+ * rounding, of the output to fp16 before its cast to fp32, is left out where the kernel that
+ * computes the output stores fp32 itself (by size and alignment). */
 void mgpuLLMDecodingContextLayer(float *input, float *qkv, float *gemm_weight, float *gemm_bias,
                                  float *ffn1_weight, float *ffn1_bias, float *ffn2_weight,
                                  float *ffn2_bias, float *output, int64_t batch, int64_t seq_len,

@@ -438,8 +438,8 @@ def pack_weight(w, stream=None):
 
 
 def matmul_ex(x, w, bias=None, residual=None, act: int = ACT_NONE, stream=None, kernel: str = "auto"):
-    """kernel "auto": mgpuMatmulEx*, i.e. hipBLASLt or one of the three hand-written kernels (gemm_mfma, gemm_ksplit,
-    gemm_f32_small) as the committed table and the fixed rule of the kernel library say; "mfma": gemm_mfma itself (fp16 /
+    """kernel "auto": mgpuMatmulEx*, i.e. one of the hand-written kernels (gemm_wide, gemm_round, gemm_mfma, gemm_ksplit,
+    gemm_f32_small) or hipBLASLt as the fixed rule of the kernel library says; "mfma": gemm_mfma's launcher by itself (fp16 /
     bf16, M a multiple of 128, N of 128 or 96, K of 32); "packed": mgpuMatmulExPacked*, w being the [N, K] copy that
     pack_weight made."""
     if stream is None and kernel in ("auto", "packed"):

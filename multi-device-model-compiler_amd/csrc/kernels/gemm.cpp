@@ -11,8 +11,8 @@
 //  * GELU is applied by an exact-erf kernel after a bias-only epilogue, because
 //    the library's fused GELU is the tanh approximation;
 //  * a call only enqueues: which of the kernels serves a shape - the library or
-//    a hand-written one (gemm_wide.hip, gemm_mfma.hip, gemm_ksplit.hip, gemm_f32_small.hip) -
-//    is a fixed rule: gemm_wide first, where it applies (wideWidth); for the rest a
+//    a hand-written one (gemm_wide.hip, gemm_round.hip, gemm_mfma.hip, gemm_ksplit.hip, gemm_f32_small.hip) -
+//    is a fixed rule: gemm_wide and gemm_round first, where they apply; for the rest a
 //    table decided offline (gemm_table.inc, written by `bench.py --tune-gemm`
 //    from measurements on an MI355X) and, for shapes the table does not hold,
 //    lines on the shape; the library runs the heuristic's first algorithm.
@@ -365,7 +365,7 @@ bool gemmWantsKMajorCast(DType dt, int64_t M, int64_t N, int64_t K, bool hasBias
 // second FFN product at a few to some 2000 tokens.  Estimates as in chooseKernel, plus what writing the planes and reading
 // them in the LayerNorm behind costs over a product and its LayerNorm, fitted to 330 splits (7 % rms for gemm_mfma's, 12 % for
 // gemm_ksplit's; us, product + LayerNorm whole / split: 77 x 768 x 3072 11.6 / 8.7, 1024 x 768 x 3072 19.9 / 17.1, 1368 x 768 x
-// 3072 23.1 / 18.8, 2048 x 512 x 2048 18.7 / 15.5).  Where the estimates differ by less than a tenth the product stays whole
+// 3072 23.1 / 18.8).  Where the estimates differ by less than a tenth the product stays whole
 // (1024 x 1024 x 2048 16.0 / 15.6): the choice is 1.7 % behind the best over 110 shapes, at worst 8 % behind the whole product.
 PartialPlan gemmPartialPlan(const void *in, const void *weight, int64_t M, int64_t N, int64_t K, bool weightKMajor) {
   PartialPlan best;

@@ -3,8 +3,8 @@
 //
 // One of the ways mgpuMatmulEx<half> (lib/Kernels/GPU/Ops.cu:134-234) is
 // served; gemm.cpp has the others and the rule that chooses.  This file has the launcher for 128-row tiles: at most one a
-// CU and a depth that is a multiple of 64 go to gemm_round.hip, more of them to gemm_wide.hip, and the kernel below is what
-// is left, depths that are an odd multiple of 32 (and one step of 64 over several tiles a CU).
+// CU go to gemm_round.hip, more of them to gemm_wide.hip; the kernel below takes what is too shallow for those two (gemmMfmaShallow),
+// several tiles a CU of fewer than 128 rows, and sizes beyond the other two's limits (gemmMfmaKernel).
 //
 // Work decomposition.  A 256-thread block (4 wavefronts) owns a 128 x 128 output
 // tile (wavefronts 2 x 2, each 64 x 64 as 2 x 2 accumulators of 32 x 32) or a

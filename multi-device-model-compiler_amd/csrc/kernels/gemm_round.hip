@@ -344,7 +344,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
     const u32x2 hi = *reinterpret_cast<const u32x2 *>(p + 4);
     // (as in gemm_wide.hip)
     if (N % 64) __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], lo[1], hi[0], hi[1]}, rows, chunkOffset(it), 0, 0);
-      else __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], lo[1], hi[0], hi[1]}, rows, chunkOffset(it), 0, 16);
+    else __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo[0], lo[1], hi[0], hi[1]}, rows, chunkOffset(it), 0, 16);
   }
 }
 
@@ -374,7 +374,7 @@ void launchWidth(const void *in, const void *weight, const void *bias, const voi
 
 } // namespace
 
-// (The callers, gemm_mfma.hip, have checked the shape and the operands.)
+// (The callers, gemm.cpp and gemm_mfma.hip, have checked the shape and the operands.)
 void gemmRound(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
                int64_t K, int act, int width, hipStream_t stream) {
   if (N % 8 || K % 8 || (K % 64 && K * N >= int64_t(1) << 30) || (act != ACT_NONE && residual) || (width != 96 && width != 128)) fail("gemmRound: internal dispatch error");

@@ -353,7 +353,8 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
 
   // LN(in . w + bias + residual), the rounded sum to sumOut when it is not null.  Where the sum is wanted and gemm_wide serves the
   // product, its epilogue adds the residual and rounds the sum once, and the LayerNorm reads and writes one matrix each instead of two
-  // (4096 x 2048 x 2048, product + LayerNorm 39.0 + 14.5 -> 42.2 + 6.8 us).
+  // (4096 x 2048 x 2048, product + LayerNorm 39.0 + 14.5 -> 42.2 + 6.8 us).  Mean and variance then come from the rounded sum, as the
+  // normalised value does either way; the kernel that adds the residual itself takes them from the fp32 sum of the rounded product.
   auto productAddNorm = [&](const PartialPlan &plan, const void *in, const void *w, const void *bias, int64_t K, bool transposed,
                             const void *residual, void *sumOut, void *out) {
     if (plan.parts) {
