@@ -73,7 +73,7 @@ void launch(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqlens, v
       fmha_fwd_kernel<T, D, NQ, true, false, PAD><<<grid, block, 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
     else
       fail("fusedMHA: internal dispatch error");
-  } else if (D == 128 && S <= 64) { // one tile of keys (80 launches 1.022 times as long as before its loads went behind the scores, 1.005 so)
+  } else if (D == 128 && S <= 64 && (PAD || blocks <= deviceComputeUnits())) { // one tile of keys (the kernel has the times)
     fmha_fwd_kernel<T, D, NQ, false, false, PAD, false, D == 128><<<grid, block, 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
   } else {
     fmha_fwd_kernel<T, D, NQ, false, false, PAD><<<grid, block, 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);

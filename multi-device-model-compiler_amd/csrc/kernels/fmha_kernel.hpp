@@ -418,9 +418,12 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
   // 186 -> 178, b8 s700 h12 d96 45.3 -> 40.9, causal b4 s2048 h32 171 -> 162; over 360 launches of 2 to 7 tiles 0.98 of the
   // time); at 64, four loads a wavefront and three wavefronts a SIMD, the causal kernel loses 3-5 %, and at 256 it spills.  So
   // written the compiler peels the first tile off the loop, 600 instructions that a launch of one unmasked tile fetches for nothing
-  // (b9 s8 h12 4.10 -> 4.28 us): such a launch has an instance with the loads in front (without a loop at all, 4.2).
+  // (b9 s8 h12 4.10 -> 4.28 us).  Such a launch has an instance of its own: the loads in front, and for padded heads no loop at all (on
+  // average against the loads in front, up to one block a CU / more: peeled 1.028 / 1.001, without a loop 1.018 / 0.996, padded 1.018 /
+  // 0.983 and 0.995 / 0.969).
   constexpr bool kLoadsBehindScores = D == 128 && !SHORT;
-  for (int kt = 0; kt < trips; kt++) {
+  constexpr bool kOneTile = SHORT && PAD;
+  for (int kt = 0; kOneTile ? kt < 1 && trips > 0 : kt < trips; kt++) {
     if (TRACE) tMark = clock64();
     // The loads of tile kt (and of nothing later) must have landed; the barrier
     // makes every wavefront's share visible and also says that everybody is
@@ -430,7 +433,7 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (TRACE && kt == 0) tFirstTile = clock64();
-    if (!kLoadsBehindScores && kt + kStages - 1 < nkt) issueTile(kt + kStages - 1);
+    if (!kOneTile && !kLoadsBehindScores && kt + kStages - 1 < nkt) issueTile(kt + kStages - 1);
 
     const uint32_t stageOff = (uint32_t)((kt % kStages) * kStageBytes);
     const int key0 = tileAt(kt) * kBN;
