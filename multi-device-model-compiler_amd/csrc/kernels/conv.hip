@@ -32,6 +32,7 @@
 #include "mgpu_ops_internal.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace mgpu {
@@ -1247,49 +1248,37 @@ FastDiv fastDiv(int d) {
 
 } // namespace
 
-// Two things beside the size decide (us, what ran before / staged, 3 x 3 unless said otherwise): whether a channel's row of the filter
-// is whole lines - IC a multiple of 32 -, since staged loads run along the rows (230 tiles from 64 channels 6.9 / 6.4, from 72 6.8 /
-// 8.1); and whether a tile has more than 16 channels, since with fewer the other kernels' filter loads touch half as many lines
-// (16 channels, 230 tiles from 128 9.1 / 9.7).  By rounds of the CUs (r, a tile each; window tiles take two beyond 400 tiles, so that
-// they waste most at r = 3):
-//  * r = 1, eight wavefronts: whole rows from 64 channels on (16 channels 14.5 / 14.8 from 256, ahead from there on where rows of the image are
-//    odd: 23 x 23 16.7 / 14.7);
-//  * r = 2: the same, 450 tiles from 32 channels 7.3 / 6.7 on four, other rows from 144 (505 from 160 22.4 / 19.1, but from 48 8.1 /
-//    8.9, 80 11.1 / 12.1), 16 channels from 192 (24.0 / 20.4; from 64 9.5 / 10.0).  The 64 x 64 tiles, from 1.5 a CU on, always (450 from
-//    40 13.3 / 8.6);
-//  * r = 3, four: all (750 from 40 channels 11.8 / 10.6; 64-channel tiles from 72 17.6 / 14.8; 16 channels from 64 15.2 / 13.0) but 16 channels from rows that are not whole;
-//  * beyond, four: whole rows, not 16 channels, not 64-channel tiles, which are as good from three a CU on (1020 from 32 11.4 / 10.5, 1500 17.1 / 15.0, but from 48 19.4 / 21.3
-//    and 16 channels from 32 13.1 / 14.8), up to eight a CU, where two accumulators are ahead (3136 tiles 28.0 / 29.7).
-//  * 5 x 5, a block's LDS holds one a CU of eight, half the channels suffice: r = 1 230 tiles from 32 9.5 / 8.0, from 40 10.2 / 10.3
-//    (16 channels 9.0 / 10.5); r = 2 330 from 20 9.8 / 9.4, 16 channels from 24 9.7 / 10.7; r = 3 750 from 24 18.1 / 14.2, 16 channels
-//    15.7 / 13.7; r = 4 1020 from 32 28.2 / 25.1, from 40 28.4 / 30.4; r = 5 1200 from 24 25.4 / 21.5; beyond 1500 from 32 40.1 / 31.4,
-//    1790 from 20 27.7 / 29.1, 16 channels 2000 from 32 37.6 / 41.0.
-//  * 7 x 7: 230 tiles from 20 11.9 / 11.7, from 64 35 / 21, 1020 from 24 43.9 / 30.4; 16 channels from 64 24.4 / 20.9, from 20 10.6 / 11.8,
-//    750 from 32 43.9 / 30.5.
-// 1 x 1 gained nothing: sixteen channels of a row are one line already.
-int convStagedWaves(int win, int64_t tiles, int64_t IC, int64_t OC, int64_t cus) {
-  const int64_t groups = IC / 2, r = (tiles + cus - 1) / cus;
-  if (IC % 2) return 0;
-  const bool whole = IC % 32 == 0, few = OC <= 16, paired = (OC - 1) % 64 >= 32; // (paired: the 64 x 64 tiles go beyond 400)
-  if (paired && r > 3) return 0;
-  if (win == 7) return groups < 8 || (few && !(whole && r <= 3)) ? 0 : r == 1 ? 8 : 4;
-  if (win == 5) {
-    if (groups < 8) return 0;
-    if (r == 1) return groups >= (few ? 64 : whole ? 16 : 24) && (whole || !few) ? 8 : 0;
-    if (r == 3) return 4;
-    if (r == 4) return whole && !few && groups >= 16 ? 4 : 0;
-    return !few && (whole || r == 2 || r == 5) ? 4 : 0;
-  }
-  if (win != 3 || groups < 16) return 0;
-  if (r == 1) return whole && groups >= (few ? 128 : 32) ? 8 : 0;
-  if (r == 2) {
-    const bool many = 2 * tiles > 3 * cus;
-    if (paired && many) return groups >= 32 ? 8 : 4;
-    if (groups < 32) return whole && !few && many ? 4 : 0;
-    return (few ? whole && groups >= 96 : whole || groups >= 72) ? 8 : 0;
-  }
-  if (r == 3) return !few || whole ? 4 : 0;
-  return whole && !few && tiles <= 8 * cus ? 4 : 0;
+// How many wavefronts share a tile of conv_staged_kernel, 0 where another kernel is faster.  By size eight or four are in question (us, what
+// ran before / four / eight, 3 x 3 unless said otherwise): from 32 channel groups up to two tiles a CU (196 tiles of 32 groups 6.81 / - / 5.98,
+// 112 of 128 20.8 / - / 16.8, 496 of 128 45.1 / 27.9 / 27.0), from 16 beyond 1.5 a CU, up to eight (1176 tiles of 96 channels 1.3 to
+// 1.6 times as fast, 3136 tiles 28.0 / 29.7), up to three where the 64 x 64 tiles are the alternative (784 15.5 / 14.9, 980 48.2 / 48.5); 5 x 5, of whose blocks of
+// eight a CU holds one, the same with half the groups (248 tiles of 32 16.5 / 13.5 / 12.0, 442 42.9 / 23.3 / 24.2); 7 x 7 from 8 groups (112 of 128
+// 156 / 85 / 75).  1 x 1 gained nothing: sixteen channels of a row are one line already.
+// Whether they gain is what an estimate says, of the logarithm of their time over the former kernel's, fitted to 2600 of 4000 shapes timed
+// on all three: the more, the longer the reduction; the more channels a tile has, whose rows are the lines that an instruction of the other
+// kernels touches; where a row of the filter is whole lines, since staged loads run along it; where taps lie apart, at a stride or
+// in short rows; and the more of their last round the other kernels waste, which take two tiles a wavefront or 64 x 64.  (us, before / staged:
+// 230 tiles from 64 channels 6.9 / 6.4, from 72 6.8 / 8.1; 16 channels from 128 9.1 / 9.7; 23 x 242 x 15 from 16 to 160, 5 x 5 of stride 2, 58 / 41.)
+// Over the 4000 it is 0.857 of the time without them, 10 more than 6 % slower; staged everywhere in question it was 0.861, 174.
+int convStagedWaves(int win, int64_t stride, int64_t pixels, int64_t IC, int64_t OC, int64_t OW, int64_t cus) {
+  if (IC % 2 || win < 3) return 0;
+  const int64_t ocTiles = (OC + 31) / 32, tiles = (pixels + 31) / 32 * ocTiles, groups = IC / 2, r = (tiles + cus - 1) / cus;
+  const bool paired = (OC - 1) % 64 >= 32; // the 64 x 64 tiles go beyond 400
+  int waves = 0;
+  if (win == 7) waves = groups < 8 || (paired && r > 3) ? 0 : r == 1 ? 8 : 4;
+  else if (tiles <= (win == 3 ? 2 * cus : cus) && groups >= (win == 3 ? 32 : 16)) waves = 8;
+  else if (win == 3) waves = groups >= 16 && 2 * tiles > 3 * cus && r <= (paired ? 3 : 8) ? 4 : 0;
+  else if (tiles > cus && (r <= 3 || !paired)) waves = groups >= (r == 4 ? 16 : 8) ? 4 : 0;
+  if (!waves) return 0;
+  // rounds of the CUs that the other kernels take, a tile each
+  auto rounds = [&](int64_t blocks, int64_t each) { return (blocks + each * cus - 1) / (each * cus) * each; };
+  const int64_t others = tiles <= 400 ? r : paired ? 4 * rounds((pixels + 63) / 64 * ((OC + 63) / 64), 1)
+                                          : rounds(tiles, tiles <= 2048 ? 2 : win == 3 ? 8 : 4);
+  static const double base[3][2] = {{0.341, 0.359}, {0.212, 0.238}, {0.190, 0.150}}; // 3 x 3, 5 x 5, 7 x 7; four, eight
+  const double channels = (double)OC / (double)(32 * ocTiles), rows = std::min(4.0, 32.0 / (double)OW);
+  const double change = base[(win - 3) / 2][waves / 8] - 0.071 * std::log((double)groups / 32.0) - 0.133 * std::log(channels) - (stride > 1 ? 0.039 : 0.0) -
+                        0.011 * rows - (IC % 32 == 0 ? 0.099 : 0.0) - 0.318 * (double)others / (double)r;
+  return change < -0.01 ? waves : 0;
 }
 
 // Do patches take a 5 x 5 or 7 x 7 from one channel or three?  From half of a row's tiles filled on (us, window tiles / patches, 7 x 7 from
@@ -1477,7 +1466,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
       const int64_t units = ((IC + 2 * Window<WIN>::HALF - 1) / (2 * Window<WIN>::HALF)) * Window<WIN>::UNITS;
       const int64_t blocks = (pixels + 63) / 64 * ((OC + 63) / 64);
       if constexpr (WIN >= 3) {
-        const int ks = convStagedWaves(WIN, tiles, IC, OC, numComputeUnits());
+        const int ks = convStagedWaves(WIN, SW, pixels, IC, OC, OW, numComputeUnits());
         if (ks == 8) return staged(win, integral_constant<int, 8>());
         if (ks == 4) return staged(win, c4);
       }

@@ -164,8 +164,8 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
             int64_t OW, int64_t PHL, int64_t PWL, int64_t PHR, int64_t PWR, int64_t SH, int64_t SW, int64_t DH,
             int64_t DW, bool hasPostAdd, bool relu, hipStream_t stream);
 // How many wavefronts share a tile of its kernel that stages the filter in LDS, 0 where another one serves the convolution (win: the
-// window's side; tiles: of 32 pixels by 32 channels).
-int convStagedWaves(int win, int64_t tiles, int64_t IC, int64_t OC, int64_t cus);
+// window's side; pixels: of the output, of all images).
+int convStagedWaves(int win, int64_t stride, int64_t pixels, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
 // Do patches of input rows in LDS serve a square convolution (rowTiles: tiles of 32 pixels of one output row by 32 channels)?
 bool convByPatches(int win, int stride, int64_t tiles, int64_t rowTiles, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
 void pool2d(const float *input, float *output, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OH, int64_t OW,

@@ -7,52 +7,52 @@ import pytest
 from test_index_bounds import internal
 
 
-@pytest.mark.parametrize("win,tiles,IC,OC,waves", [
-    (3, 256, 64, 32, 8),     # a round of the CUs, rows of the filter of whole lines
-    (3, 256, 72, 32, 0),
-    (3, 256, 32, 32, 0),
-    (3, 230, 128, 16, 0),    # half of a tile's channels at most
-    (3, 230, 256, 16, 8),
-    (3, 450, 32, 24, 4),
-    (3, 450, 48, 32, 0),
-    (3, 450, 96, 32, 8),
-    (3, 450, 144, 32, 8),
-    (3, 450, 40, 64, 4),     # instead of 64 x 64 tiles
-    (3, 450, 72, 64, 8),
-    (3, 384, 40, 64, 0),
-    (3, 512, 96, 16, 0),
-    (3, 512, 192, 16, 8),
-    (3, 750, 40, 32, 4),     # three tiles a CU
-    (3, 750, 40, 16, 0),
-    (3, 750, 64, 16, 4),
-    (3, 769, 40, 32, 0),
-    (3, 1500, 64, 32, 4),
-    (3, 1500, 64, 16, 0),
-    (3, 1500, 64, 64, 0),
-    (3, 2049, 64, 32, 0),
-    (3, 450, 33, 32, 0),
-    (5, 230, 32, 32, 8),
-    (5, 230, 40, 32, 0),
-    (5, 230, 48, 32, 8),
-    (5, 230, 48, 16, 0),
-    (5, 330, 16, 32, 4),
-    (5, 330, 24, 16, 0),
-    (5, 750, 24, 16, 4),
-    (5, 1020, 32, 32, 4),
-    (5, 1020, 40, 32, 0),
-    (5, 1200, 24, 32, 4),
-    (5, 1500, 24, 32, 0),
-    (5, 10125, 32, 32, 4),
-    (7, 230, 18, 32, 8),
-    (7, 230, 18, 16, 0),
-    (7, 750, 32, 16, 4),
-    (7, 1020, 32, 16, 0),
-    (7, 1020, 18, 32, 4),
-    (7, 1020, 18, 64, 0),
+@pytest.mark.parametrize("win,stride,tiles,IC,OC,OW,waves", [
+    (3, 1, 256, 64, 32, 32, 8),
+    (3, 1, 256, 72, 32, 32, 0),
+    (3, 1, 256, 128, 32, 32, 8),
+    (3, 1, 256, 62, 32, 32, 0),
+    (3, 1, 230, 128, 16, 32, 8),
+    (3, 1, 230, 256, 16, 32, 8),
+    (3, 1, 230, 256, 8, 32, 0),
+    (3, 2, 230, 80, 32, 4, 8),
+    (3, 1, 230, 80, 32, 64, 0),
+    (3, 1, 384, 40, 64, 64, 0),
+    (3, 1, 450, 40, 64, 64, 4),
+    (3, 1, 450, 72, 64, 64, 8),
+    (3, 1, 512, 160, 32, 32, 8),
+    (3, 1, 513, 160, 32, 32, 4),
+    (3, 1, 750, 40, 32, 32, 4),
+    (3, 1, 768, 40, 64, 32, 4),
+    (3, 1, 770, 40, 64, 32, 0),
+    (3, 1, 1500, 64, 32, 64, 4),
+    (3, 1, 1500, 48, 32, 64, 0),
+    (3, 1, 2048, 64, 32, 64, 4),
+    (3, 1, 2049, 64, 32, 64, 0),
+    (3, 1, 450, 129, 32, 32, 0),
+    (5, 1, 256, 32, 32, 32, 8),
+    (5, 1, 257, 32, 32, 32, 4),
+    (5, 1, 256, 40, 32, 32, 8),
+    (5, 2, 256, 40, 32, 8, 8),
+    (5, 1, 256, 30, 32, 8, 0),
+    (5, 1, 330, 16, 32, 32, 4),
+    (5, 1, 330, 14, 32, 32, 0),
+    (5, 2, 1020, 32, 32, 32, 4),
+    (5, 1, 1020, 24, 32, 32, 0),
+    (5, 2, 1220, 16, 32, 8, 4),
+    (5, 1, 1200, 32, 64, 32, 0),
+    (7, 1, 256, 16, 32, 32, 8),
+    (7, 1, 257, 16, 32, 32, 4),
+    (7, 1, 256, 14, 32, 32, 0),
+    (7, 1, 256, 18, 8, 32, 0),
+    (7, 1, 1020, 18, 32, 32, 4),
+    (7, 1, 1020, 18, 64, 32, 0),
+    (1, 1, 256, 256, 32, 32, 0),
 ])
-def test_wavefronts_a_tile(pkg, win, tiles, IC, OC, waves):
-    ask = internal(pkg, "_ZN4mgpu15convStagedWavesEillll", ctypes.c_int, ctypes.c_int, *[ctypes.c_int64] * 4)
-    assert ask(win, tiles, IC, OC, 256) == waves
+def test_wavefronts_a_tile(pkg, win, stride, tiles, IC, OC, OW, waves):
+    """On either side of the lines on tiles, channel groups, channels a tile, whole lines of the filter, stride and short rows."""
+    ask = internal(pkg, "_ZN4mgpu15convStagedWavesEillllll", ctypes.c_int, ctypes.c_int, *[ctypes.c_int64] * 6)
+    assert ask(win, stride, tiles // -(-OC // 32) * 32, IC, OC, OW, 256) == waves
 
 
 @pytest.mark.parametrize("win,stride,tiles,rowTiles,IC,OC,OW,patches", [

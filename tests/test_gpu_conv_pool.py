@@ -61,19 +61,22 @@ def test_conv2d_of_few_taps_four_pixels_a_lane(pkg, gpu, oracle, rng, N, IC, H, 
 
 @pytest.mark.parametrize("N,IC,H,W,OC,K,pad,stride,dilation,relu,add", [
     # eight wavefronts a tile: 80 and 48 groups of channels (shares that are no whole chunks), 73 (cut shares, a last piece half past
-    # the filter's end), 25 (5 x 5), a last channel tile of one, images smaller than a tile; the smallest that take it
+    # the filter's end), 25 (5 x 5), a last channel tile of one, images smaller than a tile
     (5, 160, 7, 7, 33, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, True), (2, 96, 9, 31, 32, (3, 3), (0, 2, 1, 0), (2, 1), (1, 2), False, False),
     (5, 146, 50, 51, 32, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, True), (3, 50, 11, 13, 40, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), True, True),
-    (1, 64, 1, 1, 17, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (1, 256, 3, 5, 1, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True),
+    (1, 256, 1, 1, 33, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (1, 256, 3, 5, 17, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True),
+    (2, 128, 7, 9, 64, (3, 3), (1, 1, 1, 1), (2, 2), (1, 1), True, False),
     # four: 17, 19 and 33 groups, one and several channel tiles, 64-channel tiles cut, the last pixel tile cut
-    (7, 34, 50, 51, 32, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (7, 38, 41, 40, 48, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False),
+    (7, 34, 50, 51, 32, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (6, 38, 41, 40, 64, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False),
     (4, 66, 41, 66, 64, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (4, 18, 30, 91, 32, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), False, True),
     (9, 32, 50, 61, 32, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), True, False),
+    (3, 70, 61, 60, 96, (3, 3), (2, 2, 2, 2), (1, 1), (2, 2), False, False),
+    (7, 38, 41, 40, 48, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False),
     # the same where rows of the filter are no whole lines, or channels few: another kernel
+    (1, 256, 3, 5, 1, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True),
     (5, 66, 7, 7, 33, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, True), (2, 70, 9, 31, 32, (3, 3), (0, 2, 1, 0), (2, 1), (1, 2), False, False),
     (1, 64, 1, 1, 1, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (3, 34, 11, 13, 40, (5, 5), (2, 2, 2, 2), (1, 1), (1, 1), True, True),
     (5, 34, 50, 51, 32, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), False, True), (8, 38, 41, 40, 48, (3, 3), (1, 1, 1, 1), (1, 1), (1, 1), True, False),
-    (3, 70, 61, 60, 96, (3, 3), (2, 2, 2, 2), (1, 1), (2, 2), False, False),
     # 7 x 7: rows and columns outside on every side, dilation, eight groups and an odd number; eight and four wavefronts
     (2, 18, 5, 6, 33, (7, 7), (3, 3, 3, 3), (1, 1), (1, 1), True, True), (3, 16, 20, 23, 40, (7, 7), (4, 6, 5, 2), (2, 1), (1, 2), False, False),
     (4, 22, 41, 60, 32, (7, 7), (3, 3, 3, 3), (1, 1), (1, 1), False, True), (3, 16, 50, 51, 64, (7, 7), (3, 3, 3, 3), (1, 1), (2, 1), True, False)])
