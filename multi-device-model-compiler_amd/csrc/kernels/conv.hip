@@ -13,8 +13,8 @@
 // columns, so that a register of an accumulator is 32 consecutive pixels of a channel: whole
 // 128-byte runs of the NCHW output.  The tap matrix is never written to memory.  Taps come
 // through buffer loads, whose bounds check answers 0 for an offset outside the image: padding costs
-// no branch and no second instruction.  Seven kernels share the work (conv2d below has the rule and
-// the measurements behind it):
+// no branch and no second instruction.  Seven kernels share the work here (conv2d below has the rule and
+// the measurements behind it), and an eighth, conv_split.hip, has the large 3 x 3 ones:
 //   few taps  (K <= 32, a network's stem)  filter in registers, wavefronts walk over pixel tiles
 //   quads     (the same, many tiles, rows of whole quads, stride 1 across)  four pixels a lane
 //   patch     (5 or 7 square from one channel or three)  input rows through LDS, once for all taps
@@ -29,6 +29,7 @@
 // of as many bytes takes 39).  Unlike the reference, asymmetric padding is honoured (it passes only
 // PHL / PWL to cuDNN).
 #include "common.hpp"
+#include "conv.hpp"
 #include "mgpu_ops_internal.hpp"
 
 #include <algorithm>
@@ -43,14 +44,8 @@ struct ConvGeo {
   int IC, H, W, KH, KW, OH, OW, PHL, PWL, SH, SW, DH, DW;
 };
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int kChunk = 16;     // taps per step of the reduction: 8 a lane half
 constexpr int kSegment = 2048; // taps the tap table holds at a time
-constexpr int kOutside = (int)0x80000000; // a byte offset past every resource: the hardware's bounds check reads 0 there
 constexpr int kNever = 0x3fff0000; // a pixel past the end takes -kNever for its first row: every tap lies outside the image
 
 // Where tap k of a pixel sits: the offset from the pixel's first tap (bytes; elements when WIDE)
@@ -62,14 +57,6 @@ struct TapNarrow {
 struct TapWide {
   int off, dh, dw, pad;
 };
-
-// Division by a number that the host knows, for dividends below 2^31: (mulhi(n, mul) + n) >> shift.
-struct FastDiv {
-  unsigned mul, shift;
-};
-__device__ __forceinline__ int divide(int n, FastDiv d) {
-  return (int)((__umulhi((unsigned)n, d.mul) + (unsigned)n) >> d.shift);
-}
 
 // Which of `count` window rows (columns), `dilation` apart from `first` on, lie outside 0 .. size - 1: bit i for the i-th.
 __device__ __forceinline__ unsigned outsideBits(int first, int size, int count, int dilation) {
@@ -87,18 +74,6 @@ __device__ __forceinline__ unsigned outsideBits(int first, int size, int count, 
 // threads at a time (gridOf in conv2d), and the last piece has blocks past the last pixel.
 constexpr int64_t kGridRow = int64_t(1) << 31;
 template <int THREADS> __device__ __forceinline__ int pixelBlock() { return (int)blockIdx.z * (int)(kGridRow / THREADS) + (int)blockIdx.x; }
-
-// A buffer resource over `elems` floats (2 GiB of them at most: no offset reaches further), for the
-// builtins and, as its four words, for inline assembly.
-constexpr int kRawBuffer = 0x00027000;
-__device__ __forceinline__ int resourceBytes(int64_t elems) { return (int)(elems * 4 < 0x7fffffff ? elems * 4 : 0x7fffffff); }
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t resource(const float *p, int64_t elems) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, resourceBytes(elems), kRawBuffer);
-}
-__device__ __forceinline__ i32x4 resourceWords(const float *p, int64_t elems) {
-  const uint64_t at = (uint64_t)(uintptr_t)p;
-  return i32x4{(int)(uint32_t)at, (int)(uint32_t)(at >> 32) & 0xffff, resourceBytes(elems), kRawBuffer};
-}
 
 // The end of a wavefront's 32 channels x PT x 32 pixels: the sum over the KS wavefronts of the tile
 // (wavefront ks of them has slot `slot0` + ks of `partial`), bias, postAdd, ReLU, store.  pix and img:
@@ -1240,12 +1215,6 @@ unsigned blocksFor(int64_t items) {
 
 bool fitsInt(int64_t v) { return v >= 0 && v <= 0x7fffffff; }
 
-FastDiv fastDiv(int d) {
-  unsigned shift = 0;
-  while ((1u << shift) < (unsigned)d) shift++;
-  return {(unsigned)((((uint64_t)1 << 32) * (((uint64_t)1 << shift) - d)) / d + 1), shift};
-}
-
 } // namespace
 
 // How many wavefronts share a tile of conv_staged_kernel, 0 where another kernel is faster.  By size eight or four are in question (us, what
@@ -1279,6 +1248,26 @@ int convStagedWaves(int win, int64_t stride, int64_t pixels, int64_t IC, int64_t
   const double change = base[(win - 3) / 2][waves / 8] - 0.071 * std::log((double)groups / 32.0) - 0.133 * std::log(channels) - (stride > 1 ? 0.039 : 0.0) -
                         0.011 * rows - (IC % 32 == 0 ? 0.099 : 0.0) - 0.318 * (double)others / (double)r;
   return change < -0.01 ? waves : 0;
+}
+
+// us that a 3 x 3 takes in the kernel that the lines of conv2d give it, where conv_split_kernel does not: each start + rounds of its tiles *
+// (a part of its own + one a channel), fitted to 500 shapes (10th and 90th percentile 0.93 and 1.06 times what was measured; two
+// groups of wavefronts on LDS tiles 0.79 and 0.98).
+double convWindowTime(int64_t stride, int64_t pixels, int64_t IC, int64_t OC, int64_t OW, int64_t cus) {
+  const int64_t tiles = (pixels + 31) / 32 * ((OC + 31) / 32), blocks = (pixels + 63) / 64 * ((OC + 63) / 64), units = (IC + 1) / 2;
+  auto rounds = [](int64_t count, int64_t each) { return (double)((count + each - 1) / each); };
+  const double channels = (double)IC;
+  const int ks = convStagedWaves(3, stride, pixels, IC, OC, OW, cus);
+  if (ks == 8) return 2.9 + rounds(tiles, cus) * (0.74 + 0.044 * channels);
+  if (ks == 4) return 2.2 + rounds(tiles, cus) * (0.83 + 0.043 * channels);
+  if (tiles <= 400) return 2.8 + rounds(tiles, cus) * 0.041 * channels;
+  if ((OC - 1) % 64 >= 32) {
+    if (blocks <= cus && units >= 64) return 7.0 + 0.156 * channels;
+    if (blocks <= 2 * cus && units >= 24) return 3.0 + rounds(blocks, cus) * 0.155 * channels;
+    return 4.75 + rounds(blocks, cus) * (0.65 + 0.159 * channels);
+  }
+  if (tiles <= 2048) return 3.0 + rounds(tiles, 2 * cus) * (0.67 + 0.087 * channels);
+  return 2.6 + rounds(tiles, 8 * cus) * (1.33 + 0.319 * channels);
 }
 
 // Do patches take a 5 x 5 or 7 x 7 from one channel or three?  From half of a row's tiles filled on (us, window tiles / patches, 7 x 7 from
@@ -1461,6 +1450,18 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     else if (IC == 1) go(integral_constant<int, 7>(), c4);
     else go(integral_constant<int, 7>(), integral_constant<int, 11>());
   } else if (squareWindow) {
+    // 3 x 3 from 32 channels on in pairs of fp16 numbers, where both estimates say that this is faster (500 shapes of 0.15 GFLOP
+    // on: taken by 268, 0.83 of the time over all of them, the largest ones 0.39, none more than 2 % slower).  (16 channels are
+    // one step: no gain, and the fp32 instructions' sums are the more exact ones.)
+    if (KH == 3 && IC >= 32 && IC % 16 == 0) {
+      const int cus = numComputeUnits();
+      const ConvSplitPlan plan = convSplitPlan((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus,
+                                               0.97 * convWindowTime(SH, pixels, IC, OC, OW, cus));
+      if (plan.strips && convSplit(plan, input, weight, bias, output, add, N, IC, H, W, OC, OH, OW, PHL, PWL, SH, SW, DH, DW, relu, stream)) {
+        MGPU_CHECK_LAUNCH("mgpuConv2d");
+        return;
+      }
+    }
     auto pick = [&](auto win) {
       constexpr int WIN = decltype(win)::value;
       const int64_t units = ((IC + 2 * Window<WIN>::HALF - 1) / (2 * Window<WIN>::HALF)) * Window<WIN>::UNITS;

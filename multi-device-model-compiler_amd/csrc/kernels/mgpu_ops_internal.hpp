@@ -168,6 +168,18 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
 int convStagedWaves(int win, int64_t stride, int64_t pixels, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
 // Do patches of input rows in LDS serve a square convolution (rowTiles: tiles of 32 pixels of one output row by 32 channels)?
 bool convByPatches(int win, int stride, int64_t tiles, int64_t rowTiles, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
+// How long the kernels above take for a 3 x 3 convolution, in us (see conv.hip).
+double convWindowTime(int64_t stride, int64_t pixels, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
+// 3 x 3 on the fp16 matrix cores in pairs of fp16 numbers (conv_split.hip), from 32 channels that are a multiple of 16 on: the tile and the
+// strips of columns that take the least time (strips 0: none less than `limit` us), and the launch (false: not for these sizes or pointers).
+struct ConvSplitPlan {
+  int tile, strips;
+  double us;
+};
+ConvSplitPlan convSplitPlan(int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit);
+bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const float *bias, float *y, const float *add, int64_t N, int64_t IC,
+               int64_t H, int64_t W, int64_t OC, int64_t OH, int64_t OW, int64_t PHL, int64_t PWL, int64_t SH, int64_t SW, int64_t DH,
+               int64_t DW, bool relu, hipStream_t stream);
 void pool2d(const float *input, float *output, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OH, int64_t OW,
             int64_t KH, int64_t KW, int64_t PHL, int64_t PWL, int64_t PHR, int64_t PWR, int64_t SH, int64_t SW,
             int64_t method, hipStream_t stream);
