@@ -95,7 +95,7 @@ template <int KS_, int CAP_> struct SplitShape {
 
 template <int KS, int CAP>
 __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__restrict__ w, const float *__restrict__ x, int IC, int OC,
-                                                              int pxTiles, int ocTiles, FastDiv byOcTiles, int H, int W, int N, int relu,
+                                                              int gridDimX, int ocTiles, FastDiv byOcTiles, int H, int W, int N, int relu,
                                                               const float *__restrict__ bias, float *__restrict__ y,
                                                               const float *__restrict__ add, SplitGeo g) {
   using S = SplitShape<KS, CAP>;
@@ -109,10 +109,10 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const bool producer = wave >= kConsumers;
   const int l32 = lane % 32, hl = lane / 32;
-  // channel tiles of the same pixels on the same XCD
-  const int slotOf = (int)blockIdx.x / 8, row8 = divide(slotOf, byOcTiles);
-  const int pxTile = __builtin_amdgcn_readfirstlane(row8 * 8 + (int)blockIdx.x % 8), ocTile = __builtin_amdgcn_readfirstlane(slotOf - row8 * ocTiles);
-  if (pxTile >= pxTiles) return;
+  // an equal run of tiles for each XCD, channel tiles of the same pixels one after another
+  const int nblk = (int)gridDimX, xcd = (int)blockIdx.x % 8, share = nblk / 8, extra = nblk % 8;
+  const int wid = xcd * share + (xcd < extra ? xcd : extra) + (int)blockIdx.x / 8;
+  const int pxTile = __builtin_amdgcn_readfirstlane(divide(wid, byOcTiles)), ocTile = __builtin_amdgcn_readfirstlane(wid - pxTile * ocTiles);
   const int oc0 = ocTile * kOC, p0 = pxTile * S::PX;
   const int steps = IC / 16;
   const int pwave = wave - kConsumers, ptid = tid - 64 * kConsumers;
@@ -526,7 +526,7 @@ bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const 
   auto fits = [](int64_t v) { return v >= 0 && v <= 0x7fffffff; };
   const int64_t strips = plan.strips, width = (OW + strips - 1) / strips, pixels = N * strips * OH * width, tilePixels = kTiles[plan.tile].pixels;
   const int64_t pitch = (width - 1) * SW + (kWin - 1) * DW + 1, rows = (OH - 1) * SH + (kWin - 1) * DH + 1;
-  const int64_t pxTiles = (pixels + tilePixels - 1) / tilePixels, ocTiles = (OC + kOC - 1) / kOC, blocks = (pxTiles + 7) / 8 * 8 * ocTiles;
+  const int64_t pxTiles = (pixels + tilePixels - 1) / tilePixels, ocTiles = (OC + kOC - 1) / kOC, blocks = pxTiles * ocTiles;
   // pixel, row and byte indices from a tile's first image on are 32 bits wide, the filter's from a channel on; a grid's threads are fewer than 2^32
   const int64_t images = (tilePixels - 2) / (OH * width) + 2;
   if (!aligned16(w) || !fits(pixels + tilePixels) || !fits(N * strips * rows + tilePixels * SH) || !fits(images * IC * H * W * 4) ||
@@ -535,7 +535,7 @@ bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const 
   const SplitGeo g{(int)OH,    (int)OW, (int)PHL, (int)PWL,   (int)SH, (int)SW, (int)DH, (int)DW, (int)strips, (int)width, (int)pitch, (int)rows, (int)pixels,
                    fastDiv((int)(OH * width)), fastDiv((int)width), fastDiv((int)strips), fastDiv((int)pitch), fastDiv((int)rows)};
   auto launch = [&](auto *kernel) {
-    kernel<<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(w, x, (int)IC, (int)OC, (int)pxTiles, (int)ocTiles, fastDiv((int)ocTiles), (int)H, (int)W,
+    kernel<<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(w, x, (int)IC, (int)OC, (int)blocks, (int)ocTiles, fastDiv((int)ocTiles), (int)H, (int)W,
                                                                   (int)N, relu, bias, y, add, g);
   };
   switch (plan.tile) {
