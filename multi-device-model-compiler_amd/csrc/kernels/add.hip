@@ -49,11 +49,11 @@ void addF32(const float *a, const float *b, float *c, int64_t n, hipStream_t str
   if (!a || !b || !c) fail("mgpuAddF32: null pointer");
   if (aligned16(a) && aligned16(b) && aligned16(c)) {
     const int64_t blocks = std::min<int64_t>((n + 1023) / 1024, kMaxStreamBlocks);
-    add_f32_vec4_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(a, b, c, n, blocks * 1024);
+    launchKernel(add_f32_vec4_kernel, dim3((unsigned)blocks), dim3(256), stream, a, b, c, n, blocks * 1024);
     MGPU_CHECK_LAUNCH("add_f32_vec4_kernel");
   } else {
     const int64_t blocks = std::min<int64_t>((n + 255) / 256, kMaxStreamBlocks);
-    add_f32_scalar_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(a, b, c, n);
+    launchKernel(add_f32_scalar_kernel, dim3((unsigned)blocks), dim3(256), stream, a, b, c, n);
     MGPU_CHECK_LAUNCH("add_f32_scalar_kernel");
   }
 }

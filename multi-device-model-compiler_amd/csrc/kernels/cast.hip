@@ -118,13 +118,13 @@ void castFromF32(void *dst, const float *src, size_t size, hipStream_t stream, c
   if (aligned16(dst) && aligned16(src) && size >= 8) {
     const size_t n8 = size / 8;
     const unsigned blocks = gridFor(n8, 256);
-    cast_f32_to_h_vec8_kernel<T><<<dim3(blocks), dim3(256), 0, stream>>>(
+    launchKernel(cast_f32_to_h_vec8_kernel<T>, dim3(blocks), dim3(256), stream,
         reinterpret_cast<u32x4 *>(d), reinterpret_cast<const f32x4 *>(src), n8, (size_t)blocks * 256);
     MGPU_CHECK_LAUNCH("cast_f32_to_h_vec8_kernel");
     done = n8 * 8;
   }
   if (done < size) {
-    cast_scalar_kernel<T, float><<<dim3(gridFor(size - done, 256)), dim3(256), 0, stream>>>(d, src, done, size);
+    launchKernel(cast_scalar_kernel<T, float>, dim3(gridFor(size - done, 256)), dim3(256), stream, d, src, done, size);
     MGPU_CHECK_LAUNCH("cast_scalar_kernel");
   }
 }
@@ -138,13 +138,13 @@ void castToF32(float *dst, const void *src, size_t size, hipStream_t stream, con
   if (aligned16(dst) && aligned16(src) && size >= 8) {
     const size_t n8 = size / 8;
     const unsigned blocks = gridFor(n8, 256);
-    cast_h_to_f32_vec8_kernel<T><<<dim3(blocks), dim3(256), 0, stream>>>(
+    launchKernel(cast_h_to_f32_vec8_kernel<T>, dim3(blocks), dim3(256), stream,
         reinterpret_cast<f32x4 *>(dst), reinterpret_cast<const u32x4 *>(s), n8, (size_t)blocks * 256);
     MGPU_CHECK_LAUNCH("cast_h_to_f32_vec8_kernel");
     done = n8 * 8;
   }
   if (done < size) {
-    cast_scalar_kernel<float, T><<<dim3(gridFor(size - done, 256)), dim3(256), 0, stream>>>(dst, s, done, size);
+    launchKernel(cast_scalar_kernel<float, T>, dim3(gridFor(size - done, 256)), dim3(256), stream, dst, s, done, size);
     MGPU_CHECK_LAUNCH("cast_scalar_kernel");
   }
 }
@@ -271,7 +271,7 @@ void castWeightsF32ToF16(CastJob *jobs, int count, hipStream_t stream) {
   }
   t.count = count;
   if (!blocks) return;
-  cast_weights_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(t);
+  launchKernel(cast_weights_kernel, dim3((unsigned)blocks), dim3(256), stream, t);
   MGPU_CHECK_LAUNCH("cast_weights_kernel");
 }
 
@@ -280,7 +280,7 @@ void transposeCastF32ToF16(void *dst, const float *src, int64_t rows, int64_t co
   if (!dst || !src) fail("transposeCastF32ToF16: null pointer");
   const dim3 grid((unsigned)((cols + 63) / 64), (unsigned)((rows + 63) / 64));
   if ((rows + 63) / 64 > 65535) fail("transposeCastF32ToF16: more than 4194240 rows");
-  transpose_cast_kernel<_Float16, float><<<grid, dim3(256), 0, stream>>>(static_cast<_Float16 *>(dst), src, rows, cols);
+  launchKernel(transpose_cast_kernel<_Float16, float>, grid, dim3(256), stream, static_cast<_Float16 *>(dst), src, rows, cols);
   MGPU_CHECK_LAUNCH("transpose_cast_kernel");
 }
 void transpose16(void *dst, const void *src, int64_t rows, int64_t cols, hipStream_t stream) {
@@ -289,21 +289,21 @@ void transpose16(void *dst, const void *src, int64_t rows, int64_t cols, hipStre
   const dim3 grid((unsigned)((cols + 63) / 64), (unsigned)((rows + 63) / 64));
   if ((rows + 63) / 64 > 65535) fail("transpose16: more than 4194240 rows");
   // as 16-bit patterns (exact through the tile's floats): fp16 and bf16 alike, NaN payloads kept
-  transpose_cast_kernel<uint16_t, uint16_t><<<grid, dim3(256), 0, stream>>>(static_cast<uint16_t *>(dst),
+  launchKernel(transpose_cast_kernel<uint16_t, uint16_t>, grid, dim3(256), stream, static_cast<uint16_t *>(dst),
                                                                         static_cast<const uint16_t *>(src), rows, cols);
   MGPU_CHECK_LAUNCH("transpose_cast_kernel");
 }
 
 void fillF16(void *dst, size_t count, float value, hipStream_t stream) {
   if (count == 0) return;
-  fill_kernel<_Float16><<<dim3(gridFor(count, 256)), dim3(256), 0, stream>>>(
+  launchKernel(fill_kernel<_Float16>, dim3(gridFor(count, 256)), dim3(256), stream,
       static_cast<_Float16 *>(dst), count, (_Float16)value);
   MGPU_CHECK_LAUNCH("fill_kernel");
 }
 
 void fillI32(int32_t *dst, size_t count, int32_t value, hipStream_t stream) {
   if (count == 0) return;
-  fill_kernel<int32_t><<<dim3(gridFor(count, 256)), dim3(256), 0, stream>>>(dst, count, value);
+  launchKernel(fill_kernel<int32_t>, dim3(gridFor(count, 256)), dim3(256), stream, dst, count, value);
   MGPU_CHECK_LAUNCH("fill_kernel");
 }
 
@@ -318,11 +318,11 @@ void addFusedQKVBiasTranspose(DType dt, void *q, void *k, void *v, void *qkv, co
     fail("addFusedQKVBiasTranspose: pointers must be 16-byte aligned");
   const size_t total = (size_t)tokens * 3 * H * (D / 8);
   if (dt == DType::F16) {
-    qkv_bias_transpose_kernel<_Float16><<<dim3(gridFor(total, 256)), dim3(256), 0, stream>>>(
+    launchKernel(qkv_bias_transpose_kernel<_Float16>, dim3(gridFor(total, 256)), dim3(256), stream,
         static_cast<_Float16 *>(q), static_cast<_Float16 *>(k), static_cast<_Float16 *>(v),
         static_cast<_Float16 *>(qkv), static_cast<const _Float16 *>(bias), S, tokens, H, D);
   } else if (dt == DType::BF16) {
-    qkv_bias_transpose_kernel<bf16_t><<<dim3(gridFor(total, 256)), dim3(256), 0, stream>>>(
+    launchKernel(qkv_bias_transpose_kernel<bf16_t>, dim3(gridFor(total, 256)), dim3(256), stream,
         static_cast<bf16_t *>(q), static_cast<bf16_t *>(k), static_cast<bf16_t *>(v),
         static_cast<bf16_t *>(qkv), static_cast<const bf16_t *>(bias), S, tokens, H, D);
   } else {
@@ -379,12 +379,12 @@ template <typename T> void geluInPlaceH(void *data, size_t n, hipStream_t stream
   size_t done = 0;
   if (aligned16(data) && n >= 8) {
     const size_t n8 = n / 8;
-    gelu_h_vec8_kernel<T><<<dim3(gridFor(n8, 256)), dim3(256), 0, stream>>>(reinterpret_cast<u32x4 *>(d), n8);
+    launchKernel(gelu_h_vec8_kernel<T>, dim3(gridFor(n8, 256)), dim3(256), stream, reinterpret_cast<u32x4 *>(d), n8);
     MGPU_CHECK_LAUNCH("gelu_h_vec8_kernel");
     done = n8 * 8;
   }
   if (done < n) {
-    gelu_scalar_kernel<T><<<dim3(gridFor(n - done, 256)), dim3(256), 0, stream>>>(d, done, n);
+    launchKernel(gelu_scalar_kernel<T>, dim3(gridFor(n - done, 256)), dim3(256), stream, d, done, n);
     MGPU_CHECK_LAUNCH("gelu_scalar_kernel");
   }
 }
@@ -395,7 +395,7 @@ void geluInPlaceBF16(void *data, size_t n, hipStream_t stream) { geluInPlaceH<bf
 
 void geluInPlaceF32(float *data, size_t n, hipStream_t stream) {
   if (n == 0) return;
-  gelu_scalar_kernel<float><<<dim3(gridFor(n, 256)), dim3(256), 0, stream>>>(data, 0, n);
+  launchKernel(gelu_scalar_kernel<float>, dim3(gridFor(n, 256)), dim3(256), stream, data, 0, n);
   MGPU_CHECK_LAUNCH("gelu_scalar_kernel");
 }
 

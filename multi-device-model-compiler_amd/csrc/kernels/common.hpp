@@ -29,6 +29,17 @@ inline void checkHipStatus(hipError_t status, const char *where) {
 #define MGPU_CHECK_HIP(expr) ::mgpu::checkHipStatus((expr), #expr)
 #define MGPU_CHECK_LAUNCH(name) ::mgpu::checkHipStatus(hipGetLastError(), name)
 
+// kernel<<<grid, block, 0, stream>>>(args...) without the push and pop of a call configuration that the syntax stands for: 2.36 ->
+// 2.16 us of host time a launch, of the 3.7 that a small call of the package takes.  Errors are left for MGPU_CHECK_LAUNCH.
+template <typename T> struct Exactly {
+  using type = T;
+};
+template <typename... P>
+inline void launchKernel(void (*kernel)(P...), dim3 grid, dim3 block, hipStream_t stream, typename Exactly<P>::type... args) {
+  void *list[] = {const_cast<void *>(static_cast<const void *>(&args))...};
+  (void)hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, list, 0, stream);
+}
+
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Streaming kernels get one block per block-sized piece of the array rather

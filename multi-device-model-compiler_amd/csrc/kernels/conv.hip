@@ -1339,7 +1339,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     const int64_t blocks = std::min((pix32 + 3) / 4, most);
     auto *kernel = add ? conv_few_taps_kernel<OCT, NS, Output::Added>
                        : through ? conv_few_taps_kernel<OCT, NS, Output::Through> : conv_few_taps_kernel<OCT, NS, Output::Cached>;
-    kernel<<<gridOf(blocks, 32 * OCT, 256), dim3(256), 0, stream>>>(
+    launchKernel(kernel, gridOf(blocks, 32 * OCT, 256), dim3(256), stream,
         input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu, (int)K, (int)pix32, (int)(4 * blocks));
   };
   const int64_t tiles128 = (pixels + 127) / 128;
@@ -1362,7 +1362,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     auto *kernel = add ? (quadStores == Output::Streamed ? conv_quads_kernel<KWC, NR, Output::Streamed, true> : conv_quads_kernel<KWC, NR, Output::Through, true>)
                    : quadStores == Output::Streamed ? conv_quads_kernel<KWC, NR, Output::Streamed, false>
                    : quadStores == Output::Cached ? conv_quads_kernel<KWC, NR, Output::Cached, false> : conv_quads_kernel<KWC, NR, Output::Through, false>;
-    kernel<<<gridOf(blocks, 32, 256), dim3(256), 0, stream>>>(input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu,
+    launchKernel(kernel, gridOf(blocks, 32, 256), dim3(256), stream, input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu,
                                                               (int)tiles128, (int)(4 * blocks));
   };
   const int64_t across = (OW + 31) / 32;
@@ -1373,27 +1373,27 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     const int64_t most = std::max<int64_t>(1, (int64_t)numComputeUnits() * 2 / ((OC + 31) / 32));
     const int64_t blocks = std::min((rowTiles + 3) / 4, most);
     auto *kernel = add ? conv_patch_kernel<KWC, NR, SWC, true> : conv_patch_kernel<KWC, NR, SWC, false>;
-    kernel<<<gridOf(blocks, 32, 256), dim3(256), 0, stream>>>(input, weight, bias, output, g, (int)OC, (int)P, (int)N, fastDiv((int)across),
+    launchKernel(kernel, gridOf(blocks, 32, 256), dim3(256), stream, input, weight, bias, output, g, (int)OC, (int)P, (int)N, fastDiv((int)across),
                                                               byOH, add, relu, (int)across, (int)rowTiles, (int)(4 * blocks));
   };
   auto window = [&](auto win, auto pts, auto kss) {
     constexpr int WIN = decltype(win)::value, PT = decltype(pts)::value, KS = decltype(kss)::value;
     const int64_t perBlock = 4 / KS * 32 * PT;
-    conv_window_kernel<WIN, PT, KS><<<gridOf((pixels + perBlock - 1) / perBlock, 32, 256), dim3(256), 0, stream>>>(
+    launchKernel(conv_window_kernel<WIN, PT, KS>, gridOf((pixels + perBlock - 1) / perBlock, 32, 256), dim3(256), stream,
         input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu);
   };
   auto staged = [&](auto win, auto kss) {
     constexpr int WIN = decltype(win)::value, KS = decltype(kss)::value;
-    conv_staged_kernel<WIN, KS><<<gridOf(pix32, 32, 64 * KS), dim3(64 * KS), 0, stream>>>(
+    launchKernel(conv_staged_kernel<WIN, KS>, gridOf(pix32, 32, 64 * KS), dim3(64 * KS), stream,
         input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu);
   };
   auto tile = [&](auto win, auto kss) {
     constexpr int WIN = decltype(win)::value, KS = decltype(kss)::value;
-    conv_tile_kernel<WIN, KS><<<gridOf((pixels + 63) / 64, 64, 256 * KS), dim3(256 * KS), 0, stream>>>(
+    launchKernel(conv_tile_kernel<WIN, KS>, gridOf((pixels + 63) / 64, 64, 256 * KS), dim3(256 * KS), stream,
         input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu);
   };
   auto table = [&](auto wide) {
-    conv_table_kernel<decltype(wide)::value><<<gridOf(pix32, 32, 256), dim3(256), 0, stream>>>(
+    launchKernel(conv_table_kernel<decltype(wide)::value>, gridOf(pix32, 32, 256), dim3(256), stream,
         input, weight, bias, add, output, g, (int)OC, (int)K, (int)P, pixels, relu);
   };
   using std::integral_constant;
@@ -1508,7 +1508,7 @@ void pool2d(const float *input, float *output, int64_t N, int64_t C, int64_t H, 
   const unsigned blocks = blocksFor(total);
   auto launch = [&](auto index) {
     using Index = decltype(index);
-    pool_kernel<Index><<<dim3(blocks), dim3(256), 0, stream>>>(input, output, (Index)total, (Index)blocks * 256, (int)H, (int)W, (int)OH,
+    launchKernel(pool_kernel<Index>, dim3(blocks), dim3(256), stream, input, output, (Index)total, (Index)blocks * 256, (int)H, (int)W, (int)OH,
                                                                (int)OW, (int)KH, (int)KW, (int)PHL, (int)PWL, (int)SH, (int)SW, method == 1);
   };
   // (the stride is added past the last index once)

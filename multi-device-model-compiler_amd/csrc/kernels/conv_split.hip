@@ -535,7 +535,7 @@ bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const 
   const SplitGeo g{(int)OH,    (int)OW, (int)PHL, (int)PWL,   (int)SH, (int)SW, (int)DH, (int)DW, (int)strips, (int)width, (int)pitch, (int)rows, (int)pixels,
                    fastDiv((int)(OH * width)), fastDiv((int)width), fastDiv((int)strips), fastDiv((int)pitch), fastDiv((int)rows)};
   auto launch = [&](auto *kernel) {
-    kernel<<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(w, x, (int)IC, (int)OC, (int)blocks, (int)ocTiles, fastDiv((int)ocTiles), (int)H, (int)W,
+    launchKernel(kernel, dim3((unsigned)blocks), dim3(kThreads), stream, w, x, (int)IC, (int)OC, (int)blocks, (int)ocTiles, fastDiv((int)ocTiles), (int)H, (int)W,
                                                                   (int)N, relu, bias, y, add, g);
   };
   switch (plan.tile) {

@@ -62,7 +62,7 @@ void launch(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqlens, v
                                : S >= (D == 256 ? 768 : 512) && blocks <= cus;
     if (halves) {
       auto *kernel = causal ? fmha_fwd_kernel<T, D, 1, true, false, PAD, true> : fmha_fwd_kernel<T, D, 1, false, false, PAD, true>;
-      kernel<<<grid, dim3(512), 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
+      launchKernel(kernel, grid, dim3(512), stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
       MGPU_CHECK_LAUNCH("fmha_fwd_kernel");
       return;
     }
@@ -70,13 +70,13 @@ void launch(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqlens, v
   if (causal) {
     // (the causal kernel exists with one 32-query block per wavefront only)
     if constexpr (NQ == 1)
-      fmha_fwd_kernel<T, D, NQ, true, false, PAD><<<grid, block, 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
+      launchKernel(fmha_fwd_kernel<T, D, NQ, true, false, PAD>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
     else
       fail("fusedMHA: internal dispatch error");
   } else if (D == 128 && S <= 64 && (PAD || blocks <= deviceComputeUnits())) { // one tile of keys (the kernel has the times)
-    fmha_fwd_kernel<T, D, NQ, false, false, PAD, false, D == 128><<<grid, block, 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
+    launchKernel(fmha_fwd_kernel<T, D, NQ, false, false, PAD, false, D == 128>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
   } else {
-    fmha_fwd_kernel<T, D, NQ, false, false, PAD><<<grid, block, 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
+    launchKernel(fmha_fwd_kernel<T, D, NQ, false, false, PAD>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
   }
   MGPU_CHECK_LAUNCH("fmha_fwd_kernel");
 }

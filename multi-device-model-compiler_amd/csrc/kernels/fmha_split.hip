@@ -344,9 +344,9 @@ void launchSplit(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqle
   auto *o = static_cast<uint16_t *>(out);
   const dim3 grid(blocks), block(64 * SplitGeo<D>::W);
   if (causal)
-    fmha_split_kernel<T, D, QG, true, PAD><<<grid, block, 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, (int)blocks, dHead);
+    launchKernel(fmha_split_kernel<T, D, QG, true, PAD>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, (int)blocks, dHead);
   else
-    fmha_split_kernel<T, D, QG, false, PAD><<<grid, block, 0, stream>>>(in, seqlens, cuSeqlens, o, S, H, nQB, c, (int)blocks, dHead);
+    launchKernel(fmha_split_kernel<T, D, QG, false, PAD>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, (int)blocks, dHead);
   MGPU_CHECK_LAUNCH("fmha_split_kernel");
 }
 

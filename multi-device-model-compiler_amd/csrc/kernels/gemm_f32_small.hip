@@ -104,11 +104,11 @@ void gemmF32Small(const float *in, const float *weight, const float *bias, const
   const int tilesM = (int)((M + 31) / 32), tilesN = (int)((N + 31) / 32);
   const dim3 grid((unsigned)(tilesM * tilesN)), block(64 * kWaves);
   if (act == ACT_RELU)
-    gemm_f32_small_kernel<ACT_RELU><<<grid, block, 0, stream>>>(in, weight, bias, residual, out, (int)M, (int)N, (int)K, tilesM);
+    launchKernel(gemm_f32_small_kernel<ACT_RELU>, grid, block, stream, in, weight, bias, residual, out, (int)M, (int)N, (int)K, tilesM);
   else if (act == ACT_GELU)
-    gemm_f32_small_kernel<ACT_GELU><<<grid, block, 0, stream>>>(in, weight, bias, residual, out, (int)M, (int)N, (int)K, tilesM);
+    launchKernel(gemm_f32_small_kernel<ACT_GELU>, grid, block, stream, in, weight, bias, residual, out, (int)M, (int)N, (int)K, tilesM);
   else
-    gemm_f32_small_kernel<ACT_NONE><<<grid, block, 0, stream>>>(in, weight, bias, residual, out, (int)M, (int)N, (int)K, tilesM);
+    launchKernel(gemm_f32_small_kernel<ACT_NONE>, grid, block, stream, in, weight, bias, residual, out, (int)M, (int)N, (int)K, tilesM);
   MGPU_CHECK_LAUNCH("gemm_f32_small_kernel");
 }
 

@@ -260,11 +260,11 @@ void launchTile(const uint16_t *a, const uint16_t *w, const uint16_t *b, const u
   const int nblk = tilesM * tilesN;
   const dim3 grid((unsigned)nblk), block(64 * kSplit);
   if (act == ACT_GELU)
-    gemm_ksplit_kernel<T, ACT_GELU, MB, NB, RING, KMAJOR><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)M, (int)N, (int)K, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<T, ACT_GELU, MB, NB, RING, KMAJOR>, grid, block, stream, a, w, b, r, o, (int)M, (int)N, (int)K, tilesM, nblk);
   else if (act == ACT_RELU)
-    gemm_ksplit_kernel<T, ACT_RELU, MB, NB, RING, KMAJOR><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)M, (int)N, (int)K, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<T, ACT_RELU, MB, NB, RING, KMAJOR>, grid, block, stream, a, w, b, r, o, (int)M, (int)N, (int)K, tilesM, nblk);
   else
-    gemm_ksplit_kernel<T, ACT_NONE, MB, NB, RING, KMAJOR><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)M, (int)N, (int)K, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<T, ACT_NONE, MB, NB, RING, KMAJOR>, grid, block, stream, a, w, b, r, o, (int)M, (int)N, (int)K, tilesM, nblk);
 }
 
 template <typename T, bool KMAJOR>
@@ -331,11 +331,11 @@ void gemmKSplitPartialF16(const void *in, const void *weight, float *planes, int
   const dim3 grid((unsigned)nblk, (unsigned)parts), block(64 * kSplit);
   const int m = (int)M, n = (int)N, k = (int)K;
   if (tile == KSplitTile::T32x32)
-    gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 1, 4, false, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 1, 4, false, true>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
   else if (tile == KSplitTile::T32x64)
-    gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 2, 3, false, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 2, 3, false, true>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
   else
-    gemm_ksplit_kernel<_Float16, ACT_NONE, 2, 2, 2, false, true><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 2, 2, 2, false, true>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
   MGPU_CHECK_LAUNCH("gemm_ksplit_kernel");
 }
 

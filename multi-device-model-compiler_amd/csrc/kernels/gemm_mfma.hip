@@ -297,11 +297,11 @@ void launchAct(const uint16_t *a, const uint16_t *w, const uint16_t *b, const ui
   const int tilesN = (int)((N + 32 * NB - 1) / (32 * NB)), tilesM = (int)((M + kBM - 1) / kBM);
   const dim3 grid((unsigned)(tilesM * tilesN)), block(256);
   if (act == ACT_GELU)
-    gemm_mfma_kernel<T, ACT_GELU, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    launchKernel(gemm_mfma_kernel<T, ACT_GELU, NB, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   else if (act == ACT_RELU)
-    gemm_mfma_kernel<T, ACT_RELU, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    launchKernel(gemm_mfma_kernel<T, ACT_RELU, NB, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   else
-    gemm_mfma_kernel<T, ACT_NONE, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+    launchKernel(gemm_mfma_kernel<T, ACT_NONE, NB, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
 }
 template <typename T, int NB>
 void launchTile(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint16_t *r, uint16_t *o, int64_t M,

@@ -353,10 +353,10 @@ void launch(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint1
             int act, hipStream_t stream) {
   const int tilesM = (int)((M + kBM - 1) / kBM), tilesN = (int)((N + 32 * NB - 1) / (32 * NB));
   const dim3 grid((unsigned)(tilesM * tilesN)), block(kThreads);
-  if (r) gemm_round_kernel<T, kResidual, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_GELU) gemm_round_kernel<T, ACT_GELU, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_RELU) gemm_round_kernel<T, ACT_RELU, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else gemm_round_kernel<T, ACT_NONE, NB, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  if (r) launchKernel(gemm_round_kernel<T, kResidual, NB, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_GELU) launchKernel(gemm_round_kernel<T, ACT_GELU, NB, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_RELU) launchKernel(gemm_round_kernel<T, ACT_RELU, NB, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else launchKernel(gemm_round_kernel<T, ACT_NONE, NB, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_round_kernel");
 }
 
@@ -389,8 +389,8 @@ void gemmRoundPartialF16(const void *in, const void *weight, float *planes, int6
   const dim3 grid((unsigned)(tilesM * tilesN), (unsigned)parts), block(kThreads);
   const auto *a = static_cast<const uint16_t *>(in), *w = static_cast<const uint16_t *>(weight);
   auto *o = reinterpret_cast<uint16_t *>(planes);
-  if (width == 128) gemm_round_kernel<_Float16, kPartial, 4, false><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else gemm_round_kernel<_Float16, kPartial, 3, false><<<grid, block, 0, stream>>>(a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  if (width == 128) launchKernel(gemm_round_kernel<_Float16, kPartial, 4, false>, grid, block, stream, a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else launchKernel(gemm_round_kernel<_Float16, kPartial, 3, false>, grid, block, stream, a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_round_kernel");
 }
 

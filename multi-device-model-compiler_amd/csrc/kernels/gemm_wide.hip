@@ -382,17 +382,17 @@ void launch(const uint16_t *a, const uint16_t *w, const uint16_t *b, const uint1
             int act, hipStream_t stream) {
   const int tilesM = (int)((M + kBM - 1) / kBM), tilesN = (int)((N + BN - 1) / BN);
   const dim3 grid((unsigned)(tilesM * tilesN)), block(kThreads);
-  if (r) gemm_wide_kernel<T, kResidual, BN, uint16_t, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_GELU) gemm_wide_kernel<T, ACT_GELU, BN, uint16_t, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else if (act == ACT_RELU) gemm_wide_kernel<T, ACT_RELU, BN, uint16_t, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else gemm_wide_kernel<T, ACT_NONE, BN, uint16_t, RAGGED><<<grid, block, 0, stream>>>(a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  if (r) launchKernel(gemm_wide_kernel<T, kResidual, BN, uint16_t, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_GELU) launchKernel(gemm_wide_kernel<T, ACT_GELU, BN, uint16_t, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else if (act == ACT_RELU) launchKernel(gemm_wide_kernel<T, ACT_RELU, BN, uint16_t, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else launchKernel(gemm_wide_kernel<T, ACT_NONE, BN, uint16_t, RAGGED>, grid, block, stream, a, w, b, r, o, (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_wide_kernel");
 }
 
 template <int BN>
 void launchToF32(const void *a, const void *w, const void *b, const void *r, float *o, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
   const int tilesM = (int)((M + kBM - 1) / kBM), tilesN = (int)((N + BN - 1) / BN);
-  gemm_wide_kernel<_Float16, kResidual, BN, float, false><<<dim3((unsigned)(tilesM * tilesN)), dim3(kThreads), 0, stream>>>(
+  launchKernel(gemm_wide_kernel<_Float16, kResidual, BN, float, false>, dim3((unsigned)(tilesM * tilesN)), dim3(kThreads), stream,
       static_cast<const uint16_t *>(a), static_cast<const uint16_t *>(w), static_cast<const uint16_t *>(b), static_cast<const uint16_t *>(r), o,
       (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_wide_kernel");

@@ -467,7 +467,7 @@ void launchRows(bool ragged, const T *input, const T *residual, const T *gamma, 
   const int64_t cap = kMaxStreamBlocks;
   if (blocks > cap) blocks = cap;
 #define MGPU_LN_ROWS(S)                                                                                                      \
-  layernorm_rows_kernel<T, LANES, VPL, RESIDUAL, RowShape::S><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>( \
+  launchKernel(layernorm_rows_kernel<T, LANES, VPL, RESIDUAL, RowShape::S>, dim3((unsigned)blocks), dim3(256), stream, \
       input, gamma, beta, normed, m, n, (int)(blocks * GROUPS), eps, residual, sumOut)
   if (ragged) MGPU_LN_ROWS(kRagged);
   else if (n / ElemTraits<T>::kVec == LANES * VPL) MGPU_LN_ROWS(kFull);
@@ -536,7 +536,7 @@ void layerNormTyped(const T *input, const T *residual, const T *gamma, const T *
     const bool pairRows = m >= 2 && vpl * ElemTraits<T>::kVec <= 32;
     if (pairRows) blocks = (blocks + 1) / 2;
 #define MGPU_LN_BLOCK(V, R, F)                                                                    \
-  layernorm_block_kernel<T, V, R, RESIDUAL, RowShape::F><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>( \
+  launchKernel(layernorm_block_kernel<T, V, R, RESIDUAL, RowShape::F>, dim3((unsigned)blocks), dim3(256), stream, \
       input, gamma, beta, normed, m, n, (int)(blocks * R), eps, residual, sumOut)
 #define MGPU_LN_SHAPES(V, R)                 \
   if (ragged) MGPU_LN_BLOCK(V, R, kRagged);  \
@@ -560,7 +560,7 @@ void layerNormTyped(const T *input, const T *residual, const T *gamma, const T *
     MGPU_CHECK_LAUNCH("layernorm_block_kernel");
     return;
   }
-  layernorm_general_kernel<T, RESIDUAL><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(
+  launchKernel(layernorm_general_kernel<T, RESIDUAL>, dim3((unsigned)blocks), dim3(256), stream,
       input, gamma, beta, normed, m, n, (int)blocks, eps, residual, sumOut);
   MGPU_CHECK_LAUNCH("layernorm_general_kernel");
 }
@@ -623,10 +623,10 @@ bool castLayerNormF32ToF16(const float *input, const void *gamma, const void *be
 #define MGPU_LN_CAST(L, V)                                                                                     \
   if (lanes == L && vpl == V) {                                                                                \
     if (full)                                                                                                  \
-      layernorm_cast_rows_kernel<_Float16, L, V, true><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(      \
+      launchKernel(layernorm_cast_rows_kernel<_Float16, L, V, true>, dim3((unsigned)blocks), dim3(256), stream,      \
           input, g, b, c, y, m, n, (int)(blocks * (256 / L)), eps);                                            \
     else                                                                                                       \
-      layernorm_cast_rows_kernel<_Float16, L, V, false><<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(     \
+      launchKernel(layernorm_cast_rows_kernel<_Float16, L, V, false>, dim3((unsigned)blocks), dim3(256), stream,     \
           input, g, b, c, y, m, n, (int)(blocks * (256 / L)), eps);                                            \
   }
   MGPU_LN_CAST(16, 1) MGPU_LN_CAST(16, 2) MGPU_LN_CAST(16, 3) MGPU_LN_CAST(16, 4)

@@ -116,7 +116,7 @@ void launch(const float *planes, const void *bias, const void *residual, const v
   auto *s = static_cast<_Float16 *>(sumOut);
   const auto kernel = N <= 512 ? partial_sums_kernel<1, PARTS, RESULT> : N <= 1024 ? partial_sums_kernel<2, PARTS, RESULT>
                                                                                    : partial_sums_kernel<4, PARTS, RESULT>;
-  kernel<<<grid, block, 0, stream>>>(planes, b, r, g, be, s, out, (int)M, (int)N, eps);
+  launchKernel(kernel, grid, block, stream, planes, b, r, g, be, s, out, (int)M, (int)N, eps);
   MGPU_CHECK_LAUNCH("partial_sums_kernel");
 }
 
