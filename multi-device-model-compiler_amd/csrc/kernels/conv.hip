@@ -564,6 +564,13 @@ __global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__
   finishTile<1, KS, uint32_t>(acc, partial, 0, ks, bias, add, y, OC, P, oc0, nFirst, img, pix, lane, relu);
 }
 
+// Scales for pairs of fp16 numbers: the largest value to 2^7 .. 2^8, where pairs hold sizes from kLeastInPairs on.  Largest values
+// beyond 2^100, or under 2^-100 and not 0, are left to the fp32 instructions.
+constexpr float kLeastInPairs = 0.25f;
+__device__ __forceinline__ bool pairsHold(float most) { return most == 0.0f || (most >= 0x1p-100f && most <= 0x1p100f); }
+__device__ __forceinline__ int pairExponent(float most) { return most == 0.0f ? 0 : 134 - (int)(__builtin_bit_cast(uint32_t, most) >> 23); }
+__device__ __forceinline__ float powerOf2(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
+
 // ---- few taps -----------------------------------------------------------------------------
 // A reduction of at most 2 NS taps (a network's stem: 3 channels, 3 x 3).  A wavefront keeps the
 // filter of its OCT x 32 channels in registers, lane half hl the taps 2 s + hl of step s, and walks
@@ -710,7 +717,12 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
 // 256 x 256 -> 64, 268 MB: 76.9 -> 65.5 us (1 x 1 from the same: 68.0 -> 49.2; a fill of as many bytes takes 39); 8 x 3 x 224 x
 // 224 -> 64 with a postAdd 87 -> 49; 8 x 3 x 128 x 128 -> 16 11.0 -> 6.7.  Stores of one tile dealt out between the matrix
 // instructions of the next measured the same, an order of tiles by XCD too, runs of tiles a wavefront 90.
-template <int KW, int NR, Output OUT, bool ADDED>
+// SPLIT: the products by the fp16 matrix instructions, operands taken apart into pairs of fp16 numbers as in conv_split.hip: six
+// steps of 32 clocks instead of 15 of 64, and fewer roundings (K = 27: error against 64 bits 1.1e-7 -> 0.67e-7).  A quad's pixels
+// have a scale of their own, each tile: whole windows that are small beside their neighbours', infinities and filters of which a
+// channel is small beside the others take the fp32 instructions.  us, before / now: 16 x 3 x 256 x 256 -> 64 59 / 54, 16 x 3 x
+// 224 x 224 -> 64 58 / 47, 4 x 3 x 224 x 224 -> 64 17.2 / 12.6, 16 x 3 x 76 x 248 -> 33 of stride 2 down 14.8 / 9.8.
+template <int KW, int NR, Output OUT, bool ADDED, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                             const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
                                                             int P, int N, FastDiv byP, FastDiv byOW, const float *__restrict__ add,
@@ -739,6 +751,30 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
   for (int r = 0; r < 16; r++) {
     const int oc = oc0 + 8 * (r / 4) + r % 4 + 4 * hl;
     bv[r] = bias[oc < OC ? oc : OC - 1];
+  }
+  // SPLIT: the lane half's taps as eight each of STEPS matrix instructions, in the order of its rows, in pairs of fp16 numbers.
+  constexpr int TAPS = NR * KW, STEPS = (TAPS + 7) / 8;
+  u32x4 ah[STEPS], al[STEPS];
+  float wDown = 1.0f;  // undoes the filter's scale
+  bool pairs = SPLIT;  // whether they hold the filter (uniform)
+  if constexpr (SPLIT) {
+    float m = 0.0f; // of the lane's channel
+#pragma unroll
+    for (int i = 0; i < TAPS; i++) m = fmaxf(m, fabsf(a[i / KW][i % KW]));
+    m = halves_max(m);
+    const float most = group_max<64>(m);
+    const int e = pairExponent(most);
+    const float scale = powerOf2(e);
+    wDown = powerOf2(-e);
+    pairs = __builtin_amdgcn_ballot_w64(!pairsHold(most) || (m > 0.0f && m * scale < kLeastInPairs)) == 0;
+#pragma unroll
+    for (int i = 0; i < 4 * STEPS; i++) {
+      auto tap = [&](int k) { return k < TAPS ? a[k / KW][k % KW] * scale : 0.0f; };
+      uint32_t hi, lo;
+      splitPair(tap(2 * i), tap(2 * i + 1), hi, lo);
+      ah[i / 4][i % 4] = hi;
+      al[i / 4][i % 4] = lo;
+    }
   }
   struct Tile {
     int pix, img, nFirst; // the lane's first pixel (-1: past the end), its image less the tile's first, that image
@@ -798,15 +834,8 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
     };
     f32x4 addend[16];
     if (ADDED && kEarly) everyChannel([&](int r, int voffset, int soffset) { addend[r] = fromPost(voffset, soffset); });
-    f32x16 acc[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-      for (int i = 0; i < 16; i++) acc[j][i] = bv[i];
-#pragma unroll
-    for (int i = 0; i < NR; i++) {
-      // the window's KW + 3 columns in order (uniform selects: PWL of them lie left of the quad)
-      float c[KW + 3];
+    // the window's KW + 3 columns of a row in order (uniform selects: PWL of them lie left of the quad)
+    auto columns = [&](int i, float (&c)[KW + 3]) {
 #pragma unroll
       for (int e = 0; e < KW + 3; e++) {
         float v = e < SIDE ? o.side[i][e] : 0.0f; // e < PWL
@@ -816,19 +845,90 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
         if (e >= 4 && e - 4 >= 0 && e - 4 < SIDE && e >= g.PWL + 4) v = o.side[i][e - 4];
         c[e] = v;
       }
+    };
+    auto store = [&](const f32x16 (&acc)[4], auto &&value) { // value(register, accumulator's)
+      everyChannel([&](int r, int voffset, int soffset) {
+        f32x4 v = {value(r, acc[0][r]), value(r, acc[1][r]), value(r, acc[2][r]), value(r, acc[3][r])};
+        if (ADDED) v += kEarly ? addend[r] : fromPost(voffset, soffset);
+        // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
+        if (relu) v = f32x4{fmaxf(v[0], 0.0f), fmaxf(v[1], 0.0f), fmaxf(v[2], 0.0f), fmaxf(v[3], 0.0f)};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, voffset, soffset,
+                                               OUT == Output::Streamed ? 2 : OUT == Output::Through ? 16 : 0);
+      });
+    };
+    if constexpr (SPLIT) {
+      // One scale for the quad, from the largest value of its windows; of each pixel's window the pairs have to hold it, too.
+      float c[NR][KW + 3], column[KW + 3], window[4];
+#pragma unroll
+      for (int e = 0; e < KW + 3; e++) column[e] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < NR; i++) {
+        columns(i, c[i]);
+#pragma unroll
+        for (int e = 0; e < KW + 3; e++) column[e] = fmaxf(column[e], fabsf(c[i][e]));
+      }
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        window[j] = column[j];
+#pragma unroll
+        for (int k = 1; k < KW; k++) window[j] = fmaxf(window[j], column[j + k]);
+        window[j] = halves_max(window[j]);
+      }
+      const float m = fmaxf(fmaxf(window[0], window[1]), fmaxf(window[2], window[3]));
+      const int e = pairExponent(m);
+      const float scale = powerOf2(e), down = powerOf2(-e) * wDown;
+      bool low = false;
+#pragma unroll
+      for (int j = 0; j < 4; j++) low |= window[j] > 0.0f && window[j] * scale < kLeastInPairs;
+      if (pairs && __builtin_amdgcn_ballot_w64(low || !pairsHold(m)) == 0) {
+#pragma unroll
+        for (int i = 0; i < NR; i++)
+#pragma unroll
+          for (int k = 0; k < KW + 3; k++) c[i][k] *= scale;
+        f32x16 acc[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          u32x4 bh[STEPS], bl[STEPS];
+#pragma unroll
+          for (int i = 0; i < 4 * STEPS; i++) {
+            auto tap = [&](int k) { return k < TAPS ? c[k / KW][k % KW + j] : 0.0f; };
+            uint32_t hi, lo;
+            splitPair(tap(2 * i), tap(2 * i + 1), hi, lo);
+            bh[i / 4][i % 4] = hi;
+            bl[i / 4][i % 4] = lo;
+          }
+          auto product = [&](const u32x4 &u, const u32x4 &v, const f32x16 &to) {
+            return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, u), __builtin_bit_cast(f16x8, v), to, 0, 0, 0);
+          };
+          // (the small products first: their roundings are small, too)
+          f32x16 sum;
+#pragma unroll
+          for (int i = 0; i < 16; i++) sum[i] = 0.0f;
+#pragma unroll
+          for (int i = 0; i < STEPS; i++) sum = product(ah[i], bl[i], product(al[i], bh[i], sum));
+#pragma unroll
+          for (int i = 0; i < STEPS; i++) sum = product(ah[i], bh[i], sum);
+          acc[j] = sum;
+        }
+        store(acc, [&](int r, float v) { return fmaf(v, down, bv[r]); });
+        return;
+      }
+    }
+    f32x16 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[j][i] = bv[i];
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+      float c[KW + 3];
+      columns(i, c);
 #pragma unroll
       for (int k = 0; k < KW; k++)
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][k], c[k + j], acc[j], 0, 0, 0);
     }
-    everyChannel([&](int r, int voffset, int soffset) {
-      f32x4 v = {acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
-      if (ADDED) v += kEarly ? addend[r] : fromPost(voffset, soffset);
-      // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
-      if (relu) v = f32x4{fmaxf(v[0], 0.0f), fmaxf(v[1], 0.0f), fmaxf(v[2], 0.0f), fmaxf(v[3], 0.0f)};
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, voffset, soffset,
-                                             OUT == Output::Streamed ? 2 : OUT == Output::Through ? 16 : 0);
-    });
+    store(acc, [](int, float v) { return v; });
   };
   Tile even, odd;
   int tile = (int)blockIdx.x * 4 + wave;
@@ -1359,9 +1459,17 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     // two blocks per CU and channel tile
     const int64_t most = std::max<int64_t>(1, (int64_t)numComputeUnits() * 2 / ((OC + 31) / 32));
     const int64_t blocks = std::min((tiles128 + 3) / 4, most);
-    auto *kernel = add ? (quadStores == Output::Streamed ? conv_quads_kernel<KWC, NR, Output::Streamed, true> : conv_quads_kernel<KWC, NR, Output::Through, true>)
-                   : quadStores == Output::Streamed ? conv_quads_kernel<KWC, NR, Output::Streamed, false>
-                   : quadStores == Output::Cached ? conv_quads_kernel<KWC, NR, Output::Cached, false> : conv_quads_kernel<KWC, NR, Output::Through, false>;
+    // Pairs of fp16 numbers from 12 taps on (of 9 they would be no more exact than the fp32 instructions, 6.5e-8 / 7.0e-8); an addend
+    // in flight leaves no registers for them.
+    auto kernelOf = [&](auto split) {
+      constexpr bool SPLIT = decltype(split)::value;
+      return quadStores == Output::Streamed ? conv_quads_kernel<KWC, NR, Output::Streamed, false, SPLIT>
+             : quadStores == Output::Cached ? conv_quads_kernel<KWC, NR, Output::Cached, false, SPLIT> : conv_quads_kernel<KWC, NR, Output::Through, false, SPLIT>;
+    };
+    auto *kernel = kernelOf(std::false_type());
+    if (add) kernel = quadStores == Output::Streamed ? conv_quads_kernel<KWC, NR, Output::Streamed, true, false> : conv_quads_kernel<KWC, NR, Output::Through, true, false>;
+    else if constexpr (KWC * NR > 8)
+      if (K >= 12) kernel = kernelOf(std::true_type());
     launchKernel(kernel, gridOf(blocks, 32, 256), dim3(256), stream, input, weight, bias, output, g, (int)OC, (int)P, (int)N, byP, byOW, add, relu,
                                                               (int)tiles128, (int)(4 * blocks));
   };

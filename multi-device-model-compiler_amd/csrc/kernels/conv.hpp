@@ -33,4 +33,15 @@ __device__ __forceinline__ i32x4 resourceWords(const float *p, int64_t elems) {
   return i32x4{(int)(uint32_t)at, (int)(uint32_t)(at >> 32) & 0xffff, resourceBytes(elems), kRawBuffer};
 }
 
+// a and b as fp16 numbers, hi, and what these leave, lo: pairs of 22 bits where lo is no smaller than fp16's normal numbers, 2^-25
+// off below.  (Four instructions; v_fma_mixlo / mixhi_f16 would be fewer where a scale comes besides, but writing half a register
+// takes them two to three times as long.)
+__device__ __forceinline__ void splitPair(float a, float b, uint32_t &hi, uint32_t &lo) {
+  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+  float ra, rb;
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(ra) : "v"(a), "v"(hi));
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(rb) : "v"(b), "v"(hi));
+  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(lo) : "v"(ra), "v"(rb));
+}
+
 } // namespace mgpu

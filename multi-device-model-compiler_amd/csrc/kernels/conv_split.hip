@@ -61,16 +61,6 @@ template <int LANES> __device__ __forceinline__ void ldsLoad16First(uint32_t off
 }
 #pragma clang diagnostic pop
 
-// a * scale and b * scale as fp16 numbers and what these leave, in pairs.  (Six instructions; v_fma_mixlo / mixhi_f16 would be
-// four, but writing half a register takes them two to three times as long.)
-__device__ __forceinline__ void splitPair(float a, float b, float scale, uint32_t &hi, uint32_t &lo) {
-  float sa = a * scale, sb = b * scale;
-  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(hi) : "v"(sa), "v"(sb));
-  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(sa) : "v"(sa), "v"(hi));
-  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(sb) : "v"(sb), "v"(hi));
-  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(lo) : "v"(sa), "v"(sb));
-}
-
 // The exponent of a scale 2^e for values whose largest has these bits (none: what to take them for where there is none).
 __device__ __forceinline__ int scaleExponent(uint32_t largest, int none) {
   const int e = (int)(largest >> 23) - 126; // 2^(e-1) <= largest < 2^e
@@ -243,7 +233,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
         if constexpr (SPLIT) {
           uint32_t hi[4], lo[4];
 #pragma unroll
-          for (int k = 0; k < 4; k++) splitPair(v[2 * k], v[2 * k + 1], scale, hi[k], lo[k]);
+          for (int k = 0; k < 4; k++) splitPair(v[2 * k] * scale, v[2 * k + 1] * scale, hi[k], lo[k]);
           *reinterpret_cast<u32x4 *>(at) = u32x4{hi[0], hi[1], hi[2], hi[3]};
           *reinterpret_cast<u32x4 *>(at + second) = u32x4{lo[0], lo[1], lo[2], lo[3]};
         } else {

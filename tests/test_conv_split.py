@@ -99,36 +99,59 @@ def test_against_the_oracle(pkg, gpu, oracle, rng, tile, N, IC, H, W, OC, pad, s
     assert np.all(np.abs(got - ref) <= 1e-5 * (1 + np.abs(ref))), np.abs(got - ref).max()
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("kind", ["normal", "tiny", "huge", "dark half", "outlier", "growing", "growing filter", "zero channels", "zero filter channels",
-                                  "dead filters", "zeros", "inf", "inf filter", "nan"])
-def test_operands_of_every_size(pkg, gpu, kind):
-    """Against 64 bits, elementwise to the size of the products summed up: what the pieces do not hold goes the fp32 way."""
+KINDS = ["normal", "tiny", "huge", "dark half", "outlier", "growing", "growing filter", "zero channels", "zero filter channels", "dead filters", "zeros",
+         "inf", "inf filter", "nan"]
+
+
+def operands(kind, N, IC, H, W, OC, device):
     import torch
-    gen = torch.Generator(device=gpu).manual_seed(len(kind))
-    r = lambda *s: torch.randn(s, device=gpu, generator=gen)  # noqa: E731
-    N, IC, H, W, OC = 2, 64, 14, 16, 40
-    x, w, b = r(N, IC, H, W), r(OC, IC, 3, 3), torch.zeros(OC, device=gpu)
+    gen = torch.Generator(device=device).manual_seed(len(kind))
+    r = lambda *s: torch.randn(s, device=device, generator=gen)  # noqa: E731
+    x, w, c = r(N, IC, H, W), r(OC, IC, 3, 3), min(IC - 1, 16)
     if kind == "tiny": x, w = x * 1e-12, w * 1e-9
     if kind == "huge": x, w = x * 1e14, w * 1e9
-    if kind == "dark half": x[:, :, :, :8] *= 1e-9
-    if kind == "outlier": x[1, 40, 3, 3] = 1e7
-    if kind == "growing": x[:, 16:] *= 1e4
-    if kind == "growing filter": w[:, 16:] *= 1e4
-    if kind == "zero channels": x[:, :16] = 0
-    if kind == "zero filter channels": w[:, :16], w[1] = 0, 1e-12 * w[1]
+    if kind == "dark half": x[:, :, :, :W // 2 + 1] *= 1e-9
+    if kind == "outlier": x[1, IC // 2, 3, 3] = 1e7
+    if kind == "growing": x[:, c:] *= 1e4
+    if kind == "growing filter": w[:, c:] *= 1e4
+    if kind == "zero channels": x[:, :c] = 0
+    if kind == "zero filter channels": w[:, :c], w[1] = 0, 1e-12 * w[1]
     if kind == "dead filters": w[::3] *= 1e-20
     if kind == "zeros": x.zero_()
-    if kind == "inf": x[0, 5, 4, 4] = float("inf")
-    if kind == "inf filter": w[3, 50, 1, 1] = float("-inf")
-    if kind == "nan": x[1, 7, 5, 6], w[2, 3, 0, 0] = float("nan"), float("nan")
+    if kind == "inf": x[0, c - 1, 4, 4] = float("inf")
+    if kind == "inf filter": w[3, c, 1, 1] = float("-inf")
+    if kind == "nan": x[1, c - 1, 5, 6], w[2, c - 1, 0, 0] = float("nan"), float("nan")
+    return x, w
+
+
+def check(got, x, w, kind):
+    """Against 64 bits, elementwise to the size of the products summed up: what the pairs do not hold goes the fp32 way."""
+    import torch
+    H, W = x.shape[2:]
     conv = lambda x, w: sum(torch.nn.functional.pad(x, (1, 1, 1, 1))[:, None, :, i:i + H, j:j + W].mul(w[None, :, :, i, j, None, None]).sum(2)  # noqa: E731
                             for i in range(3) for j in range(3))
-    ref, size = conv(x.double(), w.double()), conv(x.double().abs(), w.double().abs())
+    ref, size, got = conv(x.double(), w.double()), conv(x.double().abs(), w.double().abs()), got.double()
+    finite = torch.isfinite(ref)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(got[~finite & ~torch.isnan(ref)], ref[~finite & ~torch.isnan(ref)])
+    # 2^-24 a product and rounding: some hundreds of them, whose errors are far from all of one sign
+    assert (got - ref).abs()[finite].le(2.0 ** -20 * size[finite]).all(), kind
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+def test_operands_of_every_size(pkg, gpu, kind):
+    import torch
+    x, w = operands(kind, 2, 64, 14, 16, 40, gpu)
     for tile in (0, 4):
-        got = split_conv(pkg, tile, 1, x, w, b, None, (1, 1, 1, 1), (1, 1), (1, 1), False).double()
-        finite = torch.isfinite(ref)
-        assert torch.equal(torch.isnan(got), torch.isnan(ref))
-        assert torch.equal(got[~finite & ~torch.isnan(ref)], ref[~finite & ~torch.isnan(ref)])
-        # 2^-24 a product and rounding: 288 products of sixteen, whose errors are far from all of one sign
-        assert (got - ref).abs()[finite].le(2.0 ** -20 * size[finite]).all(), kind
+        check(split_conv(pkg, tile, 1, x, w, torch.zeros(40, device=gpu), None, (1, 1, 1, 1), (1, 1), (1, 1), False), x, w, kind)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("IC", [2, 3])
+def test_operands_of_every_size_in_a_stem(pkg, gpu, kind, IC):
+    """The kernel of few taps and four pixels a lane, on the same terms (512 tiles of 128 pixels x 32 channels)."""
+    import torch
+    x, w = operands(kind, 2, IC, 64, 64, 250, gpu)
+    check(pkg.conv2d(x, w, torch.zeros(250, device=gpu), pad=(1, 1, 1, 1)), x, w, kind)
