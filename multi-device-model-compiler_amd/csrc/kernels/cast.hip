@@ -7,6 +7,7 @@
 // wide side and the grid is sized to the array.  Round to nearest even.
 // The transpose replaces add_fusedQKV_bias_transpose_kernel
 // (lib/Kernels/GPU/Transpose.cu:5-84).
+#include "cast_table.hpp"
 #include "common.hpp"
 #include "mgpu_ops_internal.hpp"
 #include "types.hpp"
@@ -15,9 +16,6 @@ namespace mgpu {
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // T is the 16-bit type (_Float16 or bf16_t); its vectors travel as 16 raw bytes.
 // (The grid's stride is an explicit argument: explicit arguments are preloaded into SGPRs,
@@ -150,79 +148,8 @@ void castToF32(float *dst, const void *src, size_t size, hipStream_t stream, con
 }
 
 
-// ---- a layer's weights in one launch --------------------------------------------------------
-// The reference layer hands over fp32 weights on every call; casting its seven arrays one by one is seven
-// launches of 2.3 us host time, most of them a few microseconds of work.  Here one grid covers them all: a block finds
-// its array among the first-block numbers in the arguments.  A plain array goes 8 elements a lane; one wanted
-// K-major (transposed) goes in 64 x 64 tiles, four rows by four columns per thread, through LDS at a pitch of
-// 68 halves: 16 bytes a lane from and to memory, 8-byte LDS accesses that meet every bank equally often
-// (d_model 2048, ffn 2048, 151 MB: 27 us, 5.6 TB/s; as seven launches of the plain cast 58 us of GPU time,
-// half of it hidden behind the LayerNorm and the first GEMM, which it slowed).
-struct CastTable {
-  CastJob job[kMaxCastJobs];
-  unsigned firstBlock[kMaxCastJobs + 1];
-  int count;
-};
-constexpr int kPlainPerBlock = 2048;
-
-__global__ __launch_bounds__(256) void cast_weights_kernel(CastTable t) {
-  __shared__ __attribute__((aligned(16))) _Float16 tile[64][68];
-  int j = 0;
-  while (j + 1 < t.count && blockIdx.x >= t.firstBlock[j + 1]) j++; // (uniform)
-  const CastJob job = t.job[j];
-  const unsigned block = blockIdx.x - t.firstBlock[j];
-  const float *src = job.src;
-  _Float16 *dst = static_cast<_Float16 *>(job.dst);
-  const int tid = threadIdx.x;
-  if (!job.kMajor) {
-    const int64_t n = job.rows * job.cols, i = (int64_t)block * kPlainPerBlock + tid * 8;
-    if (job.vector && i + 8 <= n) {
-      const f32x4 lo = *reinterpret_cast<const f32x4 *>(src + i), hi = *reinterpret_cast<const f32x4 *>(src + i + 4);
-      const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      *reinterpret_cast<u32x4 *>(dst + i) = ElemTraits<_Float16>::pack(v);
-    } else {
-      for (int e = 0; e < 8; e++)
-        if (i + e < n) dst[i + e] = (_Float16)src[i + e];
-    }
-    return;
-  }
-  const int64_t tilesC = (job.cols + 63) / 64;
-  const int64_t r0 = (int64_t)(block / tilesC) * 64, c0 = (int64_t)(block % tilesC) * 64;
-  const bool whole = job.vector && r0 + 64 <= job.rows && c0 + 64 <= job.cols; // (uniform)
-  const int q = tid % 16, w = tid / 16; // this thread: rows 4 w.., columns 4 q..
-  f32x4 v[4];
-  if (whole) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const f32x4 *>(src + (r0 + 4 * w + i) * job.cols + c0 + 4 * q);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int64_t r = r0 + 4 * w + i, c = c0 + 4 * q + e;
-        v[i][e] = r < job.rows && c < job.cols ? src[r * job.cols + c] : 0.0f;
-      }
-  }
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const f16x4 col = {(_Float16)v[0][e], (_Float16)v[1][e], (_Float16)v[2][e], (_Float16)v[3][e]};
-    *reinterpret_cast<f16x4 *>(&tile[4 * q + e][4 * w]) = col;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int c = tid / 8 + 32 * i, r = 8 * (tid % 8);
-    const f16x4 lo = *reinterpret_cast<const f16x4 *>(&tile[c][r]), hi = *reinterpret_cast<const f16x4 *>(&tile[c][r + 4]);
-    _Float16 *out = dst + (c0 + c) * job.rows + r0 + r;
-    if (whole) {
-      *reinterpret_cast<f16x8 *>(out) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    } else if (c0 + c < job.cols) {
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        if (r0 + r + e < job.rows) out[e] = e < 4 ? lo[e % 4] : hi[e % 4];
-    }
-  }
-}
+// ---- a layer's weights in one launch (cast_table.hpp) ---------------------------------------
+__global__ __launch_bounds__(256) void cast_weights_kernel(CastTable t) { castTableBlock(t, blockIdx.x); }
 
 // dst[c][r] = T(src[r][c]) for a row-major rows x cols matrix: 64 x 64 tiles through LDS (one
 // padding column against bank conflicts), coalesced on both sides.  Runs once per weight array
@@ -255,9 +182,9 @@ void castBF16ToF32(float *dst, const void *src, size_t size, hipStream_t stream)
   castToF32<bf16_t>(dst, src, size, stream, "castBF16ToF32");
 }
 
-void castWeightsF32ToF16(CastJob *jobs, int count, hipStream_t stream) {
+unsigned castTable(CastJob *jobs, int count, CastTable &t) {
   if (count < 0 || count > kMaxCastJobs) fail("castWeightsF32ToF16: too many arrays");
-  CastTable t{};
+  t = CastTable{};
   uint64_t blocks = 0;
   for (int j = 0; j < count; j++) {
     CastJob &job = jobs[j];
@@ -270,8 +197,14 @@ void castWeightsF32ToF16(CastJob *jobs, int count, hipStream_t stream) {
     if (blocks > 0x7fffffffu) fail("castWeightsF32ToF16: weights too large for one launch");
   }
   t.count = count;
+  return (unsigned)blocks;
+}
+
+void castWeightsF32ToF16(CastJob *jobs, int count, hipStream_t stream) {
+  CastTable t;
+  const unsigned blocks = castTable(jobs, count, t);
   if (!blocks) return;
-  launchKernel(cast_weights_kernel, dim3((unsigned)blocks), dim3(256), stream, t);
+  launchKernel(cast_weights_kernel, dim3(blocks), dim3(256), stream, t);
   MGPU_CHECK_LAUNCH("cast_weights_kernel");
 }
 

@@ -404,6 +404,22 @@ void gemmPartialF16(const PartialPlan &plan, const void *in, const void *weight,
   else gemmKSplitPartialF16(in, weight, planes, M, N, K, plan.tile, plan.parts, stream);
 }
 
+bool matmulResidualF32(const void *input, const void *weight, const void *bias, const void *residual, float *output, int64_t M, int64_t N,
+                       int64_t K, bool weightKMajor, hipStream_t stream) {
+  if (!bias || !residual || !aligned16(output)) return false;
+  // (gemm_wide wherever it can go, also on shallow products: its unrounded result saves a pass)
+  const int wide = weightKMajor || K % 64 ? 0 : wideWidth(DType::F16, input, weight, bias, residual, output, M, N, K, ACT_NONE);
+  if (wide) {
+    gemmWideResidualF32(input, weight, bias, residual, output, M, N, K, wide, stream);
+    return true;
+  }
+  const Choice choice = chooseKernel(DType::F16, input, weight, bias, residual, output, M, N, K, true, ACT_NONE, true, weightKMajor);
+  if (choice.kernel == GemmKernel::Round) gemmRoundResidualF32(input, weight, bias, residual, output, M, N, K, choice.width, stream);
+  else if (choice.kernel == GemmKernel::KSplit) gemmKSplitResidualF32(input, weight, bias, residual, output, M, N, K, choice.tile, weightKMajor, stream);
+  else return false;
+  return true;
+}
+
 void matmulEx(DType dt, const void *input, const void *weight, const void *bias, void *output,
               const void *residual, int64_t M, int64_t N, int64_t K, bool hasBias, int act,
               bool hasResidual, hipStream_t stream, bool weightKMajor) {

@@ -13,8 +13,9 @@
 // MFMA formulation and operand reads are those of gemm_mfma.hip: the transposed product
 // out^T[n, m] = W^T[n, k] . in^T[k, m] with W^T through the transposing LDS read.
 //
-// PARTIAL: the blocks of grid row y take the y-th share of the reduction and write their fp32 sums to plane y of `out`
-// (float [gridDim.y][M][N]; partial_sums.hip adds the planes up and has the epilogue).
+// Result::Planes: the blocks of grid row y take the y-th share of the reduction and write their fp32 sums to plane y of `out`
+// (float [gridDim.y][M][N]; partial_sums.hip adds the planes up and has the epilogue).  Result::F32: the rounded result, widened (the
+// bits of a cast behind the kernel).
 #include "common.hpp"
 #include "mfma.hpp"
 #include "mgpu_ops_internal.hpp"
@@ -28,7 +29,8 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 
 constexpr int kSplit = 8; // wavefronts of a block
 
-template <typename T, int ACT, int MB, int NB, int RING, bool KMAJOR, bool PARTIAL = false>
+enum class Result { Half, Planes, F32 };
+template <typename T, int ACT, int MB, int NB, int RING, bool KMAJOR, Result RESULT = Result::Half>
 __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
                                                                  const uint16_t *__restrict__ bias, const uint16_t *residual, uint16_t *out,
                                                                  int M, int N, int K, int tilesM, int nblk) {
@@ -54,7 +56,7 @@ __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint1
   const int l32 = lane % 32, hl = lane / 32;
 
   int chunks = (K + 31) / 32, firstChunk = 0;
-  if (PARTIAL) {
+  if (RESULT == Result::Planes) {
     firstChunk = chunks * (int)blockIdx.y / (int)gridDim.y;
     chunks = chunks * ((int)blockIdx.y + 1) / (int)gridDim.y - firstChunk;
   }
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint1
     float4v x = *reinterpret_cast<const float4v *>(part);
 #pragma unroll
     for (int s = 1; s < KS; s++) x += *reinterpret_cast<const float4v *>(part + s * kWave);
-    if (PARTIAL) {
+    if (RESULT == Result::Planes) {
       *reinterpret_cast<float4v *>(reinterpret_cast<float *>(out) + ((size_t)blockIdx.y * M + m) * N + n) = x;
       continue;
     }
@@ -249,6 +251,12 @@ __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint1
     v4 o;
 #pragma unroll
     for (int i = 0; i < 4; i++) o[i] = Mm::narrow(x[i]);
+    if (RESULT == Result::F32) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[i] = Mm::widen(o[i]);
+      *reinterpret_cast<float4v *>(reinterpret_cast<float *>(out) + (size_t)m * N + n) = x;
+      continue;
+    }
     *reinterpret_cast<v4 *>(out + (size_t)m * N + n) = o;
   }
 }
@@ -331,12 +339,34 @@ void gemmKSplitPartialF16(const void *in, const void *weight, float *planes, int
   const dim3 grid((unsigned)nblk, (unsigned)parts), block(64 * kSplit);
   const int m = (int)M, n = (int)N, k = (int)K;
   if (tile == KSplitTile::T32x32)
-    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 1, 4, false, true>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 1, 4, false, Result::Planes>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
   else if (tile == KSplitTile::T32x64)
-    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 2, 3, false, true>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 2, 3, false, Result::Planes>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
   else
-    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 2, 2, 2, false, true>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 2, 2, 2, false, Result::Planes>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
   MGPU_CHECK_LAUNCH("gemm_ksplit_kernel");
+}
+
+namespace {
+template <bool KMAJOR>
+void launchToF32(const void *in, const void *weight, const void *bias, const void *residual, float *out, int64_t M, int64_t N, int64_t K,
+                 KSplitTile tile, hipStream_t stream) {
+  auto go = [&](auto *kernel, int bm, int bn) {
+    const int tilesM = (int)((M + bm - 1) / bm), nblk = tilesM * (int)((N + bn - 1) / bn);
+    launchKernel(kernel, dim3((unsigned)nblk), dim3(64 * kSplit), stream, static_cast<const uint16_t *>(in), static_cast<const uint16_t *>(weight),
+        static_cast<const uint16_t *>(bias), static_cast<const uint16_t *>(residual), reinterpret_cast<uint16_t *>(out), (int)M, (int)N, (int)K, tilesM, nblk);
+  };
+  if (tile == KSplitTile::T32x32) go(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 1, 4, KMAJOR, Result::F32>, 32, 32);
+  else if (tile == KSplitTile::T32x64) go(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 2, 3, KMAJOR, Result::F32>, 32, 64);
+  else go(gemm_ksplit_kernel<_Float16, ACT_NONE, 2, 2, 2, KMAJOR, Result::F32>, 64, 64);
+  MGPU_CHECK_LAUNCH("gemm_ksplit_kernel");
+}
+} // namespace
+
+void gemmKSplitResidualF32(const void *in, const void *weight, const void *bias, const void *residual, float *out, int64_t M, int64_t N,
+                           int64_t K, KSplitTile tile, bool weightKMajor, hipStream_t stream) {
+  if (weightKMajor) launchToF32<true>(in, weight, bias, residual, out, M, N, K, tile, stream);
+  else launchToF32<false>(in, weight, bias, residual, out, M, N, K, tile, stream);
 }
 
 } // namespace mgpu

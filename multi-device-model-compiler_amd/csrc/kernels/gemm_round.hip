@@ -36,6 +36,7 @@ template <int NB> __host__ __device__ constexpr int wSwz(int row) { return NB ==
 constexpr int kResidual = 3; // + residual in its place
 constexpr int kPartial = 4;  // the blocks of grid row y take the y-th share of the reduction and write their fp32 sums to
                              // plane y of `out` (float [gridDim.y][M][N]; partial_sums.hip adds them up and has the epilogue)
+constexpr int kResidualF32 = 5; // + residual, the rounded result widened to fp32 (the bits of a cast behind the kernel)
 template <typename T, int ACT, int NB, bool RAGGED>
 __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
                                                                  const uint16_t *__restrict__ bias, const uint16_t *residual, uint16_t *out,
@@ -43,6 +44,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
   using M = Mma<T>;
   using v8 = typename M::v8;
   using v4 = typename M::v4;
+  constexpr bool RESIDUAL = ACT == kResidual || ACT == kResidualF32;
   constexpr int BN = 32 * NB;
   constexpr int kA = kBM * 128, kW = 64 * BN * 2, kStage = kA + kW; // a step of 64: 16 KiB of input rows, 16 or 12 of the weight
   constexpr int kRing = 5, kAhead = kRing - 1;
@@ -267,7 +269,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
   auto chunkCol = [&](int it) { return (it * 128 + khalf * 64 + lane) % kChunks; };
   auto chunkOffset = [&](int it) { return nw + 8 * chunkCol(it) < N ? (uint32_t)(chunkRow(it) * N * 2 + chunkCol(it) * 16) : 0x40000000u; };
   u32x4 rraw[kMine];
-  if (ACT == kResidual) { // on its way under the last matrix instructions
+  if (RESIDUAL) { // on its way under the last matrix instructions
     const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(residual + partAt), 0, partBytes, 0x00020000);
 #pragma unroll
     for (int it = 0; it < kMine; it++) rraw[it] = __builtin_amdgcn_raw_buffer_load_b128(rows, chunkOffset(it), 0, 0);
@@ -294,7 +296,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
         for (int i = 0; i < 4; i++) x[i] = khalf ? acc[nb][mb][4 * g + i] : acc[nb][mb][8 + 4 * g + i];
         *slot(mover, (nb * MB + mb) * 2 + g) = x;
       }
-  if (ACT == kResidual) {
+  if (RESIDUAL) {
 #pragma unroll
     for (int it = 0; it < kMine; it++) { // (8-byte accesses: the staging stride is no multiple of 16 bytes)
       uint16_t *p = &stage[chunkRow(it) * kOutStride + 8 * chunkCol(it)];
@@ -320,10 +322,16 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
           continue;
         }
         uint16_t *p = &stage[row * kOutStride + col];
-        if (ACT == kResidual) {
+        if (RESIDUAL) {
           const v4 r = *reinterpret_cast<const v4 *>(p);
 #pragma unroll
           for (int i = 0; i < 4; i++) x[i] += M::widen(r[i]);
+        }
+        if (ACT == kResidualF32) {
+#pragma unroll
+          for (int i = 0; i < 4; i++) x[i] = M::widen(M::narrow(x[i]));
+          if (mw + row < M_ && nw + col < N) *reinterpret_cast<float4v *>(reinterpret_cast<float *>(out) + (size_t)(mw + row) * N + nw + col) = x;
+          continue;
         }
         v4 o;
 #pragma unroll
@@ -334,7 +342,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
         }
         *reinterpret_cast<v4 *>(p) = o;
       }
-  if (ACT == kPartial) return;
+  if (ACT == kPartial || ACT == kResidualF32) return;
   __syncthreads();
   const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(out + partAt, 0, partBytes, 0x00020000);
 #pragma unroll
@@ -380,6 +388,21 @@ void gemmRound(DType dt, const void *in, const void *weight, const void *bias, c
   if (N % 8 || K % 8 || (K % 64 && K * N >= int64_t(1) << 30) || (act != ACT_NONE && residual) || (width != 96 && width != 128)) fail("gemmRound: internal dispatch error");
   if (dt == DType::F16) launchWidth<_Float16>(in, weight, bias, residual, out, M, N, K, act, width, stream);
   else launchWidth<bf16_t>(in, weight, bias, residual, out, M, N, K, act, width, stream);
+}
+
+void gemmRoundResidualF32(const void *in, const void *weight, const void *bias, const void *residual, float *out, int64_t M, int64_t N,
+                          int64_t K, int width, hipStream_t stream) {
+  if (N % 8 || K % 8 || (K % 64 && K * N >= int64_t(1) << 30) || !residual || (width != 96 && width != 128)) fail("gemmRound: internal dispatch error");
+  const int tilesM = (int)((M + kBM - 1) / kBM), tilesN = (int)((N + width - 1) / width);
+  auto go = [&](auto *kernel) {
+    launchKernel(kernel, dim3((unsigned)(tilesM * tilesN)), dim3(kThreads), stream, static_cast<const uint16_t *>(in), static_cast<const uint16_t *>(weight),
+        static_cast<const uint16_t *>(bias), static_cast<const uint16_t *>(residual), reinterpret_cast<uint16_t *>(out), (int)N, (int)K, tilesN, tilesM, (int)M);
+  };
+  if (width == 128 && K % 64) go(gemm_round_kernel<_Float16, kResidualF32, 4, true>);
+  else if (width == 128) go(gemm_round_kernel<_Float16, kResidualF32, 4, false>);
+  else if (K % 64) go(gemm_round_kernel<_Float16, kResidualF32, 3, true>);
+  else go(gemm_round_kernel<_Float16, kResidualF32, 3, false>);
+  MGPU_CHECK_LAUNCH("gemm_round_kernel");
 }
 
 void gemmRoundPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, int width, int parts,

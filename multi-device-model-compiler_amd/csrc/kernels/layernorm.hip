@@ -11,9 +11,12 @@
 // Rows wider than a wavefront can hold live in the registers of a whole block
 // (layernorm_block_kernel); rows beyond 256 x 16 vectors and rows shorter than one vector
 // take the general block-per-row kernel.
+#include "cast_table.hpp"
 #include "common.hpp"
 #include "mgpu_ops_internal.hpp"
 #include "types.hpp"
+
+#include <algorithm>
 
 namespace mgpu {
 
@@ -60,9 +63,10 @@ struct RowVectors {
 // (VPL of them, the last ones predicated off when the row is shorter; kFull
 // says that the row fills all of them, which removes every predicate and with
 // it the branches that would sit between the loads).
-template <typename T, int LANES, int VPL, bool RESIDUAL, RowShape SHAPE>
+// TO: the result's type, T or (whole vectors) float, which holds the result as rounded to T.
+template <typename T, int LANES, int VPL, bool RESIDUAL, RowShape SHAPE, typename TO = T>
 __global__ __launch_bounds__(256) void layernorm_rows_kernel(
-    const T *__restrict__ input, const T *__restrict__ gamma, const T *__restrict__ beta, T *__restrict__ normed,
+    const T *__restrict__ input, const T *__restrict__ gamma, const T *__restrict__ beta, TO *__restrict__ normed,
     int m, int nArg, int rowStep, float eps, const T *__restrict__ residual, T *__restrict__ sumOut) {
   // Argument order: the first 14 dwords are preloaded into SGPRs, and what the path to the
   // first row load needs comes first; rowStep (rows per trip of the grid) stands in for
@@ -152,7 +156,7 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
     // (4096, 768) 3.93 -> 3.80 us, (262144, 768) fp32 266 -> 263.5 us, the fp32 headline unchanged.
     const float rstd = __builtin_amdgcn_rsqf(var + eps);
 
-    T *yr = normed + (size_t)row * n;
+    TO *yr = normed + (size_t)row * n;
     T *sr = (RESIDUAL && sumOut) ? sumOut + (size_t)row * n : nullptr;
 #pragma unroll
     for (int k = 0; k < VPL; k++) {
@@ -172,7 +176,15 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
         }
 #pragma unroll
         for (int e = 0; e < VEC; e++) y[e] = (x[k][e] - mean) * rstd * g[e] + b[e];
-        Rows::store(Tr::pack(y), yr, k == VPL - 1, v, n);
+        if constexpr (std::is_same<T, TO>::value) {
+          Rows::store(Tr::pack(y), yr, k == VPL - 1, v, n);
+        } else {
+          static_assert(!Rows::kRagged && std::is_same<TO, float>::value, "whole vectors of floats");
+          Tr::unpack(Tr::pack(y), y);
+#pragma unroll
+          for (int q = 0; q < VEC / 4; q++)
+            __builtin_nontemporal_store(f32x4{y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]}, reinterpret_cast<f32x4 *>(yr) + v * (VEC / 4) + q);
+        }
       }
     }
   }
@@ -186,11 +198,8 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(
 // bits.  Lane l of a group holds the 8-element vectors l, l + LANES, ... (two
 // 16-byte loads each).
 template <typename T, int LANES, int VPL, bool FULL>
-__global__ __launch_bounds__(256) void layernorm_cast_rows_kernel(const float *__restrict__ input,
-                                                                  const T *__restrict__ gamma,
-                                                                  const T *__restrict__ beta, T *__restrict__ castOut,
-                                                                  T *__restrict__ normed, int m, int nArg, int rowStep,
-                                                                  float eps) {
+__device__ __forceinline__ void castNormRows(const float *__restrict__ input, const T *__restrict__ gamma, const T *__restrict__ beta,
+                                             T *__restrict__ castOut, T *__restrict__ normed, int m, int nArg, int rowStep, float eps) {
   using Tr = ElemTraits<T>;
   constexpr int VEC = Tr::kVec; // 8
   constexpr int GROUPS = 256 / LANES;
@@ -282,6 +291,24 @@ __global__ __launch_bounds__(256) void layernorm_cast_rows_kernel(const float *_
       }
     }
   }
+}
+
+template <typename T, int LANES, int VPL, bool FULL>
+__global__ __launch_bounds__(256) void layernorm_cast_rows_kernel(const float *__restrict__ input, const T *__restrict__ gamma,
+                                                                  const T *__restrict__ beta, T *__restrict__ castOut,
+                                                                  T *__restrict__ normed, int m, int n, int rowStep, float eps) {
+  castNormRows<T, LANES, VPL, FULL>(input, gamma, beta, castOut, normed, m, n, rowStep, eps);
+}
+
+// The same in the first rowBlocks blocks, a layer's weights in the others: a launch less (2 x 93 tokens of 768 40.0 -> 35.9 us with
+// the fp32 result from the last kernel's epilogue), and the end of the one hides behind the other (8 x 512 of 2048 262 -> 257).
+template <typename T, int LANES, int VPL, bool FULL>
+__global__ __launch_bounds__(256) void layernorm_cast_weights_kernel(const float *__restrict__ input, const T *__restrict__ gamma,
+                                                                     const T *__restrict__ beta, T *__restrict__ castOut,
+                                                                     T *__restrict__ normed, int m, int n, int rowBlocks, float eps,
+                                                                     CastTable weights) {
+  if (blockIdx.x < (unsigned)rowBlocks) castNormRows<T, LANES, VPL, FULL>(input, gamma, beta, castOut, normed, m, n, rowBlocks * (256 / LANES), eps);
+  else castTableBlock(weights, blockIdx.x - (unsigned)rowBlocks);
 }
 
 // Rows too wide for one wavefront's registers: the same scheme with a whole
@@ -601,11 +628,36 @@ void layerNorm(DType dt, const void *input, const void *residual, const void *ga
   }
 }
 
-bool castLayerNormF32ToF16(const float *input, const void *gamma, const void *beta, void *castOut, void *normed,
-                           float eps, int m, int n, hipStream_t stream) {
-  if (m < 0 || n < 0) fail("castLayerNorm: negative shape");
-  if (m == 0 || n == 0) return true;
-  if (!input || !gamma || !beta || !castOut || !normed) fail("castLayerNorm: null pointer");
+bool layerNormF16ToF32(const void *input, const void *residual, const void *gamma, const void *beta, float *normed, float eps, int m, int n,
+                       hipStream_t stream) {
+  const int nvec = n / 8;
+  if (n % 8 || nvec > 64 * kMaxVPL || !aligned16(input) || !aligned16(residual) || !aligned16(gamma) || !aligned16(beta) || !aligned16(normed))
+    return false;
+  // (lane groups as in layerNormTyped)
+  const int lanes = nvec <= 16 * 4 ? 16 : nvec <= 32 * 4 ? 32 : 64;
+  const int vpl = (nvec + lanes - 1) / lanes;
+  const bool full = nvec == lanes * vpl;
+  const int64_t blocks = std::min<int64_t>(((int64_t)m * lanes + 255) / 256, kMaxStreamBlocks);
+  auto launch = [&](auto *kernel) {
+    launchKernel(kernel, dim3((unsigned)blocks), dim3(256), stream, static_cast<const _Float16 *>(input), static_cast<const _Float16 *>(gamma),
+        static_cast<const _Float16 *>(beta), normed, m, n, (int)(blocks * (256 / lanes)), eps, static_cast<const _Float16 *>(residual), nullptr);
+  };
+#define MGPU_LN_F32(L, V)                                                                                                \
+  if (lanes == L && vpl == V) {                                                                                          \
+    if (full) launch(layernorm_rows_kernel<_Float16, L, V, true, RowShape::kFull, float>);                               \
+    else launch(layernorm_rows_kernel<_Float16, L, V, true, RowShape::kVectors, float>);                                 \
+  }
+  MGPU_LN_F32(16, 1) MGPU_LN_F32(16, 2) MGPU_LN_F32(16, 3) MGPU_LN_F32(16, 4)
+  MGPU_LN_F32(32, 3) MGPU_LN_F32(32, 4)
+  MGPU_LN_F32(64, 3) MGPU_LN_F32(64, 4) MGPU_LN_F32(64, 5) MGPU_LN_F32(64, 6) MGPU_LN_F32(64, 7) MGPU_LN_F32(64, 8)
+#undef MGPU_LN_F32
+  MGPU_CHECK_LAUNCH("layernorm_rows_kernel");
+  return true;
+}
+
+// (jobs: null, or a layer's weights to cast in the same launch)
+static bool castLayerNorm(CastJob *jobs, int count, const float *input, const void *gamma, const void *beta, void *castOut, void *normed,
+                          float eps, int m, int n, hipStream_t stream) {
   const int nvec = n / 8;
   if (n % 8 || nvec > 64 * kMaxVPL || !aligned16(input) || !aligned16(gamma) || !aligned16(beta) ||
       !aligned16(castOut) || !aligned16(normed))
@@ -620,14 +672,26 @@ bool castLayerNormF32ToF16(const float *input, const void *gamma, const void *be
   const auto *b = static_cast<const _Float16 *>(beta);
   auto *c = static_cast<_Float16 *>(castOut);
   auto *y = static_cast<_Float16 *>(normed);
-#define MGPU_LN_CAST(L, V)                                                                                     \
-  if (lanes == L && vpl == V) {                                                                                \
-    if (full)                                                                                                  \
-      launchKernel(layernorm_cast_rows_kernel<_Float16, L, V, true>, dim3((unsigned)blocks), dim3(256), stream,      \
-          input, g, b, c, y, m, n, (int)(blocks * (256 / L)), eps);                                            \
-    else                                                                                                       \
-      launchKernel(layernorm_cast_rows_kernel<_Float16, L, V, false>, dim3((unsigned)blocks), dim3(256), stream,     \
-          input, g, b, c, y, m, n, (int)(blocks * (256 / L)), eps);                                            \
+  CastTable table;
+  int64_t grid = blocks;
+  if (jobs) {
+    grid += castTable(jobs, count, table);
+    if (grid > 0x7fffffff) return false;
+  }
+  auto launch = [&](auto lanesTag, auto vplTag, auto fullTag) {
+    constexpr int L = decltype(lanesTag)::value, V = decltype(vplTag)::value;
+    constexpr bool FULL = decltype(fullTag)::value;
+    if (jobs)
+      launchKernel(layernorm_cast_weights_kernel<_Float16, L, V, FULL>, dim3((unsigned)grid), dim3(256), stream,
+          input, g, b, c, y, m, n, (int)blocks, eps, table);
+    else
+      launchKernel(layernorm_cast_rows_kernel<_Float16, L, V, FULL>, dim3((unsigned)grid), dim3(256), stream,
+          input, g, b, c, y, m, n, (int)(blocks * (256 / L)), eps);
+  };
+#define MGPU_LN_CAST(L, V)                                                                                                    \
+  if (lanes == L && vpl == V) {                                                                                               \
+    if (full) launch(std::integral_constant<int, L>(), std::integral_constant<int, V>(), std::true_type());                    \
+    else launch(std::integral_constant<int, L>(), std::integral_constant<int, V>(), std::false_type());                        \
   }
   MGPU_LN_CAST(16, 1) MGPU_LN_CAST(16, 2) MGPU_LN_CAST(16, 3) MGPU_LN_CAST(16, 4)
   MGPU_LN_CAST(32, 3) MGPU_LN_CAST(32, 4)
@@ -635,6 +699,19 @@ bool castLayerNormF32ToF16(const float *input, const void *gamma, const void *be
 #undef MGPU_LN_CAST
   MGPU_CHECK_LAUNCH("layernorm_cast_rows_kernel");
   return true;
+}
+
+bool castLayerNormF32ToF16(const float *input, const void *gamma, const void *beta, void *castOut, void *normed,
+                           float eps, int m, int n, hipStream_t stream) {
+  if (m < 0 || n < 0) fail("castLayerNorm: negative shape");
+  if (m == 0 || n == 0) return true;
+  if (!input || !gamma || !beta || !castOut || !normed) fail("castLayerNorm: null pointer");
+  return castLayerNorm(nullptr, 0, input, gamma, beta, castOut, normed, eps, m, n, stream);
+}
+
+bool castWeightsLayerNormF32ToF16(CastJob *jobs, int count, const float *input, const void *gamma, const void *beta, void *castOut,
+                                  void *normed, float eps, int m, int n, hipStream_t stream) {
+  return castLayerNorm(jobs, count, input, gamma, beta, castOut, normed, eps, m, n, stream);
 }
 
 } // namespace mgpu

@@ -19,16 +19,15 @@
 //    capture, so the graph owns its temporaries and a later eager call that
 //    grows (frees and replaces) the stream's arena cannot pull memory from
 //    under a graph that is still replayed;
-//  * one kernel casts all seven weight and bias arrays, on the caller's stream
+//  * one kernel casts all seven weight and bias arrays and the input, with its LayerNorm where that comes first, on the caller's stream
 //    (the reference casts each on a side stream; here the casts are bound by
 //    memory, so beside a GEMM they only slow it, and their launches and events
 //    were half of the host time of a small layer: 4096 x 2048 321 -> 289 us,
 //    240 x 768 112 -> 47 us); it writes K-major the weights whose GEMM is the
 //    library's, which has faster kernels for that layout.  The gamma = 1 /
 //    beta = 0 vectors are written once per model width, not per call;
-//  * the final fp16 -> fp32 cast runs after the last GEMM on the caller's
-//    stream (the reference issues it on the side stream without waiting for
-//    that GEMM: LLM.cu:136-141).
+//  * the final fp16 -> fp32 cast is the last GEMM's or LayerNorm's epilogue, and a kernel behind it only where that has none
+//    (the reference issues it on the side stream without waiting for that GEMM: LLM.cu:136-141).
 //
 // bertEncoderLayerF16 is the post-LN BERT encoder layer on fp16 tensors (GELU,
 // learned LayerNorm affine, optional key-padding lengths); the reference has
@@ -327,13 +326,7 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
       cachedReady[i] = cw.pending();
     }
   } else {
-    CastJob jobs[7];
-    for (int i = 0; i < 7; i++) {
-      Operand &op = ops[i];
-      op.half = arena.at(op.slot);
-      jobs[i] = CastJob{op.src, op.half, op.rows, op.cols ? op.cols : 1, op.cols && kMajor[op.group], false};
-    }
-    castWeightsF32ToF16(jobs, 7, stream);
+    for (Operand &op : ops) op.half = arena.at(op.slot);
   }
   auto join = [&](int group) {
     for (int i = 0; i < 7; i++)
@@ -349,6 +342,23 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
   } else { // under capture, first use of this width: the pair lives in the arena
     fillF16(arena.at(oGamma), d, 1.0f, stream);
     fillF16(arena.at(oBeta), d, 0.0f, stream);
+  }
+
+  // The casts: the weights' and, in the same launch, the input's - with its LayerNorm where that comes first and the width allows
+  // (fp16 copy of the input, the residual of the second LayerNorm, and its LayerNorm: one kernel where the width allows, else the
+  // reference's two).
+  {
+    CastJob jobs[8];
+    int count = 0;
+    if (!useCache)
+      for (const Operand &op : ops) jobs[count++] = CastJob{op.src, op.half, op.rows, op.cols ? op.cols : 1, op.cols && kMajor[op.group], false};
+    const bool fused = norm_first && (count ? castWeightsLayerNormF32ToF16(jobs, count, input, gamma, beta, arena.at(oX), arena.at(oLn), 1e-5f, (int)M, (int)d, stream)
+                                            : castLayerNormF32ToF16(input, gamma, beta, arena.at(oX), arena.at(oLn), 1e-5f, (int)M, (int)d, stream));
+    if (!fused) {
+      jobs[count++] = CastJob{input, arena.at(oX), M, d, false, false};
+      castWeightsF32ToF16(jobs, count, stream);
+      if (norm_first) layerNorm(DType::F16, arena.at(oX), nullptr, gamma, beta, nullptr, arena.at(oLn), 1e-5f, (int)M, (int)d, stream);
+    }
   }
 
   // LN(in . w + bias + residual), the rounded sum to sumOut when it is not null.  Where the sum is wanted and gemm_wide serves the
@@ -373,13 +383,6 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
 
   if (norm_first) {
     // y = x + proj(attention(LN(x))), out = y + ffn(LN(y))
-    // fp16 copy of the input (the residual of the second LayerNorm) and its
-    // LayerNorm: one kernel where the width allows, else the reference's two.
-    if (!castLayerNormF32ToF16(input, gamma, beta, arena.at(oX), arena.at(oLn), 1e-5f, (int)M, (int)d, stream)) {
-      castF32ToF16(arena.at(oX), input, M * d, stream);
-      layerNorm(DType::F16, arena.at(oX), nullptr, gamma, beta, nullptr, arena.at(oLn), 1e-5f, (int)M, (int)d, stream);
-    }
-
     join(0);
     matmulEx(DType::F16, arena.at(oLn), wqkvH, nullptr, arena.at(oQkv), nullptr, M, 3 * d,
              d, false, ACT_NONE, false, stream, kMajor[0]);
@@ -402,10 +405,8 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
       arena.release(stream);
       return;
     }
-    // (or from gemm_wide's accumulators: 4096 x 2048 x 2048 42.2 + 11.2 for the cast behind it -> 40.5 us)
-    const int wide = kMajor[3] || ffn % 64 || reinterpret_cast<uintptr_t>(output) % 16 ? 0 : gemmWideWidth(DType::F16, M, d, ffn, ACT_NONE, true);
-    if (wide) {
-      gemmWideResidualF32(arena.at(oF), w2H, b2H, arena.at(oY), output, M, d, ffn, wide, stream);
+    // (or from the product's accumulators: 4096 x 2048 x 2048 42.2 + 11.2 for the cast behind it -> 40.5 us)
+    if (matmulResidualF32(arena.at(oF), w2H, b2H, arena.at(oY), output, M, d, ffn, kMajor[3], stream)) {
       arena.release(stream);
       return;
     }
@@ -416,7 +417,6 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
     // flag, Ops.h:43-48, and never reads it):  h = LN(x + proj(attention(x))),
     // out = LN(h + ffn(h)), both LayerNorms with gamma = 1 / beta = 0 at eps 1e-5 like the
     // pre-LN ones, every intermediate stored in fp16 where the pre-LN path stores it.
-    castF32ToF16(arena.at(oX), input, M * d, stream);
     join(0);
     matmulEx(DType::F16, arena.at(oX), wqkvH, nullptr, arena.at(oQkv), nullptr, M, 3 * d,
              d, false, ACT_NONE, false, stream, kMajor[0]);
@@ -435,7 +435,12 @@ void decodingContextLayer(float *input, float *qkv, float *gemm_weight, float *g
       arena.release(stream);
       return;
     }
-    productAddNorm(ffn2Plan, arena.at(oF), w2H, b2H, ffn, kMajor[3], arena.at(oY), nullptr, arena.at(oOut));
+    matmulEx(DType::F16, arena.at(oF), w2H, b2H, arena.at(oProj), nullptr, M, d, ffn, true, ACT_NONE, false, stream, kMajor[3]);
+    if (layerNormF16ToF32(arena.at(oProj), arena.at(oY), gamma, beta, output, 1e-5f, (int)M, (int)d, stream)) {
+      arena.release(stream);
+      return;
+    }
+    layerNorm(DType::F16, arena.at(oProj), arena.at(oY), gamma, beta, nullptr, arena.at(oOut), 1e-5f, (int)M, (int)d, stream);
   }
 
   castF16ToF32(output, arena.at(oOut), M * d, stream);

@@ -45,6 +45,9 @@ void castBF16ToF32(float *dst, const void *src, size_t size, hipStream_t stream)
 // dst[c][r] = src[r][c] of a row-major rows x cols matrix (fp32 -> fp16; any 16-bit type, bit for bit)
 void transposeCastF32ToF16(void *dst, const float *src, int64_t rows, int64_t cols, hipStream_t stream);
 void transpose16(void *dst, const void *src, int64_t rows, int64_t cols, hipStream_t stream);
+// LayerNorm of the sum of fp16 rows, rounded to fp16, in fp32 (m, n > 0); false, and nothing launched, for rows that are not whole aligned vectors or too wide.
+bool layerNormF16ToF32(const void *input, const void *residual, const void *gamma, const void *beta, float *normed, float eps, int m, int n,
+                       hipStream_t stream);
 // fp32 arrays to fp16, up to kMaxCastJobs of them in one launch; kMajor: dst[c][r] = src[r][c].
 struct CastJob {
   const float *src;
@@ -55,6 +58,9 @@ struct CastJob {
 };
 constexpr int kMaxCastJobs = 8;
 void castWeightsF32ToF16(CastJob *jobs, int count, hipStream_t stream);
+// The same and castLayerNormF32ToF16 (m, n > 0) in one launch; false, and nothing launched, where that one would be.
+bool castWeightsLayerNormF32ToF16(CastJob *jobs, int count, const float *input, const void *gamma, const void *beta, void *castOut,
+                                  void *normed, float eps, int m, int n, hipStream_t stream);
 void fillF16(void *dst, size_t count, float value, hipStream_t stream);
 void fillI32(int32_t *dst, size_t count, int32_t value, hipStream_t stream);
 
@@ -72,6 +78,10 @@ void gemmDeinit();
 void matmulEx(DType dt, const void *input, const void *weight, const void *bias, void *output,
               const void *residual, int64_t M, int64_t N, int64_t K, bool hasBias, int act,
               bool hasResidual, hipStream_t stream, bool weightKMajor = false);
+// fp16 operands, in . weight + bias + residual in fp32 on the kernel that matmulEx would run (rounded to fp16 on the way, except by
+// gemm_wide); false, and nothing launched, where that one has no such epilogue.
+bool matmulResidualF32(const void *input, const void *weight, const void *bias, const void *residual, float *output, int64_t M, int64_t N,
+                       int64_t K, bool weightKMajor, hipStream_t stream);
 // Which kernel matmulEx runs a product on (K, N > 0; 16-byte aligned operands), and the width at which gemm_wide serves it, 0 where
 // it does not.
 enum class GemmKernel { Library, Mfma, KSplit, F32Small, Wide, Round };
@@ -122,6 +132,8 @@ int gemmRoundWidth(DType dt, const void *in, const void *weight, const void *bia
                    int64_t K);
 void gemmRound(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
                int64_t K, int act, int width, hipStream_t stream);
+void gemmRoundResidualF32(const void *in, const void *weight, const void *bias, const void *residual, float *out, int64_t M, int64_t N, int64_t K,
+                          int width, hipStream_t stream);
 void gemmRoundPartialF16(const void *in, const void *weight, float *planes, int64_t M, int64_t N, int64_t K, int width, int parts,
                          hipStream_t stream);
 
@@ -133,6 +145,8 @@ bool gemmKSplitSupports(DType dt, const void *in, const void *weight, const void
                         int64_t N, int64_t K);
 void gemmKSplit(DType dt, const void *in, const void *weight, const void *bias, const void *residual, void *out, int64_t M, int64_t N,
                 int64_t K, int act, KSplitTile tile, bool weightKMajor, hipStream_t stream);
+void gemmKSplitResidualF32(const void *in, const void *weight, const void *bias, const void *residual, float *out, int64_t M, int64_t N,
+                           int64_t K, KSplitTile tile, bool weightKMajor, hipStream_t stream);
 // A GEMM whose reduction is split over blocks: `parts` fp32 planes [M, N] of partial sums (16-byte aligned), added up by
 // one of the kernels of partial_sums.hip.  gemmPartialPlan: parts = 0 where the shape is better served whole.
 struct PartialPlan {
