@@ -28,8 +28,8 @@ int deviceComputeUnits() {
 }
 
 // dHead: head dimension in memory; D: the tile geometry it runs in (dHead == D, or a
-// smaller multiple of 8 with the PAD instantiation).
-template <typename T, int D, int NQ, bool PAD>
+// smaller multiple of 8, up to USED, with the PAD instantiation).
+template <typename T, int D, int NQ, bool PAD, int USED = D>
 void launch(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqlens, void *out, int B, int S, int H,
             int dHead, float scale, bool causal, hipStream_t stream) {
   constexpr int BM = 128 * NQ;
@@ -61,7 +61,7 @@ void launch(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqlens, v
     const bool halves = causal ? S >= 512 && !pair && 2 * blocks <= cus * (nQB >= 12 ? 4 : nQB >= 8 ? 3 : 2)
                                : S >= (D == 256 ? 768 : 512) && blocks <= cus;
     if (halves) {
-      auto *kernel = causal ? fmha_fwd_kernel<T, D, 1, true, false, PAD, true> : fmha_fwd_kernel<T, D, 1, false, false, PAD, true>;
+      auto *kernel = causal ? fmha_fwd_kernel<T, D, 1, true, false, PAD, true, false, USED> : fmha_fwd_kernel<T, D, 1, false, false, PAD, true, false, USED>;
       launchKernel(kernel, grid, dim3(512), stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
       MGPU_CHECK_LAUNCH("fmha_fwd_kernel");
       return;
@@ -70,13 +70,13 @@ void launch(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqlens, v
   if (causal) {
     // (the causal kernel exists with one 32-query block per wavefront only)
     if constexpr (NQ == 1)
-      launchKernel(fmha_fwd_kernel<T, D, NQ, true, false, PAD>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
+      launchKernel(fmha_fwd_kernel<T, D, NQ, true, false, PAD, false, false, USED>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
     else
       fail("fusedMHA: internal dispatch error");
   } else if (D == 128 && S <= 64 && (PAD || blocks <= deviceComputeUnits())) { // one tile of keys (the kernel has the times)
-    launchKernel(fmha_fwd_kernel<T, D, NQ, false, false, PAD, false, D == 128>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
+    launchKernel(fmha_fwd_kernel<T, D, NQ, false, false, PAD, false, D == 128, USED>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
   } else {
-    launchKernel(fmha_fwd_kernel<T, D, NQ, false, false, PAD>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
+    launchKernel(fmha_fwd_kernel<T, D, NQ, false, false, PAD, false, false, USED>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, order, (int)blocks, dHead, nullptr);
   }
   MGPU_CHECK_LAUNCH("fmha_fwd_kernel");
 }
@@ -97,8 +97,16 @@ void launchForHeadDim(const void *qkv, const int32_t *seqlens, const int32_t *cu
   else if (dHead == 64) launch<T, 64, 1, false>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
   else if (dHead == 128) launch<T, 128, 1, false>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
   else if (dHead == 256) launch<T, 256, 1, false>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
+  // Sizes in between go in classes, each without the matrix steps that only filler would feed.  The lines lie where a step of 16 or 32
+  // saves most at sizes in use (us, the whole geometry / the class: 32 of 64 20.6 / 16.2 at b15 s934 h4, 80 of 128 83.6 / 66.9 at b9 s1351 h8, 160 of
+  // 256 111 / 82 at b8 s535 h32; over 150 launches 32: 0.87 of the time, 40: 0.96, 72 and 80: 0.93, 96: 0.94, 144 and 160: 0.87).
+  else if (dHead <= 32) launch<T, 64, 1, true, 32>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
+  else if (dHead <= 48) launch<T, 64, 1, true, 48>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
   else if (dHead < 64) launch<T, 64, 1, true>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
+  else if (dHead <= 80) launch<T, 128, 1, true, 80>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
+  else if (dHead <= 96) launch<T, 128, 1, true, 96>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
   else if (dHead < 128) launch<T, 128, 1, true>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
+  else if (dHead <= 160) launch<T, 256, 1, true, 160>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
   else launch<T, 256, 1, true>(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
 }
 

@@ -135,9 +135,10 @@ constexpr float kSumFloor = 0.015625f;
 // elements long; a lane whose 16-byte chunk of a K or V row lies beyond dHead
 // fetches chunk 0 of that row instead (in bounds, finite wherever the row is),
 // Q is zero there, so the scores do not see the K filler, and the O^T rows the V
-// filler feeds are never stored.
+// filler feeds are never stored.  USED: the k-steps and O^T rows that hold nothing but
+// filler are left out, dHead <= USED.
 // SHORT: no sequence is longer than a tile of keys (kLoadsBehindScores has the reason).
-template <typename T, int D, int NQ, bool CAUSAL, bool TRACE = false, bool PAD = false, bool HALVES = false, bool SHORT = false>
+template <typename T, int D, int NQ, bool CAUSAL, bool TRACE = false, bool PAD = false, bool HALVES = false, bool SHORT = false, int USED = D>
 __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) ? 3 : 2) void fmha_fwd_kernel(const uint16_t *__restrict__ qkv,
                                                               const int32_t *__restrict__ seqlens,
                                                               const int32_t *__restrict__ cuSeqlens,
@@ -157,6 +158,7 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
   using v8 = typename M::v8;
   using v4 = typename M::v4;
   using G = Geo<D>;
+  constexpr int DC = (USED + 15) / 16, DB = (USED + 31) / 32, KF = DC < G::KF ? DC : G::KF, VF = DB < G::VF ? DB : G::VF;
   constexpr int BM = 128 * NQ;
   constexpr int kBN = G::kBN;
   constexpr int kStages = G::kStages, kTileBytes = G::kTileBytes, kStageBytes = G::kStageBytes, LPW = G::LPW;
@@ -352,13 +354,13 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
     if (t < nkt) issueTile(t);
 
   // Q as the B operand: lane (query l32, k-slots = d 16c + 8hl .. +7).
-  v8 qf[NQ][G::DC];
+  v8 qf[NQ][DC];
 #pragma unroll
   for (int qi = 0; qi < NQ; qi++) {
     int row = q0 + qi * 32 + l32;
     row = row < rows ? row : rows - 1;
 #pragma unroll
-    for (int c = 0; c < G::DC; c++) {
+    for (int c = 0; c < DC; c++) {
       if (!PAD || 2 * c + hl < validChunks)
         qf[qi][c] = *reinterpret_cast<const v8 *>(qbase + (size_t)row * tokBytes + (16 * c + 8 * hl) * 2);
       else
@@ -381,20 +383,20 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
     return (uint32_t)((4 * half + j) * G::rowBytes + chunk * 16 + 8 * (r % 2));
   };
   // (as with the movers' offsets: kept in registers, or recomputed per tile at D = 256)
-  uint32_t kfrag[G::KF], vfrag[G::VF];
+  uint32_t kfrag[KF], vfrag[VF];
 #pragma unroll
-  for (int c = 0; c < G::KF; c++) kfrag[c] = kRecomputeOffsets ? 0u : kfragOf(c, l32, hl);
+  for (int c = 0; c < KF; c++) kfrag[c] = kRecomputeOffsets ? 0u : kfragOf(c, l32, hl);
 #pragma unroll
-  for (int db = 0; db < G::VF; db++) vfrag[db] = kRecomputeOffsets ? 0u : vfragOf(db, lane);
+  for (int db = 0; db < VF; db++) vfrag[db] = kRecomputeOffsets ? 0u : vfragOf(db, lane);
 
-  f32x16 accO[NQ][G::DB];
+  f32x16 accO[NQ][DB];
   float m_run[NQ], l_run[NQ]; // stale reference maximum (raw score units), this lane's share of the running sum
 #pragma unroll
   for (int qi = 0; qi < NQ; qi++) {
     m_run[qi] = 0.0f;
     l_run[qi] = 0.0f;
 #pragma unroll
-    for (int db = 0; db < G::DB; db++)
+    for (int db = 0; db < DB; db++)
 #pragma unroll
       for (int i = 0; i < 16; i++) accO[qi][db][i] = 0.0f;
   }
@@ -410,7 +412,7 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
 #pragma unroll
     for (int qi = 0; qi < NQ; qi++)
 #pragma unroll
-      for (int c = 0; c < G::DC; c++) asm volatile("" ::"v"(qf[qi][c]));
+      for (int c = 0; c < DC; c++) asm volatile("" ::"v"(qf[qi][c]));
   }
   // Where the loads of the next tile go out: right behind the barrier they keep a wavefront from its score MFMAs until the
   // address path has taken all of them (16 cycles an instruction, 8 of every wavefront at head_dim 128); behind the scores the wait
@@ -458,14 +460,14 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
 
     // Operand pointers in the LDS address space: one add per tile, the rest
     // of every address is an instruction immediate.
-    const lds_u8 *kp[G::KF], *vp[G::VF];
+    const lds_u8 *kp[KF], *vp[VF];
     int ln = lane;
     if (kRecomputeOffsets) asm volatile("" : "+v"(ln));
 #pragma unroll
-    for (int c = 0; c < G::KF; c++)
+    for (int c = 0; c < KF; c++)
       kp[c] = (const lds_u8 *)(uintptr_t)(ldsBase + stageOff + (kRecomputeOffsets ? kfragOf(c, ln % 32, ln / 32) : kfrag[c]));
 #pragma unroll
-    for (int db = 0; db < G::VF; db++)
+    for (int db = 0; db < VF; db++)
       vp[db] = (const lds_u8 *)(uintptr_t)(ldsBase + stageOff + kTileBytes + (kRecomputeOffsets ? vfragOf(db, ln) : vfrag[db]));
 
     if (TRACE) {
@@ -480,8 +482,8 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
 #pragma unroll
       for (int kb = 0; kb < G::KB; kb++) {
 #pragma unroll
-        for (int c = 0; c < G::DC; c++) {
-          const v8 a = *reinterpret_cast<const v8 __attribute__((address_space(3))) *>(kp[c % G::KF] + (c / G::KF) * 256 +
+        for (int c = 0; c < DC; c++) {
+          const v8 a = *reinterpret_cast<const v8 __attribute__((address_space(3))) *>(kp[c % KF] + (c / KF) * 256 +
                                                                                         kb * 32 * G::rowBytes);
 #pragma unroll
           for (int qi = 0; qi < NQ; qi++) {
@@ -559,7 +561,7 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
         m_run[qi] = m_new;
         l_run[qi] *= alpha;
 #pragma unroll
-        for (int db = 0; db < G::DB; db++)
+        for (int db = 0; db < DB; db++)
 #pragma unroll
           for (int i = 0; i < 16; i++) accO[qi][db][i] *= alpha;
         lsum = makeP(m_new);
@@ -575,12 +577,12 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
     // ---- O^T += V^T P^T ----------------------------------------------------
     __builtin_amdgcn_s_setprio(2);
 #pragma unroll
-    for (int db = 0; db < G::DB; db++) {
+    for (int db = 0; db < DB; db++) {
 #pragma unroll
       for (int kb = 0; kb < G::KB; kb++) {
 #pragma unroll
         for (int m = 0; m < 2; m++) {
-          const lds_u8 *p = vp[db % G::VF] + (db / G::VF) * 256 + (32 * kb + 16 * m) * G::rowBytes;
+          const lds_u8 *p = vp[db % VF] + (db / VF) * 256 + (32 * kb + 16 * m) * G::rowBytes;
           const v4 lo = M::readTr(p);                    // k-slots 0..3: keys +4hl+0..3
           const v4 hi = M::readTr(p + 8 * G::rowBytes);  // k-slots 4..7: keys +8+4hl+0..3
           const v8 a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -591,7 +593,7 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
     }
     __builtin_amdgcn_s_setprio(0);
     if (TRACE) {
-      asm volatile("" ::"v"(accO[NQ - 1][G::DB - 1][15]));
+      asm volatile("" ::"v"(accO[NQ - 1][DB - 1][15]));
       cPV += clock64() - tMark;
     }
   }
@@ -604,7 +606,7 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
     l_run[0] = halves_sum(l_run[0]);
     if (half == 1) {
 #pragma unroll
-      for (int db = 0; db < G::DB; db++)
+      for (int db = 0; db < DB; db++)
 #pragma unroll
         for (int i = 0; i < 16; i++) mine[64 * (16 * db + i)] = accO[0][db][i];
       mine[64 * (D / 2)] = m_run[0];
@@ -617,7 +619,7 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
       const float e0 = __builtin_amdgcn_exp2f((m0 - m) * scale_log2e), e1 = l1 != 0.0f ? __builtin_amdgcn_exp2f((m1 - m) * scale_log2e) : 0.0f;
       l_run[0] = l_run[0] * e0 + l1 * e1;
 #pragma unroll
-      for (int db = 0; db < G::DB; db++)
+      for (int db = 0; db < DB; db++)
 #pragma unroll
         for (int i = 0; i < 16; i++) accO[0][db][i] = accO[0][db][i] * e0 + mine[64 * (16 * db + i)] * e1;
     }
@@ -631,7 +633,7 @@ __global__ __launch_bounds__(HALVES ? 512 : 256, (CAUSAL && D == 64 && !HALVES) 
     const float l = HALVES ? l_run[qi] : halves_sum(l_run[qi]);
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
-    for (int db = 0; db < G::DB; db++)
+    for (int db = 0; db < DB; db++)
 #pragma unroll
       for (int g = 0; g < 4; g++) {
         v4 o;

@@ -37,7 +37,8 @@ template <int D> struct SplitGeo {
   static_assert(kLdsBytes <= 160 * 1024, "LDS of a CU");
 };
 
-template <typename T, int D, int QG, bool CAUSAL, bool PAD>
+// (PAD, USED: see fmha_kernel.hpp)
+template <typename T, int D, int QG, bool CAUSAL, bool PAD, int USED>
 __global__ __launch_bounds__(64 * SplitGeo<D>::W, 1) void fmha_split_kernel(const uint16_t *__restrict__ qkv,
                                                                             const int32_t *__restrict__ seqlens,
                                                                             const int32_t *__restrict__ cuSeqlens,
@@ -48,6 +49,7 @@ __global__ __launch_bounds__(64 * SplitGeo<D>::W, 1) void fmha_split_kernel(cons
   using v4 = typename M::v4;
   using G = Geo<D>;
   using SG = SplitGeo<D>;
+  constexpr int DC = (USED + 15) / 16, DB = (USED + 31) / 32, KF = DC < G::KF ? DC : G::KF, VF = DB < G::VF ? DB : G::VF;
   constexpr int W = SG::W, KS = W / QG, R = SG::R, LPT = SG::LPT, kTileBytes = SG::kTileBytes;
   const int kD = PAD ? dHead : D;
   const int validChunks = PAD ? dHead / 8 : G::CPR;
@@ -89,12 +91,12 @@ __global__ __launch_bounds__(64 * SplitGeo<D>::W, 1) void fmha_split_kernel(cons
   const int n = tiles > ks ? (tiles - ks + KS - 1) / KS : 0;
 
   // Q as the B operand: lane (query l32, k-slots = d 16c + 8hl .. +7).
-  v8 qf[G::DC];
+  v8 qf[DC];
   {
     int row = q0 + l32;
     row = row < rows ? row : rows - 1;
 #pragma unroll
-    for (int c = 0; c < G::DC; c++) {
+    for (int c = 0; c < DC; c++) {
       if (!PAD || 2 * c + hl < validChunks)
         qf[c] = *reinterpret_cast<const v8 *>(qbase + (size_t)row * tokBytes + (16 * c + 8 * hl) * 2);
       else
@@ -136,25 +138,25 @@ __global__ __launch_bounds__(64 * SplitGeo<D>::W, 1) void fmha_split_kernel(cons
     }
 
   // ---- operand addresses inside a tile, as in fmha_kernel.hpp ---------------------------------------------
-  uint32_t kfrag[G::KF], vfrag[G::VF];
+  uint32_t kfrag[KF], vfrag[VF];
 #pragma unroll
-  for (int c = 0; c < G::KF; c++) kfrag[c] = (uint32_t)(l32 * G::rowBytes + (((2 * c + hl) ^ G::kSwz(l32)) * 16));
+  for (int c = 0; c < KF; c++) kfrag[c] = (uint32_t)(l32 * G::rowBytes + (((2 * c + hl) ^ G::kSwz(l32)) * 16));
 #pragma unroll
-  for (int db = 0; db < G::VF; db++) {
+  for (int db = 0; db < VF; db++) {
     const int g = lane / 16, L = lane % 16, r = L % 4, j = L / 4;
     const int chunk = (4 * db + 2 * (g % 2) + r / 2) ^ G::vSwz(4 * hl + j);
     vfrag[db] = (uint32_t)((4 * hl + j) * G::rowBytes + chunk * 16 + 8 * (r % 2));
   }
 
-  f32x16 accO[G::DB];
+  f32x16 accO[DB];
   float m_run = 0.0f, l_run = 0.0f; // reference maximum (raw score units), this lane's share of the row sum
 #pragma unroll
-  for (int db = 0; db < G::DB; db++)
+  for (int db = 0; db < DB; db++)
 #pragma unroll
     for (int i = 0; i < 16; i++) accO[db][i] = 0.0f;
   // (a use of every Q register here keeps the wait for them out of the loop)
 #pragma unroll
-  for (int c = 0; c < G::DC; c++) asm volatile("" ::"v"(qf[c]));
+  for (int c = 0; c < DC; c++) asm volatile("" ::"v"(qf[c]));
 
   // The loads are counted by hand.  In flight, in order: K j, V j, K j+1, V j+1, ... up to tile j+R-1; the K of tile j+R
   // follows the scores of tile j, its V the product with V of tile j.
@@ -169,9 +171,9 @@ __global__ __launch_bounds__(64 * SplitGeo<D>::W, 1) void fmha_split_kernel(cons
 #pragma unroll
     for (int i = 0; i < 16; i++) accS[i] = 0.0f;
 #pragma unroll
-    for (int c = 0; c < G::DC; c++) {
-      const lds_u8 *kp = (const lds_u8 *)(uintptr_t)(stage + kfrag[c % G::KF]);
-      const v8 a = *reinterpret_cast<const v8 __attribute__((address_space(3))) *>(kp + (c / G::KF) * 256);
+    for (int c = 0; c < DC; c++) {
+      const lds_u8 *kp = (const lds_u8 *)(uintptr_t)(stage + kfrag[c % KF]);
+      const v8 a = *reinterpret_cast<const v8 __attribute__((address_space(3))) *>(kp + (c / KF) * 256);
       accS = M::run(a, qf[c], accS);
     }
     const bool more = j + R < n;
@@ -220,7 +222,7 @@ __global__ __launch_bounds__(64 * SplitGeo<D>::W, 1) void fmha_split_kernel(cons
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
-      for (int db = 0; db < G::DB; db++)
+      for (int db = 0; db < DB; db++)
 #pragma unroll
         for (int i = 0; i < 16; i++) accO[db][i] *= alpha;
       lsum = makeP(m_new);
@@ -246,10 +248,10 @@ __global__ __launch_bounds__(64 * SplitGeo<D>::W, 1) void fmha_split_kernel(cons
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
 #pragma unroll
-    for (int db = 0; db < G::DB; db++)
+    for (int db = 0; db < DB; db++)
 #pragma unroll
       for (int m = 0; m < 2; m++) {
-        const lds_u8 *p = (const lds_u8 *)(uintptr_t)(stage + kTileBytes + vfrag[db % G::VF]) + (db / G::VF) * 256 + 16 * m * G::rowBytes;
+        const lds_u8 *p = (const lds_u8 *)(uintptr_t)(stage + kTileBytes + vfrag[db % VF]) + (db / VF) * 256 + 16 * m * G::rowBytes;
         const v4 lo = M::readTr(p);
         const v4 hi = M::readTr(p + 8 * G::rowBytes);
         accO[db] = M::run(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pf[m], accO[db]);
@@ -265,7 +267,7 @@ __global__ __launch_bounds__(64 * SplitGeo<D>::W, 1) void fmha_split_kernel(cons
   float *part = reinterpret_cast<float *>(smem); // [W][32][OS]
   float *ml = part + W * 32 * SG::OS;            // [W][32] pairs (reference, row sum)
 #pragma unroll
-  for (int db = 0; db < G::DB; db++)
+  for (int db = 0; db < DB; db++)
 #pragma unroll
     for (int g = 0; g < 4; g++)
       *reinterpret_cast<f32x4 *>(&part[(wave * 32 + l32) * SG::OS + 32 * db + 8 * g + 4 * hl]) =
@@ -334,7 +336,7 @@ int splitGroups(int D, int B, int S, int H, bool causal) {
   return causal && S >= 2048 && blocks2 <= 2 * cus ? 2 : 0;
 }
 
-template <typename T, int D, int QG, bool PAD>
+template <typename T, int D, int QG, bool PAD, int USED = D>
 void launchSplit(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqlens, void *out, int B, int S, int H,
                  int dHead, float scale, bool causal, hipStream_t stream) {
   const int nQB = (S + 32 * QG - 1) / (32 * QG);
@@ -344,9 +346,9 @@ void launchSplit(const void *qkv, const int32_t *seqlens, const int32_t *cuSeqle
   auto *o = static_cast<uint16_t *>(out);
   const dim3 grid(blocks), block(64 * SplitGeo<D>::W);
   if (causal)
-    launchKernel(fmha_split_kernel<T, D, QG, true, PAD>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, (int)blocks, dHead);
+    launchKernel(fmha_split_kernel<T, D, QG, true, PAD, USED>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, (int)blocks, dHead);
   else
-    launchKernel(fmha_split_kernel<T, D, QG, false, PAD>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, (int)blocks, dHead);
+    launchKernel(fmha_split_kernel<T, D, QG, false, PAD, USED>, grid, block, stream, in, seqlens, cuSeqlens, o, S, H, nQB, c, (int)blocks, dHead);
   MGPU_CHECK_LAUNCH("fmha_split_kernel");
 }
 
@@ -355,8 +357,13 @@ bool launchGeometry(const void *qkv, const int32_t *seqlens, const int32_t *cuSe
                     int dHead, float scale, bool causal, hipStream_t stream) {
   const int groups = splitGroups(D, B, S, H, causal);
   if (groups == 0) return false;
-  const auto launch = groups == 1 ? (dHead == D ? launchSplit<T, D, 1, false> : launchSplit<T, D, 1, true>)
-                                  : (dHead == D ? launchSplit<T, D, 2, false> : launchSplit<T, D, 2, true>);
+  constexpr int kFew = D == 64 ? 32 : D == 128 ? 80 : 160, kSome = D == 64 ? 48 : D == 128 ? 96 : 160; // (as in fmha.hip)
+  auto pick = [&](auto qg) {
+    constexpr int QG = decltype(qg)::value;
+    return dHead == D ? launchSplit<T, D, QG, false> : dHead <= kFew ? launchSplit<T, D, QG, true, kFew>
+           : dHead <= kSome ? launchSplit<T, D, QG, true, kSome> : launchSplit<T, D, QG, true>;
+  };
+  const auto launch = groups == 1 ? pick(std::integral_constant<int, 1>()) : pick(std::integral_constant<int, 2>());
   launch(qkv, seqlens, cuSeqlens, out, B, S, H, dHead, scale, causal, stream);
   return true;
 }
