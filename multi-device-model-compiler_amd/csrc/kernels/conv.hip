@@ -1370,6 +1370,16 @@ double convWindowTime(int64_t stride, int64_t pixels, int64_t IC, int64_t OC, in
   return 2.6 + rounds(tiles, 8 * cus) * (1.33 + 0.319 * channels);
 }
 
+// us on few tiles, a closer fit there: 1100 launches of up to 325 tiles (10th and 90th percentile 0.81 to 0.93 and 1.06 to 1.10).
+double convFewTilesTime(int win, int64_t stride, int64_t pixels, int64_t IC, int64_t OC, int64_t OW, int64_t cus) {
+  const int64_t tiles = (pixels + 31) / 32 * ((OC + 31) / 32);
+  const int ks = convStagedWaves(win, stride, pixels, IC, OC, OW, cus);
+  if (ks == 4 || tiles > 400) return 0.0;
+  const double rounds = (double)((tiles + cus - 1) / cus), channels = (double)IC;
+  if (ks == 8) return win == 3 ? 3.6 + rounds * 0.0444 * channels : win == 5 ? 3.14 + rounds * (0.335 + 0.1305 * channels) : 2.65 + rounds * (0.97 + 0.275 * channels);
+  return win == 3 ? 3.75 + rounds * 0.0355 * channels : win == 5 ? 3.56 + rounds * 0.131 * channels : 4.16 + rounds * 0.284 * channels;
+}
+
 // Do patches take a 5 x 5 or 7 x 7 from one channel or three?  From half of a row's tiles filled on (us, window tiles / patches, 7 x 7 from
 // 3 channels unless said otherwise: 1 x 224 x 224 -> 64 of stride 2 13.0 / 7.4, 16 x 256 x 256 94 / 57, 4 x 112 x 112 -> 32 14.2 / 10.3, 2 x
 // 28 x 28 -> 96 7.5 / 6.9; 32 x 28 x 28 -> 64 from 1 12.3 / 5.7; 5 x 5 16 x 128 x 128 -> 64 55 / 33; but rows of 10 13.1 / 16.4).  From one
@@ -1561,14 +1571,26 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     // 3 x 3 from 32 channels on in pairs of fp16 numbers, where both estimates say that this is faster (500 shapes of 0.15 GFLOP
     // on: taken by 268, 0.83 of the time over all of them, the largest ones 0.39, none more than 2 % slower).  (16 channels are
     // one step: no gain, and the fp32 instructions' sums are the more exact ones.)
+    ConvSplitPlan split{0, 0, 0.0};
     if (KH == 3 && IC >= 32 && IC % 16 == 0) {
       const int cus = numComputeUnits();
-      const ConvSplitPlan plan = convSplitPlan((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus,
-                                               0.97 * convWindowTime(SH, pixels, IC, OC, OW, cus));
-      if (plan.strips && convSplit(plan, input, weight, bias, output, add, N, IC, H, W, OC, OH, OW, PHL, PWL, SH, SW, DH, DW, relu, stream)) {
+      split = convSplitPlan((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus, 0.97 * convWindowTime(SH, pixels, IC, OC, OW, cus));
+    }
+    // Few tiles on quarters or halves of them, where the estimates say so by 8 % (570 launches of up to 1300 quarters: 0.81 of the time on
+    // average, the best choice everywhere would be 0.80, three of them 3 to 6 % slower; by 5 % 20 of them would be, of 24 channels).
+    if (KH >= 3) {
+      const int cus = numComputeUnits();
+      const double others = convFewTilesTime((int)KH, SH, pixels, IC, OC, OW, cus);
+      const ConvSmallPlan small = convSmallPlan((int)KH, pixels, IC, OC, cus);
+      if (small.ocSide && small.us < 0.92 * (split.strips ? std::min(others, 1.05 * split.us) : others) &&
+          convSmall((int)KH, small.ocSide, input, weight, bias, output, add, N, IC, H, W, OC, OH, OW, PHL, PWL, SH, SW, DH, DW, relu, stream)) {
         MGPU_CHECK_LAUNCH("mgpuConv2d");
         return;
       }
+    }
+    if (split.strips && convSplit(split, input, weight, bias, output, add, N, IC, H, W, OC, OH, OW, PHL, PWL, SH, SW, DH, DW, relu, stream)) {
+      MGPU_CHECK_LAUNCH("mgpuConv2d");
+      return;
     }
     auto pick = [&](auto win) {
       constexpr int WIN = decltype(win)::value;

@@ -14,7 +14,7 @@
 // out^T[n, m] = W^T[n, k] . in^T[k, m] with W^T through the transposing LDS read.
 //
 // Result::Planes: the blocks of grid row y take the y-th share of the reduction and write their fp32 sums to plane y of `out`
-// (float [gridDim.y][M][N]; partial_sums.hip adds the planes up and has the epilogue).  Result::F32: the rounded result, widened (the
+// (float [parts][M][N]; partial_sums.hip adds the planes up and has the epilogue).  Result::F32: the rounded result, widened (the
 // bits of a cast behind the kernel).
 #include "common.hpp"
 #include "mfma.hpp"
@@ -57,8 +57,9 @@ __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint1
 
   int chunks = (K + 31) / 32, firstChunk = 0;
   if (RESULT == Result::Planes) {
-    firstChunk = chunks * (int)blockIdx.y / (int)gridDim.y;
-    chunks = chunks * ((int)blockIdx.y + 1) / (int)gridDim.y - firstChunk;
+    const uint32_t perPart = partialShare(residual);
+    firstChunk = (int)__umulhi((uint32_t)(chunks * (int)blockIdx.y), perPart);
+    chunks = (int)__umulhi((uint32_t)(chunks * ((int)blockIdx.y + 1)), perPart) - firstChunk;
   }
   const int c0 = firstChunk + chunks * ks / KS, c1 = firstChunk + chunks * (ks + 1) / KS;
 
@@ -334,16 +335,17 @@ void gemmKSplitPartialF16(const void *in, const void *weight, float *planes, int
   const auto *a = static_cast<const uint16_t *>(in);
   const auto *w = static_cast<const uint16_t *>(weight);
   auto *o = reinterpret_cast<uint16_t *>(planes);
+  const uint16_t *share = partialShareArgument(parts);
   const int bm = tile == KSplitTile::T64x64 ? 64 : 32, bn = tile == KSplitTile::T32x32 ? 32 : 64;
   const int tilesM = (int)((M + bm - 1) / bm), nblk = tilesM * (int)((N + bn - 1) / bn);
   const dim3 grid((unsigned)nblk, (unsigned)parts), block(64 * kSplit);
   const int m = (int)M, n = (int)N, k = (int)K;
   if (tile == KSplitTile::T32x32)
-    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 1, 4, false, Result::Planes>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 1, 4, false, Result::Planes>, grid, block, stream, a, w, nullptr, share, o, m, n, k, tilesM, nblk);
   else if (tile == KSplitTile::T32x64)
-    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 2, 3, false, Result::Planes>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 1, 2, 3, false, Result::Planes>, grid, block, stream, a, w, nullptr, share, o, m, n, k, tilesM, nblk);
   else
-    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 2, 2, 2, false, Result::Planes>, grid, block, stream, a, w, nullptr, nullptr, o, m, n, k, tilesM, nblk);
+    launchKernel(gemm_ksplit_kernel<_Float16, ACT_NONE, 2, 2, 2, false, Result::Planes>, grid, block, stream, a, w, nullptr, share, o, m, n, k, tilesM, nblk);
   MGPU_CHECK_LAUNCH("gemm_ksplit_kernel");
 }
 

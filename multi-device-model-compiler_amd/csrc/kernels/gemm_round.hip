@@ -35,7 +35,7 @@ template <int NB> __host__ __device__ constexpr int wSwz(int row) { return NB ==
 // ACT: the activation, or one of
 constexpr int kResidual = 3; // + residual in its place
 constexpr int kPartial = 4;  // the blocks of grid row y take the y-th share of the reduction and write their fp32 sums to
-                             // plane y of `out` (float [gridDim.y][M][N]; partial_sums.hip adds them up and has the epilogue)
+                             // plane y of `out` (float [parts][M][N]; partial_sums.hip adds them up and has the epilogue)
 constexpr int kResidualF32 = 5; // + residual, the rounded result widened to fp32 (the bits of a cast behind the kernel)
 template <typename T, int ACT, int NB, bool RAGGED>
 __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
@@ -77,8 +77,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
   const char *wg = reinterpret_cast<const char *>(weight) + (size_t)n0 * 2;
   int steps = RAGGED ? (K + 63) / 64 : K / 64;
   if (ACT == kPartial) {
-    const int first = steps * (int)blockIdx.y / (int)gridDim.y;
-    steps = steps * ((int)blockIdx.y + 1) / (int)gridDim.y - first;
+    const uint32_t perPart = partialShare(residual);
+    const int first = (int)__umulhi((uint32_t)(steps * (int)blockIdx.y), perPart);
+    steps = (int)__umulhi((uint32_t)(steps * ((int)blockIdx.y + 1)), perPart) - first;
     ag += (size_t)first * 128;
     wg += (size_t)first * 128 * N;
   }
@@ -412,8 +413,8 @@ void gemmRoundPartialF16(const void *in, const void *weight, float *planes, int6
   const dim3 grid((unsigned)(tilesM * tilesN), (unsigned)parts), block(kThreads);
   const auto *a = static_cast<const uint16_t *>(in), *w = static_cast<const uint16_t *>(weight);
   auto *o = reinterpret_cast<uint16_t *>(planes);
-  if (width == 128) launchKernel(gemm_round_kernel<_Float16, kPartial, 4, false>, grid, block, stream, a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else launchKernel(gemm_round_kernel<_Float16, kPartial, 3, false>, grid, block, stream, a, w, nullptr, nullptr, o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  if (width == 128) launchKernel(gemm_round_kernel<_Float16, kPartial, 4, false>, grid, block, stream, a, w, nullptr, partialShareArgument(parts), o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else launchKernel(gemm_round_kernel<_Float16, kPartial, 3, false>, grid, block, stream, a, w, nullptr, partialShareArgument(parts), o, (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_round_kernel");
 }
 

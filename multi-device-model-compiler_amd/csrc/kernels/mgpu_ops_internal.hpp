@@ -194,6 +194,18 @@ ConvSplitPlan convSplitPlan(int N, int IC, int OC, int OH, int OW, int SH, int S
 bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const float *bias, float *y, const float *add, int64_t N, int64_t IC,
                int64_t H, int64_t W, int64_t OC, int64_t OH, int64_t OW, int64_t PHL, int64_t PWL, int64_t SH, int64_t SW, int64_t DH,
                int64_t DW, bool relu, hipStream_t stream);
+// How long the same take for 3 x 3, 5 x 5 or 7 x 7 on few tiles, in us; 0: not few.
+double convFewTilesTime(int win, int64_t stride, int64_t pixels, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
+// 3 x 3, 5 x 5 or 7 x 7 on tiles of 16 pixels (conv_small.hip), from channels that are a multiple of 4: the output channels of a tile, 16 or 32, that
+// take the least time (0: none) and the launch (false: not for these sizes).
+struct ConvSmallPlan {
+  int ocSide;
+  double us;
+};
+ConvSmallPlan convSmallPlan(int win, int64_t pixels, int64_t IC, int64_t OC, int64_t cus);
+bool convSmall(int win, int ocSide, const float *x, const float *w, const float *bias, float *y, const float *add, int64_t N, int64_t IC, int64_t H, int64_t W,
+               int64_t OC, int64_t OH, int64_t OW, int64_t PHL, int64_t PWL, int64_t SH, int64_t SW, int64_t DH, int64_t DW, bool relu,
+               hipStream_t stream);
 void pool2d(const float *input, float *output, int64_t N, int64_t C, int64_t H, int64_t W, int64_t OH, int64_t OW,
             int64_t KH, int64_t KW, int64_t PHL, int64_t PWL, int64_t PHR, int64_t PWR, int64_t SH, int64_t SW,
             int64_t method, hipStream_t stream);
