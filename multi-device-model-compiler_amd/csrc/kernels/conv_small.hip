@@ -194,9 +194,10 @@ ConvSmallPlan convSmallPlan(int win, int64_t pixels, int64_t IC, int64_t OC, int
   ConvSmallPlan best{0, 0.0};
   if (IC % kGroup) return best;
   for (int i = 0; i < (win == 7 ? 1 : 2); i++) {
-    const int64_t side = kSide << i, tiles = (pixels + kSide - 1) / kSide * ((OC + side - 1) / side);
+    const int64_t side = kSide << i, rounds = ((pixels + kSide - 1) / kSide * ((OC + side - 1) / side) + cus - 1) / cus;
+    if (rounds > 2) continue; // (of which the fit knows too little: 4914 pixels of 64 -> 64 in three 10.2 -> 10.7 us)
     const double *t = time[i][(win - 3) / 2];
-    const double us = t[0] + (double)((tiles + cus - 1) / cus * ((IC + kGroup * kShares - 1) / (kGroup * kShares))) * t[1];
+    const double us = t[0] + (double)(rounds * ((IC + kGroup * kShares - 1) / (kGroup * kShares))) * t[1];
     if (!best.ocSide || us < best.us) best = ConvSmallPlan{(int)side, us};
   }
   return best;

@@ -18,7 +18,9 @@ class Plan(ctypes.Structure):
     (3, 16 * 16 + 1, 64, 256, 32),   # a tile more: halves in one round
     (3, 16 * 16, 64, 257, 32),
     (3, 32 * 16, 64, 256, 32),
-    (3, 32 * 16 + 1, 128, 256, 16),  # three rounds against two
+    (3, 32 * 16 + 1, 128, 256, 32),  # two rounds of halves
+    (3, 64 * 16, 128, 256, 32),
+    (3, 64 * 16 + 1, 128, 256, 0),   # a third: the tiles of 32 x 32 fill the chip as well
     (5, 300, 64, 256, 32),
     (7, 300, 64, 256, 16),           # no halves of it
     (7, 300, 62, 256, 0),
