@@ -30,6 +30,9 @@ constexpr int kGroup = 4;  // channels at a time
 
 struct SmallGeo {
   int IC, H, W, OW, PHL, PWL, SH, SW, DH, DW;
+  int blocks, inner; // tiles; those side by side that are counted first, of pixels where the filter is the larger operand, else of channels
+  FastDiv byInner;
+  bool pixelsFirst;
 };
 
 template <int WIN, int OT> struct Small {
@@ -55,7 +58,12 @@ __global__ __launch_bounds__(64 * kShares, 2) void conv_small_kernel(const float
   const int tid = threadIdx.x, lane = tid % 64;
   const int share = __builtin_amdgcn_readfirstlane(tid / 64);
   const int l16 = lane % 16, quarter = lane / 16;
-  const int oc0 = blockIdx.y * S::ROWS, q0 = blockIdx.x * kSide;
+  // An equal run of tiles for each XCD, those one after another that share the larger operand, which then comes into one L2 (168 pixels
+  // of 256 -> 512, 7 x 7, 26 MB of filter: 90 us with every eighth tile on an XCD, 84 so; over 300 launches 0.97 of the time).
+  const int xcd = (int)blockIdx.x % 8, run = g.blocks / 8, extra = g.blocks % 8;
+  const int wid = xcd * run + (xcd < extra ? xcd : extra) + (int)blockIdx.x / 8;
+  const int outer = __builtin_amdgcn_readfirstlane(divide(wid, g.byInner)), inner = wid - outer * g.inner;
+  const int oc0 = (g.pixelsFirst ? outer : inner) * S::ROWS, q0 = (g.pixelsFirst ? inner : outer) * kSide;
   const int HW4 = g.H * g.W * 4, pixels = N * P;
   const int nFirst = __builtin_amdgcn_readfirstlane(divide(q0, byP));
 
@@ -211,13 +219,14 @@ bool convSmall(int win, int ocSide, const float *x, const float *w, const float 
   const int64_t P = OH * OW, pixels = N * P, tiles = (pixels + kSide - 1) / kSide, ocTiles = (OC + ocSide - 1) / ocSide;
   // byte offsets from a tile's first image and filter row on are 32 bits wide; a grid's threads are fewer than 2^32
   const int64_t images = (kSide - 2) / P + 2;
-  if (IC % kGroup || !fits(pixels + kSide) || !fits(images * IC * H * W * 4) || !fits(ocSide * IC * win * win * 4) || ocTiles > 65535 ||
-      tiles * (64 * kShares) >= (int64_t(1) << 32))
+  if (IC % kGroup || !fits(pixels + kSide) || !fits(images * IC * H * W * 4) || !fits(ocSide * IC * win * win * 4) || tiles * ocTiles * (64 * kShares) >= (int64_t(1) << 32))
     return false;
-  const SmallGeo g{(int)IC, (int)H, (int)W, (int)OW, (int)PHL, (int)PWL, (int)SH, (int)SW, (int)DH, (int)DW};
+  const bool pixelsFirst = OC * win * win > N * H * W;
+  const int inner = (int)(pixelsFirst ? tiles : ocTiles);
+  const SmallGeo g{(int)IC, (int)H, (int)W, (int)OW, (int)PHL, (int)PWL, (int)SH, (int)SW, (int)DH, (int)DW, (int)(tiles * ocTiles), inner, fastDiv(inner), pixelsFirst};
   auto *kernel = ocSide == 32 ? (win == 3 ? conv_small_kernel<3, 2> : conv_small_kernel<5, 2>)
                  : win == 3 ? conv_small_kernel<3, 1> : win == 5 ? conv_small_kernel<5, 1> : conv_small_kernel<7, 1>;
-  launchKernel(kernel, dim3((unsigned)tiles, (unsigned)ocTiles), dim3(64 * kShares), stream, x, w, (int)OC, (int)P, (int)N, fastDiv((int)P), fastDiv((int)OW),
+  launchKernel(kernel, dim3((unsigned)(tiles * ocTiles)), dim3(64 * kShares), stream, x, w, (int)OC, (int)P, (int)N, fastDiv((int)P), fastDiv((int)OW),
                bias, y, add, relu, g);
   return true;
 }
