@@ -1576,6 +1576,14 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
       const int cus = numComputeUnits();
       split = convSplitPlan((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus, 0.97 * convWindowTime(SH, pixels, IC, OC, OW, cus));
     }
+    // 5 x 5 from 16 channels on likewise.  What the other kernels take is estimated low, by the matrix instructions of the rounds alone (0.131 to
+    // 0.25 us a round and channel were measured; 0.124 leaves some launches of one or two rounds with them: 248 tiles from 256 40 / 44 us, 567 from
+    // 16 9.9 / 9.7, 288 from 16 7.7 / 8.4, but 264 from 64 19.5 / 16.0, 438 from 32 12.5 / 10.8, 876 from 128 84 / 35).
+    if (KH == 5 && IC >= 16 && IC % 8 == 0) {
+      const int cus = numComputeUnits();
+      const double others = 3.0 + (double)((tiles + cus - 1) / cus) * 0.124 * (double)IC;
+      split = convSplitPlan5((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus, 0.97 * others);
+    }
     // Few tiles on quarters or halves of them, where the estimates say so by 8 % (570 launches of up to 1300 quarters: 0.81 of the time on
     // average, the best choice everywhere would be 0.80, three of them 3 to 6 % slower; by 5 % 20 of them would be, of 24 channels).
     if (KH >= 3) {

@@ -1,4 +1,4 @@
-// 3 x 3 convolution of fp32 tensors on the fp16 matrix cores, with fp32's accuracy.
+// 3 x 3 and 5 x 5 convolution of fp32 tensors on the fp16 matrix cores, with fp32's accuracy.
 //
 // Every operand is taken apart into two fp16 numbers, v = scale * x = hi + lo with hi = fp16(v), lo = fp16(v - hi) and a scale
 // that is a power of two: 22 bits of the 24, and three products, hi.hi + (hi.lo + lo.hi), sum up in fp32.  What is left out is
@@ -7,7 +7,7 @@
 // pixels, K taps): 0.9e-7 to 2.2e-7 for K = 288 to 2304, 1.2e-7 to 5.7e-7 with the fp32 instructions on the same shapes.
 //
 // What fp32 has and fp16 pairs have not is range.  The scales come from the block's own operands - one for its pixels, one for each
-// output channel's filter, each from the largest value in its first sixteen input channels, which they put to 2^7 .. 2^8 -, so
+// output channel's filter, each from the largest value in its first step of input channels, which they put to 2^7 .. 2^8 -, so
 // that tensors of any size fit, and the block checks while it converts: a value beyond 65504 (infinities; 256 times what the
 // first channels hold), or a window whose largest value is under 2^-9 of them, and the block does its tile again with the fp32
 // instructions, which read the same LDS.  (NaNs need no check: they come through both ways.)
@@ -25,6 +25,12 @@
 // A consumer has 32 channels x 64 pixels; one, two or four of them share pixels and split the nine positions (tiles of 256, 128
 // and 64 pixels).  us, before / now, 3 x 3 pad 1: 12 x 256 x 10 x 46 -> 256 83 / 34, 12 x 256 x 240 x 36 -> 16 151 / 67, 17 x 128 x
 // 15 x 33 -> 128 46 / 20, 32 x 64 x 56 x 56 -> 64 77 / 53, 23 x 256 x 12 x 10 -> 256 40 / 25, 5 x 256 x 36 x 9 -> 256 26 / 21.
+//
+// 5 x 5: sixteen channels of its 25 positions, twice and as they are, would not fit the LDS.  A step has eight, and a matrix instruction's
+// sixteen products are two positions, one a lane half; the 26th is a filler of zeros, filter and pixels.  The consumers' reads set the
+// pace (1.7 us a step of 128 pixels, of which the matrix instructions are 0.5; three sets of operands on their way in place of two
+// spill).  us, before / now, stride 1 pad 2: 8 x 128 x 21 x 42 -> 128 81 / 34, 16 x 64 x 46 x 46 -> 64 120 / 56, 8 x 32 x 60 x 60 -> 64
+// 43 / 26, 4 x 256 x 30 x 30 -> 256 156 / 62.  Error against 64 bits 0.7e-7 to 1.6e-7 for K = 400 to 3200, 0.8e-7 to 2.1e-7 before.
 #include "common.hpp"
 #include "conv.hpp"
 #include "mfma.hpp"
@@ -37,7 +43,6 @@ namespace mgpu {
 namespace {
 
 constexpr int kConsumers = 4, kProducers = 8, kThreads = 64 * (kConsumers + kProducers);
-constexpr int kWin = 3, kTaps = kWin * kWin; // the window
 constexpr int kOC = 32;                      // output channels of a block
 constexpr int kPT = 2;                       // tiles of 32 pixels of a consumer
 constexpr int kTop = 8;                      // scaled maxima lie under 2^8
@@ -68,28 +73,32 @@ __device__ __forceinline__ int scaleExponent(uint32_t largest, int none) {
 }
 __device__ __forceinline__ float powerOf2(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
 
-// KS: consumers that share their pixels; CAP: staged pixels at most
-template <int KS_, int CAP_> struct SplitShape {
+// WIN: the window; KS: consumers that share their pixels; CAP: staged pixels at most
+template <int WIN, int KS_, int CAP_> struct SplitShape {
+  static constexpr int TAPS = WIN * WIN, CH = WIN == 3 ? 16 : 8, OCTETS = CH / 8; // positions; input channels of a step
+  // Matrix instructions' sets of sixteen products: a position of sixteen channels, or two of eight (the last one has a filler beside it).
+  static constexpr int PAIRED = 3 - OCTETS, SETS = (TAPS + PAIRED - 1) / PAIRED;
   static constexpr int KS = KS_, CAP = CAP_, PXW = kConsumers / KS, PX = 32 * kPT * PXW;
-  static constexpr int UNIT = 2 * 2 * kOC * 16 + 80; // bytes of a position's filter values (the 80: positions side by side on different banks)
-  static constexpr int FILTER = kTaps * UNIT, PIXELS = 2 * 2 * CAP * 16;
-  static constexpr int ROW = 16 * kTaps, PITCH = ROW + 4; // words of a channel's filter in a step
+  static constexpr int UNIT = OCTETS * 2 * kOC * 16 + 80; // bytes of a position's filter values (the 80: positions side by side on different banks)
+  static constexpr int HALF = OCTETS == 2 ? 2 * kOC * 16 : UNIT; // from the values of a lane half to the other's
+  static constexpr int FILTER = SETS * PAIRED * UNIT, PIXELS = OCTETS * 2 * CAP * 16;
+  static constexpr int ROW = CH * TAPS, PITCH = ROW + 4; // words of a channel's filter in a step
   static constexpr int RAW = kOC * PITCH * 4, RAWS = 3;
   static constexpr int LDS = 2 * (FILTER + PIXELS) + RAWS * RAW;
   static constexpr int RPW = kOC / kProducers; // filter rows a producer moves
-  static constexpr int ITEMS = kOC * 2 * kTaps; // eight channels of a position of a filter
-  static constexpr int WI = (ITEMS + 64 * kProducers - 1) / (64 * kProducers), PI = 2 * CAP / (64 * kProducers);
-  static_assert(CAP % (32 * kProducers) == 0 && ITEMS % 64 == 0, "whole wavefronts");
+  static constexpr int ITEMS = kOC * OCTETS * TAPS; // eight channels of a position of a filter
+  static constexpr int WI = (ITEMS + 64 * kProducers - 1) / (64 * kProducers), PI = (OCTETS * CAP + 64 * kProducers - 1) / (64 * kProducers);
+  static_assert(CAP % 64 == 0 && ROW % 4 == 0 && ROW / 4 <= 64 && LDS + 1024 <= 160 * 1024, "whole wavefronts; a CU's LDS");
   static_assert(KS == 1 || kConsumers * kPT * 16 * 64 * 4 <= LDS, "the partial sums take the buffers' place");
 };
 
-template <int KS, int CAP>
+template <int WIN, int KS, int CAP>
 __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__restrict__ w, const float *__restrict__ x, int IC, int OC,
                                                               int gridDimX, int ocTiles, FastDiv byOcTiles, int H, int W, int N, int relu,
                                                               const float *__restrict__ bias, float *__restrict__ y,
                                                               const float *__restrict__ add, SplitGeo g) {
-  using S = SplitShape<KS, CAP>;
-  constexpr int PXW = S::PXW, PI = S::PI, WI = S::WI, RPW = S::RPW;
+  using S = SplitShape<WIN, KS, CAP>;
+  constexpr int PXW = S::PXW, PI = S::PI, WI = S::WI, RPW = S::RPW, TAPS = S::TAPS, SETS = S::SETS;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[S::LDS];
   __shared__ uint32_t wMax[kOC], xMax;
   __shared__ int wExp[kOC], bad, small;
@@ -104,7 +113,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
   const int wid = xcd * share + (xcd < extra ? xcd : extra) + (int)blockIdx.x / 8;
   const int pxTile = __builtin_amdgcn_readfirstlane(divide(wid, byOcTiles)), ocTile = __builtin_amdgcn_readfirstlane(wid - pxTile * ocTiles);
   const int oc0 = ocTile * kOC, p0 = pxTile * S::PX;
-  const int steps = IC / 16;
+  const int steps = IC / S::CH;
   const int pwave = wave - kConsumers, ptid = tid - 64 * kConsumers;
 
   // ---- the filter, as it is, into a ring of three steps.  (Past the last step it is loaded once more, and so are the pixels: a load
@@ -118,7 +127,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
 #pragma unroll
     for (int i = 0; i < RPW; i++) {
       const int row = pwave * RPW + i, oc = oc0 + row < OC ? oc0 + row : OC - 1; // (a channel past the end is not stored)
-      ldsLoad16First<S::ROW / 4>((uint32_t)lane * 16, from + (int64_t)oc * (IC * kTaps * 4), rawAt + slot * S::RAW + row * (S::PITCH * 4));
+      ldsLoad16First<S::ROW / 4>((uint32_t)lane * 16, from + (int64_t)oc * (IC * TAPS * 4), rawAt + slot * S::RAW + row * (S::PITCH * 4));
     }
   };
   if (producer) {
@@ -140,7 +149,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
   // Staged input rows: from the first one of the tile's first pixel to the last one of its last, over the images.
   const Pixel first = pixelOf(p0), last = pixelOf((p0 + S::PX < g.pixels ? p0 + S::PX : g.pixels) - 1);
   const int r0 = first.image * g.rows + first.row * g.SH;
-  const int staged = (last.image * g.rows + last.row * g.SH + (kWin - 1) * g.DH - r0 + 1) * g.pitch;
+  const int staged = (last.image * g.rows + last.row * g.SH + (WIN - 1) * g.DH - r0 + 1) * g.pitch;
   const int blocks = __builtin_amdgcn_readfirstlane((staged + 63) / 64), plane = blocks * 64; // ... in pieces of 64 pixels
   const int n0 = __builtin_amdgcn_readfirstlane(divide(first.image, g.byStrips));
   const int HW = H * W;
@@ -159,7 +168,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
       const int r = divide(px, g.byPitch), c = px - r * g.pitch;
       const int vr = r0 + r, image = divide(vr, g.byRows), ih = vr - image * g.rows - g.PHL;
       const int n = divide(image, g.byStrips), iw = (image - n * g.strips) * g.stripW * g.SW + c - g.PWL;
-      const bool in = half < 2 && px < staged && n < N && (unsigned)ih < (unsigned)H && (unsigned)iw < (unsigned)W;
+      const bool in = half < S::OCTETS && px < staged && n < N && (unsigned)ih < (unsigned)H && (unsigned)iw < (unsigned)W;
       xoff[i] = in ? ((n - n0) * IC * HW + half * 8 * HW + ih * W + iw) * 4 : kOutside;
       xlds[i] = (half * 2 * plane + px) * 16;
     }
@@ -168,18 +177,19 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
     bool wused[WI];
 #pragma unroll
     for (int i = 0; i < WI; i++) {
-      const int e = i * 64 * kProducers + ptid, pair = e / kTaps, tap = e - pair * kTaps;
+      const int at = i * 64 * kProducers + ptid, e = at < S::ITEMS ? at : S::ITEMS - 1; // (past the end: the last one again)
+      const int pair = e / TAPS, tap = e - pair * TAPS;
       wused[i] = i * 64 * kProducers + pwave * 64 < S::ITEMS; // (uniform)
-      wch[i] = pair / 2;
-      wraw[i] = wch[i] * S::PITCH + pair % 2 * (8 * kTaps) + tap;
-      wlds[i] = tap * S::UNIT + (pair % 2 * 2 * kOC + wch[i]) * 16;
+      wch[i] = pair / S::OCTETS;
+      wraw[i] = wch[i] * S::PITCH + pair % S::OCTETS * (8 * TAPS) + tap;
+      wlds[i] = tap * S::UNIT + (pair % S::OCTETS * 2 * kOC + wch[i]) * 16;
     }
     const auto image = resource(x + (int64_t)n0 * IC * HW, (int64_t)(N - n0) * IC * HW);
     struct Pieces {
       float v[PI][8];
     };
     auto loadPixels = [&](Pieces &p, int step) {
-      const int at = step * 16 * HW * 4;
+      const int at = step * S::CH * HW * 4;
 #pragma unroll
       for (int i = 0; i < PI; i++)
 #pragma unroll
@@ -207,7 +217,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
         float m = 0.0f;
         const int row = pwave * RPW + lane / LPR;
 #pragma unroll
-        for (int i = 0; i < S::ROW / LPR; i++) m = fmaxf(m, fabsf(raw[row * S::PITCH + i * LPR + lane % LPR]));
+        for (int i = 0; i < S::ROW; i += LPR) m = fmaxf(m, fabsf(raw[row * S::PITCH + (i + LPR <= S::ROW || i + lane % LPR < S::ROW ? i + lane % LPR : i)]));
         m = group_max<LPR>(m);
         if (lane % LPR == 0) {
           wMax[row] = __builtin_bit_cast(uint32_t, m);
@@ -248,7 +258,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
 #pragma unroll
           for (int i = 0; i < PI; i++) {
             if constexpr (SPLIT) xmost[i] = largest(p.v[i], xmost[i]);
-            if (piece(i) < 2 * blocks) put(p.v[i], xs, at + xlds[i], plane * 16);
+            if (piece(i) < S::OCTETS * blocks) put(p.v[i], xs, at + xlds[i], plane * 16);
           }
           loadPixels(p, atMost(s + 2));
           at = smem + (s & 1) * S::FILTER;
@@ -257,7 +267,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
             if (!wused[i]) continue;
             float v[8];
 #pragma unroll
-            for (int k = 0; k < 8; k++) v[k] = raw[slot * (S::RAW / 4) + wraw[i] + k * kTaps];
+            for (int k = 0; k < 8; k++) v[k] = raw[slot * (S::RAW / 4) + wraw[i] + k * TAPS];
             if constexpr (SPLIT) wmost[i] = largest(v, wmost[i]);
             put(v, SPLIT ? ws[i] : 1.0f, at + wlds[i], kOC * 16);
           }
@@ -279,7 +289,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
         bool fault = false, low = false;
 #pragma unroll
         for (int i = 0; i < PI; i++)
-          if (piece(i) < 2 * blocks) {
+          if (piece(i) < S::OCTETS * blocks) {
             fault |= xmost[i] * xs >= kMost;
             low |= xmost[i] > 0.0f && xmost[i] * xs < kLeast;
           }
@@ -298,7 +308,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
           float *maxima = reinterpret_cast<float *>(smem);
 #pragma unroll
           for (int i = 0; i < PI; i++)
-            if (piece(i) < 2 * blocks) maxima[piece(i) * 64 + lane] = xmost[i];
+            if (piece(i) < S::OCTETS * blocks) maxima[piece(i) * 64 + lane] = xmost[i];
           __syncthreads();
           __syncthreads();
         }
@@ -319,9 +329,14 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
     const int q = p0 + (pw * kPT + t) * 32 + l32;
     const Pixel p = pixelOf(q < g.pixels ? q : p0);
     const int n = divide(p.image, g.byStrips), col = (p.image - n * g.strips) * g.stripW + p.col;
-    bbase[t] = ((p.image * g.rows + p.row * g.SH - r0) * g.pitch + p.col * g.SW) * 16 + hl * (2 * 16) * plane;
+    bbase[t] = ((p.image * g.rows + p.row * g.SH - r0) * g.pitch + p.col * g.SW) * 16 + (S::OCTETS == 2 ? hl * (2 * 16) * plane : 0);
     pix[t] = q < g.pixels && col < g.OW ? p.row * g.OW + col : -1;
     img[t] = n - n0;
+  }
+  // The filler position's filter values are zeros, and taken for its pixels too (an infinity times 0 would be none).
+  constexpr int kFiller = TAPS * S::UNIT;
+  if constexpr (S::PAIRED == 2) {
+    if (tid < 2 * 64) *reinterpret_cast<u32x4 *>(smem + tid / 64 * S::FILTER + kFiller + tid % 64 * 16) = u32x4{0u, 0u, 0u, 0u};
   }
   f32x16 acc[kPT];
   auto multiply = [&](auto splitTag) -> bool { // false: the pieces did not hold everything
@@ -334,16 +349,19 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
     struct Operands {
       f16x8 ah, al, bh[kPT], bl[kPT]; // not SPLIT: eight channels as two times four floats
     };
-    auto read = [&](Operands &o, int step, int tap) {
-      const unsigned char *wat = smem + (step & 1) * S::FILTER + hl * (2 * kOC * 16) + l32 * 16 + tap * S::UNIT;
-      const unsigned char *xat = pixelBuf + (step & 1) * S::PIXELS;
-      const int ky = tap / kWin, kx = tap - ky * kWin, off = (ky * g.DH * g.pitch + kx * g.DW) * 16;
+    auto read = [&](Operands &o, int step, int set) {
+      const unsigned char *wat = smem + (step & 1) * S::FILTER + hl * S::HALF + l32 * 16 + set * (S::PAIRED * S::UNIT);
+      const int pixelsAt = 2 * S::FILTER + (step & 1) * S::PIXELS;
+      const int tap = S::PAIRED == 2 ? 2 * set + hl : set;
+      const int ky = tap / WIN, kx = tap - ky * WIN, off = (ky * g.DH * g.pitch + kx * g.DW) * 16;
+      const bool filler = S::PAIRED == 2 && tap == TAPS;
       o.ah = *reinterpret_cast<const f16x8 *>(wat);
       o.al = *reinterpret_cast<const f16x8 *>(wat + kOC * 16);
 #pragma unroll
       for (int t = 0; t < kPT; t++) {
-        o.bh[t] = *reinterpret_cast<const f16x8 *>(xat + bbase[t] + off);
-        o.bl[t] = *reinterpret_cast<const f16x8 *>(xat + bbase[t] + off + plane * 16);
+        const int at = filler ? kFiller : pixelsAt + bbase[t] + off;
+        o.bh[t] = *reinterpret_cast<const f16x8 *>(smem + at);
+        o.bl[t] = *reinterpret_cast<const f16x8 *>(smem + at + (filler ? 0 : plane * 16));
       }
     };
     auto mma = [&](const Operands &o) {
@@ -369,19 +387,19 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
     if constexpr (SPLIT) __syncthreads();
     __syncthreads();
     for (int s = 0; s < steps; s++) {
-      // positions from, from + KS, ...: dealt out in turns
-      const int from = KS == 1 ? 0 : (ks + s * (kTaps % KS)) % KS;
+      // sets from, from + KS, ...: dealt out in turns
+      const int from = KS == 1 ? 0 : (ks + s * (SETS % KS)) % KS;
       Operands even, odd;
       read(even, s, from);
-      int tap = from;
+      int set = from;
 #pragma nounroll
-      for (; tap + KS < kTaps; tap += 2 * KS) {
-        read(odd, s, tap + KS);
+      for (; set + KS < SETS; set += 2 * KS) {
+        read(odd, s, set + KS);
         mma(even);
-        read(even, s, tap + 2 * KS < kTaps ? tap + 2 * KS : from);
+        read(even, s, set + 2 * KS < SETS ? set + 2 * KS : from);
         mma(odd);
       }
-      if (tap < kTaps) mma(even);
+      if (set < SETS) mma(even);
       __syncthreads();
     }
     if constexpr (SPLIT) {
@@ -394,9 +412,9 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
 #pragma unroll
         for (int t = 0; t < kPT; t++) {
           float m = 0.0f;
-          const int base = bbase[t] / 16 - hl * plane; // (a lane half has a plane of pixels and one of lower pieces each)
-          for (int ky = 0; ky < kWin; ky++)
-            for (int kx = 0; kx < kWin; kx++) m = fmaxf(m, maxima[base + ky * g.DH * g.pitch + kx * g.DW]);
+          const int base = bbase[t] / 16 - (S::OCTETS == 2 ? hl * plane : 0); // (a lane half has a plane of pixels and one of lower pieces each)
+          for (int ky = 0; ky < WIN; ky++)
+            for (int kx = 0; kx < WIN; kx++) m = fmaxf(m, maxima[base + ky * g.DH * g.pitch + kx * g.DW]);
           m = halves_max(m);
           fault |= pix[t] >= 0 && m > 0.0f && m * powerOf2(xe) < kLeast;
         }
@@ -472,23 +490,24 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
   }
 }
 
-// The tiles, and what a launch in them takes: us = start + rounds of the CUs * (block + step * IC / 16), fitted to 800 launches of
-// each of the larger two, 450 and 280 of the others (a tenth to a ninetieth percentile of 0.93 to 1.08 times what was measured).
+// The tiles, and what a launch in them takes: us = start + rounds of the CUs * (block + step * steps), fitted to 800 launches of
+// each of the larger two of 3 x 3, 450 and 280 of the others (a tenth to a ninetieth percentile of 0.93 to 1.08 times what was measured), and
+// to 80 of 5 x 5.
 struct SplitTile {
   int pixels, cap;
   double start, block, step;
 };
-constexpr SplitTile kTiles[] = {{64, 256, 1.5, 4.7, 0.89}, {64, 512, 1.5, 5.1, 1.08}, {128, 256, 1.4, 5.5, 1.10}, {128, 512, 1.3, 6.0, 1.20}, {256, 512, 0.7, 7.5, 1.42}};
+constexpr SplitTile kTiles[] = {{64, 256, 1.5, 4.7, 0.89}, {64, 512, 1.5, 5.1, 1.08}, {128, 256, 1.4, 5.5, 1.10}, {128, 512, 1.3, 6.0, 1.20}, {256, 512, 0.7, 7.5, 1.42},
+                                {64, 384, 1.4, 4.45, 1.173}, {128, 384, 1.2, 5.1, 1.68}};
+constexpr int kTiles3 = 5, kTiles5 = 2; // of 3 x 3, and behind them of 5 x 5
 
-} // namespace
-
-// The cheapest of them, if it takes less than `limit` us.
-ConvSplitPlan convSplitPlan(int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit) {
+// The cheapest of tiles first .. first + count - 1, if it takes less than `limit` us.
+ConvSplitPlan cheapest(int first, int count, int win, int step, int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit) {
   ConvSplitPlan best{0, 0, limit};
-  const int ocTiles = (OC + kOC - 1) / kOC, below = (kWin - 1) * DH + 1; // below: rows of a window
-  for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); i++) {
+  const int ocTiles = (OC + kOC - 1) / kOC, below = (win - 1) * DH + 1; // below: rows of a window
+  for (int i = first; i < first + count; i++) {
     const SplitTile &tile = kTiles[i];
-    const double round = tile.block + tile.step * (IC / 16);
+    const double round = tile.block + tile.step * (IC / step);
     if (tile.start + round >= best.us) continue;
     // the widest strips whose staged rows fit (none narrower than 8 beside others: their halo would be most of them)
     for (int strips = (OW + tile.cap - 1) / tile.cap, width; width = (OW + strips - 1) / strips, strips == 1 || width >= 8;
@@ -496,7 +515,7 @@ ConvSplitPlan convSplitPlan(int N, int IC, int OC, int OH, int OW, int SH, int S
       // rows that the tile's pixels lie in at most, and images; where one of these ends, its last window's rows come besides
       const int64_t rows = std::min<int64_t>((tile.pixels - 2) / width + 2, (int64_t)N * strips * OH);
       const int64_t images = std::min<int64_t>((tile.pixels - 2) / ((int64_t)OH * width) + 2, rows);
-      const int64_t staged = ((rows - 1) * SH + below + (images - 1) * std::max(0, below - SH)) * ((int64_t)(width - 1) * SW + (kWin - 1) * DW + 1);
+      const int64_t staged = ((rows - 1) * SH + below + (images - 1) * std::max(0, below - SH)) * ((int64_t)(width - 1) * SW + (win - 1) * DW + 1);
       if (staged <= tile.cap) {
         const int64_t blocks = ((int64_t)N * strips * OH * width + tile.pixels - 1) / tile.pixels * ocTiles;
         const double us = tile.start + (double)((blocks + cus - 1) / cus) * round;
@@ -509,18 +528,28 @@ ConvSplitPlan convSplitPlan(int N, int IC, int OC, int OH, int OW, int SH, int S
   return best;
 }
 
+} // namespace
+
+ConvSplitPlan convSplitPlan(int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit) {
+  return cheapest(0, kTiles3, 3, 16, N, IC, OC, OH, OW, SH, SW, DH, DW, cus, limit);
+}
+ConvSplitPlan convSplitPlan5(int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit) {
+  return cheapest(kTiles3, kTiles5, 5, 8, N, IC, OC, OH, OW, SH, SW, DH, DW, cus, limit);
+}
+
 // Launches it; false where its indices would not fit.
 bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const float *bias, float *y, const float *add, int64_t N, int64_t IC,
                int64_t H, int64_t W, int64_t OC, int64_t OH, int64_t OW, int64_t PHL, int64_t PWL, int64_t SH, int64_t SW, int64_t DH,
                int64_t DW, bool relu, hipStream_t stream) {
   auto fits = [](int64_t v) { return v >= 0 && v <= 0x7fffffff; };
   const int64_t strips = plan.strips, width = (OW + strips - 1) / strips, pixels = N * strips * OH * width, tilePixels = kTiles[plan.tile].pixels;
-  const int64_t pitch = (width - 1) * SW + (kWin - 1) * DW + 1, rows = (OH - 1) * SH + (kWin - 1) * DH + 1;
+  const int win = plan.tile < kTiles3 ? 3 : 5, taps = win * win;
+  const int64_t pitch = (width - 1) * SW + (win - 1) * DW + 1, rows = (OH - 1) * SH + (win - 1) * DH + 1;
   const int64_t pxTiles = (pixels + tilePixels - 1) / tilePixels, ocTiles = (OC + kOC - 1) / kOC, blocks = pxTiles * ocTiles;
   // pixel, row and byte indices from a tile's first image on are 32 bits wide, the filter's from a channel on; a grid's threads are fewer than 2^32
   const int64_t images = (tilePixels - 2) / (OH * width) + 2;
   if (!aligned16(w) || !fits(pixels + tilePixels) || !fits(N * strips * rows + tilePixels * SH) || !fits(images * IC * H * W * 4) ||
-      !fits(images * OC * OH * OW * 4) || !fits(IC * kTaps * 4) || blocks * kThreads >= (int64_t(1) << 32))
+      !fits(images * OC * OH * OW * 4) || !fits(IC * taps * 4) || blocks * kThreads >= (int64_t(1) << 32))
     return false;
   const SplitGeo g{(int)OH,    (int)OW, (int)PHL, (int)PWL,   (int)SH, (int)SW, (int)DH, (int)DW, (int)strips, (int)width, (int)pitch, (int)rows, (int)pixels,
                    fastDiv((int)(OH * width)), fastDiv((int)width), fastDiv((int)strips), fastDiv((int)pitch), fastDiv((int)rows)};
@@ -529,11 +558,13 @@ bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const 
                                                                   (int)N, relu, bias, y, add, g);
   };
   switch (plan.tile) {
-  case 0: launch(conv_split_kernel<4, 256>); break;
-  case 1: launch(conv_split_kernel<4, 512>); break;
-  case 2: launch(conv_split_kernel<2, 256>); break;
-  case 3: launch(conv_split_kernel<2, 512>); break;
-  default: launch(conv_split_kernel<1, 512>);
+  case 0: launch(conv_split_kernel<3, 4, 256>); break;
+  case 1: launch(conv_split_kernel<3, 4, 512>); break;
+  case 2: launch(conv_split_kernel<3, 2, 256>); break;
+  case 3: launch(conv_split_kernel<3, 2, 512>); break;
+  case 4: launch(conv_split_kernel<3, 1, 512>); break;
+  case 5: launch(conv_split_kernel<5, 4, 384>); break;
+  default: launch(conv_split_kernel<5, 2, 384>);
   }
   return true;
 }
