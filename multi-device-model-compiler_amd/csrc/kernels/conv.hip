@@ -1576,13 +1576,14 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
       const int cus = numComputeUnits();
       split = convSplitPlan((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus, 0.97 * convWindowTime(SH, pixels, IC, OC, OW, cus));
     }
-    // 5 x 5 from 16 channels on likewise.  What the other kernels take is estimated low, by the matrix instructions of the rounds alone (0.131 to
-    // 0.25 us a round and channel were measured; 0.124 leaves some launches of one or two rounds with them: 248 tiles from 256 40 / 44 us, 567 from
-    // 16 9.9 / 9.7, 288 from 16 7.7 / 8.4, but 264 from 64 19.5 / 16.0, 438 from 32 12.5 / 10.8, 876 from 128 84 / 35).
-    if (KH == 5 && IC >= 16 && IC % 8 == 0) {
+    // 5 x 5 and 7 x 7 from 16 channels on likewise.  What the other kernels take is estimated low, by the matrix instructions of the rounds alone
+    // (5 x 5 0.131 to 0.25 us a round and channel were measured, 7 x 7 0.262 to 0.36; this leaves some launches of one or two rounds with them.
+    // us, other kernels / this, tiles of 32 x 32 - 5 x 5: 248 from 256 channels 40 / 42, 288 from 16 7.7 / 8.0, but 264 from 64 19.5 / 15.0, 438 from 32 12.5 / 10.3, 876 from
+    // 128 84 / 30; 7 x 7: 256 from 128 38.7 / 47.6, 210 from 64 20.7 / 26.8, but 286 from 64 38.5 / 27.1, 324 from 32 20.9 / 16.5, 545 from 16 19.4 / 12.8).
+    if (KH >= 5 && IC >= 16 && IC % (KH == 5 ? 8 : 4) == 0) {
       const int cus = numComputeUnits();
-      const double others = 3.0 + (double)((tiles + cus - 1) / cus) * 0.124 * (double)IC;
-      split = convSplitPlan5((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus, 0.97 * others);
+      const double others = 3.0 + (double)((tiles + cus - 1) / cus) * (KH == 5 ? 0.124 : 0.26) * (double)IC;
+      split = (KH == 5 ? convSplitPlan5 : convSplitPlan7)((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus, 0.97 * others);
     }
     // Few tiles on quarters or halves of them, where the estimates say so by 8 % (570 launches of up to 1300 quarters: 0.81 of the time on
     // average, the best choice everywhere would be 0.80, three of them 3 to 6 % slower; by 5 % 20 of them would be, of 24 channels).

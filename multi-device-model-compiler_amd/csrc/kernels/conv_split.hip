@@ -1,4 +1,4 @@
-// 3 x 3 and 5 x 5 convolution of fp32 tensors on the fp16 matrix cores, with fp32's accuracy.
+// 3 x 3, 5 x 5 and 7 x 7 convolution of fp32 tensors on the fp16 matrix cores, with fp32's accuracy.
 //
 // Every operand is taken apart into two fp16 numbers, v = scale * x = hi + lo with hi = fp16(v), lo = fp16(v - hi) and a scale
 // that is a power of two: 22 bits of the 24, and three products, hi.hi + (hi.lo + lo.hi), sum up in fp32.  What is left out is
@@ -26,11 +26,14 @@
 // and 64 pixels).  us, before / now, 3 x 3 pad 1: 12 x 256 x 10 x 46 -> 256 83 / 34, 12 x 256 x 240 x 36 -> 16 151 / 67, 17 x 128 x
 // 15 x 33 -> 128 46 / 20, 32 x 64 x 56 x 56 -> 64 77 / 53, 23 x 256 x 12 x 10 -> 256 40 / 25, 5 x 256 x 36 x 9 -> 256 26 / 21.
 //
-// 5 x 5: sixteen channels of its 25 positions, twice and as they are, would not fit the LDS.  A step has eight, and a matrix instruction's
-// sixteen products are two positions, one a lane half; the 26th is a filler of zeros, filter and pixels.  The consumers' reads set the
-// pace (1.7 us a step of 128 pixels, of which the matrix instructions are 0.5; three sets of operands on their way in place of two
-// spill).  us, before / now, stride 1 pad 2: 8 x 128 x 21 x 42 -> 128 81 / 34, 16 x 64 x 46 x 46 -> 64 120 / 56, 8 x 32 x 60 x 60 -> 64
-// 43 / 26, 4 x 256 x 30 x 30 -> 256 156 / 62.  Error against 64 bits 0.7e-7 to 1.6e-7 for K = 400 to 3200, 0.8e-7 to 2.1e-7 before.
+// 5 x 5 and 7 x 7: sixteen channels of their positions, twice and as they are, would not fit the LDS.  A step has eight or four, and a matrix
+// instruction's sixteen products are two positions, one a lane half, or four, two side by side in a lane's sixteen bytes.  Positions past the
+// window are fillers of zeros, filter and pixels.  The consumers' reads set the pace (1.5 us a step of 128 pixels, of which the matrix
+// instructions are 0.5; three sets of operands on their way in place of two spill; positions' distances by the vector unit in place of
+// scalars took 5 x 5 1.7 us, two positions of 7 x 7 that may lie in different rows, by four reads in place of two, 2.4).  us, before / now, stride 1:
+// 5 x 5 8 x 128 x 21 x 42 -> 128 81 / 30, 16 x 64 x 46 x 46 -> 64 120 / 51, 8 x 32 x 60 x 60 -> 64 43 / 24, 4 x 256 x 30 x 30 -> 256 156 / 55; 7 x 7,
+// tiles of 32 x 32, 1296 from 64 channels 140 / 61, 819 from 32 41 / 20, 432 from 128 70 / 46, 545 from 16 19.4 / 12.8.  Error against 64 bits 0.7e-7 to 1.6e-7
+// for K = 400 to 3200, 0.8e-7 to 2.1e-7 before; 7 x 7 0.9e-7 to 2.3e-7, 1.3e-7 to 3.4e-7 before.
 #include "common.hpp"
 #include "conv.hpp"
 #include "mfma.hpp"
@@ -75,18 +78,21 @@ __device__ __forceinline__ float powerOf2(int e) { return __builtin_bit_cast(flo
 
 // WIN: the window; KS: consumers that share their pixels; CAP: staged pixels at most
 template <int WIN, int KS_, int CAP_> struct SplitShape {
-  static constexpr int TAPS = WIN * WIN, CH = WIN == 3 ? 16 : 8, OCTETS = CH / 8; // positions; input channels of a step
-  // Matrix instructions' sets of sixteen products: a position of sixteen channels, or two of eight (the last one has a filler beside it).
-  static constexpr int PAIRED = 3 - OCTETS, SETS = (TAPS + PAIRED - 1) / PAIRED;
+  static constexpr int TAPS = WIN * WIN, CH = WIN == 3 ? 16 : WIN == 5 ? 8 : 4; // positions; input channels of a step
+  // Sixteen bytes hold eight channels of a position, or four of two.  A matrix instruction's set of sixteen products is two of them: a position
+  // of sixteen channels, two of eight (the last one with a filler beside it), or four of four, two and two side by side in a window row, of which
+  // the eighth is a filler.
+  static constexpr int OCTETS = CH == 16 ? 2 : 1, CPS = CH < 8 ? CH : 8, BESIDE = 8 / CPS; // channels and positions in sixteen bytes
+  static constexpr int PAIRED = 3 - OCTETS, UNITS = BESIDE == 2 ? WIN * 4 : TAPS, SETS = (UNITS + PAIRED - 1) / PAIRED;
   static constexpr int KS = KS_, CAP = CAP_, PXW = kConsumers / KS, PX = 32 * kPT * PXW;
-  static constexpr int UNIT = OCTETS * 2 * kOC * 16 + 80; // bytes of a position's filter values (the 80: positions side by side on different banks)
+  static constexpr int UNIT = OCTETS * 2 * kOC * 16 + 80; // bytes of a unit's filter values (the 80: units side by side on different banks)
   static constexpr int HALF = OCTETS == 2 ? 2 * kOC * 16 : UNIT; // from the values of a lane half to the other's
-  static constexpr int FILTER = SETS * PAIRED * UNIT, PIXELS = OCTETS * 2 * CAP * 16;
+  static constexpr int FILTER = SETS * PAIRED * UNIT, PXB = 2 * CPS, PIXELS = OCTETS * 2 * CAP * PXB; // PXB: bytes of a pixel's pieces
   static constexpr int ROW = CH * TAPS, PITCH = ROW + 4; // words of a channel's filter in a step
   static constexpr int RAW = kOC * PITCH * 4, RAWS = 3;
   static constexpr int LDS = 2 * (FILTER + PIXELS) + RAWS * RAW;
   static constexpr int RPW = kOC / kProducers; // filter rows a producer moves
-  static constexpr int ITEMS = kOC * OCTETS * TAPS; // eight channels of a position of a filter
+  static constexpr int ITEMS = kOC * OCTETS * UNITS; // sixteen bytes of a filter
   static constexpr int WI = (ITEMS + 64 * kProducers - 1) / (64 * kProducers), PI = (OCTETS * CAP + 64 * kProducers - 1) / (64 * kProducers);
   static_assert(CAP % 64 == 0 && ROW % 4 == 0 && ROW / 4 <= 64 && LDS + 1024 <= 160 * 1024, "whole wavefronts; a CU's LDS");
   static_assert(KS == 1 || kConsumers * kPT * 16 * 64 * 4 <= LDS, "the partial sums take the buffers' place");
@@ -98,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
                                                               const float *__restrict__ bias, float *__restrict__ y,
                                                               const float *__restrict__ add, SplitGeo g) {
   using S = SplitShape<WIN, KS, CAP>;
-  constexpr int PXW = S::PXW, PI = S::PI, WI = S::WI, RPW = S::RPW, TAPS = S::TAPS, SETS = S::SETS;
+  constexpr int PXW = S::PXW, PI = S::PI, WI = S::WI, RPW = S::RPW, TAPS = S::TAPS, SETS = S::SETS, CPS = S::CPS, PXB = S::PXB;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[S::LDS];
   __shared__ uint32_t wMax[kOC], xMax;
   __shared__ int wExp[kOC], bad, small;
@@ -170,34 +176,35 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
       const int n = divide(image, g.byStrips), iw = (image - n * g.strips) * g.stripW * g.SW + c - g.PWL;
       const bool in = half < S::OCTETS && px < staged && n < N && (unsigned)ih < (unsigned)H && (unsigned)iw < (unsigned)W;
       xoff[i] = in ? ((n - n0) * IC * HW + half * 8 * HW + ih * W + iw) * 4 : kOutside;
-      xlds[i] = (half * 2 * plane + px) * 16;
+      xlds[i] = (half * 2 * plane + px) * PXB;
     }
-    // ... and eight channels of a position of the filter
+    // ... and sixteen bytes of the filter
     int wraw[WI], wlds[WI], wch[WI];
-    bool wused[WI];
+    bool wused[WI], wlast[WI]; // wlast: its second position is a filler
 #pragma unroll
     for (int i = 0; i < WI; i++) {
       const int at = i * 64 * kProducers + ptid, e = at < S::ITEMS ? at : S::ITEMS - 1; // (past the end: the last one again)
-      const int pair = e / TAPS, tap = e - pair * TAPS;
+      const int pair = e / S::UNITS, unit = e - pair * S::UNITS;
       wused[i] = i * 64 * kProducers + pwave * 64 < S::ITEMS; // (uniform)
       wch[i] = pair / S::OCTETS;
-      wraw[i] = wch[i] * S::PITCH + pair % S::OCTETS * (8 * TAPS) + tap;
-      wlds[i] = tap * S::UNIT + (pair % S::OCTETS * 2 * kOC + wch[i]) * 16;
+      wraw[i] = wch[i] * S::PITCH + pair % S::OCTETS * (8 * TAPS) + (S::BESIDE == 2 ? unit / 4 * WIN + unit % 4 * 2 : unit);
+      wlast[i] = S::BESIDE == 2 && unit % 4 == 3;
+      wlds[i] = unit * S::UNIT + (pair % S::OCTETS * 2 * kOC + wch[i]) * 16;
     }
     const auto image = resource(x + (int64_t)n0 * IC * HW, (int64_t)(N - n0) * IC * HW);
     struct Pieces {
-      float v[PI][8];
+      float v[PI][CPS];
     };
     auto loadPixels = [&](Pieces &p, int step) {
       const int at = step * S::CH * HW * 4;
 #pragma unroll
       for (int i = 0; i < PI; i++)
 #pragma unroll
-        for (int k = 0; k < 8; k++) p.v[i][k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(image, xoff[i], at + k * HW * 4, 0));
+        for (int k = 0; k < CPS; k++) p.v[i][k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(image, xoff[i], at + k * HW * 4, 0));
     };
-    auto largest = [](const float (&v)[8], float m) {
+    auto largest = [](const auto &v, float m) {
 #pragma unroll
-      for (int k = 0; k < 8; k++) m = fmaxf(m, fabsf(v[k]));
+      for (const float f : v) m = fmaxf(m, fabsf(f));
       return m;
     };
     auto produce = [&](auto splitTag) { // the operands of every step, in pieces or as they are
@@ -210,7 +217,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
       }
       loadPixels(even, 0);
       loadPixels(odd, atMost(1));
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PI * 8 + RPW) : "memory"); // the filter of the first step has arrived
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PI * CPS + RPW) : "memory"); // the filter of the first step has arrived
       __syncthreads();
       if constexpr (SPLIT) {
         constexpr int LPR = 64 / RPW; // lanes a row
@@ -247,8 +254,27 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
           *reinterpret_cast<u32x4 *>(at) = u32x4{hi[0], hi[1], hi[2], hi[3]};
           *reinterpret_cast<u32x4 *>(at + second) = u32x4{lo[0], lo[1], lo[2], lo[3]};
         } else {
-          *reinterpret_cast<f32x4 *>(at) = f32x4{v[0], v[1], v[2], v[3]};
-          *reinterpret_cast<f32x4 *>(at + second) = f32x4{v[4], v[5], v[6], v[7]};
+          constexpr int FIRST = CPS / 2; // a position's channels come half and half
+          *reinterpret_cast<f32x4 *>(at) = f32x4{v[0], v[1], v[FIRST == 4 ? 2 : 4], v[FIRST == 4 ? 3 : 5]};
+          *reinterpret_cast<f32x4 *>(at + second) = f32x4{v[FIRST], v[FIRST + 1], v[6], v[7]};
+        }
+      };
+      auto putPixel = [&](const float (&v)[CPS], unsigned char *at) {
+        if constexpr (CPS == 8) {
+          put(v, xs, at, plane * PXB);
+        } else {
+          u32x2 hi, lo;
+          if constexpr (SPLIT) {
+            uint32_t h[2], l[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++) splitPair(v[2 * k] * xs, v[2 * k + 1] * xs, h[k], l[k]);
+            hi = u32x2{h[0], h[1]}, lo = u32x2{l[0], l[1]};
+          } else {
+            hi = u32x2{__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1])};
+            lo = u32x2{__builtin_bit_cast(uint32_t, v[2]), __builtin_bit_cast(uint32_t, v[3])};
+          }
+          *reinterpret_cast<u32x2 *>(at) = hi;
+          *reinterpret_cast<u32x2 *>(at + plane * PXB) = lo;
         }
       };
       int slot = 0;
@@ -258,7 +284,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
 #pragma unroll
           for (int i = 0; i < PI; i++) {
             if constexpr (SPLIT) xmost[i] = largest(p.v[i], xmost[i]);
-            if (piece(i) < S::OCTETS * blocks) put(p.v[i], xs, at + xlds[i], plane * 16);
+            if (piece(i) < S::OCTETS * blocks) putPixel(p.v[i], at + xlds[i]);
           }
           loadPixels(p, atMost(s + 2));
           at = smem + (s & 1) * S::FILTER;
@@ -267,13 +293,16 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
             if (!wused[i]) continue;
             float v[8];
 #pragma unroll
-            for (int k = 0; k < 8; k++) v[k] = raw[slot * (S::RAW / 4) + wraw[i] + k * TAPS];
+            for (int k = 0; k < 8; k++) {
+              v[k] = raw[slot * (S::RAW / 4) + wraw[i] + k % CPS * TAPS + k / CPS];
+              if (k >= CPS && wlast[i]) v[k] = 0.0f;
+            }
             if constexpr (SPLIT) wmost[i] = largest(v, wmost[i]);
             put(v, SPLIT ? ws[i] : 1.0f, at + wlds[i], kOC * 16);
           }
           loadFilter(atMost(s + 2), slot == 0 ? 2 : slot - 1); // (everybody is done with what was there: a step ago)
           slot = slot == 2 ? 0 : slot + 1;
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * 8 + RPW) : "memory"); // the filter of step s + 1 has arrived
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * CPS + RPW) : "memory"); // the filter of step s + 1 has arrived
         }
         __syncthreads();
       };
@@ -329,13 +358,14 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
     const int q = p0 + (pw * kPT + t) * 32 + l32;
     const Pixel p = pixelOf(q < g.pixels ? q : p0);
     const int n = divide(p.image, g.byStrips), col = (p.image - n * g.strips) * g.stripW + p.col;
-    bbase[t] = ((p.image * g.rows + p.row * g.SH - r0) * g.pitch + p.col * g.SW) * 16 + (S::OCTETS == 2 ? hl * (2 * 16) * plane : 0);
+    bbase[t] = ((p.image * g.rows + p.row * g.SH - r0) * g.pitch + p.col * g.SW) * PXB + (S::OCTETS == 2 ? hl * (2 * 16) * plane : 0);
     pix[t] = q < g.pixels && col < g.OW ? p.row * g.OW + col : -1;
     img[t] = n - n0;
   }
-  // The filler position's filter values are zeros, and taken for its pixels too (an infinity times 0 would be none).
-  constexpr int kFiller = TAPS * S::UNIT;
-  if constexpr (S::PAIRED == 2) {
+  // The filler unit's filter values are zeros, which are taken for its pixels too (an infinity times 0 would be none).
+  constexpr bool FILLED = S::UNITS % S::PAIRED != 0;
+  constexpr int kFiller = S::UNITS * S::UNIT;
+  if constexpr (FILLED) {
     if (tid < 2 * 64) *reinterpret_cast<u32x4 *>(smem + tid / 64 * S::FILTER + kFiller + tid % 64 * 16) = u32x4{0u, 0u, 0u, 0u};
   }
   f32x16 acc[kPT];
@@ -352,16 +382,34 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
     auto read = [&](Operands &o, int step, int set) {
       const unsigned char *wat = smem + (step & 1) * S::FILTER + hl * S::HALF + l32 * 16 + set * (S::PAIRED * S::UNIT);
       const int pixelsAt = 2 * S::FILTER + (step & 1) * S::PIXELS;
-      const int tap = S::PAIRED == 2 ? 2 * set + hl : set;
-      const int ky = tap / WIN, kx = tap - ky * WIN, off = (ky * g.DH * g.pitch + kx * g.DW) * 16;
-      const bool filler = S::PAIRED == 2 && tap == TAPS;
+      const unsigned char *xat = smem + pixelsAt;
+      // (by scalars, and a selection between the lane halves)
+      auto distance = [&](int unit) {
+        const int ky = S::BESIDE == 2 ? unit / 4 : unit / WIN, kx = S::BESIDE == 2 ? unit % 4 * 2 : unit - ky * WIN;
+        return (ky * g.DH * g.pitch + kx * g.DW) * PXB;
+      };
+      const int off = S::PAIRED == 2 && hl ? distance(2 * set + 1) : distance(S::PAIRED * set);
+      const bool filler = FILLED && hl && set == SETS - 1;
       o.ah = *reinterpret_cast<const f16x8 *>(wat);
       o.al = *reinterpret_cast<const f16x8 *>(wat + kOC * 16);
 #pragma unroll
       for (int t = 0; t < kPT; t++) {
-        const int at = filler ? kFiller : pixelsAt + bbase[t] + off;
-        o.bh[t] = *reinterpret_cast<const f16x8 *>(smem + at);
-        o.bl[t] = *reinterpret_cast<const f16x8 *>(smem + at + (filler ? 0 : plane * 16));
+        if constexpr (S::PAIRED == 1) {
+          o.bh[t] = *reinterpret_cast<const f16x8 *>(xat + bbase[t] + off);
+          o.bl[t] = *reinterpret_cast<const f16x8 *>(xat + bbase[t] + off + plane * PXB);
+          continue;
+        }
+        const int at = filler ? kFiller : pixelsAt + bbase[t] + off, lower = at + (filler ? 0 : plane * PXB);
+        if constexpr (S::BESIDE == 1) {
+          o.bh[t] = *reinterpret_cast<const f16x8 *>(smem + at);
+          o.bl[t] = *reinterpret_cast<const f16x8 *>(smem + lower);
+        } else { // (eight bytes of either pixel; behind the last one of a row lies what is none of the window's)
+          const f16x4 none = {}, *h = reinterpret_cast<const f16x4 *>(smem + at), *l = reinterpret_cast<const f16x4 *>(smem + lower);
+          f16x4 h1 = h[1], l1 = l[1];
+          if (hl && set % 2) h1 = none, l1 = none;
+          o.bh[t] = __builtin_shufflevector(h[0], h1, 0, 1, 2, 3, 4, 5, 6, 7);
+          o.bl[t] = __builtin_shufflevector(l[0], l1, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
       }
     };
     auto mma = [&](const Operands &o) {
@@ -412,7 +460,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
 #pragma unroll
         for (int t = 0; t < kPT; t++) {
           float m = 0.0f;
-          const int base = bbase[t] / 16 - (S::OCTETS == 2 ? hl * plane : 0); // (a lane half has a plane of pixels and one of lower pieces each)
+          const int base = bbase[t] / PXB - (S::OCTETS == 2 ? hl * plane : 0); // (a lane half has a plane of pixels and one of lower pieces each)
           for (int ky = 0; ky < WIN; ky++)
             for (int kx = 0; kx < WIN; kx++) m = fmaxf(m, maxima[base + ky * g.DH * g.pitch + kx * g.DW]);
           m = halves_max(m);
@@ -492,14 +540,14 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
 
 // The tiles, and what a launch in them takes: us = start + rounds of the CUs * (block + step * steps), fitted to 800 launches of
 // each of the larger two of 3 x 3, 450 and 280 of the others (a tenth to a ninetieth percentile of 0.93 to 1.08 times what was measured), and
-// to 80 of 5 x 5.
+// to some 40 each of 5 x 5 and 7 x 7 (0.95 to 1.04).
 struct SplitTile {
   int pixels, cap;
   double start, block, step;
 };
 constexpr SplitTile kTiles[] = {{64, 256, 1.5, 4.7, 0.89}, {64, 512, 1.5, 5.1, 1.08}, {128, 256, 1.4, 5.5, 1.10}, {128, 512, 1.3, 6.0, 1.20}, {256, 512, 0.7, 7.5, 1.42},
-                                {64, 384, 1.4, 4.45, 1.173}, {128, 384, 1.2, 5.1, 1.68}};
-constexpr int kTiles3 = 5, kTiles5 = 2; // of 3 x 3, and behind them of 5 x 5
+                                {64, 384, 1.2, 4.6, 1.085}, {128, 384, 1.2, 5.1, 1.49}, {64, 704, 1.1, 4.85, 1.247}, {128, 704, 0.75, 5.7, 1.55}};
+constexpr int kTiles3 = 5, kTiles5 = 2, kTiles7 = 2; // of 3 x 3, and behind them of 5 x 5 and 7 x 7
 
 // The cheapest of tiles first .. first + count - 1, if it takes less than `limit` us.
 ConvSplitPlan cheapest(int first, int count, int win, int step, int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit) {
@@ -536,6 +584,10 @@ ConvSplitPlan convSplitPlan(int N, int IC, int OC, int OH, int OW, int SH, int S
 ConvSplitPlan convSplitPlan5(int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit) {
   return cheapest(kTiles3, kTiles5, 5, 8, N, IC, OC, OH, OW, SH, SW, DH, DW, cus, limit);
 }
+ConvSplitPlan convSplitPlan7(int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit) {
+  if (DW != 1) return ConvSplitPlan{0, 0, limit}; // (two positions of a row come as sixteen bytes side by side)
+  return cheapest(kTiles3 + kTiles5, kTiles7, 7, 4, N, IC, OC, OH, OW, SH, SW, DH, DW, cus, limit);
+}
 
 // Launches it; false where its indices would not fit.
 bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const float *bias, float *y, const float *add, int64_t N, int64_t IC,
@@ -543,12 +595,12 @@ bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const 
                int64_t DW, bool relu, hipStream_t stream) {
   auto fits = [](int64_t v) { return v >= 0 && v <= 0x7fffffff; };
   const int64_t strips = plan.strips, width = (OW + strips - 1) / strips, pixels = N * strips * OH * width, tilePixels = kTiles[plan.tile].pixels;
-  const int win = plan.tile < kTiles3 ? 3 : 5, taps = win * win;
+  const int win = plan.tile < kTiles3 ? 3 : plan.tile < kTiles3 + kTiles5 ? 5 : 7, taps = win * win;
   const int64_t pitch = (width - 1) * SW + (win - 1) * DW + 1, rows = (OH - 1) * SH + (win - 1) * DH + 1;
   const int64_t pxTiles = (pixels + tilePixels - 1) / tilePixels, ocTiles = (OC + kOC - 1) / kOC, blocks = pxTiles * ocTiles;
   // pixel, row and byte indices from a tile's first image on are 32 bits wide, the filter's from a channel on; a grid's threads are fewer than 2^32
   const int64_t images = (tilePixels - 2) / (OH * width) + 2;
-  if (!aligned16(w) || !fits(pixels + tilePixels) || !fits(N * strips * rows + tilePixels * SH) || !fits(images * IC * H * W * 4) ||
+  if ((win == 7 && DW != 1) || !aligned16(w) || !fits(pixels + tilePixels) || !fits(N * strips * rows + tilePixels * SH) || !fits(images * IC * H * W * 4) ||
       !fits(images * OC * OH * OW * 4) || !fits(IC * taps * 4) || blocks * kThreads >= (int64_t(1) << 32))
     return false;
   const SplitGeo g{(int)OH,    (int)OW, (int)PHL, (int)PWL,   (int)SH, (int)SW, (int)DH, (int)DW, (int)strips, (int)width, (int)pitch, (int)rows, (int)pixels,
@@ -564,7 +616,9 @@ bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const 
   case 3: launch(conv_split_kernel<3, 2, 512>); break;
   case 4: launch(conv_split_kernel<3, 1, 512>); break;
   case 5: launch(conv_split_kernel<5, 4, 384>); break;
-  default: launch(conv_split_kernel<5, 2, 384>);
+  case 6: launch(conv_split_kernel<5, 2, 384>); break;
+  case 7: launch(conv_split_kernel<7, 4, 704>); break;
+  default: launch(conv_split_kernel<7, 2, 704>);
   }
   return true;
 }

@@ -184,8 +184,7 @@ int convStagedWaves(int win, int64_t stride, int64_t pixels, int64_t IC, int64_t
 bool convByPatches(int win, int stride, int64_t tiles, int64_t rowTiles, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
 // How long the kernels above take for a 3 x 3 convolution, in us (see conv.hip).
 double convWindowTime(int64_t stride, int64_t pixels, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
-// 3 x 3 and 5 x 5 on the fp16 matrix cores in pairs of fp16 numbers (conv_split.hip), from 32 channels that are a multiple of 16 on, or 16 that are
-// one of 8: the tile and the strips of columns that take the least time (strips 0: none less than `limit` us), and the launch (false: not for
+// 3 x 3, 5 x 5 and 7 x 7 on the fp16 matrix cores in pairs of fp16 numbers (conv_split.hip), of channels that are a multiple of 16, 8 and 4: the tile and the strips of columns that take the least time (strips 0: none less than `limit` us), and the launch (false: not for
 // these sizes or pointers).
 struct ConvSplitPlan {
   int tile, strips;
@@ -193,6 +192,7 @@ struct ConvSplitPlan {
 };
 ConvSplitPlan convSplitPlan(int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit);
 ConvSplitPlan convSplitPlan5(int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit);
+ConvSplitPlan convSplitPlan7(int N, int IC, int OC, int OH, int OW, int SH, int SW, int DH, int DW, int cus, double limit);
 bool convSplit(const ConvSplitPlan &plan, const float *x, const float *w, const float *bias, float *y, const float *add, int64_t N, int64_t IC,
                int64_t H, int64_t W, int64_t OC, int64_t OH, int64_t OW, int64_t PHL, int64_t PWL, int64_t SH, int64_t SW, int64_t DH,
                int64_t DW, bool relu, hipStream_t stream);
