@@ -1568,9 +1568,9 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     else if (IC == 1) go(integral_constant<int, 7>(), c4);
     else go(integral_constant<int, 7>(), integral_constant<int, 11>());
   } else if (squareWindow) {
-    // 3 x 3 from 32 channels on in pairs of fp16 numbers, where both estimates say that this is faster (500 shapes of 0.15 GFLOP
-    // on: taken by 268, 0.83 of the time over all of them, the largest ones 0.39, none more than 2 % slower).  (16 channels are
-    // one step: no gain, and the fp32 instructions' sums are the more exact ones.)
+    // 3 x 3 from 32 channels on in three bf16 numbers, where both estimates say that this is faster (700 shapes: taken by 267, 0.91 of the
+    // time over all of them where the best choice everywhere would be 0.907, the largest ones 0.5 to 0.6, two 5 to 6 % slower).  (16 channels are one
+    // step: no gain.)
     ConvSplitPlan split{0, 0, 0.0};
     if (KH == 3 && IC >= 32 && IC % 16 == 0) {
       const int cus = numComputeUnits();
@@ -1578,12 +1578,12 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     }
     // 5 x 5 and 7 x 7 from 16 channels on likewise.  What the other kernels take is estimated low, by the matrix instructions of the rounds alone
     // (5 x 5 0.131 to 0.25 us a round and channel were measured, 7 x 7 0.262 to 0.36; this leaves some launches of one or two rounds with them.
-    // us, other kernels / this, tiles of 32 x 32 - 5 x 5: 248 from 256 channels 40 / 42, 288 from 16 7.7 / 8.0, but 264 from 64 19.5 / 15.0, 438 from 32 12.5 / 10.3, 876 from
-    // 128 84 / 30; 7 x 7: 256 from 128 38.7 / 47.6, 210 from 64 20.7 / 26.8, but 286 from 64 38.5 / 27.1, 324 from 32 20.9 / 16.5, 545 from 16 19.4 / 12.8).
+    // 500 shapes each: taken by 168 and 175, 0.886 and 0.908 of the time over all of them where the best choice would be 0.875 and 0.902, none
+    // slower; an estimate a tenth higher, 0.881 and 0.905, is up to 10 % wrong).
     if (KH >= 5 && IC >= 16 && IC % (KH == 5 ? 8 : 4) == 0) {
       const int cus = numComputeUnits();
-      const double others = 3.0 + (double)((tiles + cus - 1) / cus) * (KH == 5 ? 0.124 : 0.26) * (double)IC;
-      split = (KH == 5 ? convSplitPlan5 : convSplitPlan7)((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus, 0.97 * others);
+      const double others = 3.0 + (double)((tiles + cus - 1) / cus) * (KH == 5 ? 0.13 : 0.27) * (double)IC;
+      split = (KH == 5 ? convSplitPlan5 : convSplitPlan7)((int)N, (int)IC, (int)OC, (int)OH, (int)OW, (int)SH, (int)SW, (int)DH, (int)DW, cus, others);
     }
     // Few tiles on quarters or halves of them, where the estimates say so by 8 % (570 launches of up to 1300 quarters: 0.81 of the time on
     // average, the best choice everywhere would be 0.80, three of them 3 to 6 % slower; by 5 % 20 of them would be, of 24 channels).

@@ -44,4 +44,15 @@ __device__ __forceinline__ void splitPair(float a, float b, uint32_t &hi, uint32
   asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(lo) : "v"(ra), "v"(rb));
 }
 
+// a and b as three bf16 numbers each, the first of which is the nearest, the second the nearest to what that leaves: all 24 bits (as long
+// as the last one is no subnormal: from 2^-110 on).
+__device__ __forceinline__ void splitTriple(float a, float b, uint32_t (&piece)[3]) {
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(piece[i]) : "v"(a), "v"(b));
+    a -= __builtin_bit_cast(float, piece[i] << 16);
+    b -= __builtin_bit_cast(float, piece[i] & 0xffff0000u);
+  }
+}
+
 } // namespace mgpu

@@ -184,8 +184,9 @@ int convStagedWaves(int win, int64_t stride, int64_t pixels, int64_t IC, int64_t
 bool convByPatches(int win, int stride, int64_t tiles, int64_t rowTiles, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
 // How long the kernels above take for a 3 x 3 convolution, in us (see conv.hip).
 double convWindowTime(int64_t stride, int64_t pixels, int64_t IC, int64_t OC, int64_t OW, int64_t cus);
-// 3 x 3, 5 x 5 and 7 x 7 on the fp16 matrix cores in pairs of fp16 numbers (conv_split.hip), of channels that are a multiple of 16, 8 and 4: the tile and the strips of columns that take the least time (strips 0: none less than `limit` us), and the launch (false: not for
-// these sizes or pointers).
+// 3 x 3, 5 x 5 and 7 x 7 on the bf16 matrix cores in three bf16 numbers (conv_split.hip), of channels that are a multiple of 16, 8 and 4: the
+// tile and the strips of columns that take the least time (strips 0: none less than `limit` us), and the launch (false: not for these
+// sizes or pointers).
 struct ConvSplitPlan {
   int tile, strips;
   double us;

@@ -1,5 +1,5 @@
-"""3 x 3 convolution in pairs of fp16 numbers (csrc/kernels/conv_split.hip): that its tiles' input rows fit their place in LDS, which
-convolutions it takes, and its results against the oracle and against 64 bits, on operands that the pairs hold and on others."""
+"""3 x 3 convolution in three bf16 numbers (csrc/kernels/conv_split.hip): that its tiles' input rows fit their place in LDS, which
+convolutions it takes, and its results against the oracle and against 64 bits, on operands of every size."""
 import ctypes
 import random
 
@@ -14,7 +14,7 @@ class Plan(ctypes.Structure):
     _fields_ = [("tile", ctypes.c_int), ("strips", ctypes.c_int), ("us", ctypes.c_double)]
 
 
-TILES = [(64, 256), (64, 512), (128, 256), (128, 512), (256, 512)]  # pixels, staged pixels at most
+TILES = [(64, 256), (64, 448), (128, 256), (128, 448), (256, 448)]  # pixels, staged pixels at most
 
 
 def plan_of(pkg, *args, limit=1e9):
@@ -101,6 +101,19 @@ def test_against_the_oracle(pkg, gpu, oracle, rng, tile, N, IC, H, W, OC, pad, s
 
 KINDS = ["normal", "tiny", "huge", "dark half", "outlier", "growing", "growing filter", "zero channels", "zero filter channels", "dead filters", "zeros",
          "inf", "inf filter", "nan"]
+# Values that are small beside others of the same window, by channel, by pixel and by image, which the filter brings up again or has alone.
+UNEVEN = ["channels 1e-4", "channels 1e-6", "channels 1e-9", "selected 1e-6", "selected 1e-12", "selected beside an outlier", "last channels", "dim image",
+          "near the smallest"]
+
+
+def uneven(kind, x, w):
+    r = float(kind.split()[-1]) if "1e-" in kind else 1e-7
+    if kind.startswith("channels"): x[:, 1::2] *= r; w[:, ::2] *= r  # noqa: E702
+    if kind.startswith("selected"): x[:, 1::2] *= r; w[:, ::2] = 0  # noqa: E702
+    if kind == "selected beside an outlier": x[:, 1, 3, 3] = 1.0
+    if kind == "last channels": x[:, -1] *= r; w[:, :-1] *= r  # noqa: E702
+    if kind == "dim image": x[1, 1::2] *= r; w[:, ::2] *= r  # noqa: E702
+    if kind == "near the smallest": x *= 1e-36; w *= 1e8  # noqa: E702
 
 
 def operands(kind, N, IC, H, W, OC, device):
@@ -121,11 +134,12 @@ def operands(kind, N, IC, H, W, OC, device):
     if kind == "inf": x[0, c - 1, 4, 4] = float("inf")
     if kind == "inf filter": w[3, c, 1, 1] = float("-inf")
     if kind == "nan": x[1, c - 1, 5, 6], w[2, c - 1, 0, 0] = float("nan"), float("nan")
+    if kind in UNEVEN: uneven(kind, x, w)
     return x, w
 
 
 def check(got, x, w, kind):
-    """Against 64 bits, elementwise to the size of the products summed up: what the pairs do not hold goes the fp32 way."""
+    """Against 64 bits, elementwise to the size of the products summed up: infinities and NaNs go the fp32 way."""
     import torch
     H, W = x.shape[2:]
     conv = lambda x, w: sum(torch.nn.functional.pad(x, (1, 1, 1, 1))[:, None, :, i:i + H, j:j + W].mul(w[None, :, :, i, j, None, None]).sum(2)  # noqa: E731
@@ -139,12 +153,25 @@ def check(got, x, w, kind):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("kind", KINDS + UNEVEN)
 def test_operands_of_every_size(pkg, gpu, kind):
     import torch
     x, w = operands(kind, 2, 64, 14, 16, 40, gpu)
     for tile in (0, 4):
         check(split_conv(pkg, tile, 1, x, w, torch.zeros(40, device=gpu), None, (1, 1, 1, 1), (1, 1), (1, 1), False), x, w, kind)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [0, 2, 4])
+def test_an_image_for_itself(pkg, gpu, tile):
+    """The bits of an image's result, whatever the images are that share its tiles."""
+    import torch
+    x, w = operands("normal", 3, 48, 7, 9, 40, gpu)
+    b = torch.randn(40, device=gpu)
+    alone = split_conv(pkg, tile, 1, x[1:2].contiguous(), w, b, None, (1, 1, 1, 1), (1, 1), (1, 1), False)
+    for value in (1.0, 1e-8, 1e8, float("inf"), float("nan")):
+        x[0], x[2] = x[0] * 1e4, value
+        assert torch.equal(split_conv(pkg, tile, 1, x, w, b, None, (1, 1, 1, 1), (1, 1), (1, 1), False)[1:2], alone), value
 
 
 @pytest.mark.gpu
