@@ -876,7 +876,7 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
       }
       const float m = fmaxf(fmaxf(window[0], window[1]), fmaxf(window[2], window[3]));
       const int e = pairExponent(m);
-      const float scale = powerOf2(e), down = powerOf2(-e) * wDown;
+      const float scale = powerOf2(e), down = powerOf2(-e); // (times wDown it may be no number: one after the other)
       bool low = false;
 #pragma unroll
       for (int j = 0; j < 4; j++) low |= window[j] > 0.0f && window[j] * scale < kLeastInPairs;
@@ -910,7 +910,7 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
           for (int i = 0; i < STEPS; i++) sum = product(ah[i], bh[i], sum);
           acc[j] = sum;
         }
-        store(acc, [&](int r, float v) { return fmaf(v, down, bv[r]); });
+        store(acc, [&](int r, float v) { return fmaf(v * down, wDown, bv[r]); });
         return;
       }
     }

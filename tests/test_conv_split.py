@@ -182,3 +182,15 @@ def test_operands_of_every_size_in_a_stem(pkg, gpu, kind, IC):
     import torch
     x, w = operands(kind, 2, IC, 64, 64, 250, gpu)
     check(pkg.conv2d(x, w, torch.zeros(250, device=gpu), pad=(1, 1, 1, 1)), x, w, kind)
+
+
+@pytest.mark.gpu
+def test_a_stem_of_nothing_beside_large_values(pkg, gpu):
+    """Where the other products overflow, a filter of zeros and a window of zeros still give the bias."""
+    import torch
+    x, w = operands("normal", 2, 3, 64, 64, 250, gpu)
+    b = torch.randn(250, device=gpu)
+    x, w = x * 1e25, w * 1e25
+    x[:, :, 8:16, 8:16], w[77] = 0, 0
+    got = pkg.conv2d(x, w, b, pad=(1, 1, 1, 1))
+    assert torch.equal(got[:, 77], b[77].expand(2, 64, 64)) and torch.equal(got[:, :, 9:15, 9:15], b[:, None, None].expand(2, 250, 6, 6))
