@@ -564,13 +564,6 @@ __global__ __launch_bounds__(64 * KS, 2) void conv_staged_kernel(const float *__
   finishTile<1, KS, uint32_t>(acc, partial, 0, ks, bias, add, y, OC, P, oc0, nFirst, img, pix, lane, relu);
 }
 
-// Scales for pairs of fp16 numbers: the largest value to 2^7 .. 2^8, where pairs hold sizes from kLeastInPairs on.  Largest values
-// beyond 2^100, or under 2^-100 and not 0, are left to the fp32 instructions.
-constexpr float kLeastInPairs = 0.25f;
-__device__ __forceinline__ bool pairsHold(float most) { return most == 0.0f || (most >= 0x1p-100f && most <= 0x1p100f); }
-__device__ __forceinline__ int pairExponent(float most) { return most == 0.0f ? 0 : 134 - (int)(__builtin_bit_cast(uint32_t, most) >> 23); }
-__device__ __forceinline__ float powerOf2(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
-
 // ---- few taps -----------------------------------------------------------------------------
 // A reduction of at most 2 NS taps (a network's stem: 3 channels, 3 x 3).  A wavefront keeps the
 // filter of its OCT x 32 channels in registers, lane half hl the taps 2 s + hl of step s, and walks
@@ -717,11 +710,11 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
 // 256 x 256 -> 64, 268 MB: 76.9 -> 65.5 us (1 x 1 from the same: 68.0 -> 49.2; a fill of as many bytes takes 39); 8 x 3 x 224 x
 // 224 -> 64 with a postAdd 87 -> 49; 8 x 3 x 128 x 128 -> 16 11.0 -> 6.7.  Stores of one tile dealt out between the matrix
 // instructions of the next measured the same, an order of tiles by XCD too, runs of tiles a wavefront 90.
-// SPLIT: the products by the fp16 matrix instructions, operands taken apart into pairs of fp16 numbers as in conv_split.hip: six
-// steps of 32 clocks instead of 15 of 64, and fewer roundings (K = 27: error against 64 bits 1.1e-7 -> 0.67e-7).  A quad's pixels
-// have a scale of their own, each tile: whole windows that are small beside their neighbours', infinities and filters of which a
-// channel is small beside the others take the fp32 instructions.  us, before / now: 16 x 3 x 256 x 256 -> 64 59 / 54, 16 x 3 x
-// 224 x 224 -> 64 58 / 47, 4 x 3 x 224 x 224 -> 64 17.2 / 12.6, 16 x 3 x 76 x 248 -> 33 of stride 2 down 14.8 / 9.8.
+// SPLIT: the products by the bf16 matrix instructions, operands taken apart into three numbers as in conv_split.hip: twelve steps of
+// 32 clocks instead of 15 of 64, and fewer roundings (K = 27: error against 64 bits 1.1e-7 -> 0.39e-7).  A tile with values so large that
+// they or their sums might be none in pieces is done again behind the others, and what is no number takes the fp32 instructions'
+// result.  us, fp32 instructions / this: 16 x 3 x 256 x 256 -> 64 54.9 / 54.2, 16 x 3 x 224 x 224 -> 64 47.9 / 40.6, 4 x 3 x 224 x 224 -> 64 16.2 / 13.9, 16
+// x 3 x 76 x 248 -> 33 19.0 / 15.1, 8 x 1 x 112 x 112 -> 64, 5 x 5, 10.7 / 8.8; of two channels 16.7 / 16.8 (16 x 2 x 128 x 128 -> 64).
 template <int KW, int NR, Output OUT, bool ADDED, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                             const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
@@ -742,39 +735,43 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
     const bool in = r < rows;
     toff[i] = in ? (ic * g.H + kh * g.DH) * g.W * 4 : 0;
     tkh[i] = in ? kh : 31;
+  }
+  auto loadFilter = [&]() { // the lane's channel, rows of its half
     const int oc = oc0 + l32 < OC ? oc0 + l32 : OC - 1;
 #pragma unroll
-    for (int k = 0; k < KW; k++) a[i][k] = in ? w[((int64_t)oc * rows + r) * KW + k] : 0.0f;
-  }
+    for (int i = 0; i < NR; i++) {
+      const int r = hl * NR + i;
+#pragma unroll
+      for (int k = 0; k < KW; k++) a[i][k] = r < rows ? w[((int64_t)oc * rows + r) * KW + k] : 0.0f;
+    }
+  };
+  loadFilter();
   float bv[16];
 #pragma unroll
   for (int r = 0; r < 16; r++) {
     const int oc = oc0 + 8 * (r / 4) + r % 4 + 4 * hl;
     bv[r] = bias[oc < OC ? oc : OC - 1];
   }
-  // SPLIT: the lane half's taps as eight each of STEPS matrix instructions, in the order of its rows, in pairs of fp16 numbers.
+  // SPLIT: the lane half's taps as eight each of STEPS matrix instructions, in the order of its rows, in pieces.
   constexpr int TAPS = NR * KW, STEPS = (TAPS + 7) / 8;
-  u32x4 ah[STEPS], al[STEPS];
-  float wDown = 1.0f;  // undoes the filter's scale
-  bool pairs = SPLIT;  // whether they hold the filter (uniform)
-  if constexpr (SPLIT) {
-    float m = 0.0f; // of the lane's channel
-#pragma unroll
-    for (int i = 0; i < TAPS; i++) m = fmaxf(m, fabsf(a[i / KW][i % KW]));
-    m = halves_max(m);
-    const float most = group_max<64>(m);
-    const int e = pairExponent(most);
-    const float scale = powerOf2(e);
-    wDown = powerOf2(-e);
-    pairs = __builtin_amdgcn_ballot_w64(!pairsHold(most) || (m > 0.0f && m * scale < kLeastInPairs)) == 0;
+  u32x4 ap[kPieces][STEPS];
+  float most = 0.0f; // pixels below this are finite in pieces, and so are their sums (uniform)
+  auto inPieces = [&](u32x4 (&piece)[kPieces][STEPS], auto &&tap) { // tap: of the lane half's, by number
 #pragma unroll
     for (int i = 0; i < 4 * STEPS; i++) {
-      auto tap = [&](int k) { return k < TAPS ? a[k / KW][k % KW] * scale : 0.0f; };
-      uint32_t hi, lo;
-      splitPair(tap(2 * i), tap(2 * i + 1), hi, lo);
-      ah[i / 4][i % 4] = hi;
-      al[i / 4][i % 4] = lo;
+      uint32_t p[kPieces];
+      splitTriple(2 * i < TAPS ? tap(2 * i) * kSplitScale : 0.0f, 2 * i + 1 < TAPS ? tap(2 * i + 1) * kSplitScale : 0.0f, p);
+#pragma unroll
+      for (int k = 0; k < kPieces; k++) piece[k][i / 4][i % 4] = p[k];
     }
+  };
+  if constexpr (SPLIT) {
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TAPS; i++) m = fmaxf(m, fabsf(a[i / KW][i % KW]));
+    m = group_max<64>(m);
+    if (m < 0x1p100f) most = fminf(0x1p100f, 0x1p74f / fmaxf(m, 0x1p-26f)); // (32 products of less than 2^74 and two scales of 2^24)
+    inPieces(ap, [&](int k) { return a[k / KW][k % KW]; });
   }
   struct Tile {
     int pix, img, nFirst; // the lane's first pixel (-1: past the end), its image less the tile's first, that image
@@ -812,7 +809,9 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
     }
   };
   const int64_t outElems = (int64_t)OC * P;
-  auto finish = [&](Tile &o) {
+  bool rest = false; // SPLIT: may there be sums that are no numbers in pieces? (uniform)
+  auto finish = [&](Tile &o, auto againTag) {
+    constexpr bool AGAIN = decltype(againTag)::value;
     const auto out = resource(y + o.nFirst * outElems, (N - o.nFirst) * outElems);
     const int at = o.pix < 0 ? kOutside : ((o.img * OC + oc0 + 4 * hl) * P + o.pix) * 4;
     int row = P * 4, channels = OC;
@@ -846,9 +845,9 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
         c[e] = v;
       }
     };
-    auto store = [&](const f32x16 (&acc)[4], auto &&value) { // value(register, accumulator's)
+    auto store = [&](const f32x16 (&acc)[4]) {
       everyChannel([&](int r, int voffset, int soffset) {
-        f32x4 v = {value(r, acc[0][r]), value(r, acc[1][r]), value(r, acc[2][r]), value(r, acc[3][r])};
+        f32x4 v = {acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
         if (ADDED) v += kEarly ? addend[r] : fromPost(voffset, soffset);
         // cuDNN's ReLU with CUDNN_NOT_PROPAGATE_NAN maps NaN to 0, as fmaxf does
         if (relu) v = f32x4{fmaxf(v[0], 0.0f), fmaxf(v[1], 0.0f), fmaxf(v[2], 0.0f), fmaxf(v[3], 0.0f)};
@@ -856,89 +855,84 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
                                                OUT == Output::Streamed ? 2 : OUT == Output::Through ? 16 : 0);
       });
     };
+    f32x16 acc[4];
     if constexpr (SPLIT) {
-      // One scale for the quad, from the largest value of its windows; of each pixel's window the pairs have to hold it, too.
-      float c[NR][KW + 3], column[KW + 3], window[4];
-#pragma unroll
-      for (int e = 0; e < KW + 3; e++) column[e] = 0.0f;
+      float c[NR][KW + 3], m = 0.0f;
 #pragma unroll
       for (int i = 0; i < NR; i++) {
         columns(i, c[i]);
 #pragma unroll
-        for (int e = 0; e < KW + 3; e++) column[e] = fmaxf(column[e], fabsf(c[i][e]));
+        for (int e = 0; e < KW + 3; e++) m = fmaxf(m, fabsf(c[i][e]));
       }
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        window[j] = column[j];
+        u32x4 bp[kPieces][STEPS];
+        inPieces(bp, [&](int k) { return c[k / KW][k % KW + j]; });
+        f32x16 sum;
 #pragma unroll
-        for (int k = 1; k < KW; k++) window[j] = fmaxf(window[j], column[j + k]);
-        window[j] = halves_max(window[j]);
+        for (int i = 0; i < 16; i++) sum[i] = 0.0f;
+        // (the small products first: their roundings are small, too)
+#pragma unroll
+        for (int order = kPieces - 1; order >= 0; order--)
+#pragma unroll
+          for (int k = 0; k <= order; k++)
+#pragma unroll
+            for (int i = 0; i < STEPS; i++)
+              sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ap[k][i]), __builtin_bit_cast(bf16x8, bp[order - k][i]), sum, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[j][i] = fmaf(sum[i], kSplitUnscale, bv[i]);
       }
-      const float m = fmaxf(fmaxf(window[0], window[1]), fmaxf(window[2], window[3]));
-      const int e = pairExponent(m);
-      const float scale = powerOf2(e), down = powerOf2(-e); // (times wDown it may be no number: one after the other)
-      bool low = false;
-#pragma unroll
-      for (int j = 0; j < 4; j++) low |= window[j] > 0.0f && window[j] * scale < kLeastInPairs;
-      if (pairs && __builtin_amdgcn_ballot_w64(low || !pairsHold(m)) == 0) {
-#pragma unroll
-        for (int i = 0; i < NR; i++)
-#pragma unroll
-          for (int k = 0; k < KW + 3; k++) c[i][k] *= scale;
-        f32x16 acc[4];
+      const bool numbers = __builtin_amdgcn_ballot_w64(!(m < most)) == 0; // (a NaN is one in either way)
+      if constexpr (AGAIN) {
+        if (numbers) return;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-          u32x4 bh[STEPS], bl[STEPS];
+          f32x16 plain;
 #pragma unroll
-          for (int i = 0; i < 4 * STEPS; i++) {
-            auto tap = [&](int k) { return k < TAPS ? c[k / KW][k % KW + j] : 0.0f; };
-            uint32_t hi, lo;
-            splitPair(tap(2 * i), tap(2 * i + 1), hi, lo);
-            bh[i / 4][i % 4] = hi;
-            bl[i / 4][i % 4] = lo;
-          }
-          auto product = [&](const u32x4 &u, const u32x4 &v, const f32x16 &to) {
-            return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, u), __builtin_bit_cast(f16x8, v), to, 0, 0, 0);
-          };
-          // (the small products first: their roundings are small, too)
-          f32x16 sum;
+          for (int i = 0; i < 16; i++) plain[i] = bv[i];
 #pragma unroll
-          for (int i = 0; i < 16; i++) sum[i] = 0.0f;
+          for (int i = 0; i < TAPS; i++) plain = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i / KW][i % KW], c[i / KW][i % KW + j], plain, 0, 0, 0);
 #pragma unroll
-          for (int i = 0; i < STEPS; i++) sum = product(ah[i], bl[i], product(al[i], bh[i], sum));
-#pragma unroll
-          for (int i = 0; i < STEPS; i++) sum = product(ah[i], bh[i], sum);
-          acc[j] = sum;
+          for (int i = 0; i < 16; i++) acc[j][i] = fabsf(acc[j][i]) < __builtin_inff() ? acc[j][i] : plain[i];
         }
-        store(acc, [&](int r, float v) { return fmaf(v * down, wDown, bv[r]); });
-        return;
+      } else {
+        rest |= !numbers;
       }
+      store(acc);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[j][i] = bv[i];
+#pragma unroll
+      for (int i = 0; i < NR; i++) {
+        float c[KW + 3];
+        columns(i, c);
+#pragma unroll
+        for (int k = 0; k < KW; k++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][k], c[k + j], acc[j], 0, 0, 0);
+      }
+      store(acc);
     }
-    f32x16 acc[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-      for (int i = 0; i < 16; i++) acc[j][i] = bv[i];
-#pragma unroll
-    for (int i = 0; i < NR; i++) {
-      float c[KW + 3];
-      columns(i, c);
-#pragma unroll
-      for (int k = 0; k < KW; k++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][k], c[k + j], acc[j], 0, 0, 0);
-    }
-    store(acc, [](int, float v) { return v; });
   };
   Tile even, odd;
   int tile = (int)blockIdx.x * 4 + wave;
   if (tile < tiles) fetch(even, tile);
   for (; tile < tiles; tile += 2 * tileStep) {
     if (tile + tileStep < tiles) fetch(odd, tile + tileStep);
-    finish(even);
+    finish(even, std::false_type());
     if (tile + tileStep >= tiles) break;
     if (tile + 2 * tileStep < tiles) fetch(even, tile + 2 * tileStep);
-    finish(odd);
+    finish(odd, std::false_type());
+  }
+  if constexpr (SPLIT) {
+    if (!rest) return;
+    loadFilter(); // (here, where the operands of the fp32 instructions cost the loop above no registers)
+    for (tile = (int)blockIdx.x * 4 + wave; tile < tiles; tile += tileStep) {
+      fetch(even, tile);
+      finish(even, std::true_type());
+    }
   }
 }
 
@@ -1469,8 +1463,8 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     // two blocks per CU and channel tile
     const int64_t most = std::max<int64_t>(1, (int64_t)numComputeUnits() * 2 / ((OC + 31) / 32));
     const int64_t blocks = std::min((tiles128 + 3) / 4, most);
-    // Pairs of fp16 numbers from 12 taps on (of 9 they would be no more exact than the fp32 instructions, 6.5e-8 / 7.0e-8); an addend
-    // in flight leaves no registers for them.
+    // In pieces from 12 taps on (fewer leave half of the sixteen products of an instruction for nothing); an addend in flight leaves no
+    // registers for them.
     auto kernelOf = [&](auto split) {
       constexpr bool SPLIT = decltype(split)::value;
       return quadStores == Output::Streamed ? conv_quads_kernel<KWC, NR, Output::Streamed, false, SPLIT>

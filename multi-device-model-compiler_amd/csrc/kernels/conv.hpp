@@ -33,23 +33,17 @@ __device__ __forceinline__ i32x4 resourceWords(const float *p, int64_t elems) {
   return i32x4{(int)(uint32_t)at, (int)(uint32_t)(at >> 32) & 0xffff, resourceBytes(elems), kRawBuffer};
 }
 
-// a and b as fp16 numbers, hi, and what these leave, lo: pairs of 22 bits where lo is no smaller than fp16's normal numbers, 2^-25
-// off below.  (Four instructions; v_fma_mixlo / mixhi_f16 would be fewer where a scale comes besides, but writing half a register
-// takes them two to three times as long.)
-__device__ __forceinline__ void splitPair(float a, float b, uint32_t &hi, uint32_t &lo) {
-  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
-  float ra, rb;
-  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(ra) : "v"(a), "v"(hi));
-  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(rb) : "v"(b), "v"(hi));
-  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(lo) : "v"(ra), "v"(rb));
-}
+// Operands in pieces (conv_split.hip has the reasons): times the one scale each, their sums times the other.
+constexpr int kPieces = 3;
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
 
 // a and b as three bf16 numbers each, the first of which is the nearest, the second the nearest to what that leaves: all 24 bits (as long
-// as the last one is no subnormal: from 2^-110 on).
+// as the last one is no subnormal: from 2^-110 on).  (v_cvt_pk_bf16_f32 by the compiler, not by inline assembly: a matrix instruction
+// that reads its result needs two wait states behind it, which the compiler sees to only for instructions that it knows.)
 __device__ __forceinline__ void splitTriple(float a, float b, uint32_t (&piece)[3]) {
 #pragma unroll
   for (int i = 0; i < 3; i++) {
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(piece[i]) : "v"(a), "v"(b));
+    piece[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
     a -= __builtin_bit_cast(float, piece[i] << 16);
     b -= __builtin_bit_cast(float, piece[i] & 0xffff0000u);
   }

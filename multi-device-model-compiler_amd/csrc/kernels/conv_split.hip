@@ -50,8 +50,6 @@ namespace {
 constexpr int kConsumers = 4, kProducers = 8, kThreads = 64 * (kConsumers + kProducers);
 constexpr int kOC = 32;                      // output channels of a block
 constexpr int kPT = 2;                       // tiles of 32 pixels of a consumer
-constexpr int kPieces = 3;                   // of an operand
-constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f; // operands are taken times the one, sums times the other
 
 struct SplitGeo {
   int OH, OW, PHL, PWL, SH, SW, DH, DW;
@@ -204,7 +202,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
 #pragma unroll
         for (int k = 0; k < PAIRS; k++) {
           uint32_t piece[kPieces];
-          splitTriple(v[2 * k] * kScale, v[2 * k + 1] * kScale, piece);
+          splitTriple(v[2 * k] * kSplitScale, v[2 * k + 1] * kSplitScale, piece);
 #pragma unroll
           for (int i = 0; i < kPieces; i++) p[i][k] = piece[i];
         }
@@ -384,7 +382,7 @@ __global__ __launch_bounds__(kThreads) void conv_split_kernel(const float *__res
     for (int i = 0; i < 16; i++) finite = finite && fabsf(acc[t][i]) < __builtin_inff();
   if (!finite) bad = 1;
 #pragma unroll
-  for (int t = 0; t < kPT; t++) acc[t] *= kUnscale;
+  for (int t = 0; t < kPT; t++) acc[t] *= kSplitUnscale;
   __syncthreads();
   if (bad) {
     f32x16 plain[kPT];

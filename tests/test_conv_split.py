@@ -175,7 +175,7 @@ def test_an_image_for_itself(pkg, gpu, tile):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("kind", KINDS + UNEVEN)
 @pytest.mark.parametrize("IC", [2, 3])
 def test_operands_of_every_size_in_a_stem(pkg, gpu, kind, IC):
     """The kernel of few taps and four pixels a lane, on the same terms (512 tiles of 128 pixels x 32 channels)."""
@@ -194,3 +194,14 @@ def test_a_stem_of_nothing_beside_large_values(pkg, gpu):
     x[:, :, 8:16, 8:16], w[77] = 0, 0
     got = pkg.conv2d(x, w, b, pad=(1, 1, 1, 1))
     assert torch.equal(got[:, 77], b[77].expand(2, 64, 64)) and torch.equal(got[:, :, 9:15, 9:15], b[:, None, None].expand(2, 250, 6, 6))
+
+
+@pytest.mark.gpu
+def test_an_image_of_a_stem_for_itself(pkg, gpu):
+    import torch
+    x, w = operands("normal", 3, 3, 61, 60, 250, gpu)  # 128 pixels of a tile lie in two images
+    b = torch.randn(250, device=gpu)
+    alone = pkg.conv2d(x, w, b, pad=(1, 1, 1, 1))[1]
+    for value in (1e-8, 1e8, float("inf")):
+        x[0], x[2] = value, value
+        assert torch.equal(pkg.conv2d(x, w, b, pad=(1, 1, 1, 1))[1], alone), value
