@@ -32,7 +32,7 @@ constexpr int kSplit = 8; // wavefronts of a block
 enum class Result { Half, Planes, F32 };
 template <typename T, int ACT, int MB, int NB, int RING, bool KMAJOR, Result RESULT = Result::Half>
 __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
-                                                                 const uint16_t *__restrict__ bias, const uint16_t *residual, uint16_t *out,
+                                                                 const uint16_t *__restrict__ bias, ResidualOrShare<RESULT == Result::Planes> residual, uint16_t *out,
                                                                  int M, int N, int K, int tilesM, int nblk) {
   using Mm = Mma<T>;
   using v8 = typename Mm::v8;
@@ -56,10 +56,9 @@ __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint1
   const int l32 = lane % 32, hl = lane / 32;
 
   int chunks = (K + 31) / 32, firstChunk = 0;
-  if (RESULT == Result::Planes) {
-    const uint32_t perPart = partialShare(residual);
-    firstChunk = (int)__umulhi((uint32_t)(chunks * (int)blockIdx.y), perPart);
-    chunks = (int)__umulhi((uint32_t)(chunks * ((int)blockIdx.y + 1)), perPart) - firstChunk;
+  if constexpr (RESULT == Result::Planes) {
+    firstChunk = divide(chunks * (int)blockIdx.y, residual);
+    chunks = divide(chunks * ((int)blockIdx.y + 1), residual) - firstChunk;
   }
   const int c0 = firstChunk + chunks * ks / KS, c1 = firstChunk + chunks * (ks + 1) / KS;
 
@@ -244,10 +243,12 @@ __global__ __launch_bounds__(64 * kSplit, 1) void gemm_ksplit_kernel(const uint1
       if (ACT == ACT_RELU) x[i] = x[i] > 0.0f ? x[i] : 0.0f;
       if (ACT == ACT_GELU) x[i] = Mm::gelu(x[i]);
     }
-    if (residual) {
-      const v4 r = *reinterpret_cast<const v4 *>(residual + (size_t)m * N + n);
+    if constexpr (RESULT != Result::Planes) {
+      if (residual) {
+        const v4 r = *reinterpret_cast<const v4 *>(residual + (size_t)m * N + n);
 #pragma unroll
-      for (int i = 0; i < 4; i++) x[i] += Mm::widen(r[i]);
+        for (int i = 0; i < 4; i++) x[i] += Mm::widen(r[i]);
+      }
     }
     v4 o;
 #pragma unroll
@@ -335,7 +336,7 @@ void gemmKSplitPartialF16(const void *in, const void *weight, float *planes, int
   const auto *a = static_cast<const uint16_t *>(in);
   const auto *w = static_cast<const uint16_t *>(weight);
   auto *o = reinterpret_cast<uint16_t *>(planes);
-  const uint16_t *share = partialShareArgument(parts);
+  const PartShare share = partShare(parts);
   const int bm = tile == KSplitTile::T64x64 ? 64 : 32, bn = tile == KSplitTile::T32x32 ? 32 : 64;
   const int tilesM = (int)((M + bm - 1) / bm), nblk = tilesM * (int)((N + bn - 1) / bn);
   const dim3 grid((unsigned)nblk, (unsigned)parts), block(64 * kSplit);

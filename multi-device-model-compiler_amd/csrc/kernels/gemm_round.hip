@@ -39,7 +39,7 @@ constexpr int kPartial = 4;  // the blocks of grid row y take the y-th share of 
 constexpr int kResidualF32 = 5; // + residual, the rounded result widened to fp32 (the bits of a cast behind the kernel)
 template <typename T, int ACT, int NB, bool RAGGED>
 __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t *__restrict__ in, const uint16_t *__restrict__ weight,
-                                                                 const uint16_t *__restrict__ bias, const uint16_t *residual, uint16_t *out,
+                                                                 const uint16_t *__restrict__ bias, ResidualOrShare<ACT == kPartial> residual, uint16_t *out,
                                                                  int N, int K, int tilesN, int tilesM, int M_) {
   using M = Mma<T>;
   using v8 = typename M::v8;
@@ -76,10 +76,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
   const char *ag = reinterpret_cast<const char *>(in) + (size_t)m0 * K * 2;
   const char *wg = reinterpret_cast<const char *>(weight) + (size_t)n0 * 2;
   int steps = RAGGED ? (K + 63) / 64 : K / 64;
-  if (ACT == kPartial) {
-    const uint32_t perPart = partialShare(residual);
-    const int first = (int)__umulhi((uint32_t)(steps * (int)blockIdx.y), perPart);
-    steps = (int)__umulhi((uint32_t)(steps * ((int)blockIdx.y + 1)), perPart) - first;
+  if constexpr (ACT == kPartial) {
+    const int first = divide(steps * (int)blockIdx.y, residual);
+    steps = divide(steps * ((int)blockIdx.y + 1), residual) - first;
     ag += (size_t)first * 128;
     wg += (size_t)first * 128 * N;
   }
@@ -270,7 +269,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_round_kernel(const uint16_t 
   auto chunkCol = [&](int it) { return (it * 128 + khalf * 64 + lane) % kChunks; };
   auto chunkOffset = [&](int it) { return nw + 8 * chunkCol(it) < N ? (uint32_t)(chunkRow(it) * N * 2 + chunkCol(it) * 16) : 0x40000000u; };
   u32x4 rraw[kMine];
-  if (RESIDUAL) { // on its way under the last matrix instructions
+  if constexpr (RESIDUAL) { // on its way under the last matrix instructions
     const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(residual + partAt), 0, partBytes, 0x00020000);
 #pragma unroll
     for (int it = 0; it < kMine; it++) rraw[it] = __builtin_amdgcn_raw_buffer_load_b128(rows, chunkOffset(it), 0, 0);
@@ -413,8 +412,8 @@ void gemmRoundPartialF16(const void *in, const void *weight, float *planes, int6
   const dim3 grid((unsigned)(tilesM * tilesN), (unsigned)parts), block(kThreads);
   const auto *a = static_cast<const uint16_t *>(in), *w = static_cast<const uint16_t *>(weight);
   auto *o = reinterpret_cast<uint16_t *>(planes);
-  if (width == 128) launchKernel(gemm_round_kernel<_Float16, kPartial, 4, false>, grid, block, stream, a, w, nullptr, partialShareArgument(parts), o, (int)N, (int)K, tilesN, tilesM, (int)M);
-  else launchKernel(gemm_round_kernel<_Float16, kPartial, 3, false>, grid, block, stream, a, w, nullptr, partialShareArgument(parts), o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  if (width == 128) launchKernel(gemm_round_kernel<_Float16, kPartial, 4, false>, grid, block, stream, a, w, nullptr, partShare(parts), o, (int)N, (int)K, tilesN, tilesM, (int)M);
+  else launchKernel(gemm_round_kernel<_Float16, kPartial, 3, false>, grid, block, stream, a, w, nullptr, partShare(parts), o, (int)N, (int)K, tilesN, tilesM, (int)M);
   MGPU_CHECK_LAUNCH("gemm_round_kernel");
 }
 

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace mgpu {
 
@@ -100,13 +101,14 @@ template <> struct ElemTraits<bf16_t> {
   }
 };
 
-// The number of planes of a product whose reduction is split over blocks (2 to 4), as ceil(2^32 / parts) in the place of the
+// The number of planes of a product whose reduction is split over blocks (2 to 4), as ceil(2^32 / parts), in the place of the
 // residual, which such a product has not: that argument is preloaded, where gridDim would be a load from the kernarg segment ahead of
 // everything else in the kernel, and 256 bytes more of it to write at every launch (BERT layer, two such products of seven kernels:
-// 77 tokens of 768 29.9 -> 29.5 us, 47 of 256 20.7 -> 20.4).  n / parts is __umulhi(n, partialShare), exactly so below 2^30.
-__device__ __forceinline__ uint32_t partialShare(const uint16_t *residual) { return (uint32_t)reinterpret_cast<uintptr_t>(residual); }
-inline const uint16_t *partialShareArgument(int parts) {
-  return reinterpret_cast<const uint16_t *>((uintptr_t)((((uint64_t)1 << 32) + (unsigned)parts - 1) / (unsigned)parts));
-}
+// 77 tokens of 768 29.9 -> 29.5 us, 47 of 256 20.7 -> 20.4).
+enum class PartShare : uint64_t {};
+template <bool PARTIAL> using ResidualOrShare = std::conditional_t<PARTIAL, PartShare, const uint16_t *>;
+inline PartShare partShare(int parts) { return PartShare((((uint64_t)1 << 32) + (unsigned)parts - 1) / (unsigned)parts); }
+// n / parts, exactly so below 2^30
+__device__ __forceinline__ int divide(int n, PartShare share) { return (int)__umulhi((uint32_t)n, (uint32_t)share); }
 
 } // namespace mgpu
