@@ -53,38 +53,49 @@ SHAPES = [  # N, IC, H, W, OC, pad (top, left, bottom, right), stride, dilation
 ]
 
 
+def small_conv(pkg, side, x, w, b, add, pad, stride, dilation, relu):
+    import torch
+    (N, IC, H, W), (OC, _, win, _) = x.shape, w.shape
+    OH, OW = ((s + pad[i] + pad[i + 2] - (win - 1) * dilation[i] - 1) // stride[i] + 1 for i, s in enumerate((H, W)))
+    pkg.ops()
+    launch = internal(pkg, "_ZN4mgpu9convSmallEiiPKfS1_S1_PfS1_lllllllllllllbP12ihipStream_t", ctypes.c_bool, ctypes.c_int, ctypes.c_int,
+                      *[ctypes.c_void_p] * 5, *[ctypes.c_int64] * 13, ctypes.c_bool, ctypes.c_void_p)
+    count = N * OC * OH * OW
+    out = torch.full((count + 64,), 7.0, device=x.device)  # 32 elements before and behind
+    assert launch(win, side, x.data_ptr(), w.data_ptr(), b.data_ptr(), out[32:].data_ptr(), add.data_ptr() if add is not None else None, N, IC, H, W, OC,
+                  OH, OW, pad[0], pad[1], *stride, *dilation, relu, torch.cuda.current_stream().cuda_stream)
+    assert torch.all(out[:32] == 7) and torch.all(out[32 + count:] == 7)
+    return out[32:32 + count].view(N, OC, OH, OW)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("win,side", [(3, 16), (3, 32), (5, 16), (5, 32), (7, 16)])
 def test_edges(pkg, gpu, oracle, shape, win, side):
-    import torch
     N, IC, H, W, OC, pad, stride, dilation = shape
     OH, OW = ((s + pad[i] + pad[i + 2] - (win - 1) * dilation[i] - 1) // stride[i] + 1 for i, s in enumerate((H, W)))
     if OH < 1 or OW < 1: pytest.skip("no such window in it")
     rng = np.random.Generator(np.random.PCG64(IC + win))
     x, w = rng.standard_normal((N, IC, H, W)).astype(np.float32), (rng.standard_normal((OC, IC, win, win)) * (IC * win * win) ** -0.5).astype(np.float32)
     b, a = rng.standard_normal(OC).astype(np.float32), rng.standard_normal((N, OC, OH, OW)).astype(np.float32)
-    pkg.ops()
-    launch = internal(pkg, "_ZN4mgpu9convSmallEiiPKfS1_S1_PfS1_lllllllllllllbP12ihipStream_t", ctypes.c_bool, ctypes.c_int, ctypes.c_int,
-                      *[ctypes.c_void_p] * 5, *[ctypes.c_int64] * 13, ctypes.c_bool, ctypes.c_void_p)
     tx, tw, tb, ta = (to_dev(t, gpu) for t in (x, w, b, a))
-    count = N * OC * OH * OW
     for add, relu in ((None, False), (a, True)):
-        out = torch.full((count + 64,), 7.0, device=gpu)  # 32 elements before and behind
-        assert launch(win, side, tx.data_ptr(), tw.data_ptr(), tb.data_ptr(), out[32:].data_ptr(), ta.data_ptr() if add is not None else None, N, IC, H, W, OC,
-                      OH, OW, pad[0], pad[1], *stride, *dilation, relu, torch.cuda.current_stream().cuda_stream)
-        assert torch.all(out[:32] == 7) and torch.all(out[32 + count:] == 7)
-        got = out[32:32 + count].view(N, OC, OH, OW).cpu().numpy()
+        got = small_conv(pkg, side, tx, tw, tb, ta if add is not None else None, pad, stride, dilation, relu).cpu().numpy()
         ref = oracle.conv2d(x, w, b, add, pad, stride, dilation, relu)
         # both sides are a sum of K products of fp32 accuracy: 2^-24 of the sum of their sizes (here about 1) times some sqrt(K)
         assert np.all(np.abs(got - ref) <= 1e-5 * (1 + np.abs(ref))), np.abs(got - ref).max()
 
 
 @pytest.mark.gpu
-def test_infinities_and_nan(pkg, gpu):
+@pytest.mark.parametrize("win,side", [(3, 16), (3, 32), (5, 16), (5, 32), (7, 16)])
+def test_infinities_and_nan(pkg, gpu, win, side):
     import torch
-    x, w, b = torch.zeros((1, 8, 6, 6), device=gpu), torch.ones((16, 8, 3, 3), device=gpu), torch.zeros(16, device=gpu)
-    x[0, 3, 1, 1], x[0, 7, 5, 5], w[5, 0, 0, 0] = float("inf"), float("nan"), float("inf")
-    got, ref = pkg.conv2d(x, w, b, pad=(1, 1, 1, 1)), torch.nn.functional.conv2d(x.double().cpu(), w.double().cpu(), padding=1).float().to(gpu)
+    gen = torch.Generator(device=gpu).manual_seed(win)
+    x, w = (torch.randint(1, 4, s, device=gpu, generator=gen).float() for s in ((2, 36, 9, 11), (33, 36, win, win)))  # (sums are whole numbers below 2^24)
+    x[0, 3, 1, 1], x[0, 35, 8, 10], x[1, 17, 4, 4], w[5, 0, 0, 0], w[32, 30, win - 1, win - 1] = (float(v) for v in ("inf", "nan", "-inf", "inf", "-inf"))
+    p = win // 2
+    got = small_conv(pkg, side, x, w, torch.zeros(33, device=gpu), None, (p, p, p, p), (1, 1), (1, 1), False)
+    ref = torch.nn.functional.conv2d(x.double().cpu(), w.double().cpu(), padding=p).float().to(gpu)
     # (outside the image a tap is 0, which an infinite filter value makes a NaN in either)
     assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[~ref.isnan()], ref[~ref.isnan()])
+    assert ref.isnan().any() and ref.isinf().any() and ref.isfinite().any()
