@@ -713,8 +713,9 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
 // SPLIT: the products by the bf16 matrix instructions, operands taken apart into three numbers as in conv_split.hip: twelve steps of
 // 32 clocks instead of 15 of 64, and fewer roundings (K = 27: error against 64 bits 1.1e-7 -> 0.39e-7).  A tile with values so large that
 // they or their sums might be none in pieces is done again behind the others, and what is no number takes the fp32 instructions'
-// result.  us, fp32 instructions / this: 16 x 3 x 256 x 256 -> 64 54.9 / 54.2, 16 x 3 x 224 x 224 -> 64 47.9 / 40.6, 4 x 3 x 224 x 224 -> 64 16.2 / 13.9, 16
-// x 3 x 76 x 248 -> 33 19.0 / 15.1, 8 x 1 x 112 x 112 -> 64, 5 x 5, 10.7 / 8.8; of two channels 16.7 / 16.8 (16 x 2 x 128 x 128 -> 64).
+// result.  us, fp32 instructions / this, outputs in turn: 16 x 3 x 256 x 256 -> 64 56.2 / 55.0, 16 x 3 x 224 x 224 -> 64 56.1 / 48.4, 4 x 3 x 224 x 224 -> 64 16.0 /
+// 12.9, 16 x 3 x 76 x 248 -> 33 18.8 / 13.3, 8 x 1 x 112 x 112 -> 64, 5 x 5, 10.6 / 8.4; of two channels 16.9 / 16.4 (16 x 2 x 128 x 128 -> 64).  Each of the four
+// pixels' taps taken apart for itself: 56.7, 50.6, 13.5, 14.7, 8.6, 16.3.
 template <int KW, int NR, Output OUT, bool ADDED, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                             const float *__restrict__ bias, float *__restrict__ y, ConvGeo g, int OC,
@@ -752,15 +753,19 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
     const int oc = oc0 + 8 * (r / 4) + r % 4 + 4 * hl;
     bv[r] = bias[oc < OC ? oc : OC - 1];
   }
-  // SPLIT: the lane half's taps as eight each of STEPS matrix instructions, in the order of its rows, in pieces.
-  constexpr int TAPS = NR * KW, STEPS = (TAPS + 7) / 8;
+  // SPLIT: the lane half's taps as eight each of STEPS matrix instructions, in pieces: of every row the pairs of neighbours, then the last
+  // ones of two rows at a time.
+  constexpr int TAPS = NR * KW, STEPS = (TAPS + 7) / 8, PAIRS = KW / 2;
   u32x4 ap[kPieces][STEPS];
   float most = 0.0f; // pixels below this are finite in pieces, and so are their sums (uniform)
-  auto inPieces = [&](u32x4 (&piece)[kPieces][STEPS], auto &&tap) { // tap: of the lane half's, by number
+  auto inOrder = [&](u32x4 (&piece)[kPieces][STEPS], auto &&pair, auto &&lasts) { // pair(row, first column), lasts(row, the next one or -1)
 #pragma unroll
     for (int i = 0; i < 4 * STEPS; i++) {
-      uint32_t p[kPieces];
-      splitTriple(2 * i < TAPS ? tap(2 * i) * kSplitScale : 0.0f, 2 * i + 1 < TAPS ? tap(2 * i + 1) * kSplitScale : 0.0f, p);
+      constexpr int OF_ROWS = NR * PAIRS;
+      const int r = 2 * (i - OF_ROWS);
+      uint32_t p[kPieces] = {0u, 0u, 0u};
+      if (i < OF_ROWS) pair(p, i / PAIRS, i % PAIRS * 2);
+      else if (r < NR) lasts(p, r, r + 1 < NR ? r + 1 : -1);
 #pragma unroll
       for (int k = 0; k < kPieces; k++) piece[k][i / 4][i % 4] = p[k];
     }
@@ -771,7 +776,10 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
     for (int i = 0; i < TAPS; i++) m = fmaxf(m, fabsf(a[i / KW][i % KW]));
     m = group_max<64>(m);
     if (m < 0x1p100f) most = fminf(0x1p100f, 0x1p74f / fmaxf(m, 0x1p-26f)); // (32 products of less than 2^74 and two scales of 2^24)
-    inPieces(ap, [&](int k) { return a[k / KW][k % KW]; });
+    inOrder(ap, [&](uint32_t (&p)[kPieces], int row, int k) { splitTriple(a[row][k] * kSplitScale, a[row][k + 1] * kSplitScale, p); },
+            [&](uint32_t (&p)[kPieces], int row, int next) {
+              splitTriple(a[row][KW - 1] * kSplitScale, next < 0 ? 0.0f : a[next < 0 ? 0 : next][KW - 1] * kSplitScale, p);
+            });
   }
   struct Tile {
     int pix, img, nFirst; // the lane's first pixel (-1: past the end), its image less the tile's first, that image
@@ -857,17 +865,35 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
     };
     f32x16 acc[4];
     if constexpr (SPLIT) {
+      // Two columns at a time are taken apart, once for the four pixels; what starts at an odd one is put together from halves.
       float c[NR][KW + 3], m = 0.0f;
+      uint32_t two[NR][(KW + 3) / 2][kPieces];
 #pragma unroll
       for (int i = 0; i < NR; i++) {
         columns(i, c[i]);
 #pragma unroll
         for (int e = 0; e < KW + 3; e++) m = fmaxf(m, fabsf(c[i][e]));
+#pragma unroll
+        for (int e = 0; e < KW + 3; e += 2) splitTriple(c[i][e] * kSplitScale, c[i][e + 1] * kSplitScale, two[i][e / 2]);
       }
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         u32x4 bp[kPieces][STEPS];
-        inPieces(bp, [&](int k) { return c[k / KW][k % KW + j]; });
+        inOrder(bp,
+                [&](uint32_t (&p)[kPieces], int row, int k) {
+#pragma unroll
+                  for (int n = 0; n < kPieces; n++) {
+                    const int e = k + j;
+                    p[n] = e % 2 ? __builtin_amdgcn_alignbit(two[row][e / 2 + 1][n], two[row][e / 2][n], 16) : two[row][e / 2][n];
+                  }
+                },
+                [&](uint32_t (&p)[kPieces], int row, int next) {
+#pragma unroll
+                  for (int n = 0; n < kPieces; n++) {
+                    const int e = KW - 1 + j;
+                    p[n] = __builtin_amdgcn_perm(next < 0 ? 0u : two[next < 0 ? 0 : next][e / 2][n], two[row][e / 2][n], e % 2 ? 0x07060302u : 0x05040100u);
+                  }
+                });
         f32x16 sum;
 #pragma unroll
         for (int i = 0; i < 16; i++) sum[i] = 0.0f;
@@ -881,6 +907,7 @@ __global__ __launch_bounds__(256, 2) void conv_quads_kernel(const float *__restr
               sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ap[k][i]), __builtin_bit_cast(bf16x8, bp[order - k][i]), sum, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[j][i] = fmaf(sum[i], kSplitUnscale, bv[i]);
+        __builtin_amdgcn_sched_barrier(0); // (one pixel after the other: 5 x 5 would spill)
       }
       const bool numbers = __builtin_amdgcn_ballot_w64(!(m < most)) == 0; // (a NaN is one in either way)
       if constexpr (AGAIN) {
