@@ -6,7 +6,7 @@
 //   conv:  y = act(conv(x, w) + bias[oc] + postAdd),  act = ReLU or identity
 //   pool:  max (padding ignored) or average that counts the padding
 //          (CUDNN_POOLING_AVERAGE_COUNT_INCLUDE_PADDING, Ops.cu:347-349)
-// The convolution is an implicit GEMM on the fp32 matrix cores
+// The convolution is an implicit GEMM, mostly on the fp32 matrix cores
 // (v_mfma_f32_32x32x2_f32: true fp32 products, fp32 accumulation):
 //   y[n][oc, p] = sum_k w[oc, k] * taps[k, p],  k = (ic, kh, kw), p = (oh, ow)
 // in 32 x 32 tiles, channels in the rows and pixels - counted over the whole batch - in the
@@ -14,7 +14,8 @@
 // 128-byte runs of the NCHW output.  The tap matrix is never written to memory.  Taps come
 // through buffer loads, whose bounds check answers 0 for an offset outside the image: padding costs
 // no branch and no second instruction.  Seven kernels share the work here (conv2d below has the rule and
-// the measurements behind it), and an eighth, conv_split.hip, has the large 3 x 3 ones:
+// the measurements behind it), with two more: conv_small.hip takes 3 x 3, 5 x 5 and 7 x 7 of few tiles, in tiles of 16 pixels, and
+// conv_split.hip the large ones, on the bf16 matrix cores in three numbers an operand, as the quads of 12 taps on are here:
 //   few taps  (K <= 32, a network's stem)  filter in registers, wavefronts walk over pixel tiles
 //   quads     (the same, many tiles, rows of whole quads, stride 1 across)  four pixels a lane
 //   patch     (5 or 7 square from one channel or three)  input rows through LDS, once for all taps
@@ -25,7 +26,7 @@
 //   table     (every other window, and images beyond 2 GiB)  tap offsets from a table in LDS
 // What bounds them: one 32x32x2 MFMA takes 64 cycles of a SIMD (157 TFLOP/s on the chip) and the
 // vector instructions of the same wavefront do not overlap with it, so the loops are built to have
-// none; the stem is bound by its output (268 MB at 16 x 3 x 256 x 256 -> 64: 65 us, a plain fill
+// none; the stem is bound by its output (268 MB at 16 x 3 x 256 x 256 -> 64: 55 us, a plain fill
 // of as many bytes takes 39).  Unlike the reference, asymmetric padding is honoured (it passes only
 // PHL / PWL to cuDNN).
 #include "common.hpp"

@@ -17,8 +17,8 @@
 // wavefronts (producers) bring operands into LDS, four (consumers) multiply, a step of sixteen input channels at a time,
 // double-buffered.  A step of 32 x 256 takes 2.35 us, of which the matrix cores are busy 0.54 and the LDS 0.53 (0.4 of that bank conflicts);
 // without conversions it would take 2.2, with half of the products 1.9.  (Eight producers, since a lone wavefront on a SIMD issues a vector
-// instruction every eight cycles only.  Operands of a step's first set asked for ahead of the last one's products: 83.5 -> 90 us on the 7 x 7
-// below.)
+// instruction every eight cycles only.  Operands of a step's first set asked for ahead of the last one's products took 95 us for 84 on the
+// first 7 x 7 below.)
 //  * Filter rows come as they are, 576 bytes of a channel and step by one load into LDS, a step ahead, of which a lane takes
 //    four channels of a position or more.  A producer converts the rows that it has loaded itself, so that they need neither a second buffer
 //    nor a barrier.  (Straight into registers a load touched seven rows: 15 cycles an instruction.)
