@@ -1623,6 +1623,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
       MGPU_CHECK_LAUNCH("mgpuConv2d");
       return;
     }
+    // (convWindowTime restates these lines for 3 x 3, and convFewTilesTime the first two: what changes here changes there.)
     auto pick = [&](auto win) {
       constexpr int WIN = decltype(win)::value;
       const int64_t units = ((IC + 2 * Window<WIN>::HALF - 1) / (2 * Window<WIN>::HALF)) * Window<WIN>::UNITS;
