@@ -712,7 +712,8 @@ __global__ __launch_bounds__(256, 2) void conv_few_taps_kernel(const float *__re
 // 224 -> 64 with a postAdd 87 -> 49; 8 x 3 x 128 x 128 -> 16 11.0 -> 6.7.  Stores of one tile dealt out between the matrix
 // instructions of the next measured the same, an order of tiles by XCD too, runs of tiles a wavefront 90.
 // SPLIT: the products by the bf16 matrix instructions, operands taken apart into three numbers as in conv_split.hip: twelve steps of
-// 32 clocks instead of 15 of 64, and fewer roundings (K = 27: error against 64 bits 1.1e-7 -> 0.39e-7).  A tile with values so large that
+// 32 clocks instead of 15 of 64, and fewer roundings (K = 27: error against 64 bits 1.1e-7 -> 0.39e-7; of a product without others, where the
+// fp32 instructions round once, 0.6e-7 -> 1.6e-7 at most).  A tile with values so large that
 // they or their sums might be none in pieces is done again behind the others, and what is no number takes the fp32 instructions'
 // result.  us, fp32 instructions / this, outputs in turn: 16 x 3 x 256 x 256 -> 64 56.2 / 55.0, 16 x 3 x 224 x 224 -> 64 56.1 / 48.4, 4 x 3 x 224 x 224 -> 64 16.0 /
 // 12.9, 16 x 3 x 76 x 248 -> 33 18.8 / 13.3, 8 x 1 x 112 x 112 -> 64, 5 x 5, 10.6 / 8.4; of two channels 16.9 / 16.4 (16 x 2 x 128 x 128 -> 64).  Each of the four

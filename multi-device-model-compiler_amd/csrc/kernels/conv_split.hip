@@ -2,12 +2,13 @@
 //
 // Every operand is taken apart into three bf16 numbers, each the nearest to what those before it leave: all 24 bits, at fp32's range
 // (the split of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
-// Computations", 2019).  Of the nine products of two such numbers six are summed up in fp32; the other three are at most 2^-23
-// of a product, whichever its size, 2^-26 in the root mean square, and of either sign.  The sums' errors, which are the larger ones, become fewer, since an instruction
-// adds sixteen products at a time where the fp32 one adds two.  Relative error against 64 bits (2-norm; N(0, 1) pixels): 0.56e-7 to 2.0e-7 for
-// 3 x 3, 0.54e-7 to 2.7e-7 for 5 x 5, 0.72e-7 to 3.2e-7 for 7 x 7, on average 0.82, 0.76 and 0.66 times that of the fp32 instructions on the same
-// shapes and never more.  (Two fp16 numbers and a scale for a block, three products, took 0.75 of the time, and lost what is small
-// beside the block's largest values: an input channel of 1e-6 of the others, weighted up again, was off by 2e-4.)
+// Computations", 2019).  Of the nine products of two such numbers six are summed up in fp32; the other three are at most 2^-23 of a
+// product, whichever its size, 2^-26 in the root mean square, and of either sign.  The sums' errors, which are the larger ones, become
+// fewer, since an instruction adds sixteen products at a time where the fp32 one adds two.  Relative error against 64 bits (2-norm;
+// N(0, 1) pixels): 0.56e-7 to 2.0e-7 for 3 x 3, 0.54e-7 to 2.7e-7 for 5 x 5, 0.72e-7 to 3.2e-7 for 7 x 7, on average 0.82, 0.76 and 0.66 times
+// that of the fp32 instructions on the same shapes and never more; of a product without others, which those round once, 0.94e-7 at
+// most to 0.6e-7.  (Two fp16 numbers and a scale for a block, three products, took 0.75 of the time, and lost what is small beside the
+// block's largest values: an input channel of 1e-6 of the others, weighted up again, was off by 2e-4.)
 //
 // Operands are multiplied by 2^24 first, so that the last piece of a number near fp32's smallest is no subnormal, and sums by 2^-48 at
 // the end.  What becomes of infinities, NaNs and products beyond 2^80 is no finite sum; a block with one does its tile again with the
