@@ -1592,7 +1592,7 @@ void conv2d(const float *input, const float *weight, const float *bias, float *o
     else go(integral_constant<int, 7>(), integral_constant<int, 11>());
   } else if (squareWindow) {
     // 3 x 3 from 32 channels on in three bf16 numbers, where both estimates say that this is faster (700 shapes: taken by 267, 0.91 of the
-    // time over all of them where the best choice everywhere would be 0.907, the largest ones 0.5 to 0.6, two 5 to 6 % slower).  (16 channels are one
+    // time over all of them where the best choice everywhere would be 0.907, 0.66 beyond 80 us, two 5 to 6 % slower).  (16 channels are one
     // step: no gain.)
     ConvSplitPlan split{0, 0, 0.0};
     if (KH == 3 && IC >= 32 && IC % 16 == 0) {
